@@ -1189,10 +1189,40 @@ static inline bool gmm_large_tiles(const GmmParams& p, int mode) {
   return tiles >= (mode == MODE_TN ? 129 : 256);
 }
 
+constexpr int64_t kRemainderMinRows = 2048;  // see gmm_use_remainder
+
+// Row-adaptive tiles (gmm_rows.hip) for 16-bit NN / NT: tiles of 64 to 256 rows x 256 columns that
+// share an expert's rows evenly, one workgroup per CU.  Measured against the 128x128 and 256x256 tiles
+// in the same process, n = rows per expert, times of both sides in us (K x M, experts):
+//   * n below 96 (NT: 128): an expert is one 128-row tile either way and its weights bound the launch;
+//     the 128x128 kernel with two workgroups per CU streams them a little faster
+//     (n 64: 375 against 399 for 4096 x 28672, 8 experts).
+//   * up to 512 rows the 128x128 kernel multiplies padding and moves twice the operands per product:
+//     n 384: 996 -> 731 (4096 x 28672, 8), 436 -> 338 (2048 x 2816, 64), NT 974 -> 765 (7168 x 4096, 32);
+//     n 160: 654 -> 380 (7168 x 4096, 32).
+//   * from 512 rows on the 256x256 tiles are the alternative.  NN gains 1-10 % as long as the
+//     reduction is long enough to carry its prologue (n 1024: 1730 -> 1681, K 7168; but 223 -> 238 at
+//     K 1024); NT loses 4-10 % (its 64-byte pieces of two operands against 128-byte ones there:
+//     1632 -> 1727, K 4096), so it stays.  From 2048 rows on the remainder launches take over.
+//   * with less than three quarters of a round of tiles, or a last round that leaves more than 30 % of
+//     all rounds idle, the smaller tiles spread better (K 2816, M 1024, 16 experts, 64 tiles: 27 -> 43).
+//   * the activation backward (NT) around 256 rows: half the experts take a second chunk of two units,
+//     whose epilogue does not overlap anything (361 -> 408 at K 7168); 128x128 tiles there.
+static inline bool gmm_rows_pays(const GmmParams& p, int mode, int epi) {
+  const int64_t n = p.N / (p.E > 0 ? p.E : 1);
+  const bool glu = epi == EPI_GLU_FWD_SILU || epi == EPI_GLU_FWD_GELU;
+  const int64_t cols = glu ? (p.F + 127) / 128 : (p.M + 255) / 256;
+  const int64_t tiles = p.E * ((n + 16 + 255) / 256) * cols;
+  const int64_t cus = gmm_grid(1), rounds = (tiles + cus - 1) / cus;
+  if (p.K < 1024 || tiles * 4 < cus * 3 || tiles * 10 < rounds * cus * 7) return false;
+  if (mode == MODE_NN) return n >= 96 && n < kRemainderMinRows && (n < 512 || p.K >= 1536);
+  if (epi != EPI_NONE && n >= 240 && n < 288) return false;
+  return n >= 128 && n < 512;
+}
+
 // The separate launch for short last row tiles pays off once an expert has many full row tiles:
 // at 4096 rows per expert (Mixtral shape) it saves 4-7 % of a GEMM, at 1024 rows per expert (64 or 32
 // experts) the main kernel with its partial tiles is 5-10 % faster than the two launches.
-constexpr int64_t kRemainderMinRows = 2048;
 static inline bool gmm_use_remainder(const GmmParams& p) {
   return p.N / (p.E > 0 ? p.E : 1) >= kRemainderMinRows;
 }
@@ -1239,6 +1269,9 @@ template <int DT, int ODT, int MODE, int EPI>
 static int launch_gmm_mode(const GmmParams& p, int dtype, int out_dtype, hipStream_t st) {
   constexpr bool half = Elem<DT>::bytes == 2;
   constexpr bool glu_fwd = EPI == EPI_GLU_FWD_SILU || EPI == EPI_GLU_FWD_GELU;
+  if constexpr (half && MODE != MODE_TN) {
+    if (gmm_rows_pays(p, MODE, EPI)) return launch_gmm_rows(p, MODE, dtype, out_dtype, EPI, st);
+  }
   if (gmm_large_tiles(p, MODE)) {
     if constexpr (MODE == MODE_TN && half) {
       (void)dtype;
@@ -1434,7 +1467,8 @@ extern "C" int gmoe_gmm_glu(const void* a, const void* w1, void* fc1, void* act_
   hipStream_t st = static_cast<hipStream_t>(stream);
   p.c2 = static_cast<unsigned char*>(act_out);
   p.F = F;
-  if (dtype != GMOE_F32 && gmm_large_tiles(p, MODE_NN) && F % 8 == 0)
+  if (dtype != GMOE_F32 && F % 8 == 0 &&
+      (gmm_large_tiles(p, MODE_NN) || gmm_rows_pays(p, MODE_NN, EPI_GLU_FWD_SILU)))
     return gmm_dispatch(p, MODE_NN, dtype, dtype, act == GMOE_ACT_SILU ? EPI_GLU_FWD_SILU : EPI_GLU_FWD_GELU, st);
   // small groups / fp32: the GEMM followed by the activation kernel
   const int rc2 = gmm_dispatch(p, MODE_NN, dtype, dtype, EPI_NONE, st);

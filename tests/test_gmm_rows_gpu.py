@@ -1,0 +1,44 @@
+"""The row-adaptive NN / NT tiles at the edges of their chunks: experts of 0 rows, of 1, of one row
+more or less than a unit (64), a tile (256) and two tiles, reductions that end inside a stage, columns
+that end inside a tile; plain, fp32 output, and with the activation and its backward fused."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+ROWS = [0, 1, 63, 64, 65, 127, 128, 129, 191, 193, 255, 256, 257, 320, 511, 513]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("K,F", [(1024, 1024), (1160, 904), (1544, 1096)])
+def test_chunk_edges(pkg, dev, dtype, K, F):
+    E, N, M = len(ROWS), sum(ROWS), 2 * F
+    g = torch.Generator(device=dev).manual_seed(K + F)
+    print("case", dtype, K, F, flush=True)
+    off = torch.tensor([0] + ROWS, device=dev).cumsum(0)
+
+    def rnd(*s, std=1.0):
+        return torch.empty(*s, device=dev).normal_(0.0, std, generator=g).to(dtype)
+
+    a, w1 = rnd(N, K), rnd(E, K, M, std=K ** -0.5)
+    wt = rnd(E, F, K, std=K ** -0.5)
+    fc1, act = pkg.ops.gmm_glu(a, w1, off)
+    plain = pkg.ops.gmm(a, w1, off)
+    plain32 = pkg.ops.gmm(a, w1, off, out_dtype=torch.float32)
+    d = pkg.ops.gmm(a, wt, off, trans_b=True)
+    d32 = pkg.ops.gmm(a, wt, off, trans_b=True, out_dtype=torch.float32)
+    dfc1 = pkg.ops.gmm_glu_bwd(a, wt, fc1, off)
+    assert torch.equal(fc1, plain) and torch.equal(act, pkg.ops.glu_fwd(fc1))
+    assert torch.equal(dfc1, pkg.ops.glu_bwd(d, fc1))
+    assert torch.equal(plain, plain32.to(dtype)) and torch.equal(d, d32.to(dtype))
+    # products of 16-bit values are exact in fp32; both sides round up to K additions of partial sums
+    # of size about one (rows of a have norm sqrt(K), columns of w norm one): 2^-24 * sqrt(K) per
+    # element typically, eight times that as the bound
+    tol = 8 * 2.0 ** -24 * K ** 0.5 * 4
+    s = 0
+    for e, n in enumerate(ROWS):
+        x = a[s:s + n].double()
+        for got, want in ((plain32, x @ w1[e].double()), (d32, x @ wt[e].double().t().contiguous())):
+            err = (got[s:s + n].double() - want).abs().max().item() if n else 0.0
+            assert err < tol, (e, n, err)
+        s += n
