@@ -15,7 +15,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB_DIR = os.path.join(HERE, "_lib")
 LIB_PATH = os.path.join(LIB_DIR, "libgalvatron_moe.so")
-SOURCES = ["route.hip", "losses.hip", "capacity.hip", "permute.hip", "glu.hip", "bias.hip", "gmm.hip", "gmm_dtl.hip", "gmm_rows.hip", "gmm_fp8s.hip", "quant.hip", "norm.hip", "gate.hip", "abi.hip"]
+SOURCES = ["route.hip", "losses.hip", "capacity.hip", "permute.hip", "glu.hip", "bias.hip", "gmm.hip", "gmm_dtl.hip", "gmm_rows.hip", "gmm_tn.hip", "gmm_fp8s.hip", "quant.hip", "norm.hip", "gate.hip", "abi.hip"]
 
 # packed-fp32 instructions are switched off for every device compilation of this library
 HIPCC_FLAGS = [
@@ -31,7 +31,7 @@ HIPCC_FLAGS = [
 # loop headers of the GEMM kernels on 64-byte boundaries: the Mixtral-shape step 0.4 % faster in the
 # same runs (the dW launches 0.9 %), the other shapes unchanged
 SOURCE_FLAGS = {"gmm.hip": ["-falign-loops=64"], "gmm_dtl.hip": ["-falign-loops=64"],
-                "gmm_rows.hip": ["-falign-loops=64"]}
+                "gmm_rows.hip": ["-falign-loops=64"], "gmm_tn.hip": ["-falign-loops=64"]}
 
 
 def _hipcc() -> str:

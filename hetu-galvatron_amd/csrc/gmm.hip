@@ -1220,6 +1220,21 @@ static inline bool gmm_rows_pays(const GmmParams& p, int mode, int epi) {
   return n >= 128 && n < 512;
 }
 
+// dW of 16-bit operands with a short reduction (gmm_tn.hip: 128x256 tiles, two workgroups per CU) against
+// the 256x256 LDS-DMA kernel, or 128x128 tiles where that one does not apply; n = rows per expert, us on
+// both sides: n 48: 302 -> 192 (14336 x 4096, 8 experts), 587 -> 381 (7168 x 4096, 32); n 384: 1098 -> 995
+// (4096 x 28672, 8), 107 -> 77 (1024 x 5632, 16); n 768: 342 -> 305 (1408 x 2048, 64), but 1573 -> 1591
+// (4096 x 28672); n 1024: 1884 -> 1935 (7168 x 4096): the operand traffic of the smaller tile takes over.
+// (Small outputs gain beyond that, n 1024: 417 -> 380 for 1408 x 2048, but with shared experts on a
+// second stream that step lost 0.6 %.)  With fewer than three quarters of a tile per CU the 128x128
+// tiles spread better (128 tiles of 1024 x 512: 13 -> 15).
+static inline bool gmm_tn_short_pays(const GmmParams& p) {
+  const int64_t n = p.N / (p.E > 0 ? p.E : 1);
+  const int64_t tiles = p.E * ((p.K + 127) / 128) * ((p.M + 255) / 256);
+  if (p.K < 128 || p.M < 256 || tiles * 4 < gmm_grid(1) * 3) return false;
+  return n <= 768;
+}
+
 // The separate launch for short last row tiles pays off once an expert has many full row tiles:
 // at 4096 rows per expert (Mixtral shape) it saves 4-7 % of a GEMM, at 1024 rows per expert (64 or 32
 // experts) the main kernel with its partial tiles is 5-10 % faster than the two launches.
@@ -1269,6 +1284,9 @@ template <int DT, int ODT, int MODE, int EPI>
 static int launch_gmm_mode(const GmmParams& p, int dtype, int out_dtype, hipStream_t st) {
   constexpr bool half = Elem<DT>::bytes == 2;
   constexpr bool glu_fwd = EPI == EPI_GLU_FWD_SILU || EPI == EPI_GLU_FWD_GELU;
+  if constexpr (half && MODE == MODE_TN) {
+    if (gmm_tn_short_pays(p)) return launch_gmm_tn_short(p, dtype, out_dtype, st);
+  }
   if constexpr (half && MODE != MODE_TN) {
     if (gmm_rows_pays(p, MODE, EPI)) return launch_gmm_rows(p, MODE, dtype, out_dtype, EPI, st);
   }

@@ -239,6 +239,9 @@ struct Fp8Scale {
 // Launches the LDS-DMA variant (gmm_dtl.hip) of the dW product (TN) for 16-bit operands.
 int launch_gmm_dtl_tn(const GmmParams& p, int dtype, int out_dtype, hipStream_t st);
 
+// Launches the dW kernel for short reductions (gmm_tn.hip) for 16-bit operands.
+int launch_gmm_tn_short(const GmmParams& p, int dtype, int out_dtype, hipStream_t st);
+
 // Launches the row-adaptive kernel (gmm_rows.hip) for 16-bit operands.
 int launch_gmm_rows(const GmmParams& p, int mode, int dtype, int out_dtype, int epi, hipStream_t st);
 

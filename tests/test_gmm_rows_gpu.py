@@ -1,4 +1,4 @@
-"""The row-adaptive NN / NT tiles at the edges of their chunks: experts of 0 rows, of 1, of one row
+"""The row-adaptive NN / NT tiles and the short-reduction TN tiles at the edges of their chunks: experts of 0 rows, of 1, of one row
 more or less than a unit (64), a tile (256) and two tiles, reductions that end inside a stage, columns
 that end inside a tile; plain, fp32 output, and with the activation and its backward fused."""
 import pytest
@@ -41,4 +41,26 @@ def test_chunk_edges(pkg, dev, dtype, K, F):
         for got, want in ((plain32, x @ w1[e].double()), (d32, x @ wt[e].double().t().contiguous())):
             err = (got[s:s + n].double() - want).abs().max().item() if n else 0.0
             assert err < tol, (e, n, err)
+        s += n
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("K,M", [(1024, 512), (1160, 904), (136, 4104)])
+def test_short_reduction_edges(pkg, dev, dtype, K, M):
+    """dW over 0, 1, a stage (32) more or less one, ... rows; output edges inside a tile."""
+    rows = [0, 1, 31, 32, 33, 63, 64, 65, 95, 97, 128, 129, 7, 0, 300, 2]
+    E, N = len(rows), sum(rows)
+    g = torch.Generator(device=dev).manual_seed(K + M)
+    print("case", dtype, K, M, flush=True)
+    off = torch.tensor([0] + rows, device=dev).cumsum(0)
+    a = torch.empty(N, K, device=dev).normal_(generator=g).to(dtype)
+    b = torch.empty(N, M, device=dev).normal_(generator=g).to(dtype)
+    got32 = pkg.ops.gmm(a, b, off, trans_a=True, out_dtype=torch.float32)
+    got = pkg.ops.gmm(a, b, off, trans_a=True)
+    assert torch.equal(got, got32.to(dtype))
+    s = 0
+    for e, n in enumerate(rows):
+        want = a[s:s + n].double().t().contiguous() @ b[s:s + n].double()
+        # exact products of values up to about 5 x 5, n fp32 additions: 2^-24 * 25 * n bounds each sum
+        assert (got32[e].double() - want).abs().max().item() <= 2.0 ** -24 * 25 * n * 4
         s += n
