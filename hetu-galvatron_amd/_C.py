@@ -6,13 +6,15 @@ The library is the only compute backend of this package: there is no Python or C
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import threading
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # GALVATRON_MOE_LIB selects another build of the same ABI (e.g. a tuning variant)
 LIB_PATH = os.environ.get("GALVATRON_MOE_LIB") or os.path.join(_HERE, "_lib", "libgalvatron_moe.so")
-ABI_VERSION = 10
+ABI_VERSION = 11
 
 GMOE_F32, GMOE_BF16, GMOE_F16, GMOE_F8E4M3 = 0, 1, 2, 3
 SCORE_SOFTMAX, SCORE_SIGMOID, SCORE_IDENTITY = 0, 1, 2
@@ -45,6 +47,7 @@ PROTOTYPES = {
     "gmoe_permute_plan": (_int, [_vp, _i64, _int, _i64, _vp, _vp, _i64, _vp, _vp, _vp, _vp, _vp]),
     "gmoe_permute_plan_static_max_slots": (_i64, []),
     "gmoe_permute_plan_static": (_int, [_vp, _i64, _int, _i64, _vp, _vp, _i64, _vp, _vp, _vp, _vp]),
+    "gmoe_expert_offsets": (_int, [_vp, _int, _vp, _vp]),
     "gmoe_permute_rows": (_int, [_vp, _int, _i64, _i64, _int, _vp, _i64, _vp, _vp, _int, _vp, _vp]),
     "gmoe_unpermute_rows": (_int, [_vp, _int, _i64, _i64, _int, _vp, _i64, _vp, _int, _vp, _vp,
                                    _vp, _vp, _vp, _vp]),
@@ -83,7 +86,9 @@ PROTOTYPES = {
 }
 
 _lib = None
+_host = None
 _lock = threading.Lock()
+HOST_PATH = os.path.join(_HERE, "_lib", "_gmoe_host.so")
 
 
 class LibraryMissingError(RuntimeError):
@@ -112,6 +117,29 @@ def lib() -> ctypes.CDLL:
                                    (got, ABI_VERSION))
             _lib = handle
     return _lib
+
+
+def host():
+    """The native autograd nodes of the layer (csrc/host.cpp), launching through `lib()`."""
+    global _host
+    if _host is not None:
+        return _host
+    lib()
+    with _lock:
+        if _host is None:
+            if not os.path.exists(HOST_PATH):
+                raise LibraryMissingError(
+                    "host module %s is missing: build it with `python %s`. This package has no "
+                    "fallback path." % (HOST_PATH, os.path.join(_HERE, "build.py")))
+            from .moe_utils import MoEAuxLossAutoScaler
+
+            loader = importlib.machinery.ExtensionFileLoader("_gmoe_host", HOST_PATH)
+            spec = importlib.util.spec_from_file_location("_gmoe_host", HOST_PATH, loader=loader)
+            module = importlib.util.module_from_spec(spec)
+            loader.exec_module(module)
+            module.bind_library(LIB_PATH, lambda: MoEAuxLossAutoScaler.main_loss_backward_scale)
+            _host = module
+    return _host
 
 
 def check(status: int, what: str) -> None:

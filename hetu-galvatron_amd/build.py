@@ -17,6 +17,9 @@ LIB_DIR = os.path.join(HERE, "_lib")
 LIB_PATH = os.path.join(LIB_DIR, "libgalvatron_moe.so")
 SOURCES = ["route.hip", "losses.hip", "capacity.hip", "permute.hip", "glu.hip", "bias.hip", "gmm.hip", "gmm_dtl.hip", "gmm_rows.hip", "gmm_tn.hip", "gmm_fp8s.hip", "quant.hip", "norm.hip", "gate.hip", "abi.hip"]
 
+HOST_SOURCE = "host.cpp"  # the native autograd nodes, a torch extension module
+HOST_PATH = os.path.join(LIB_DIR, "_gmoe_host.so")
+
 # packed-fp32 instructions are switched off for every device compilation of this library
 HIPCC_FLAGS = [
     "-O3",
@@ -50,6 +53,27 @@ def _run(cmd):
     return out
 
 
+def build_host() -> str:
+    """Compile csrc/host.cpp against the installed torch (host code only)."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    os.makedirs(LIB_DIR, exist_ok=True)
+    torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    include = [*cpp_extension.include_paths(), "/opt/rocm/include", sysconfig.get_paths()["include"]]
+    tmp = HOST_PATH + ".tmp"
+    _run([shutil.which("g++") or "g++", "-O2", "-fPIC", "-shared", "-std=c++17", "-w",
+          "-DTORCH_EXTENSION_NAME=_gmoe_host", "-DTORCH_API_INCLUDE_EXTENSION_H", "-D__HIP_PLATFORM_AMD__=1",
+          "-DUSE_ROCM=1", "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI),
+          *["-I" + d for d in include], os.path.join(CSRC, HOST_SOURCE), "-o", tmp,
+          "-L" + torch_lib, "-Wl,-rpath," + torch_lib, "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch", "-ltorch_python",
+          "-ldl"])
+    os.replace(tmp, HOST_PATH)
+    return HOST_PATH
+
+
 def build_library(verbose: bool = False, extra_flags=()) -> str:
     """Compile every source under csrc/ and link the shared library.  Always recompiles."""
     hipcc = _hipcc()
@@ -62,10 +86,12 @@ def build_library(verbose: bool = False, extra_flags=()) -> str:
         out = _run([hipcc, *HIPCC_FLAGS, *SOURCE_FLAGS.get(src, ()), *extra_flags, "-c", os.path.join(CSRC, src), "-o", obj])
         return src, out
 
-    with ThreadPoolExecutor(max_workers=min(4, len(SOURCES))) as pool:
+    with ThreadPoolExecutor(max_workers=5) as pool:
+        host = pool.submit(build_host)
         for src, out in pool.map(compile_one, zip(SOURCES, objs)):
             if verbose and out.strip():
                 print("[%s]\n%s" % (src, out))
+        host.result()
     tmp = LIB_PATH + ".tmp"
     _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", tmp, *objs])
     os.replace(tmp, LIB_PATH)

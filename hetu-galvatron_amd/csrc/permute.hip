@@ -648,6 +648,38 @@ static inline bool prob_dtype_ok(int dt) { return dt == GMOE_F32 || dt == GMOE_B
 
 using namespace gmoe;
 
+// One workgroup scans the counts 256 at a time.
+__global__ __launch_bounds__(256) void expert_offsets_kernel(const long long* counts, int E, long long* offsets) {
+  __shared__ long long wave_tot[4];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  long long run = 0;
+  for (int base = 0; base < E; base += 256) {
+    const int e = base + tid;
+    const long long own = e < E ? counts[e] : 0;
+    long long incl = own;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const long long o = __shfl_up(incl, d);
+      if (lane >= d) incl += o;
+    }
+    if (lane == 63) wave_tot[wave] = incl;
+    __syncthreads();
+    long long before = run;
+    for (int w = 0; w < wave; ++w) before += wave_tot[w];
+    if (e < E) offsets[e] = before + incl - own;
+    run += wave_tot[0] + wave_tot[1] + wave_tot[2] + wave_tot[3];
+    __syncthreads();
+  }
+  if (tid == 0) offsets[E] = run;
+}
+
+extern "C" int gmoe_expert_offsets(const int64_t* tokens_per_expert, int E, int64_t* expert_offsets, void* stream) {
+  GMOE_CHECK_ARG(tokens_per_expert != nullptr && expert_offsets != nullptr && E >= 1 && E <= 65536);
+  hipLaunchKernelGGL(expert_offsets_kernel, dim3(1), dim3(256), 0, static_cast<hipStream_t>(stream),
+                     reinterpret_cast<const long long*>(tokens_per_expert), E, reinterpret_cast<long long*>(expert_offsets));
+  return gmoe_launch_status();
+}
+
 extern "C" int64_t gmoe_permute_plan_workspace_bytes(int64_t T, int E) {
   const int64_t NC = (T + kChunkTokens - 1) / kChunkTokens;
   return 2 * (int64_t)E * (NC > 0 ? NC : 1) * (int64_t)sizeof(int);

@@ -17,8 +17,8 @@ from typing import Tuple
 
 import torch
 
-from . import ops
-from .moe_utils import _PermuteRows, _UnpermuteRows, _SortChunks
+from . import _C, ops
+from .moe_utils import _SortChunks
 
 
 def row_id_map_reference_layout(row_id_map: torch.Tensor) -> torch.Tensor:
@@ -54,7 +54,7 @@ def moe_permute(inp: torch.Tensor, routing_map: torch.Tensor, num_out_tokens: in
         # "no tokens are dropped": the size is data dependent, one host read
         num_out_tokens = int(routing_map.bool().sum().item())
     plan = ops.permute_plan(routing_map, num_out_tokens, want_sorted=False)
-    out = _PermuteRows.apply(inp.contiguous(), plan.dst_map, plan.n_out, False)
+    out = _C.host().permute_rows(inp, plan.dst_map, plan.n_out, False)
     return out, plan.dst_map
 
 
@@ -79,7 +79,7 @@ def moe_unpermute(inp: torch.Tensor, row_id_map: torch.Tensor, merging_probs: to
         assert restore_shape[0] == num_tokens and restore_shape[1] == inp.shape[1]
     if merging_probs is not None:
         merging_probs = merging_probs.contiguous()
-    return _UnpermuteRows.apply(inp.contiguous(), row_id_map, merging_probs, num_tokens, False)
+    return _C.host().combine(inp, row_id_map, merging_probs, False, None, None)
 
 
 def moe_sort_chunks_by_index(inp: torch.Tensor, split_sizes: torch.Tensor,

@@ -13,48 +13,18 @@ import torch
 import torch.nn.functional as F
 from torch.nn.parameter import Parameter
 
-from . import ops
+from . import _C, ops
 from .config import MoEConfig
 from .grouped_gemm import ops as gg_ops
 
 
-class _GLU(torch.autograd.Function):
-    """act(y[:, :F]) * y[:, F:]  (mlp.py:52-57; backward transformer/fused_kernels.py:157-162)."""
-
-    @staticmethod
-    def forward(ctx, y, act):
-        ctx.save_for_backward(y)
-        ctx.act = act
-        return ops.glu_fwd(y, act)
-
-    @staticmethod
-    def backward(ctx, grad_out):
-        (y,) = ctx.saved_tensors
-        return ops.glu_bwd(grad_out.contiguous(), y, ctx.act), None
-
-
-class _GLUFp8Store(torch.autograd.Function):
-    """The same activation with its input kept as float8_e4m3fn for the backward
-    (SwiGLUFunction with fp8_input_store, transformer/fused_kernels.py:190-204): a quarter (fp32)
-    or half (16-bit) of the saved bytes, the gradient computed on the rounded input."""
-
-    @staticmethod
-    def forward(ctx, y, act):
-        out, y8 = ops.glu_fwd_fp8store(y, act)
-        ctx.save_for_backward(y8)
-        ctx.act = act
-        return out
-
-    @staticmethod
-    def backward(ctx, grad_out):
-        (y8,) = ctx.saved_tensors
-        return ops.glu_bwd_fp8in(grad_out.contiguous(), y8, ctx.act), None
-
-
 def glu(y: torch.Tensor, act: str = "silu", fp8_input_store: bool = False) -> torch.Tensor:
+    """act(y[:, :F]) * y[:, F:]  (mlp.py:52-57; backward transformer/fused_kernels.py:157-162).
+    `fp8_input_store`: the input is kept as float8_e4m3fn for the backward (SwiGLUFunction with
+    fp8_input_store, transformer/fused_kernels.py:190-204): a quarter (fp32) or half (16-bit) of the saved
+    bytes, the gradient computed on the rounded input."""
     shape = y.shape
-    fn = _GLUFp8Store if fp8_input_store else _GLU
-    out = fn.apply(y.reshape(-1, shape[-1]).contiguous(), act)
+    out = _C.host().glu(y.reshape(-1, shape[-1]).contiguous(), act, fp8_input_store)
     return out.view(*shape[:-1], shape[-1] // 2)
 
 
@@ -99,7 +69,7 @@ def bias_swiglu_impl(input, bias, fp8_input_store=False):
     return glu(input, "silu", fp8_input_store)
 
 
-class _FusedGatedExperts(torch.autograd.Function):
+class _FusedGatedExperts:
     """out = gmm(act(gmm(x, w1)[:, :F]) * gmm(x, w1)[:, F:], w2) with the activation fused into the
     first GEMM's epilogue and its backward into the epilogue of the d(act) GEMM
     (same math, op by op, as moe/mlp.py:106-112 and its autograd)."""
@@ -114,33 +84,9 @@ class _FusedGatedExperts(torch.autograd.Function):
     fuse_backward = True
 
     @staticmethod
-    def forward(ctx, x, w1, w2, batch_sizes, act):
+    def apply(x, w1, w2, batch_sizes, act):
         offsets = ops.expert_offsets_from_batch_sizes(batch_sizes, x.device)
-        x = x.contiguous()
-        w1 = w1.contiguous()
-        w2 = w2.contiguous()
-        fc1, h = ops.gmm_glu(x, w1, offsets, act)
-        out = ops.gmm(h, w2, offsets)
-        ctx.save_for_backward(x, w1, w2, fc1, h, offsets)
-        ctx.act = act
-        return out
-
-    @staticmethod
-    def backward(ctx, grad_out):
-        x, w1, w2, fc1, h, offsets = ctx.saved_tensors
-        grad_out = grad_out.contiguous()
-        dx = dw1 = dw2 = None
-        if _FusedGatedExperts.fuse_backward:
-            dfc1 = ops.gmm_glu_bwd(grad_out, w2, fc1, offsets, ctx.act)
-        else:
-            dfc1 = ops.glu_bwd(ops.gmm(grad_out, w2, offsets, trans_b=True), fc1, ctx.act)
-        if ctx.needs_input_grad[2]:
-            dw2 = ops.gmm(h, grad_out, offsets, trans_a=True)
-        if ctx.needs_input_grad[0]:
-            dx = ops.gmm(dfc1, w1, offsets, trans_b=True)
-        if ctx.needs_input_grad[1]:
-            dw1 = ops.gmm(x, dfc1, offsets, trans_a=True)
-        return dx, dw1, dw2, None, None
+        return _C.host().gated_experts(x, w1, w2, offsets, act, _FusedGatedExperts.fuse_backward)
 
 
 def fused_gated_experts(x, w1, w2, batch_sizes, act: str = "silu"):
@@ -148,58 +94,16 @@ def fused_gated_experts(x, w1, w2, batch_sizes, act: str = "silu"):
     return _FusedGatedExperts.apply(x, w1, w2, batch_sizes, act)
 
 
-class _Fp8GatedExperts(torch.autograd.Function):
-    """The gated expert MLP on block-scaled fp8 weights (frozen): forward and the gradient of the
-    input only.  Weight layouts are those of GroupedMLP, [E,H,2F] and [E,F,H]; the dX GEMMs read the
-    same fp8 tensors with the transposed-operand flag."""
-
-    @staticmethod
-    def _gemm(a, w_q, w_scale, offsets, fp8_activations, trans_b=False):
-        if fp8_activations:
-            # the rows are quantised too (a power-of-two scale per row and 128 elements) and the
-            # product runs on the block-scaled fp8 MFMA
-            a_q, a_scale = ops.quantize_fp8_rows(a)
-            return ops.gmm_fp8a(a_q, a_scale, w_q, w_scale, offsets, trans_b=trans_b)
-        return ops.gmm_fp8w(a, w_q, w_scale, offsets, trans_b=trans_b)
-
-    @staticmethod
-    def forward(ctx, x, w1_q, w1_scale, w2_q, w2_scale, batch_sizes, act, fp8_activations):
-        offsets = ops.expert_offsets_from_batch_sizes(batch_sizes, x.device)
-        gemm = _Fp8GatedExperts._gemm
-        x = x.contiguous()
-        fc1 = gemm(x, w1_q, w1_scale, offsets, fp8_activations)
-        if fp8_activations:
-            # activation and row quantiser in one pass: the activation is needed as fp8 rows only
-            h_q, h_scale = ops.glu_fwd_quantize_fp8_rows(fc1, act)
-            out = ops.gmm_fp8a(h_q, h_scale, w2_q, w2_scale, offsets)
-        else:
-            out = gemm(ops.glu_fwd(fc1, act), w2_q, w2_scale, offsets, False)
-        ctx.save_for_backward(w1_q, w1_scale, w2_q, w2_scale, fc1, offsets)
-        ctx.act = act
-        ctx.fp8_activations = fp8_activations
-        return out
-
-    @staticmethod
-    def backward(ctx, grad_out):
-        w1_q, w1_scale, w2_q, w2_scale, fc1, offsets = ctx.saved_tensors
-        gemm = _Fp8GatedExperts._gemm
-        dact = gemm(grad_out.contiguous(), w2_q, w2_scale, offsets, ctx.fp8_activations, trans_b=True)
-        if ctx.fp8_activations and (fc1.shape[1] // 2) % 128 == 0:
-            d_q, d_scale = ops.glu_bwd_quantize_fp8_rows(dact, fc1, ctx.act)
-            dx = ops.gmm_fp8a(d_q, d_scale, w1_q, w1_scale, offsets, trans_b=True)
-        else:
-            dx = gemm(ops.glu_bwd(dact, fc1, ctx.act), w1_q, w1_scale, offsets, ctx.fp8_activations,
-                      trans_b=True)
-        return dx, None, None, None, None, None, None, None
-
-
 def fp8_gated_experts(x, w1_q, w1_scale, w2_q, w2_scale, batch_sizes, act: str = "silu",
                       fp8_activations: bool = False):
     """x [N,H] bf16; (w1_q [E,H,2F], w1_scale) and (w2_q [E,F,H], w2_scale) from
     ops.quantize_fp8_block; batch_sizes [E] -> [N,H] bf16.  `fp8_activations`: the rows entering each
     of the four products are quantised to fp8 as well (ops.quantize_fp8_rows) and the products run on
-    the fp8 MFMA; off by default, where the bf16 rows are multiplied with the exactly widened weights."""
-    return _Fp8GatedExperts.apply(x, w1_q, w1_scale, w2_q, w2_scale, batch_sizes, act, fp8_activations)
+    the fp8 MFMA; off by default, where the bf16 rows are multiplied with the exactly widened weights.
+    The weights are frozen: the gradient is that of x only, its products read the same fp8 tensors with the
+    transposed-operand flag."""
+    offsets = ops.expert_offsets_from_batch_sizes(batch_sizes, x.device)
+    return _C.host().fp8_gated_experts(x, w1_q, w1_scale, w2_q, w2_scale, offsets, act, fp8_activations)
 
 
 def _act_name(config: MoEConfig) -> str:

@@ -23,7 +23,7 @@ from typing import Optional
 
 import torch
 
-from . import ops
+from . import _C, ops
 
 HAVE_TE = True  # the fused path is always available here
 
@@ -91,36 +91,13 @@ class _ZLoss(torch.autograd.Function):
         return ops.score_stats_bwd(logits, 1, "softmax", z_scale=ctx.factor, grad_loss=g), None
 
 
-class _SeqAuxLoss(torch.autograd.Function):
-    """coeff * mean_b sum_e (count[b,e] * E / (S k)) * mean_s score[s,b,e] of `x` [S*B, E], where
-    the scores are x itself (score_fn "identity") or computed from x as logits inside the kernel.
-    One statistics launch forward, one gradient launch backward."""
-
-    @staticmethod
-    def forward(ctx, x, routing_map, batch_size, seq_length, topk, coeff, score_fn):
-        x = x.contiguous()
-        loss, counts, _ = ops.seq_aux_loss(x, routing_map.contiguous(), batch_size, seq_length, topk,
-                                           coeff, score_fn)
-        ctx.save_for_backward(x, counts)
-        ctx.cfg = (batch_size, seq_length, topk, coeff, score_fn)
-        return loss
-
-    @staticmethod
-    def backward(ctx, grad_loss):
-        x, counts = ctx.saved_tensors
-        batch_size, seq_length, topk, coeff, score_fn = ctx.cfg
-        grad_loss = grad_loss.detach().to(torch.float32).reshape(1).contiguous()
-        dx = ops.seq_aux_loss_bwd(x, counts, batch_size, seq_length, topk, coeff, score_fn, grad_loss)
-        return dx, None, None, None, None, None, None
-
-
 def sequence_load_balancing_loss_func(probs, routing_map, batch_size, seq_length, topk,
                                       moe_aux_loss_coeff, sequence_partition_group=None):
     """Per-sequence load-balancing loss (moe_utils.py:62-112); `probs` [S*B, E] are the routing
     scores, token (s, b) in row s*B + b.  Differentiable in `probs`."""
     _no_sequence_partition(sequence_partition_group)
-    return _SeqAuxLoss.apply(probs, routing_map.bool(), batch_size, seq_length, topk,
-                             moe_aux_loss_coeff, "identity")
+    return _C.host().seq_aux_loss(probs, routing_map.bool(), batch_size, seq_length, topk,
+                                  moe_aux_loss_coeff, "identity")
 
 
 def z_loss_func(logits, z_loss_coeff):
@@ -187,63 +164,13 @@ class MoEAuxLossAutoScaler(torch.autograd.Function):
 # Permute / unpermute
 # ---------------------------------------------------------------------------------------------
 
-class _PermuteRows(torch.autograd.Function):
-    """permuted[dst_map[t,e]] = tokens[t]; backward sums the k gradients of a token in fp32."""
-
-    @staticmethod
-    def forward(ctx, tokens, dst_map, n_out, padded):
-        out, _ = ops.permute_rows(tokens, dst_map, n_out, zero_fill=padded)
-        ctx.save_for_backward(dst_map)
-        ctx.num_tokens = tokens.shape[0]
-        return out
-
-    @staticmethod
-    def backward(ctx, grad_permuted):
-        (dst_map,) = ctx.saved_tensors
-        grad, _ = ops.unpermute_rows(grad_permuted.contiguous(), dst_map, ctx.num_tokens)
-        return grad, None, None, None
-
-
-class _UnpermuteRows(torch.autograd.Function):
-    """out[t] = sum_e permuted[dst_map[t,e]] * probs[t,e]  (+ addend[t]) (+ residual[t])."""
-
-    @staticmethod
-    def forward(ctx, permuted, dst_map, probs, num_tokens, padded, residual=None, addend=None):
-        out, _ = ops.unpermute_rows(permuted, dst_map, num_tokens, merging_probs=probs,
-                                    residual=residual, addend=addend)
-        ctx.with_residual = residual is not None
-        ctx.with_addend = addend is not None
-        ctx.with_probs = probs is not None
-        ctx.padded = padded
-        ctx.n_out = permuted.shape[0]
-        if ctx.with_probs:
-            ctx.save_for_backward(permuted, dst_map, probs)
-        else:
-            ctx.save_for_backward(dst_map)
-        return out
-
-    @staticmethod
-    def backward(ctx, grad_out):
-        grad_out = grad_out.contiguous()
-        if ctx.with_probs:
-            permuted, dst_map, probs = ctx.saved_tensors
-            gp, gprobs = ops.unpermute_rows_bwd(grad_out, permuted, dst_map, probs,
-                                                zero_fill=ctx.padded)
-            return (gp, None, gprobs, None, None, (grad_out if ctx.with_residual else None),
-                    (grad_out if ctx.with_addend else None))
-        (dst_map,) = ctx.saved_tensors
-        gp, _ = ops.permute_rows(grad_out, dst_map, ctx.n_out, zero_fill=ctx.padded)
-        return (gp, None, None, None, None, (grad_out if ctx.with_residual else None),
-                (grad_out if ctx.with_addend else None))
-
-
 def scale_rows(x: torch.Tensor, row_scale: torch.Tensor) -> torch.Tensor:
     """x [T,H] * row_scale [T] (or [T,1]) with one rounding, differentiable in both: the combine
     kernels with the identity map (their backward yields the per-row dot products the scale's
     gradient needs)."""
     T = x.shape[0]
-    return _UnpermuteRows.apply(x.contiguous(), ops.identity_map(T, x.device),
-                                row_scale.reshape(T, 1).contiguous(), T, False)
+    return _C.host().combine(x, ops.identity_map(T, x.device), row_scale.reshape(T, 1).contiguous(), False,
+                             None, None)
 
 
 def _as_int(n) -> int:
@@ -275,7 +202,7 @@ def permute(tokens, routing_map, num_out_tokens: Optional[int] = None, fused: bo
     """
     assert tokens.dim() == 2 and routing_map.dim() == 2
     plan = _plan_for(routing_map, num_out_tokens, drop_and_pad)
-    permuted = _PermuteRows.apply(tokens.contiguous(), plan.dst_map, plan.n_out, plan.padded)
+    permuted = _C.host().permute_rows(tokens, plan.dst_map, plan.n_out, plan.padded)
     if fused:
         return permuted, plan.dst_map
     mapping = plan.sorted_indices
@@ -313,8 +240,7 @@ def unpermute(permuted_tokens: torch.Tensor, sorted_indices: torch.Tensor, resto
         probs = probs.contiguous()
     if residual is not None:
         residual = residual.reshape(num_tokens, hidden).contiguous()
-    return _UnpermuteRows.apply(permuted_tokens.contiguous(), plan.dst_map, probs, num_tokens,
-                                plan.padded, residual)
+    return _C.host().combine(permuted_tokens, plan.dst_map, probs, plan.padded, residual, None)
 
 
 class _SortChunks(torch.autograd.Function):
@@ -342,47 +268,6 @@ def sort_chunks_by_idxs(input: torch.Tensor, split_sizes: torch.Tensor, sorted_i
 # ---------------------------------------------------------------------------------------------
 # Router
 # ---------------------------------------------------------------------------------------------
-
-class _RouteTopK(torch.autograd.Function):
-    """probs, routing_map, tokens_per_expert = route(logits); differentiable in logits."""
-
-    @staticmethod
-    def forward(ctx, logits, k, score_fn, pre_softmax, scaling, expert_bias, num_groups, group_topk,
-                aux_scale=0.0, z_scale=0.0, want_stats=False, selection_scores=None):
-        """aux_scale / z_scale: factors of the load-balancing and z-loss gradients that the backward
-        adds to dlogits (times MoEAuxLossAutoScaler.main_loss_backward_scale), fused into the same
-        kernel instead of separate softmax / logsumexp graphs.  stats = [sum_t scores | sum_t lse^2].
-        selection_scores [T,E] fp32 (no gradient): ranked by the top-k instead of the scores."""
-        probs, rmap, counts, stats, _ = ops.route_topk(
-            logits, k, score_fn, pre_softmax, scaling, expert_bias, num_groups, group_topk,
-            want_stats=want_stats, selection_scores=selection_scores)
-        ctx.save_for_backward(logits, rmap, counts)
-        ctx.cfg = (k, score_fn, pre_softmax, scaling, float(aux_scale), float(z_scale))
-        if stats is None:
-            stats = logits.new_zeros((0,), dtype=torch.float32)
-        ctx.mark_non_differentiable(rmap, counts, stats)
-        # without this autograd fills a zero gradient for each of the three (three fill launches)
-        ctx.set_materialize_grads(False)
-        return probs, rmap, counts, stats
-
-    @staticmethod
-    def backward(ctx, dprobs, _dmap, _dcounts, _dstats):
-        logits, rmap, counts = ctx.saved_tensors
-        k, score_fn, pre_softmax, scaling, aux_scale, z_scale = ctx.cfg
-        if dprobs is None:
-            if aux_scale == 0.0 and z_scale == 0.0:
-                return (None,) * 12
-            dprobs = torch.zeros_like(logits)
-        loss_scale = None
-        if aux_scale != 0.0 or z_scale != 0.0:
-            loss_scale = MoEAuxLossAutoScaler.main_loss_backward_scale
-            if loss_scale is not None:
-                loss_scale = loss_scale.detach().to(device=logits.device, dtype=torch.float32)
-                loss_scale = loss_scale.reshape(-1)[:1].contiguous()
-        dlogits = ops.route_topk_bwd(logits, k, score_fn, pre_softmax, scaling, rmap,
-                                     dprobs.contiguous(), counts, aux_scale, z_scale, loss_scale)
-        return (dlogits,) + (None,) * 11
-
 
 def group_limited_topk(scores, topk, num_tokens, num_experts, num_groups, group_topk):
     """moe_utils.py:372-427: top-k restricted to the `group_topk` best expert groups, a group being
@@ -420,32 +305,14 @@ def topk_softmax_with_capacity(
         raise ValueError(f"Invalid drop_policy: {drop_policy}")
     if expert_bias is not None:
         expert_bias = expert_bias.detach().to(torch.float32).contiguous()
-    probs, routing_map, tokens_per_expert, _ = _RouteTopK.apply(
-        logits.contiguous(), topk, score_function, use_pre_softmax, scaling_factor, expert_bias,
-        num_groups, group_topk)
+    probs, routing_map, tokens_per_expert, _ = _C.host().route_topk(
+        logits, topk, score_function, use_pre_softmax, scaling_factor, expert_bias, num_groups, group_topk,
+        0.0, 0.0, False, None)
     if capacity_factor is None:
         return probs, routing_map, tokens_per_expert
     final_probs, final_map = apply_expert_capacity(probs, routing_map, topk, capacity_factor,
                                                    pad_to_capacity, drop_policy)
     return final_probs, final_map, tokens_per_expert
-
-
-class _CapacitySelect(torch.autograd.Function):
-    """probs * kept with kept chosen by the HIP selection kernel; d probs = grad * kept."""
-
-    @staticmethod
-    def forward(ctx, probs, routing_map, capacity, by_position, pad):
-        out_probs, kept = ops.capacity_select(probs.contiguous(), routing_map.contiguous(), capacity,
-                                              by_position, pad)
-        ctx.save_for_backward(kept)
-        ctx.mark_non_differentiable(kept)
-        ctx.set_materialize_grads(False)
-        return out_probs, kept
-
-    @staticmethod
-    def backward(ctx, grad_probs, _grad_kept):
-        (kept,) = ctx.saved_tensors
-        return (None if grad_probs is None else grad_probs * kept), None, None, None, None
 
 
 def apply_expert_capacity(probs, routing_map, topk, capacity_factor, pad_to_capacity=False,
@@ -457,8 +324,8 @@ def apply_expert_capacity(probs, routing_map, topk, capacity_factor, pad_to_capa
         raise ValueError(f"Invalid drop_policy: {drop_policy}")
     expert_capacity = get_capacity(num_tokens * topk, num_experts, capacity_factor)
     expert_capacity = max(1, min(expert_capacity, num_tokens))
-    return _CapacitySelect.apply(probs, routing_map, expert_capacity, drop_policy == "position",
-                                 pad_to_capacity)
+    return _C.host().capacity_select(probs, routing_map, expert_capacity, drop_policy == "position",
+                                     pad_to_capacity)
 
 
 # ---------------------------------------------------------------------------------------------
@@ -476,15 +343,21 @@ def get_moe_layer_wise_logging_tracker():
 def aux_losses_tracker_slot(name: str, layer_idx: int, num_layers: int, device):
     """One-element fp32 view of `tracker[name]["values"][layer_idx - 1]` (created on first use), for
     kernels that add a loss value to it on the device; None when layer_idx is None."""
+    values = aux_losses_tracker_values(name, layer_idx, num_layers, device)
+    return None if values is None else values.narrow(0, layer_idx - 1, 1)
+
+
+def aux_losses_tracker_values(name: str, layer_idx: int, num_layers: int, device):
+    """`tracker[name]["values"]`, fp32 [num_layers] (created on first use); None when layer_idx is None."""
     if layer_idx is None:
         return None
-    tracker = get_moe_layer_wise_logging_tracker()
-    entry = tracker.setdefault(name, {})
-    if "values" not in entry:
+    entry = _MOE_LAYER_WISE_LOGGING_TRACKER.get(name)
+    if entry is None or "values" not in entry:
+        entry = _MOE_LAYER_WISE_LOGGING_TRACKER.setdefault(name, {})
         entry["values"] = torch.zeros(num_layers, device=device)
     entry.setdefault("reduce_group", None)
     entry.setdefault("avg_group", None)
-    return entry["values"].narrow(0, layer_idx - 1, 1)
+    return entry["values"]
 
 
 def save_to_aux_losses_tracker(name: str, loss: torch.Tensor, layer_idx: int, num_layers: int,

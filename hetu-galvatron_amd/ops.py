@@ -313,24 +313,9 @@ def permute_plan(routing_map: torch.Tensor, n_out: int, capacity: int = 0,
     assert routing_map.dim() == 2
     if routing_map.dtype != torch.bool:
         routing_map = routing_map.bool()
-    routing_map = routing_map.contiguous()
-    dev = _check_dev(routing_map)
     T, E = routing_map.shape
-    L = _C.lib()
-    dst_map = torch.empty((T, E), dtype=torch.int32, device=dev)
-    # rows that stay unwritten (padding of a fixed-capacity block) read as token 0
-    sorted_indices = (torch.zeros if capacity > 0 else torch.empty)(
-        (n_out,), dtype=torch.int64, device=dev) if want_sorted else None
-    row_id_map = torch.empty((E, T), dtype=torch.int64, device=dev) if want_row_id_map else None
-    counts = torch.empty((E,), dtype=torch.int64, device=dev)
-    offsets = torch.empty((E + 1,), dtype=torch.int64, device=dev)
-    ws = torch.empty((max(1, L.gmoe_permute_plan_workspace_bytes(T, E)),), dtype=torch.uint8,
-                     device=dev)
-    with _on(dev):
-        st = L.gmoe_permute_plan(_ptr(routing_map), T, E, int(capacity), _ptr(dst_map),
-                                 _ptr(sorted_indices), int(n_out), _ptr(row_id_map), _ptr(counts),
-                                 _ptr(offsets), _ptr(ws), _stream(dev))
-    _C.check(st, "gmoe_permute_plan")
+    dst_map, sorted_indices, row_id_map, counts, offsets = _C.host().permute_plan(
+        routing_map.contiguous(), int(n_out), int(capacity), want_sorted, want_row_id_map)
     return PermutePlan(dst_map, sorted_indices, row_id_map, counts, offsets, T, E, int(n_out),
                        padded=capacity > 0)
 
@@ -571,6 +556,9 @@ def expert_offsets_from_batch_sizes(batch_sizes: torch.Tensor, device) -> torch.
     cached = getattr(batch_sizes, "_gmoe_offsets", None)
     if cached is not None and cached.device == torch.device(device):
         return cached
+    device = torch.device(device)
+    if batch_sizes.device == device:
+        return _C.host().expert_offsets(batch_sizes.to(torch.int64).contiguous())
     bs = batch_sizes.to(torch.int64)
     off = torch.zeros(bs.numel() + 1, dtype=torch.int64, device=bs.device)
     torch.cumsum(bs, 0, out=off[1:])
@@ -892,85 +880,11 @@ def gate_supported(x: torch.Tensor, weight: torch.Tensor) -> bool:
             and (E <= 16 or (H % 8 == 0 and E <= 4096)))
 
 
-def _gate_padded_experts(E: int) -> int:
-    """Beyond 16 experts the projection runs as dense products whose rows are 16-byte multiples:
-    the expert count is padded to a multiple of 8 with zero rows of the weight."""
-    return E if E <= 16 else (E + 7) // 8 * 8
-
-
-def _pad_rows(t: torch.Tensor, rows: int) -> torch.Tensor:
-    out = t.new_zeros((rows,) + tuple(t.shape[1:]))
-    out[: t.shape[0]].copy_(t)
-    return out
-
-
-def _pad_cols(t: torch.Tensor, cols: int) -> torch.Tensor:
-    out = t.new_zeros((t.shape[0], cols))
-    out[:, : t.shape[1]].copy_(t)
-    return out
-
-
 def gate_fwd(x: torch.Tensor, weight: torch.Tensor, out_dtype: Optional[torch.dtype] = None):
     """logits [.., E] = x [.., H] @ weight[E, H]^T (gmoe_gate_fwd); out_dtype = x.dtype or float32."""
-    dev = _check_dev(x, weight)
-    E, H = weight.shape
-    assert x.shape[-1] == H and x.dtype == weight.dtype
-    out_dtype = out_dtype or x.dtype
-    x2 = x.reshape(-1, H)
-    T = x2.shape[0]
-    E_real = E
-    E = _gate_padded_experts(E)
-    if E != E_real:
-        weight = _pad_rows(weight, E)
-    logits = torch.empty((T, E), dtype=out_dtype, device=dev)
-    with _on(dev):
-        nbytes = _C.lib().gmoe_gate_fwd_workspace_bytes(T, H, E, _dt(x2))
-        if nbytes < 0:
-            raise RuntimeError("gmoe_gate_fwd: unsupported shape T=%d H=%d E=%d" % (T, H, E))
-        ws = torch.empty((nbytes,), dtype=torch.uint8, device=dev) if nbytes else None
-        st = _C.lib().gmoe_gate_fwd(_ptr(x2), _ptr(weight), T, H, E, _dt(x2), _ptr(logits), _dt(logits),
-                                    _ptr(ws), nbytes, _stream(dev))
-    _C.check(st, "gmoe_gate_fwd")
-    if E != E_real:
-        logits = logits[:, :E_real].contiguous()
-    return logits.view(*x.shape[:-1], E_real)
+    return _C.host().gate_fwd(x, weight, out_dtype or x.dtype)
 
 
 def gate_bwd(dlogits: torch.Tensor, x: torch.Tensor, weight: torch.Tensor, need_dx=True, need_dw=True):
     """(dx, dweight) of gate_fwd (gmoe_gate_bwd_input, gmoe_gate_bwd_weight)."""
-    dev = _check_dev(dlogits, x, weight)
-    E, H = weight.shape
-    x2, dl = x.reshape(-1, H), dlogits.reshape(-1, E)
-    T = x2.shape[0]
-    assert dl.shape[0] == T
-    E_real = E
-    E = _gate_padded_experts(E)
-    if E != E_real:
-        # zero weight rows and zero gradient columns for the padding experts: dx is unchanged and the
-        # padding rows of dw are dropped
-        weight, dl = _pad_rows(weight, E), _pad_cols(dl, E)
-    L = _C.lib()
-    dx = dw = None
-    with _on(dev):
-        if need_dx:
-            dx = torch.empty_like(x2)
-            nbytes = L.gmoe_gate_bwd_input_workspace_bytes(T, H, E, _dt(x2), _dt(dl))
-            if nbytes < 0:
-                raise RuntimeError("gmoe_gate_bwd_input: unsupported shape T=%d H=%d E=%d" % (T, H, E))
-            ws = torch.empty((nbytes,), dtype=torch.uint8, device=dev) if nbytes else None
-            st = L.gmoe_gate_bwd_input(_ptr(dl), _dt(dl), _ptr(weight), T, H, E, _dt(x2), _ptr(dx),
-                                       _ptr(ws), nbytes, _stream(dev))
-            _C.check(st, "gmoe_gate_bwd_input")
-            dx = dx.view(x.shape)
-        if need_dw:
-            rows = L.gmoe_gate_bwd_workspace_rows(T, H, E, _dt(x2))
-            if rows < 0:
-                raise RuntimeError("gmoe_gate_bwd_weight: unsupported shape T=%d H=%d E=%d" % (T, H, E))
-            ws = torch.empty((max(rows, 1), E * H), dtype=torch.float32, device=dev)
-            dw = torch.empty_like(weight)
-            st = L.gmoe_gate_bwd_weight(_ptr(dl), _dt(dl), _ptr(x2), T, H, E, _dt(x2), _ptr(dw), _ptr(ws),
-                                        rows, _stream(dev))
-            _C.check(st, "gmoe_gate_bwd_weight")
-            if E != E_real:
-                dw = dw[:E_real].contiguous()
-    return dx, dw
+    return _C.host().gate_bwd(dlogits, x, weight, need_dx, need_dw)

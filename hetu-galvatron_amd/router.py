@@ -13,35 +13,25 @@ from __future__ import annotations
 
 import torch
 
-from . import ops
+from . import _C, ops
 from .config import MoEConfig
 from .moe_utils import (
     MoEAuxLossAutoScaler,
-    _RouteTopK,
-    _SeqAuxLoss,
     apply_expert_capacity,
-    aux_losses_tracker_slot,
+    aux_losses_tracker_values,
     save_to_aux_losses_tracker,
     z_loss_func,
 )
 
 
-class _GateProjection(torch.autograd.Function):
+class _GateProjection:
     """F.linear(input.to(router_dtype), weight.to(router_dtype)) (router.py:49-68) on the HIP gate
     kernels; gradients come back in the dtypes of input and weight, as autograd of the casts gives."""
 
     @staticmethod
-    def forward(ctx, x, weight, router_dtype):
+    def apply(x, weight, router_dtype):
         x = x.contiguous()
-        ctx.save_for_backward(x, weight)
-        return ops.gate_fwd(x, weight, out_dtype=router_dtype)
-
-    @staticmethod
-    def backward(ctx, dlogits):
-        x, weight = ctx.saved_tensors
-        dx, dw = ops.gate_bwd(dlogits.contiguous(), x, weight, need_dx=ctx.needs_input_grad[0],
-                              need_dw=ctx.needs_input_grad[1])
-        return dx, dw, None
+        return _C.host().gate_projection(ops.gate_fwd(x, weight, out_dtype=router_dtype), x, weight)
 
 
 class Router(torch.nn.Module):
@@ -151,8 +141,9 @@ class TopKRouter(Router):
         bias = None if plain or score_function != "sigmoid" else self.expert_bias
         if bias is not None:
             bias = bias.detach().to(torch.float32).contiguous()
-        probs, routing_map, counts, stats = _RouteTopK.apply(
-            logits.contiguous(), self.topk, score_function, pre_softmax,
+        host = _C.host()
+        probs, routing_map, counts, stats = host.route_topk(
+            logits, self.topk, score_function, pre_softmax,
             None if plain else cfg.moe_router_topk_scaling_factor, bias,
             None if plain else cfg.moe_router_num_groups, None if plain else cfg.moe_router_group_topk,
             aux_scale, z_scale, want_stats, selection)
@@ -161,24 +152,21 @@ class TopKRouter(Router):
         # unless tokens are dropped afterwards
         count_here = self.enable_expert_bias and torch.is_grad_enabled() and capacity is None
         if want_stats or count_here:
-            with torch.no_grad():
-                dev = logits.device
-                track_aux, track_z = aux_scale != 0.0, z_scale != 0.0
-                aux, z = ops.router_bookkeeping(
-                    stats if want_stats else None, counts, E,
-                    aux_factor=E * aux_coeff / (T * T * self.topk) if track_aux else 0.0,
-                    z_factor=z_coeff / T if track_z else 0.0, want_aux=track_aux, want_z=track_z,
-                    aux_slot=aux_losses_tracker_slot("load_balancing_loss", self.layer_idx,
-                                                     cfg.num_layers, dev) if track_aux else None,
-                    aux_slot_scale=1.0 / aux_coeff if track_aux else 1.0,
-                    z_slot=aux_losses_tracker_slot("z_loss", self.layer_idx, cfg.num_layers, dev)
-                    if track_z else None,
-                    z_slot_scale=1.0 / z_coeff if track_z and z_coeff else 1.0,
-                    local_tokens=self.local_tokens_per_expert if count_here else None)
-                if track_aux:
-                    self.last_aux_loss = aux
-                if track_z:
-                    self.last_z_loss = z
+            dev = logits.device
+            track_aux, track_z = aux_scale != 0.0, z_scale != 0.0
+            aux, z = host.bookkeeping(
+                stats, counts, E * aux_coeff / (T * T * self.topk) if track_aux else 0.0,
+                z_coeff / T if track_z else 0.0, track_aux, track_z,
+                aux_losses_tracker_values("load_balancing_loss", self.layer_idx, cfg.num_layers, dev)
+                if track_aux else None,
+                aux_losses_tracker_values("z_loss", self.layer_idx, cfg.num_layers, dev) if track_z else None,
+                (self.layer_idx or 1) - 1, 1.0 / aux_coeff if track_aux else 1.0,
+                1.0 / z_coeff if track_z and z_coeff else 1.0,
+                self.local_tokens_per_expert if count_here else None)
+            if track_aux:
+                self.last_aux_loss = aux
+            if track_z:
+                self.last_z_loss = z
         if capacity is not None:
             probs, routing_map = apply_expert_capacity(
                 probs, routing_map, self.topk, capacity, cfg.moe_pad_expert_input_to_capacity,
@@ -197,12 +185,12 @@ class TopKRouter(Router):
         sum per token (top-1: plain sigmoid).  The routing kernel with k = E: every expert selected."""
         E = logits.shape[-1]
         if self.score_function == "softmax":
-            return _RouteTopK.apply(logits.float().contiguous(), E, "softmax", True, None, None, None,
-                                    None)[0]
+            return _C.host().route_topk(logits.float(), E, "softmax", True, None, None, None, None, 0.0, 0.0,
+                                        False, None)[0]
         if self.score_function == "sigmoid":
             if self.topk > 1:
-                return _RouteTopK.apply(logits.contiguous(), E, "sigmoid", False, None, None, None,
-                                        None)[0]
+                return _C.host().route_topk(logits, E, "sigmoid", False, None, None, None, None, 0.0, 0.0, False,
+                                            None)[0]
             return torch.sigmoid(logits)
         raise ValueError(f"Invalid score_function: {self.score_function}")
 
@@ -251,8 +239,8 @@ class TopKRouter(Router):
         probs, routing_map, _ = self._route(logits, 0.0, z_coeff)
         coeff = self.config.moe_aux_loss_coeff
         if self.training and torch.is_grad_enabled() and coeff != 0:
-            aux_loss = _SeqAuxLoss.apply(logits, routing_map, bsz, seq_length, self.topk, coeff,
-                                         self.score_function)
+            aux_loss = _C.host().seq_aux_loss(logits, routing_map, bsz, seq_length, self.topk, coeff,
+                                              self.score_function)
             self.last_aux_loss = aux_loss.detach()
             save_to_aux_losses_tracker("load_balancing_loss", self.last_aux_loss / coeff,
                                        self.layer_idx, self.config.num_layers)

@@ -18,9 +18,9 @@ from typing import List, Optional
 
 import torch
 
-from . import ops
+from . import _C, ops
 from .config import MoEConfig
-from .moe_utils import _PermuteRows, _UnpermuteRows, get_capacity
+from .moe_utils import get_capacity
 
 
 class MoETokenDispatcher:
@@ -88,7 +88,7 @@ class MoEAllGatherTokenDispatcher(MoETokenDispatcher):
         # of the permuted rows): with a capacity factor >= 1 the bound above is T*k, yet tokens may
         # have been dropped and the rows past the last offset exist
         self._zero_fill = not dropless
-        permuted = _PermuteRows.apply(hidden_states.contiguous(), plan.dst_map, n_out, self._zero_fill)
+        permuted = _C.host().permute_rows(hidden_states, plan.dst_map, n_out, self._zero_fill)
         self.reversed_local_input_permutation_mapping = plan.dst_map
         return permuted, _attach_offsets(plan.tokens_per_expert, plan.expert_offsets)
 
@@ -105,8 +105,7 @@ class MoEAllGatherTokenDispatcher(MoETokenDispatcher):
             if bias.dim() == 1:  # a single local expert hands back its [H] bias (moe/mlp.py:184-186)
                 from .mlp import expand_bias
                 bias = expand_bias(bias, plan.n_out)
-            unpermuted_bias = _UnpermuteRows.apply(bias.contiguous(), plan.dst_map, self.local_probs,
-                                                   plan.num_tokens, self._zero_fill, None, None)
+            unpermuted_bias = _C.host().combine(bias, plan.dst_map, self.local_probs, self._zero_fill, None, None)
             unpermuted_bias = unpermuted_bias.view(self.hidden_shape)
         else:
             assert bias is None, "the experts returned a bias although add_bias_linear is off"
@@ -116,8 +115,7 @@ class MoEAllGatherTokenDispatcher(MoETokenDispatcher):
             shared = shared.reshape(plan.num_tokens, -1).contiguous()
         # gate weighting and the k-way reduction in one pass, fp32 accumulation
         # (token_dispatcher.py:233-244 does a multiply followed by scatter_add_)
-        out = _UnpermuteRows.apply(hidden_states.contiguous(), plan.dst_map, self.local_probs,
-                                   plan.num_tokens, self._zero_fill, residual, shared)
+        out = _C.host().combine(hidden_states, plan.dst_map, self.local_probs, self._zero_fill, residual, shared)
         return out.view(self.hidden_shape), unpermuted_bias
 
 
@@ -173,8 +171,7 @@ class MoEAlltoAllTokenDispatcher(MoETokenDispatcher):
                                 capacity=self.capacity if self.drop_and_pad else 0, want_sorted=False)
         self._plan = plan
         bounded = self.config.moe_expert_capacity_factor is not None
-        permuted = _PermuteRows.apply(hidden_states.contiguous(), plan.dst_map, plan.n_out,
-                                      plan.padded or bounded)
+        permuted = _C.host().permute_rows(hidden_states, plan.dst_map, plan.n_out, plan.padded or bounded)
         self.reversed_local_input_permutation_mapping = plan.dst_map
         return permuted, _attach_offsets(plan.tokens_per_expert, plan.expert_offsets)
 
@@ -186,8 +183,6 @@ class MoEAlltoAllTokenDispatcher(MoETokenDispatcher):
             residual = residual.reshape(plan.num_tokens, -1).contiguous()
         if shared is not None:
             shared = shared.reshape(plan.num_tokens, -1).contiguous()
-        out = _UnpermuteRows.apply(hidden_states.contiguous(), plan.dst_map, self.probs.contiguous(),
-                                   plan.num_tokens,
-                                   plan.padded or self.config.moe_expert_capacity_factor is not None,
-                                   residual, shared)
+        out = _C.host().combine(hidden_states, plan.dst_map, self.probs.contiguous(),
+                                plan.padded or self.config.moe_expert_capacity_factor is not None, residual, shared)
         return out.view(self.hidden_shape), None

@@ -22,7 +22,7 @@
 extern "C" {
 #endif
 
-#define GMOE_ABI_VERSION 10
+#define GMOE_ABI_VERSION 11
 
 typedef enum {
   GMOE_F32 = 0,
@@ -204,6 +204,11 @@ int gmoe_permute_plan_static(const uint8_t* routing_map, int64_t T, int E, int64
                              int32_t* dst_map, int64_t* sorted_indices, int64_t sorted_cap,
                              int64_t* row_id_map, int64_t* tokens_per_expert,
                              int64_t* expert_offsets, void* stream);
+
+/* expert_offsets [E+1] = exclusive prefix sums of tokens_per_expert [E] (both int64, on the device): the
+ * table the grouped GEMMs walk, for callers that hold only the counts (the `batch_sizes` of
+ * `grouped_gemm.ops.gmm`, moe/mlp.py:106-112).  1 <= E <= 65536. */
+int gmoe_expert_offsets(const int64_t* tokens_per_expert, int E, int64_t* expert_offsets, void* stream);
 
 /* Row scatter: permuted[dst_map[t,e]] = tokens[t] for every routed (t,e).  Replaces
  * `tokens.index_select(0, sorted_indices)` (moe/moe_utils.py:275) and `_permute_kernel`
