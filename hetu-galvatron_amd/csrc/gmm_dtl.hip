@@ -94,6 +94,7 @@ __global__ __launch_bounds__(kGemmThreads) void gmm_dtl_kernel(GmmParams p) {
   constexpr int NM = 16;  // MFMAs per K step
   constexpr int RA = OpA::READS_PER_FRAG, RB = OpB::READS_PER_FRAG;
   constexpr int NREAD = WT * RA + WT * RB;  // LDS reads per K step
+  static_assert(NREAD == NM && LOADS_PER_TILE == NM / 2, "one read per MFMA, a copy after every fourth");
 
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
 
@@ -185,45 +186,35 @@ __global__ __launch_bounds__(kGemmThreads) void gmm_dtl_kernel(GmmParams p) {
         const unsigned char* cur = lds + (kt & (NST - 1)) * STAGE_BYTES;
         const unsigned char* nxt = lds + ((kt + 1) & (NST - 1)) * STAGE_BYTES;
         const uint32_t st3 = lds0 + (uint32_t)(((kt + 3) & (NST - 1)) * STAGE_BYTES);
-        // ---- K step 0: MFMAs on buffer 0; read step 1 into buffer 1; request tile kt+3 ------
+        // ---- K step 0: MFMAs on buffer 0; read step 1 into buffer 1; request a of tile kt+3 ---
+        // One fragment read per MFMA and a copy after every fourth: the stage of tile kt-1 is free for
+        // both steps, and copies spread over both are 1-2 % faster than all eight at the end of this
+        // one (dW of fc1 on the Mixtral shape 6.20 -> 6.14 ms, 1.09 -> 1.06 ms for 8192 x 2048 x 11264).
         static_for<0, NM>([&](auto m_c) {
           constexpr int m = decltype(m_c)::value;
           // boustrophedon order over the fragments: one operand changes per MFMA
           constexpr int mi = m / WT, mj = (mi & 1) ? WT - 1 - m % WT : m % WT;
           Mma<DT>::run(fa[0][mi], fb[0][mj], acc[mi][mj]);
           GMOE_SCHED_FENCE();
-          constexpr int n_ops = NREAD + LOADS_PER_TILE;
-          constexpr int op_begin = (m * n_ops + NM - 1) / NM;
-          constexpr int op_end = ((m + 1) * n_ops + NM - 1) / NM;
-          static_for<op_begin, op_end>([&](auto op_c) {
-            constexpr int op = decltype(op_c)::value;
-            if constexpr (op < NREAD) {
-              frag_read(op_c, std::integral_constant<int, 1>{}, std::integral_constant<int, 1>{}, cur);
-            } else if constexpr (op - NREAD < 4) {
-              oa.template issue<op - NREAD>(kt + 3, st3, wave);
-            } else {
-              ob.template issue<op - NREAD - 4>(kt + 3, st3 + OPER_BYTES, wave);
-            }
-          });
+          frag_read(m_c, std::integral_constant<int, 1>{}, std::integral_constant<int, 1>{}, cur);
+          if constexpr (m % 4 == 2) oa.template issue<m / 4>(kt + 3, st3, wave);
+
           GMOE_SCHED_FENCE();
         });
-        // tile kt+1 must have landed (tiles kt+2 and kt+3 may still be in flight); the barrier
+        // tile kt+1 must have landed (kt+2 and the half of kt+3 may still be in flight); the barrier
         // also tells everyone that this tile's stage has been read for the last time
-        wait_dma_outstanding<2 * LOADS_PER_TILE>();
+        wait_dma_outstanding<LOADS_PER_TILE + 4>();
         __syncthreads();
         GMOE_SCHED_FENCE();
-        // ---- K step 1: MFMAs on buffer 1; read step 0 of tile kt+1 into buffer 0 -------------
+        // ---- K step 1: MFMAs on buffer 1; read step 0 of tile kt+1 into buffer 0; request b of kt+3
         static_for<0, NM>([&](auto m_c) {
           constexpr int m = decltype(m_c)::value;
           // boustrophedon order over the fragments: one operand changes per MFMA
           constexpr int mi = m / WT, mj = (mi & 1) ? WT - 1 - m % WT : m % WT;
           Mma<DT>::run(fa[1][mi], fb[1][mj], acc[mi][mj]);
           GMOE_SCHED_FENCE();
-          constexpr int op_begin = (m * NREAD + NM - 1) / NM;
-          constexpr int op_end = ((m + 1) * NREAD + NM - 1) / NM;
-          static_for<op_begin, op_end>([&](auto op_c) {
-            frag_read(op_c, std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{}, nxt);
-          });
+          frag_read(m_c, std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{}, nxt);
+          if constexpr (m % 4 == 2) ob.template issue<m / 4>(kt + 3, st3 + OPER_BYTES, wave);
           GMOE_SCHED_FENCE();
         });
       }
