@@ -497,7 +497,7 @@ extern "C" int64_t gmoe_gate_fwd_workspace_bytes(int64_t T, int64_t H, int E, in
   using namespace gmoe;
   if (gate_status(T, H, E, dtype, dtype, false) != GMOE_OK) return -1;
   if (E <= kGateFwdMaxE) return 0;
-  return gmm_dense_workspace_floats(T, H, E, MODE_NT) * 4;
+  return gmm_dense_workspace_floats(T, H, E, MODE_NT, dtype) * 4;
 }
 
 extern "C" int gmoe_gate_fwd(const void* x, const void* weight, int64_t T, int64_t H, int E, int dtype,

@@ -485,6 +485,80 @@ __device__ inline int resolve_row_part(const GmmParams& p, int k_tiles, int* cou
   return use ? ROWS_REMAINDER : ROWS_NONE;
 }
 
+// tile_cum[e] = tiles of the experts before e, tile_cum[E] all of them: one pass over the offset table, a
+// thread owns kPer consecutive experts, the per-thread sums are scanned with wavefront shuffles and four
+// wavefront totals in LDS.  Ends with a barrier.
+template <int MODE, int BM>
+__device__ __forceinline__ void build_tile_cum(const GmmParams& p, int part, int nt_cnt, int mt_fixed,
+                                               int* tile_cum) {
+  constexpr int kPer = kMaxGroupsLds / kGemmThreads;
+  __shared__ int wave_tot[kGemmThreads / 64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, E = p.E;
+  int cnt[kPer], local = 0;
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    const int e = tid * kPer + j;
+    int c = 0;
+    if (e < E) {
+      long long n = group_begin(p, e + 1) - group_begin(p, e), skip;
+      if (MODE != MODE_TN) expert_row_part(n, part, skip, n);
+      const long long mt = MODE == MODE_TN ? mt_fixed : (n + BM - 1) / BM;
+      c = (int)(mt * nt_cnt);
+    }
+    cnt[j] = c;
+    local += c;
+  }
+  int incl = local;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int o = __shfl_up(incl, d);
+    if (lane >= d) incl += o;
+  }
+  if (lane == 63) wave_tot[wave] = incl;
+  __syncthreads();
+  int run = incl - local;
+  for (int w = 0; w < wave; ++w) run += wave_tot[w];
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    const int e = tid * kPer + j;
+    if (e <= E) tile_cum[e] = run;
+    run += cnt[j];
+  }
+  if (tid == kGemmThreads - 1) tile_cum[E] = run;  // experts past E add nothing: the total
+  __syncthreads();
+}
+
+// Pieces the reduction of every tile of a 128x128 launch is cut into, 1 for none: a K tile of a tile that
+// has its CU to itself costs `us_per_k_tile`, a split launch 6 us for the second kernel and 0.026 us per
+// piece for the 128 KiB of partial sums written and read again; it cannot end before the weights have been
+// streamed (`stream_us`).  Measured on both sides of the line: 128 tiles of 44 K tiles 27 unsplit against
+// 32 us in four pieces, 64 tiles of 16 K tiles 13 against 21, 96 tiles of 64 K tiles 45 against 32, fp32
+// 4 tiles of 16 K tiles 36 against 14; 256 tiles of 224 K tiles (940 MB of weights) 159 against 193.
+__host__ __device__ inline int split_pieces(float us_per_k_tile, long long k_tiles, long long tiles, long long slots,
+                                            float stream_us) {
+  if (tiles <= 0) return 1;
+  long long most = slots / tiles;
+  if (most > kMaxSplit) most = kMaxSplit;
+  if (most > k_tiles) most = k_tiles;
+  if (most < 2) return 1;
+  const float whole = us_per_k_tile * (float)k_tiles, per_piece = 0.026f * (float)tiles;
+  long long s = (long long)(sqrtf(whole / per_piece) + 0.5f);
+  s = s < 2 ? 2 : (s > most ? most : s);
+  const float split = whole / (float)s > stream_us ? whole / (float)s : stream_us;
+  return whole - split > 6.f + per_piece * (float)s ? (int)s : 1;
+}
+__host__ __device__ inline float weight_stream_us(int64_t E, int64_t K, int64_t M, int elem_bytes) {
+  return (float)(E * K * M * elem_bytes) / 6.5e6f;  // 6.5 TB/s
+}
+__host__ __device__ constexpr float split_us_per_k_tile(int elem_bytes) { return elem_bytes == 2 ? 0.42f : 2.1f; }
+// What both kernels of a split launch use: depends on launch parameters and the tile count only.
+__device__ __forceinline__ int split_count(const GmmParams& p, float us_per_k_tile, long long total_tiles,
+                                           long long k_tiles, long long tile_elems) {
+  if (p.split_slots == 0) return 1;
+  const int s = split_pieces(us_per_k_tile, k_tiles, total_tiles, p.split_slots, p.stream_us);
+  return (long long)s * total_tiles * tile_elems <= p.ws_floats ? s : 1;
+}
+
 // The row passes of the fused activation backward's epilogue, out of line so that its registers are
 // allocated apart from the main loop's: the tile of d(act) is staged in LDS (CTile layout); the fc1
 // rows of the next batch of passes are requested before the current batch is computed and stored.
@@ -608,66 +682,17 @@ __global__ __launch_bounds__(kGemmThreads, (BM == 128 && BN == 128) ? 2 : 1) voi
     if (part == ROWS_NONE) return;  // the launch with 256-row tiles takes every row
   }
 
-  {
-    // tiles per expert -> exclusive prefix in one pass: a thread owns kPer consecutive experts, the
-    // per-thread sums are scanned with wavefront shuffles and four wavefront totals in LDS
-    constexpr int kPer = kMaxGroupsLds / kGemmThreads;
-    __shared__ int wave_tot[kGemmThreads / 64];
-    int cnt[kPer], local = 0;
-#pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-      const int e = tid * kPer + j;
-      int c = 0;
-      if (e < E) {
-        long long n = group_begin(p, e + 1) - group_begin(p, e), skip;
-        if (MODE != MODE_TN) expert_row_part(n, part, skip, n);
-        const long long mt = MODE == MODE_TN ? mt_fixed : (n + BM - 1) / BM;
-        c = (int)(mt * nt_cnt);
-      }
-      cnt[j] = c;
-      local += c;
-    }
-    int incl = local;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const int o = __shfl_up(incl, d);
-      if (lane >= d) incl += o;
-    }
-    if (lane == 63) wave_tot[wave] = incl;
-    __syncthreads();
-    int run = incl - local;
-    for (int w = 0; w < wave; ++w) run += wave_tot[w];
-#pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-      const int e = tid * kPer + j;
-      if (e <= E) tile_cum[e] = run;
-      run += cnt[j];
-    }
-    if (tid == kGemmThreads - 1) tile_cum[E] = run;  // experts past E add nothing: the total
-  }
-  __syncthreads();
+  build_tile_cum<MODE, BM>(p, part, nt_cnt, mt_fixed, tile_cum);
   const long long total_tiles = tile_cum[E];
 
   // A launch with few tiles and a long reduction (the short last row tiles of the experts) leaves
-  // most CUs idle while each workgroup walks the whole K range.  With a workspace it runs twice:
-  // SPLIT_PARTIAL cuts the reduction of every tile into S pieces, one workgroup each, which store
-  // their fp32 accumulators; SPLIT_REDUCE adds the S partial tiles in order and runs the epilogue.
-  // S depends only on launch parameters and the tile count, so both launches agree on it.
+  // most CUs idle while each workgroup walks the whole K range.  With a workspace the reduction of
+  // every tile is cut into S pieces, one workgroup each, which store their fp32 accumulators;
+  // gmm_split_reduce_kernel adds the S partial tiles in order.
   constexpr bool CAN_SPLIT = MODE != MODE_TN && EPI == EPI_NONE && !BQ && SMALL;
   constexpr long long TILE_ELEMS = (long long)BM * BN;
-  int S = 1;
-  if constexpr (CAN_SPLIT) {
-    if (p.phase != SPLIT_OFF && total_tiles > 0) {
-      const long long kt_all = (K + BK - 1) / BK;
-      long long want = p.split_slots / total_tiles;
-      if (want > kMaxSplit) want = kMaxSplit;
-      if (want > kt_all) want = kt_all;
-      if (want >= 2 && want * total_tiles * TILE_ELEMS <= p.ws_floats) S = (int)want;
-    }
-    if (p.phase == SPLIT_REDUCE && S == 1) return;  // the first launch did everything
-  }
-  const bool reduce_phase = CAN_SPLIT && p.phase == SPLIT_REDUCE;
-  const long long total_work = (S > 1 && !reduce_phase) ? total_tiles * S : total_tiles;
+  const int S = CAN_SPLIT ? split_count(p, split_us_per_k_tile(ES), total_tiles, (K + BK - 1) / BK, TILE_ELEMS) : 1;
+  const long long total_work = total_tiles * S;
 
   // Workgroup w runs on XCD w%8.  Give XCD x the consecutive positions [x*G/8, (x+1)*G/8) of
   // every whole round of G = gridDim.x tiles (G is a multiple of 8).  The tiles of the last, partial
@@ -686,8 +711,8 @@ __global__ __launch_bounds__(kGemmThreads, (BM == 128 && BN == 128) ? 2 : 1) voi
       if (slot >= share || v >= total_work) break;
     }
     GMOE_PROBE_TILE_BEGIN();
-    const long long s = (S > 1 && !reduce_phase) ? v / S : v;
-    const int chunk = (S > 1 && !reduce_phase) ? (int)(v % S) : 0;
+    const long long s = S > 1 ? v / S : v;
+    const int chunk = S > 1 ? (int)(v % S) : 0;
     while (tile_cum[e + 1] <= s) ++e;
     long long row0 = group_begin(p, e);
     long long n_e = group_begin(p, e + 1) - row0;
@@ -749,9 +774,9 @@ __global__ __launch_bounds__(kGemmThreads, (BM == 128 && BN == 128) ? 2 : 1) voi
       if (S > 1) {
         const int64_t kt_all = (K + BK - 1) / BK;
         const int64_t per = (kt_all + S - 1) / S * BK;
-        k0 = reduce_phase ? K : chunk * per;
+        k0 = chunk * per;
         if (k0 > K) k0 = K;
-        k_lim = reduce_phase ? 0 : (k0 + per < K ? per : K - k0);
+        k_lim = k0 + per < K ? per : K - k0;
       }
       la.init(p.a + (row0 * K + k0) * ES, K, (int64_t)mt * BM, n_e, k_lim, tid);
       if (MODE == MODE_NN)
@@ -912,35 +937,18 @@ __global__ __launch_bounds__(kGemmThreads, (BM == 128 && BN == 128) ? 2 : 1) voi
       if (S > 1) {
         // partial tiles of tile s: S slots of BM x BN floats, each in accumulator order
         // [fragment][quad][thread] so that a wavefront moves 1 KiB per instruction
-        float* slot = p.ws + s * S * TILE_ELEMS;
-        if (!reduce_phase) {
-          float* mine = slot + (long long)chunk * TILE_ELEMS;
+        float* mine = p.ws + (s * S + chunk) * TILE_ELEMS;
 #pragma unroll
-          for (int i = 0; i < WTM; ++i)
+        for (int i = 0; i < WTM; ++i)
 #pragma unroll
-            for (int j = 0; j < WTN; ++j)
+          for (int j = 0; j < WTN; ++j)
 #pragma unroll
-              for (int vq = 0; vq < 4; ++vq) {
-                const f32x4 q = {acc[i][j][4 * vq], acc[i][j][4 * vq + 1], acc[i][j][4 * vq + 2],
-                                 acc[i][j][4 * vq + 3]};
-                *reinterpret_cast<f32x4*>(mine + ((((i * WTN + j) * 4 + vq) * kGemmThreads) + tid) * 4) = q;
-              }
-          continue;
-        }
-        for (int c = 0; c < S; ++c) {
-          const float* part = slot + (long long)c * TILE_ELEMS;
-#pragma unroll
-          for (int i = 0; i < WTM; ++i)
-#pragma unroll
-            for (int j = 0; j < WTN; ++j)
-#pragma unroll
-              for (int vq = 0; vq < 4; ++vq) {
-                const f32x4 q = *reinterpret_cast<const f32x4*>(
-                    part + ((((i * WTN + j) * 4 + vq) * kGemmThreads) + tid) * 4);
-#pragma unroll
-                for (int t = 0; t < 4; ++t) acc[i][j][4 * vq + t] += q[t];
-              }
-        }
+            for (int vq = 0; vq < 4; ++vq) {
+              const f32x4 q = {acc[i][j][4 * vq], acc[i][j][4 * vq + 1], acc[i][j][4 * vq + 2],
+                               acc[i][j][4 * vq + 3]};
+              *reinterpret_cast<f32x4*>(mine + ((((i * WTN + j) * 4 + vq) * kGemmThreads) + tid) * 4) = q;
+            }
+        continue;
       }
     }
 
@@ -1146,6 +1154,54 @@ __global__ __launch_bounds__(kGemmThreads, (BM == 128 && BN == 128) ? 2 : 1) voi
   GMOE_PROBE_WORKGROUP_END();
 }
 
+// Adds the partial tiles of a split launch (128x128 tiles of gmm_kernel, NN / NT) in order and rounds.
+// A workgroup takes a quarter of a tile, one 32x32 fragment of each of its four wavefronts, so that a
+// launch of 64 tiles reads its 32 MB on 256 CUs and not on 64 (46 -> 17 us for both launches of
+// 2048 x 2816 x 1024 over 16 experts).
+template <int DT, int ODT, int MODE>
+__global__ __launch_bounds__(kGemmThreads) void gmm_split_reduce_kernel(GmmParams p) {
+  constexpr int BM = 128, BN = 128, BK = 128 / Elem<DT>::bytes, WTN = 2, OES = Elem<ODT>::bytes;
+  constexpr long long TILE_ELEMS = (long long)BM * BN;
+  __shared__ int tile_cum[kMaxGroupsLds + 1];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave >> 1, wn = wave & 1;
+  const int64_t M = p.M;
+  const int nt_cnt = (int)((M + BN - 1) / BN), k_tiles = (int)((p.K + BK - 1) / BK);
+  const int part = resolve_row_part(p, k_tiles, tile_cum);
+  if (part == ROWS_NONE) return;
+  build_tile_cum<MODE, BM>(p, part, nt_cnt, 0, tile_cum);
+  const long long total_tiles = tile_cum[p.E];
+  const int S = split_count(p, split_us_per_k_tile(Elem<DT>::bytes), total_tiles, k_tiles, TILE_ELEMS);
+  if (S == 1) return;  // the first launch did everything
+  int e = 0;
+  for (long long item = blockIdx.x; item < total_tiles * 4; item += gridDim.x) {
+    const long long s = item / 4;
+    const int i = (int)(item & 3) / WTN, j = (int)(item & 3) % WTN;
+    while (tile_cum[e + 1] <= s) ++e;
+    long long row0 = group_begin(p, e), n_e = group_begin(p, e + 1) - row0, begin;
+    expert_row_part(n_e, part, begin, n_e);
+    row0 += begin;
+    int mt, nt;
+    strip_order(s - tile_cum[e], (int)((n_e + BM - 1) / BM), nt_cnt, mt, nt);
+    const float* slot = p.ws + s * S * TILE_ELEMS + (int64_t)(((i * WTN + j) * 4 * kGemmThreads) + tid) * 4;
+    f32x4 sum[4] = {};
+#pragma unroll 4
+    for (int c = 0; c < S; ++c)
+#pragma unroll
+      for (int vq = 0; vq < 4; ++vq)
+        sum[vq] += *reinterpret_cast<const f32x4*>(slot + c * TILE_ELEMS + vq * kGemmThreads * 4);
+    const int64_t m = (int64_t)mt * BM + wm * 64 + i * 32 + (lane & 31);
+    if (m >= n_e) continue;
+#pragma unroll
+    for (int vq = 0; vq < 4; ++vq) {
+      const int64_t n = (int64_t)nt * BN + wn * 64 + j * 32 + 8 * vq + 4 * (lane >> 5);
+      if (n >= M) continue;
+      unsigned char* dst = p.c + ((row0 + m) * M + n) * OES;
+      if (ODT == GMOE_F32) *reinterpret_cast<f32x4*>(dst) = sum[vq];
+      else *reinterpret_cast<u32x2*>(dst) = pack4<ODT>(sum[vq][0], sum[vq][1], sum[vq][2], sum[vq][3]);
+    }
+  }
+}
+
 // Persistent grid: blocks_per_cu workgroups per CU, a multiple of 8 (one share per XCD).
 static int gmm_grid(int blocks_per_cu) {
   const int grid = (gmoe_cu_count() / 8) * 8 * blocks_per_cu;
@@ -1242,12 +1298,30 @@ static inline bool gmm_use_remainder(const GmmParams& p) {
   return p.N / (p.E > 0 ? p.E : 1) >= kRemainderMinRows;
 }
 
-// A 128x128-tile NN / NT launch whose tiles (an upper bound from the host-side sizes) fill at most
-// half of those slots while every tile walks at least 16 K tiles: worth a split into two phases.
-static inline bool gmm_few_tiles_long_k(const GmmParams& p) {
-  const int64_t row_tiles = (p.N + 127) / 128 + p.E;  // every expert may end in a partial tile
-  const int64_t tiles = row_tiles * ((p.M + 127) / 128);
-  return tiles * 2 <= kSplitSlots && p.K >= 1024;
+// Whether a 128x128-tile NN / NT launch is worth a split reduction, from the host-side sizes (an expert
+// has at least one row tile, and its last one is half full on average); the kernels decide again from the
+// tiles there are.
+static inline bool gmm_split_pays(const GmmParams& p, int dtype) {
+  const int es = dtype == GMOE_F32 ? 4 : 2;
+  const int64_t least = p.N < p.E ? p.N : p.E, average = (p.N + 127) / 128 + p.E / 2;
+  const int64_t tiles = (average > least ? average : least) * ((p.M + 127) / 128);
+  return split_pieces(split_us_per_k_tile(es), (p.K * es + 127) / 128, tiles, kSplitSlots,
+                      weight_stream_us(p.E, p.K, p.M, es)) > 1;
+}
+
+// A split launch with 128x128 tiles: the pieces, then their sums.
+template <int DT, int ODT, int MODE>
+static int launch_gmm_split(const GmmParams& p, hipStream_t st) {
+  GmmParams r = p;
+  const int64_t slots = p.ws_floats / (128 * 128);
+  r.split_slots = (int)(slots < kSplitSlots ? slots : kSplitSlots);
+  // the rows left to a remainder launch belong to some of the experts only: no bound from their weights
+  r.stream_us = p.row_part == ROWS_ALL ? weight_stream_us(p.E, p.K, p.M, Elem<DT>::bytes) : 0.f;
+  const int rc = launch_gmm_cfg<DT, ODT, MODE, 128, 128, EPI_NONE>(r, st, 2);
+  if (rc != GMOE_OK) return rc;
+  // at most split_slots / 2 tiles are split, four quarters each
+  hipLaunchKernelGGL((gmm_split_reduce_kernel<DT, ODT, MODE>), dim3(2 * r.split_slots), dim3(kGemmThreads), 0, st, r);
+  return gmoe_launch_status();
 }
 
 // The launch with 128-row tiles for the rows a ROWS_MAIN launch leaves out.
@@ -1257,14 +1331,7 @@ static int launch_gmm_remainder(const GmmParams& p, hipStream_t st) {
   r.row_part = ROWS_AUTO_REMAINDER;
   if (p.ws == nullptr || p.ws_floats < 2 * 128 * 128)
     return launch_gmm_cfg<DT, ODT, MODE, 128, 128, EPI_NONE>(r, st, 2);
-  // few tiles, each with the whole reduction: split it over the idle CUs, then add the pieces
-  const int64_t slots = p.ws_floats / (128 * 128);
-  r.split_slots = (int)(slots < kSplitSlots ? slots : kSplitSlots);
-  r.phase = SPLIT_PARTIAL;
-  const int rc = launch_gmm_cfg<DT, ODT, MODE, 128, 128, EPI_NONE>(r, st, 2);
-  if (rc != GMOE_OK) return rc;
-  r.phase = SPLIT_REDUCE;
-  return launch_gmm_cfg<DT, ODT, MODE, 128, 128, EPI_NONE>(r, st, 2);
+  return launch_gmm_split<DT, ODT, MODE>(r, st);  // few tiles, each with the whole reduction
 }
 
 // One kernel per (type, mode, size).  Groups large enough for 256x256 tiles (TFLOP/s measured on the
@@ -1320,17 +1387,8 @@ static int launch_gmm_mode(const GmmParams& p, int dtype, int out_dtype, hipStre
     return GMOE_ERR_UNSUPPORTED;  // the caller runs the GEMM and the activation kernel instead
   } else {
     if constexpr (MODE != MODE_TN && EPI == EPI_NONE) {
-      if (gmm_few_tiles_long_k(p) && p.ws != nullptr && p.ws_floats >= 2 * 128 * 128) {
-        // fewer tiles than workgroup slots and a long reduction: split it (see SPLIT_PARTIAL)
-        GmmParams r = p;
-        const int64_t slots = p.ws_floats / (128 * 128);
-        r.split_slots = (int)(slots < kSplitSlots ? slots : kSplitSlots);
-        r.phase = SPLIT_PARTIAL;
-        const int rc = launch_gmm_cfg<DT, ODT, MODE, 128, 128, EPI_NONE>(r, st, 2);
-        if (rc != GMOE_OK) return rc;
-        r.phase = SPLIT_REDUCE;
-        return launch_gmm_cfg<DT, ODT, MODE, 128, 128, EPI_NONE>(r, st, 2);
-      }
+      if (p.ws != nullptr && p.ws_floats >= 2 * 128 * 128 && gmm_split_pays(p, dtype))
+        return launch_gmm_split<DT, ODT, MODE>(p, st);
     }
     return launch_gmm_cfg<DT, ODT, MODE, 128, 128, EPI>(p, st, 2);
   }
@@ -1401,7 +1459,7 @@ static int gmm_check(GmmParams& p, const void* a, const void* b, void* c, const 
   p.ws = nullptr;
   p.ws_floats = 0;
   p.split_slots = 0;
-  p.phase = SPLIT_OFF;
+  p.stream_us = 0.f;
   p.main_grid = 0;
   return GMOE_OK;
 }
@@ -1419,14 +1477,14 @@ int gmm_dense(const void* a, const void* b, void* c, int64_t N, int64_t K, int64
   return gmm_dispatch(p, mode, dtype, out_dtype, EPI_NONE, st);
 }
 
-int64_t gmm_dense_workspace_floats(int64_t N, int64_t K, int64_t M, int mode) {
+int64_t gmm_dense_workspace_floats(int64_t N, int64_t K, int64_t M, int mode, int dtype) {
   if (mode == MODE_TN || N < 1) return 0;
   GmmParams p;
   p.E = 1;
   p.N = N;
   p.K = K;
   p.M = M;
-  const bool split = (gmm_large_tiles(p, mode) && gmm_use_remainder(p)) || gmm_few_tiles_long_k(p);
+  const bool split = (gmm_large_tiles(p, mode) && gmm_use_remainder(p)) || gmm_split_pays(p, dtype);
   return split ? (int64_t)kSplitSlots * 128 * 128 : 0;
 }
 
@@ -1451,7 +1509,7 @@ extern "C" int64_t gmoe_gmm_workspace_bytes(int E, int64_t N, int64_t K, int64_t
   p.K = K;
   p.M = M;
   const int mode = trans_b ? MODE_NT : MODE_NN;
-  const bool split = (gmm_large_tiles(p, mode) && gmm_use_remainder(p)) || gmm_few_tiles_long_k(p);
+  const bool split = (gmm_large_tiles(p, mode) && gmm_use_remainder(p)) || gmm_split_pays(p, dtype);
   return split ? (int64_t)kSplitSlots * 128 * 128 * 4 : 0;
 }
 

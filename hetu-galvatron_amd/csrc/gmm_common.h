@@ -72,11 +72,11 @@ struct GmmParams {
   const unsigned char* a_scale;  // fp8 activations: power-of-two row scales, dwords [K/128][N]
   int row_part;              // NN / NT: which rows of every expert this launch covers (ROWS_*)
   int64_t F;
-  // split reduction of a launch with few tiles (see SPLIT_* in gmm.hip): fp32 partial tiles
+  // split reduction of a launch with few tiles (see split_count in gmm.hip): fp32 partial tiles
   float* ws;
   int64_t ws_floats;
   int split_slots;           // tiles x splits this launch may spread over; 0 = never split
-  int phase;                 // SPLIT_OFF, SPLIT_PARTIAL, SPLIT_REDUCE
+  float stream_us;           // time the weights take to stream: a split launch cannot be faster
   int main_grid;             // ROWS_AUTO_*: workgroups of the launch with 256-row tiles
 };
 // First row of group e.  A null offset table means one group holding all N rows (dense GEMM on the
@@ -84,7 +84,6 @@ struct GmmParams {
 __device__ __forceinline__ long long group_begin(const GmmParams& p, int e) {
   return p.offsets ? p.offsets[e] : (e > 0 ? (long long)p.N : 0ll);
 }
-enum { SPLIT_OFF = 0, SPLIT_PARTIAL = 1, SPLIT_REDUCE = 2 };
 constexpr int kMaxSplit = 8;
 
 // A launch with 256-row tiles leaves an expert's last n % 256 rows, when they are at most kRemRows,
@@ -253,11 +252,11 @@ bool gmm_fp8_skinny_applies(const GmmParams& p, bool any_row_count = false);
 // One dense product on the grouped kernels (gmm.hip): a single group of all N rows, no offset
 // table.  mode MODE_NN: c [N,M] = a [N,K] @ b [K,M]; MODE_NT: c = a @ b^T with b [M,K]; MODE_TN:
 // c [K,M] = a^T @ b with a [N,K], b [N,M].  K and M multiples of 8.
-// ws / ws_floats: optional fp32 workspace of gmm_dense_workspace_floats(N, K, M, mode) floats; with
+// ws / ws_floats: optional fp32 workspace of gmm_dense_workspace_floats(N, K, M, mode, dtype) floats; with
 // it an NN / NT product with few output tiles and a long reduction is split over the idle CUs.
 int gmm_dense(const void* a, const void* b, void* c, int64_t N, int64_t K, int64_t M, int mode,
               int dtype, int out_dtype, hipStream_t st, float* ws = nullptr, int64_t ws_floats = 0);
-int64_t gmm_dense_workspace_floats(int64_t N, int64_t K, int64_t M, int mode);
+int64_t gmm_dense_workspace_floats(int64_t N, int64_t K, int64_t M, int mode, int dtype);
 
 // c [groups][K,M] = a_g^T @ b_g over the row ranges [offsets[g], offsets[g+1]) of a [N,K] and
 // b [N,M] (offsets: groups + 1 device values): the grouped weight-gradient product, also used to cut
