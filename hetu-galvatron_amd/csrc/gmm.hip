@@ -1276,18 +1276,19 @@ static inline bool gmm_rows_pays(const GmmParams& p, int mode, int epi) {
   return n >= 128 && n < 512;
 }
 
-// dW of 16-bit operands with a short reduction (gmm_tn.hip: 128x256 tiles, two workgroups per CU) against
-// the 256x256 LDS-DMA kernel, or 128x128 tiles where that one does not apply; n = rows per expert, us on
-// both sides: n 48: 302 -> 192 (14336 x 4096, 8 experts), 587 -> 381 (7168 x 4096, 32); n 384: 1098 -> 995
-// (4096 x 28672, 8), 107 -> 77 (1024 x 5632, 16); n 768: 342 -> 305 (1408 x 2048, 64), but 1573 -> 1591
-// (4096 x 28672); n 1024: 1884 -> 1935 (7168 x 4096): the operand traffic of the smaller tile takes over.
-// (Small outputs gain beyond that, n 1024: 417 -> 380 for 1408 x 2048, but with shared experts on a
-// second stream that step lost 0.6 %.)  With fewer than three quarters of a tile per CU the 128x128
-// tiles spread better (128 tiles of 1024 x 512: 13 -> 15).
+// dW of 16-bit operands with a short reduction and few output tiles (gmm_tn.hip: 128x256 tiles, two
+// workgroups per CU) against the 256x256 LDS-DMA kernel, or 128x128 tiles where that one does not apply;
+// n = rows per expert, us on both sides.  From one round of 256x256 tiles on that kernel, whose tiles run
+// into each other, is the faster one at any n: n 383: 911 against 999 (4096 x 28672, 8 experts), n 256:
+// 213 against 240 (2048 x 4096, 32), n 640: 65 against 65 (2816 x 1024, 16).  Below that, and where its rows
+// would be padding (K under 512), the smaller tiles spread better: 128 tiles of 256x256, 20 -> 15
+// (1024 x 1024, 8), 240: 16.3 -> 15.1 (640 x 1280, 16), 384 x 4096 over 64 experts 120 -> 110.  More than
+// 768 rows are left to the 256x256 tiles (n 1024: 1884 against 1935), fewer than three quarters of a tile
+// per CU to 128x128 ones (128 tiles of 1024 x 512: 13 against 15).
 static inline bool gmm_tn_short_pays(const GmmParams& p) {
-  const int64_t n = p.N / (p.E > 0 ? p.E : 1);
-  const int64_t tiles = p.E * ((p.K + 127) / 128) * ((p.M + 255) / 256);
-  if (p.K < 128 || p.M < 256 || tiles * 4 < gmm_grid(1) * 3) return false;
+  const int64_t n = p.N / (p.E > 0 ? p.E : 1), col_tiles = (p.M + 255) / 256;
+  if (p.K < 128 || p.M < 256 || p.E * ((p.K + 127) / 128) * col_tiles * 4 < gmm_grid(1) * 3) return false;
+  if (p.K >= 512 && p.E * ((p.K + 255) / 256) * col_tiles >= gmm_grid(1)) return false;
   return n <= 768;
 }
 

@@ -14,6 +14,12 @@
 //     issued while tile t is multiplied, i.e. a request has about three tiles of MFMAs to land.
 //     One barrier per K tile; the copies are tracked by hand (vmcnt), the compiler tracks the
 //     LDS reads.
+//   * The K tiles of all of a workgroup's output tiles form one sequence: the last three of a tile
+//     request the first three of the next, and the stores of a tile are left in flight under the next
+//     tile's MFMAs.  Before, each tile waited for its first copies and for its stores with idle matrix
+//     cores, about 10 us of 36 at 1024 rows per expert: dW of 7168 x 4096 over 32 experts 1930 -> 1752 us
+//     (1098 TFLOP/s), 2048 x 2816 over 64 786 -> 707, 1408 x 2048 over 64 433 -> 393; with 4096 rows per
+//     expert the launches are bound by the chip's power and unchanged (6050 us).
 //   * Both operands have the reduction index (the token) as the slow dimension in memory; they are
 //     stored in LDS as they are in memory, [k][outer], and the MFMA fragments are read with the
 //     transposing LDS load ds_read_b64_tr_b16: a group of 16 lanes reads a 4(k) x 16(outer) block
@@ -39,18 +45,15 @@ typedef short s16x4 __attribute__((ext_vector_type(4)));
 // ---- operand stored outer-contiguous: LDS tile [32 k][256 outer], 512 bytes per k row ----------
 // The 64-byte segment sg of row k sits at segment position sg ^ f(k), f(k) = (k & 3) | ((k >> 1) & 4):
 // the 8 rows one transposing read touches (k0..k0+3 and k0+8..k0+11) land in 8 different segments.
+// What a lane needs of an operand whatever the output tile; the tile itself is a buffer resource.
 struct TransOperand {
-  u32x4 rsrc;
   uint32_t voff[4];
-  uint32_t row_bytes;
+  uint32_t stage_bytes;  // global bytes between consecutive K tiles
   uint32_t frag_k;       // byte offset of the lane's first k row
   uint32_t frag_seg[4];  // byte offset of the lane's 8 bytes inside a k row, per fragment
 
-  // src: the expert's operand (row 0 = first reduction index); the tile starts at outer index o0.
-  __device__ __forceinline__ void init(const unsigned char* src, int64_t ld, int64_t o0,
-                                       int64_t k_limit, int wave, int lane, int sub_col0) {
-    rsrc = make_raw_rsrc(src + o0 * 2, k_limit * ld * 2 - o0 * 2);
-    row_bytes = (uint32_t)(ld * 2);
+  __device__ __forceinline__ void init(int64_t ld, int wave, int lane, int sub_col0) {
+    stage_bytes = (uint32_t)(ld * 2 * BKT);
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const int krow = (wave * 4 + q) * 2 + (lane >> 5);
@@ -68,10 +71,14 @@ struct TransOperand {
       frag_seg[j] = (uint32_t)((((seg0 + j) ^ f) * 64) + half * 32 + (s & 3) * 8);
     }
   }
+  // Offset of K tile kt inside the resource, clamped to its end: whole K tiles past the last row read as zero.
+  __device__ __forceinline__ uint32_t offset(const u32x4& rsrc, int kt) const {
+    const uint64_t o = (uint64_t)(uint32_t)kt * stage_bytes;
+    return o < rsrc[2] ? (uint32_t)o : rsrc[2];
+  }
   template <int q>
-  __device__ __forceinline__ void issue(int kt, uint32_t lds_tile, int wave) const {
-    dma16(lds_tile + (uint32_t)((wave * 4 + q) * 1024), voff[q], rsrc,
-          (uint32_t)(kt * BKT) * row_bytes);
+  __device__ __forceinline__ void issue(const u32x4& rsrc, uint32_t off, uint32_t lds_tile, int wave) const {
+    dma16(lds_tile + (uint32_t)((wave * 4 + q) * 1024), voff[q], rsrc, off);
   }
   static constexpr int READS_PER_FRAG = 2;
   // half h (4 of the 8 k values) of fragment j of K step ks
@@ -86,14 +93,34 @@ struct TransOperand {
   }
 };
 
+// An accumulator element, read where it is used: left to the compiler, all 256 are copied to the vector
+// registers at the head of the epilogue, which do not hold them beside the next tile's fragments.
+__device__ __forceinline__ float acc_read(float a) {
+  float v;
+  asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v) : "a"(a));
+  return v;
+}
+
+// One stretch of a workgroup's work: the reduction rows of one output tile, or of one segment of them (a
+// buffer resource spans at most 2 GiB; an expert with more rows is walked in segments, the accumulators
+// carried across).
+struct Work {
+  u32x4 ra, rb;  // the operands' rows, from the tile's first column on
+  int kt_cnt;    // K tiles, at least NST - 1: the copies reach one stretch ahead, never two
+  int e, mt, nt; // e < 0: none left
+  bool last;     // the tile's last stretch
+};
+
 template <int DT, int ODT>
 __global__ __launch_bounds__(kGemmThreads) void gmm_dtl_kernel(GmmParams p) {
   typedef TransOperand OpA;
   typedef TransOperand OpB;
+  typedef __attribute__((address_space(4))) const long long const_i64;
   constexpr int WT = 4;   // 32x32 accumulators per wavefront in each direction
   constexpr int NM = 16;  // MFMAs per K step
   constexpr int RA = OpA::READS_PER_FRAG, RB = OpB::READS_PER_FRAG;
   constexpr int NREAD = WT * RA + WT * RB;  // LDS reads per K step
+  constexpr int STORES = ODT == GMOE_F32 ? 0 : 32;  // result stores of a tile left in flight, per wavefront
   static_assert(NREAD == NM && LOADS_PER_TILE == NM / 2, "one read per MFMA, a copy after every fourth");
 
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
@@ -109,83 +136,113 @@ __global__ __launch_bounds__(kGemmThreads) void gmm_dtl_kernel(GmmParams p) {
   const int nt_cnt = (int)((M + BN - 1) / BN);
   const int mt_cnt = (int)((K + BM - 1) / BM);
 
-  // every expert has the same mt_cnt x nt_cnt grid of output tiles
-  const long long per_expert = (long long)mt_cnt * nt_cnt;
-  const long long total_tiles = per_expert * E;
+  // every expert has the same mt_cnt x nt_cnt grid of output tiles (32-bit: the output they tile is memory)
+  const int per_expert = mt_cnt * nt_cnt;
+  const int total_tiles = per_expert * E;
   // workgroup w runs on XCD w % 8: XCD x takes the positions [x*G/8, (x+1)*G/8) of every whole round
   // of G = gridDim.x tiles; the last, partial round is dealt to the XCDs in equal consecutive shares
   const int G = gridDim.x;
   const int xcd = blockIdx.x % 8, slot = blockIdx.x / 8;
-  const long long whole = total_tiles / G * G;  // tiles in whole rounds
-  auto tail_tile = [&]() -> long long {
-    const long long share = (total_tiles - whole + 7) / 8;
-    const long long t = whole + xcd * share + slot;
+  const int whole = total_tiles / G * G;  // tiles in whole rounds
+  auto tail_tile = [&]() -> int {
+    const int share = (total_tiles - whole + 7) / 8;
+    const int t = whole + xcd * share + slot;
     return (slot < share && t < total_tiles) ? t : -1;
   };
-  const long long first = (long long)xcd * (G / 8) + slot;
+  const int first = xcd * (G / 8) + slot;
+  const int64_t seg_rows = tn_segment_rows(K, M, 2);
 
-  for (long long s = first < whole ? first : tail_tile(); s >= 0;
-       s = s >= whole ? -1 : (s + G < whole ? s + G : tail_tile())) {
-    const int e = (int)(s / per_expert);
-    const long long row0 = group_begin(p, e);
-    const long long n_e = group_begin(p, e + 1) - row0;
-    int mt, nt;
-    strip_order(s - e * per_expert, mt_cnt, nt_cnt, mt, nt);
+  OpA oa;
+  OpB ob;
+  oa.init(K, wave, lane, wm * 128);
+  ob.init(M, wave, lane, wn * 128);
 
-    f32x16 acc[WT][WT];
+  int s = first < whole ? first : tail_tile();  // the tile and segment `fetch` takes next
+  int64_t seg0 = 0;
+  auto fetch = [&](Work& w) {
+    if (s < 0) {
+      w.ra = w.rb = make_raw_rsrc(p.a, 0);
+      w.e = -1;
+      return;
+    }
+    const int e = s / per_expert;
+    // scalar loads: a vector load's wait would drain the copies in flight
+    const_i64* off = (const_i64*)(p.offsets);
+    const long long row0 = off ? off[e] : 0, n_e = (off ? off[e + 1] : (long long)p.N) - row0;
+    const int q = s - e * per_expert, strip = q / (mt_cnt * kStripTiles), rem = q - strip * mt_cnt * kStripTiles;
+    const int n0 = strip * kStripTiles, width = nt_cnt - n0 < kStripTiles ? nt_cnt - n0 : kStripTiles;
+    w.e = e;
+    w.mt = rem / width;
+    w.nt = n0 + rem % width;
+    const int64_t left = n_e - seg0, k_lim = left < seg_rows ? left : seg_rows;
+    w.ra = make_raw_rsrc(p.a + ((row0 + seg0) * K + (int64_t)w.mt * BM) * 2, (k_lim * K - (int64_t)w.mt * BM) * 2);
+    w.rb = make_raw_rsrc(p.b + ((row0 + seg0) * M + (int64_t)w.nt * BN) * 2, (k_lim * M - (int64_t)w.nt * BN) * 2);
+    const int kt = (int)((k_lim + BKT - 1) / BKT);
+    w.kt_cnt = kt < NST - 1 ? NST - 1 : kt;
+    w.last = left <= seg_rows;
+    if (w.last) {
+      s = s >= whole ? -1 : (s + G < whole ? s + G : tail_tile());
+      seg0 = 0;
+    } else {
+      seg0 += seg_rows;
+    }
+  };
+
+  f32x16 acc[WT][WT];
+  auto clear = [&]() {
 #pragma unroll
     for (int i = 0; i < WT; ++i)
 #pragma unroll
       for (int j = 0; j < WT; ++j)
 #pragma unroll
         for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+  };
+  u32x4 fa[2][WT], fb[2][WT];
+  // read operation r of K step ks of the tile at `stage` into fragment buffer `buf`
+  auto frag_read = [&](auto r_c, auto ks_c, auto buf_c, const unsigned char* stage) {
+    constexpr int r = decltype(r_c)::value, ks = decltype(ks_c)::value, buf = decltype(buf_c)::value;
+    if constexpr (r < WT * RA) {
+      oa.template read<r / RA, ks, r % RA>(stage, fa[buf][r / RA]);
+    } else {
+      constexpr int rb = r - WT * RA;
+      ob.template read<rb / RB, ks, rb % RB>(stage + OPER_BYTES, fb[buf][rb / RB]);
+    }
+  };
 
-    // a buffer resource spans at most 2 GiB: an expert with more rows than that is walked in
-    // segments (one segment in all but extreme cases), the accumulators carried across
-    const int64_t seg_rows = tn_segment_rows(K, M, 2);
-    for (int64_t seg0 = 0; seg0 < n_e; seg0 += seg_rows) {
-    OpA oa;
-    OpB ob;
-    const int64_t k_lim = n_e - seg0 < seg_rows ? n_e - seg0 : seg_rows;
-    oa.init(p.a + (row0 + seg0) * K * 2, K, (int64_t)mt * BM, k_lim, wave, lane, wm * 128);
-    ob.init(p.b + (row0 + seg0) * M * 2, M, (int64_t)nt * BN, k_lim, wave, lane, wn * 128);
+  Work cur;
+  fetch(cur);
+  if (cur.e < 0) return;
+  // ---- prologue, once per workgroup: K tiles 0..2 in flight, wait for tile 0, fragments of its step 0
+  static_for<0, NST - 1>([&](auto t_c) {
+    constexpr int t = decltype(t_c)::value;
+    const uint32_t st = lds0 + t * STAGE_BYTES, offa = oa.offset(cur.ra, t), offb = ob.offset(cur.rb, t);
+    static_for<0, 4>([&](auto q) { oa.template issue<decltype(q)::value>(cur.ra, offa, st, wave); });
+    static_for<0, 4>([&](auto q) { ob.template issue<decltype(q)::value>(cur.rb, offb, st + OPER_BYTES, wave); });
+  });
+  wait_dma_outstanding<2 * LOADS_PER_TILE>();
+  __syncthreads();
+  static_for<0, NREAD>([&](auto r) {
+    frag_read(r, std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{}, lds);
+  });
 
-    const int kt_cnt = (int)((k_lim + BKT - 1) / BKT);
-    u32x4 fa[2][WT], fb[2][WT];
-
-    // copy K tile kt into its stage (all 8 instructions of this wavefront)
-    auto issue_tile = [&](int kt) {
-      const uint32_t st = lds0 + (uint32_t)((kt & (NST - 1)) * STAGE_BYTES);
-      static_for<0, 4>([&](auto q) { oa.template issue<decltype(q)::value>(kt, st, wave); });
-      static_for<0, 4>(
-          [&](auto q) { ob.template issue<decltype(q)::value>(kt, st + OPER_BYTES, wave); });
-    };
-    // read operation r of K step ks of the tile at `stage` into fragment buffer `buf`
-    auto frag_read = [&](auto r_c, auto ks_c, auto buf_c, const unsigned char* stage) {
-      constexpr int r = decltype(r_c)::value, ks = decltype(ks_c)::value, buf = decltype(buf_c)::value;
-      if constexpr (r < WT * RA) {
-        oa.template read<r / RA, ks, r % RA>(stage, fa[buf][r / RA]);
-      } else {
-        constexpr int rb = r - WT * RA;
-        ob.template read<rb / RB, ks, rb % RB>(stage + OPER_BYTES, fb[buf][rb / RB]);
-      }
-    };
-
-    if (kt_cnt > 0) {
-      // ---- prologue: tiles 0..2 in flight, wait for tile 0, fragments of its step 0 ------------
-      issue_tile(0);
-      issue_tile(1);
-      issue_tile(2);
-      wait_dma_outstanding<2 * LOADS_PER_TILE>();
-      __syncthreads();
-      static_for<0, NREAD>([&](auto r) {
-        frag_read(r, std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{}, lds);
-      });
-
-      for (int kt = 0; kt < kt_cnt; ++kt) {
-        const unsigned char* cur = lds + (kt & (NST - 1)) * STAGE_BYTES;
-        const unsigned char* nxt = lds + ((kt + 1) & (NST - 1)) * STAGE_BYTES;
-        const uint32_t st3 = lds0 + (uint32_t)(((kt + 3) & (NST - 1)) * STAGE_BYTES);
+  // The K tiles of all stretches form one sequence through the NST stages: the last three of a stretch
+  // request the first three of the next, so that neither the first copies of a tile nor the stores of the
+  // tile before are waited for with idle matrix cores.
+  bool stored = false;  // the tile before left its STORES in flight
+  int g = 0;            // K tiles done, all stretches
+  for (;;) {
+    Work nx;
+    clear();
+    for (;;) {
+      fetch(nx);
+      for (int kt = 0; kt < cur.kt_cnt; ++kt, ++g) {
+        const unsigned char* here = lds + (g & (NST - 1)) * STAGE_BYTES;
+        const unsigned char* nxt = lds + ((g + 1) & (NST - 1)) * STAGE_BYTES;
+        const uint32_t st3 = lds0 + (uint32_t)(((g + 3) & (NST - 1)) * STAGE_BYTES);
+        const bool own = kt + 3 < cur.kt_cnt;
+        const int kt3 = own ? kt + 3 : kt + 3 - cur.kt_cnt;
+        const u32x4 ra = own ? cur.ra : nx.ra, rb = own ? cur.rb : nx.rb;
+        const uint32_t offa = oa.offset(ra, kt3), offb = ob.offset(rb, kt3);
         // ---- K step 0: MFMAs on buffer 0; read step 1 into buffer 1; request a of tile kt+3 ---
         // One fragment read per MFMA and a copy after every fourth: the stage of tile kt-1 is free for
         // both steps, and copies spread over both are 1-2 % faster than all eight at the end of this
@@ -196,14 +253,15 @@ __global__ __launch_bounds__(kGemmThreads) void gmm_dtl_kernel(GmmParams p) {
           constexpr int mi = m / WT, mj = (mi & 1) ? WT - 1 - m % WT : m % WT;
           Mma<DT>::run(fa[0][mi], fb[0][mj], acc[mi][mj]);
           GMOE_SCHED_FENCE();
-          frag_read(m_c, std::integral_constant<int, 1>{}, std::integral_constant<int, 1>{}, cur);
-          if constexpr (m % 4 == 2) oa.template issue<m / 4>(kt + 3, st3, wave);
-
+          frag_read(m_c, std::integral_constant<int, 1>{}, std::integral_constant<int, 1>{}, here);
+          if constexpr (m % 4 == 2) oa.template issue<m / 4>(ra, offa, st3, wave);
           GMOE_SCHED_FENCE();
         });
-        // tile kt+1 must have landed (kt+2 and the half of kt+3 may still be in flight); the barrier
-        // also tells everyone that this tile's stage has been read for the last time
-        wait_dma_outstanding<LOADS_PER_TILE + 4>();
+        // tile kt+1 must have landed (kt+2 and the half of kt+3 may still be in flight, and for the first
+        // two tiles of a stretch the stores issued between their requests); the barrier also tells everyone
+        // that this tile's stage has been read for the last time
+        if (stored && kt < 2) wait_dma_outstanding<LOADS_PER_TILE + 4 + STORES>();
+        else wait_dma_outstanding<LOADS_PER_TILE + 4>();
         __syncthreads();
         GMOE_SCHED_FENCE();
         // ---- K step 1: MFMAs on buffer 1; read step 0 of tile kt+1 into buffer 0; request b of kt+3
@@ -214,64 +272,87 @@ __global__ __launch_bounds__(kGemmThreads) void gmm_dtl_kernel(GmmParams p) {
           Mma<DT>::run(fa[1][mi], fb[1][mj], acc[mi][mj]);
           GMOE_SCHED_FENCE();
           frag_read(m_c, std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{}, nxt);
-          if constexpr (m % 4 == 2) ob.template issue<m / 4>(kt + 3, st3 + OPER_BYTES, wave);
+          if constexpr (m % 4 == 2) ob.template issue<m / 4>(rb, offb, st3 + OPER_BYTES, wave);
           GMOE_SCHED_FENCE();
         });
       }
-      // every copy has landed and every wavefront is done with LDS before the next tile reuses it
-      wait_dma_outstanding<0>();
-      __syncthreads();
+      if (cur.last) break;
+      stored = false;
+      cur = nx;
     }
-    }
+    stored = STORES > 0;
 
     // ---- epilogue: lane holds row (lane%32), columns 8*(v/4) + 4*(lane/32) + v%4 of each 32x32 ----
     constexpr int OES = Elem<ODT>::bytes;
-    unsigned char* c_base = p.c + (int64_t)e * K * M * OES;
-    const int64_t c_rows = K;
+    unsigned char* c_tile = p.c + ((int64_t)cur.e * K + (int64_t)cur.mt * BM) * M * OES;
+    const int64_t c_rows = K - (int64_t)cur.mt * BM;
     if constexpr (ODT != GMOE_F32) {
-      using CT = CTile<BN>;
-      stage_acc_lds<ODT, WT, WT, BN>(lds, acc, wm * 128, wn * 128, lane);
-      __syncthreads();
-      const int cc = tid % CT::chunks, r0 = tid / CT::chunks;
-      const int64_t n = (int64_t)nt * BN + cc * 8;
-#pragma unroll 8
-      for (int it = 0; it < BM / CT::rows_per_pass; ++it) {
-        const int row = it * CT::rows_per_pass + r0;
-        const int64_t m = (int64_t)mt * BM + row;
-        if (m < c_rows && n < M)
-          st16(c_base + (m * M + n) * OES, ctile_read16(lds + row * CT::pitch + cc * 16));
-      }
-      __syncthreads();  // the next tile's copies overwrite the staged values
-      continue;
-    }
+      // 32 rows x 128 columns at a time through the wavefront's own 2 x 4 KiB of the stage that was read
+      // last: the pieces its own copies fill next, so no barrier is needed.  The 16-byte piece c of row r
+      // sits in slot c ^ (r & 15).  The buffer stores carry no condition (rows and columns that do not
+      // exist are out of the resource), so STORES of them are in flight.
+      unsigned char* mine = lds + ((g - 1) & (NST - 1)) * STAGE_BYTES + wave * 4096;
+      const auto rc = __builtin_amdgcn_make_buffer_rsrc(
+          c_tile, 0, (int)((c_rows < BM ? c_rows : BM) * M * OES), 0x00020000);
+      asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // the last MFMA's result, read by acc_read
+      GMOE_SCHED_FENCE();
+      int ln = lane;
+      asm volatile("" : "+v"(ln));  // the addresses below are computed here, not kept through the main loop
+      const int64_t n = (int64_t)cur.nt * BN + wn * 128 + (ln & 15) * 8;
+      uint32_t vo = n < M ? (uint32_t)(((wm * 128 + (ln >> 4)) * M + n) * OES) : kOob;
+      const uint32_t four_rows = (uint32_t)(4 * M * OES);
+      const int r = ln & 31;
+      unsigned char* w = mine + (r >> 4) * OPER_BYTES + (r & 15) * 256 + 8 * (ln >> 5);
 #pragma unroll
-    for (int i = 0; i < WT; ++i) {
-      const int64_t m = (int64_t)mt * BM + wm * 128 + i * 32 + (lane & 31);
-      if (m >= c_rows) continue;
+      for (int i = 0; i < WT; ++i) {
 #pragma unroll
-      for (int j = 0; j < WT; ++j) {
+        for (int j = 0; j < WT; ++j)
 #pragma unroll
-        for (int vq = 0; vq < 4; ++vq) {
-          const int64_t n = (int64_t)nt * BN + wn * 128 + j * 32 + 8 * vq + 4 * (lane >> 5);
-          if (n >= M) continue;
-          unsigned char* dst = c_base + (m * M + n) * OES;
-          const float v0 = acc[i][j][4 * vq], v1 = acc[i][j][4 * vq + 1];
-          const float v2 = acc[i][j][4 * vq + 2], v3 = acc[i][j][4 * vq + 3];
-          if (ODT == GMOE_F32)
-            *reinterpret_cast<f32x4*>(dst) = f32x4{v0, v1, v2, v3};
-          else
-            *reinterpret_cast<u32x2*>(dst) = pack4<ODT>(v0, v1, v2, v3);
+          for (int vq = 0; vq < 4; ++vq)
+            *reinterpret_cast<u32x2*>(w + ((j * 4 + vq) ^ (r & 15)) * 16) =
+                pack4<ODT>(acc_read(acc[i][j][4 * vq]), acc_read(acc[i][j][4 * vq + 1]),
+                           acc_read(acc[i][j][4 * vq + 2]), acc_read(acc[i][j][4 * vq + 3]));
+        GMOE_SCHED_FENCE();
+        u32x4 v[8];
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+          const int row = t * 4 + (ln >> 4);
+          v[t] = *reinterpret_cast<const u32x4*>(mine + (row >> 4) * OPER_BYTES + (row & 15) * 256 +
+                                                 (((ln & 15) ^ (row & 15)) * 16));
         }
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+          __builtin_amdgcn_raw_buffer_store_b128(v[t], rc, (int)vo, 0, 0);
+          vo += four_rows;
+        }
+        GMOE_SCHED_FENCE();
       }
+    } else {
+#pragma unroll
+      for (int i = 0; i < WT; ++i) {
+        const int64_t m = wm * 128 + i * 32 + (lane & 31);
+        if (m >= c_rows) continue;
+#pragma unroll
+        for (int j = 0; j < WT; ++j)
+#pragma unroll
+          for (int vq = 0; vq < 4; ++vq) {
+            const int64_t n = (int64_t)cur.nt * BN + wn * 128 + j * 32 + 8 * vq + 4 * (lane >> 5);
+            if (n < M)
+              *reinterpret_cast<f32x4*>(c_tile + (m * M + n) * OES) =
+                  f32x4{acc[i][j][4 * vq], acc[i][j][4 * vq + 1], acc[i][j][4 * vq + 2], acc[i][j][4 * vq + 3]};
+          }
+      }
+      wait_dma_outstanding<0>();  // an unknown number of stores: the counted waits start anew
     }
+    if (nx.e < 0) break;
+    cur = nx;
   }
+  wait_dma_outstanding<0>();  // nothing may land in LDS after the workgroup has ended
 }
 
 template <int DT, int ODT>
 static int launch_cfg(const GmmParams& p, hipStream_t st) {
-  // the K-tile stages, reused by the epilogue as one 256-row tile of 16-bit results
-  constexpr size_t stages = (size_t)NST * STAGE_BYTES, ctile = (size_t)BM * CTile<BN>::pitch;
-  constexpr size_t smem = stages > ctile ? stages : ctile;
+  constexpr size_t smem = (size_t)NST * STAGE_BYTES;
   auto kern = gmm_dtl_kernel<DT, ODT>;
   static std::atomic<uint64_t> done_mask{0};
   if (!gmoe_once_per_device(done_mask, [&] {

@@ -1,12 +1,11 @@
 // Grouped weight-gradient product (TN) of 16-bit operands for short reductions on gfx950:
 //   c[e] = a[rows_e]^T @ b[rows_e],  a [N,K], b [N,M], c [E,K,M]: the contract of gmm_dtl.hip.
 //
-// With few rows per expert a 256x256 tile is mostly prologue and epilogue (383 rows: 12 stages of 32
-// rows, 10 us of multiplying against 7 us around it), and one workgroup per CU leaves the matrix
-// cores idle meanwhile.  Here a tile is 128x256 and two workgroups share a CU (72 KiB of LDS, at most
+// For outputs of less than a round of 256x256 tiles, whose CUs then have nothing to hide a tile's prologue
+// and epilogue under.  Here a tile is 128x256 and two workgroups share a CU (72 KiB of LDS, at most
 // 256 registers each): one multiplies while the other copies its first stages or writes its result.
-// The price is half again as much operand traffic per product, so long reductions stay with
-// gmm_dtl.hip.
+// The price is half again as much operand traffic per product, so long reductions and large outputs
+// stay with gmm_dtl.hip (the rule with both sides' times is gmm_tn_short_pays in gmm.hip).
 #include "gmm_common.h"
 
 namespace gmoe {

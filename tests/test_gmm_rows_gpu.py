@@ -45,7 +45,7 @@ def test_chunk_edges(pkg, dev, dtype, K, F):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("K,M", [(1024, 512), (1160, 904), (136, 4104)])
+@pytest.mark.parametrize("K,M", [(1024, 512), (1160, 904), (136, 4104), (1160, 520)])
 def test_short_reduction_edges(pkg, dev, dtype, K, M):
     """dW over 0, 1, a stage (32) more or less one, ... rows; output edges inside a tile."""
     rows = [0, 1, 31, 32, 33, 63, 64, 65, 95, 97, 128, 129, 7, 0, 300, 2]
@@ -63,4 +63,27 @@ def test_short_reduction_edges(pkg, dev, dtype, K, M):
         want = a[s:s + n].double().t().contiguous() @ b[s:s + n].double()
         # exact products of values up to about 5 x 5, n fp32 additions: 2^-24 * 25 * n bounds each sum
         assert (got32[e].double() - want).abs().max().item() <= 2.0 ** -24 * 25 * n * 4
+        s += n
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("K,M", [(1160, 904), (520, 4104)])
+def test_long_reduction_edges(pkg, dev, dtype, K, M):
+    """dW on 256x256 tiles, whose copies run ahead into the next tile: experts with no rows, with less
+    than the copies' three stages (96 rows) and with many, in turn; output edges inside a tile."""
+    rows = [0, 1, 31, 3000, 32, 33, 95, 96, 97, 0, 0, 4097, 7, 2500, 65, 5000]
+    E, N = len(rows), sum(rows)
+    g = torch.Generator(device=dev).manual_seed(K + M)
+    print("case", dtype, K, M, flush=True)
+    off = torch.tensor([0] + rows, device=dev).cumsum(0)
+    a = torch.empty(N, K, device=dev).normal_(generator=g).to(dtype)
+    b = torch.empty(N, M, device=dev).normal_(generator=g).to(dtype)
+    got32 = pkg.ops.gmm(a, b, off, trans_a=True, out_dtype=torch.float32)
+    got = pkg.ops.gmm(a, b, off, trans_a=True)
+    assert torch.equal(got, got32.to(dtype))
+    s = 0
+    for e, n in enumerate(rows):
+        want = a[s:s + n].double().t().contiguous() @ b[s:s + n].double()
+        # as above; the sums of a long reduction stay within a few sqrt(n)
+        assert (got32[e].double() - want).abs().max().item() <= 2.0 ** -24 * 25 * min(n, 100 * n ** 0.5) * 4
         s += n
