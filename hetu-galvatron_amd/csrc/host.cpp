@@ -183,6 +183,7 @@ Tensor glu_bwd(const Tensor& grad, const Tensor& y, int act) {
 Tensor unpermute_rows(const Tensor& permuted, const Tensor& dst_map, const Tensor& probs, const Tensor& residual,
                       const Tensor& addend) {
   require_gpu(permuted, dst_map, probs, residual, addend);
+  REQUIRE(permuted.dim() == 2 && dst_map.dim() == 2, "combine: permuted rows [N,H], destination map [T,E]");
   const int64_t T = dst_map.size(0), E = dst_map.size(1), H = permuted.size(1);
   REQUIRE(dst_map.scalar_type() == at::kInt, "int32 destination map");
   for (const Tensor& t : {residual, addend})
@@ -199,6 +200,7 @@ Tensor unpermute_rows(const Tensor& permuted, const Tensor& dst_map, const Tenso
 }
 Tensor permute_rows(const Tensor& tokens, const Tensor& dst_map, int64_t n_out, bool zero_fill) {
   require_gpu(tokens, dst_map);
+  REQUIRE(tokens.dim() == 2 && dst_map.dim() == 2, "permute: tokens [T,H], destination map [T,E]");
   const int64_t T = tokens.size(0), H = tokens.size(1);
   REQUIRE(dst_map.scalar_type() == at::kInt && dst_map.size(0) == T, "int32 destination map [T,E]");
   Tensor out = zero_fill ? at::zeros({n_out, H}, tokens.options()) : empty_of(tokens, {n_out, H});
@@ -287,6 +289,7 @@ Tensor pad_dim(const Tensor& t, int64_t dim, int64_t n) {
 
 Tensor gate_fwd(const Tensor& x, const Tensor& weight_in, at::ScalarType out_type) {
   require_gpu(x, weight_in);
+  REQUIRE(weight_in.dim() == 2, "gate: weight [E,H]");
   const int64_t H = weight_in.size(1), E_real = weight_in.size(0), E = padded_experts(E_real);
   REQUIRE(x.size(-1) == H && x.scalar_type() == weight_in.scalar_type(), "gate: x [..,H] and weight [E,H] of one type");
   const int64_t T = H > 0 ? x.numel() / H : 0;
@@ -309,6 +312,8 @@ Tensor gate_fwd(const Tensor& x, const Tensor& weight_in, at::ScalarType out_typ
 std::pair<Tensor, Tensor> gate_bwd(const Tensor& dlogits_in, const Tensor& x, const Tensor& weight_in, bool need_dx,
                                    bool need_dw) {
   require_gpu(dlogits_in, x, weight_in);
+  REQUIRE(weight_in.dim() == 2 && (weight_in.size(1) == 0 || x.numel() % weight_in.size(1) == 0),
+          "gate: weight [E,H] and x of whole rows");
   const int64_t H = weight_in.size(1), E_real = weight_in.size(0), E = padded_experts(E_real);
   const int64_t T = H > 0 ? x.numel() / H : 0;
   Tensor dl = dlogits_in.reshape({-1, E_real});
@@ -458,10 +463,11 @@ std::pair<OptTensor, OptTensor> bookkeeping(const Tensor& stats, const Tensor& c
   REQUIRE(!local.defined() || local.scalar_type() == at::kFloat, "fp32 token counts");
   auto slot = [&](const OptTensor& values) -> float* {
     if (!values.has_value()) return nullptr;
-    REQUIRE(values->is_cuda() && values->scalar_type() == at::kFloat && index >= 0 && index < values->numel() &&
-                values->is_contiguous(),
+    // a negative index counts from the end, as indexing a tensor does
+    const int64_t n = values->numel(), slot = index < 0 ? index + n : index;
+    REQUIRE(values->is_cuda() && values->scalar_type() == at::kFloat && slot >= 0 && slot < n && values->is_contiguous(),
             "tracker values: fp32 on the GPU, one per layer");
-    return values->data_ptr<float>() + index;
+    return values->data_ptr<float>() + slot;
   };
   OptTensor aux, z;
   if (want_aux) aux = empty_of(counts, {}, at::kFloat);
@@ -482,6 +488,7 @@ struct SeqAuxLoss : Function<SeqAuxLoss> {
                         int64_t k, double coeff, int64_t score_fn) {
     const Tensor x = x_in.contiguous(), rmap = rmap_in.contiguous();
     require_gpu(x, rmap);
+    REQUIRE(x.dim() == 2, "sequence loss: scores [S*B,E]");
     const int64_t T = x.size(0), E = x.size(1);
     REQUIRE(T == B * S && rmap.sizes() == x.sizes() && rmap.scalar_type() == at::kBool,
             "sequence loss: scores [S*B,E] with a bool map");
@@ -520,9 +527,9 @@ struct CapacitySelect : Function<CapacitySelect> {
                                bool by_position, bool pad) {
     const Tensor probs = probs_in.contiguous(), rmap = rmap_in.contiguous();
     require_gpu(probs, rmap);
-    REQUIRE(rmap.sizes() == probs.sizes() && (rmap.scalar_type() == at::kBool || rmap.scalar_type() == at::kByte) &&
+    REQUIRE(probs.dim() == 2 && rmap.sizes() == probs.sizes() && (rmap.scalar_type() == at::kBool || rmap.scalar_type() == at::kByte) &&
                 capacity >= 1,
-            "capacity selection: a bool map like the probs, capacity >= 1");
+            "capacity selection: probs [T,E], a bool map like them, capacity >= 1");
     c10::DeviceGuard on(probs.device());
     Tensor out = at::empty_like(probs), kept = empty_of(probs, probs.sizes(), at::kBool);
     check(L.gmoe_capacity_select(ptr(probs), dt(probs), ptr_as<uint8_t>(rmap), probs.size(0), (int)probs.size(1),
@@ -728,6 +735,7 @@ Fp8Rows fp8_rows_like(const Tensor& t, int64_t N, int64_t K) {
 }
 Fp8Rows quantize_rows(const Tensor& x) {
   require_gpu(x);
+  REQUIRE(x.dim() == 2, "fp8 rows: [N,K]");
   Fp8Rows r = fp8_rows_like(x, x.size(0), x.size(1));
   check(L.gmoe_quantize_fp8_rows(ptr(x), dt(x), x.size(0), x.size(1), ptr(r.q), ptr_as<int32_t>(r.scale), stream_of(x)),
         "gmoe_quantize_fp8_rows");

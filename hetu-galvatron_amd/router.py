@@ -160,7 +160,7 @@ class TopKRouter(Router):
                 aux_losses_tracker_values("load_balancing_loss", self.layer_idx, cfg.num_layers, dev)
                 if track_aux else None,
                 aux_losses_tracker_values("z_loss", self.layer_idx, cfg.num_layers, dev) if track_z else None,
-                (self.layer_idx or 1) - 1, 1.0 / aux_coeff if track_aux else 1.0,
+                (0 if self.layer_idx is None else self.layer_idx - 1), 1.0 / aux_coeff if track_aux else 1.0,
                 1.0 / z_coeff if track_z and z_coeff else 1.0,
                 self.local_tokens_per_expert if count_here else None)
             if track_aux:

@@ -1,0 +1,47 @@
+"""Argument forms of the native autograd nodes: what the tensor-level checks refuse, and the slot of the
+loss tracker that a layer index names."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture()
+def routing_map(dev):
+    return torch.tensor([[1, 0], [0, 1], [1, 0], [0, 1]], dtype=torch.bool, device=dev)
+
+
+def test_rows_of_another_rank_are_refused(pkg, dev, routing_map):
+    host = pkg._C.host()
+    plan = pkg.ops.permute_plan(routing_map, 4, want_sorted=False)
+    cube = torch.zeros(4, 8, 16, device=dev)
+    scores = torch.rand(4, 2, 3, device=dev)
+    calls = [
+        lambda: host.permute_rows(cube, plan.dst_map, 4, False),
+        lambda: pkg.unpermute(cube, plan.dst_map, (4, 8)),
+        lambda: host.gate_fwd(cube, cube.view(8, 16, 4), torch.float32),
+        lambda: host.seq_aux_loss(scores, scores > 0.5, 2, 2, 1, 0.01, "identity"),
+        lambda: host.capacity_select(scores, scores > 0.5, 1, False, False),
+    ]
+    for call in calls:
+        with pytest.raises((AssertionError, ValueError)):
+            call()
+
+
+@pytest.mark.parametrize("layer_idx, slot", [(None, None), (0, 2), (1, 0), (3, 2)])
+def test_tracker_slot(pkg, dev, layer_idx, slot):
+    """values[layer_idx - 1], counted from the end for layer 0; no entry without a layer index."""
+    cfg = pkg.MoEConfig(hidden_size=64, num_moe_experts=4, moe_ffn_hidden_size=64, moe_router_topk=2,
+                        moe_router_load_balancing_type="aux_loss", moe_aux_loss_coeff=0.01, num_layers=3,
+                        params_dtype=torch.float32)
+    router = pkg.GalvatronMoERouter(cfg, layer_idx=layer_idx, device=dev).train().router
+    tracker = pkg.moe_utils.get_moe_layer_wise_logging_tracker()
+    tracker.clear()
+    router.routing(torch.randn(8, 1, 4, generator=torch.Generator().manual_seed(5)).to(dev).requires_grad_(True))
+    values = tracker.pop("load_balancing_loss", {}).get("values")
+    if slot is None:
+        assert values is None
+        return
+    expected = torch.zeros(3)
+    expected[slot] = router.last_aux_loss.item() / 0.01
+    torch.testing.assert_close(values.cpu(), expected, rtol=1e-6, atol=0)
