@@ -992,117 +992,46 @@ __global__ __launch_bounds__(kGemmThreads, (BM == 128 && BN == 128) ? 2 : 1) voi
       // C = d(act) is not stored: with fc1 = [gate | up] read back, the tile of
       // d(fc1) = [d * act'(gate) * up | d * act(gate)] is written instead (d rounded to the
       // storage type first, as a separate activation-backward kernel would see it)
-      static_assert(MODE == MODE_NT && DT == ODT, "fused activation backward follows the dX GEMM");
+      static_assert(MODE == MODE_NT && DT == ODT && DT != GMOE_F32, "16-bit: follows the dX GEMM; fp32: gmm_f32.hip");
       constexpr bool gelu = EPI == EPI_GLU_BWD_GELU;
       const int64_t F = M;
       const unsigned char* fc1 = p.aux + row0 * 2 * F * OES;
       unsigned char* dfc1 = p.c + row0 * 2 * F * OES;
-      if constexpr (DT != GMOE_F32) {
-        // d goes through LDS so that fc1 is read and d(fc1) written in 16-byte, row-contiguous
-        // pieces (the accumulator layout would touch 32 rows per instruction, 8 bytes each)
-        using CT = CTile<BN>;
-        stage_acc_lds<DT, WTM, WTN, BN>(lds, acc, wm * (BM / 2), wn * (BN / 2), lane);
-        __syncthreads();
-        const int cc = tid % CT::chunks, r0 = tid / CT::chunks;
-        const int64_t n = (int64_t)nt * BN + cc * 8;
-        if ((int64_t)mt * BM + BM <= n_e && (int64_t)nt * BN + BN <= F) {
-          // a whole tile: the passes without guards, two at a time, the next two requested ahead
-          // (15.9 instead of 30.5 us per tile: a CU with four wavefronts has too few bytes in
-          // flight when every batch of loads is waited for before the next is requested)
-          const int64_t o0 = (((int64_t)mt * BM + r0) * 2 * F + n) * OES;
-          glu_bwd_tile_rows<DT, BM, BN, gelu, 2>(lds, fc1 + o0, dfc1 + o0, 2 * F * OES, F * OES, cc, r0);
-          __syncthreads();  // the next tile's prologue writes stage 0
-          continue;
-        }
-#pragma unroll 4
-        for (int it = 0; it < BM / CT::rows_per_pass; ++it) {
-          const int row = it * CT::rows_per_pass + r0;
-          const int64_t m = (int64_t)mt * BM + row;
-          if (m >= n_e || n >= F) continue;
-          const int64_t og = (m * 2 * F + n) * OES, ou = og + F * OES;
-          float d[8], g[8], u[8], dg[8], du[8];
-          Vec16<DT>::unpack(ctile_read16(lds + row * CT::pitch + cc * 16), d);
-          Vec16<DT>::unpack(ld16_nt(fc1 + og), g);
-          Vec16<DT>::unpack(ld16_nt(fc1 + ou), u);
-#pragma unroll
-          for (int q = 0; q < 8; ++q) {
-            dg[q] = d[q] * glu_act_grad(g[q], gelu) * u[q];
-            du[q] = d[q] * glu_act(g[q], gelu);
-          }
-          st16(dfc1 + og, Vec16<DT>::pack(dg));
-          st16(dfc1 + ou, Vec16<DT>::pack(du));
-        }
+      // d goes through LDS so that fc1 is read and d(fc1) written in 16-byte, row-contiguous
+      // pieces (the accumulator layout would touch 32 rows per instruction, 8 bytes each)
+      using CT = CTile<BN>;
+      stage_acc_lds<DT, WTM, WTN, BN>(lds, acc, wm * (BM / 2), wn * (BN / 2), lane);
+      __syncthreads();
+      const int cc = tid % CT::chunks, r0 = tid / CT::chunks;
+      const int64_t n = (int64_t)nt * BN + cc * 8;
+      if ((int64_t)mt * BM + BM <= n_e && (int64_t)nt * BN + BN <= F) {
+        // a whole tile: the passes without guards, two at a time, the next two requested ahead
+        // (15.9 instead of 30.5 us per tile: a CU with four wavefronts has too few bytes in
+        // flight when every batch of loads is waited for before the next is requested)
+        const int64_t o0 = (((int64_t)mt * BM + r0) * 2 * F + n) * OES;
+        glu_bwd_tile_rows<DT, BM, BN, gelu, 2>(lds, fc1 + o0, dfc1 + o0, 2 * F * OES, F * OES, cc, r0);
         __syncthreads();  // the next tile's prologue writes stage 0
         continue;
       }
-      if (SMALL && !gelu && (int64_t)mt * BM + BM <= n_e && (int64_t)nt * BN + BN <= F) {
-        // a whole tile, straight from the accumulators: the 8 fc1 loads of the next 32x32 block are
-        // requested before the current block is computed and stored (fc1 and d(fc1) may alias as
-        // far as the compiler knows, so in the guarded loop below every load waits for the stores
-        // before it: 22 us per tile with one 16-byte load in flight per lane).  Not for the large
-        // tiles and the GELU form, which have no registers to spare for the second set of loads.
-        const unsigned char* src = fc1 + (((int64_t)mt * BM + wm * (BM / 2) + (lane & 31)) * 2 * F +
-                                          (int64_t)nt * BN + wn * (BN / 2) + 4 * (lane >> 5)) * OES;
-        unsigned char* dst = dfc1 + (src - fc1);
-        f32x4 gq[2][4], uq[2][4];
-        auto request = [&](auto buf_c, auto blk_c) {
-          constexpr int BUF = decltype(buf_c)::value, i = decltype(blk_c)::value / WTN, j = decltype(blk_c)::value % WTN;
+#pragma unroll 4
+      for (int it = 0; it < BM / CT::rows_per_pass; ++it) {
+        const int row = it * CT::rows_per_pass + r0;
+        const int64_t m = (int64_t)mt * BM + row;
+        if (m >= n_e || n >= F) continue;
+        const int64_t og = (m * 2 * F + n) * OES, ou = og + F * OES;
+        float d[8], g[8], u[8], dg[8], du[8];
+        Vec16<DT>::unpack(ctile_read16(lds + row * CT::pitch + cc * 16), d);
+        Vec16<DT>::unpack(ld16_nt(fc1 + og), g);
+        Vec16<DT>::unpack(ld16_nt(fc1 + ou), u);
 #pragma unroll
-          for (int vq = 0; vq < 4; ++vq) {
-            const int64_t o = ((int64_t)i * 32 * 2 * F + j * 32 + 8 * vq) * OES;
-            gq[BUF][vq] = *reinterpret_cast<const f32x4*>(src + o);
-            uq[BUF][vq] = *reinterpret_cast<const f32x4*>(src + o + F * OES);
-          }
-        };
-        request(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{});
-        GMOE_SCHED_FENCE();
-        static_for<0, NM>([&](auto blk_c) {
-          constexpr int blk = decltype(blk_c)::value, i = blk / WTN, j = blk % WTN, BUF = blk & 1;
-          if constexpr (blk + 1 < NM)
-            request(std::integral_constant<int, (blk + 1) & 1>{}, std::integral_constant<int, blk + 1>{});
-          GMOE_SCHED_FENCE();
-#pragma unroll
-          for (int vq = 0; vq < 4; ++vq) {
-            const int64_t o = ((int64_t)i * 32 * 2 * F + j * 32 + 8 * vq) * OES;
-            f32x4 dg, du;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              const float d = acc[i][j][4 * vq + q];
-              dg[q] = d * glu_act_grad(gq[BUF][vq][q], gelu) * uq[BUF][vq][q];
-              du[q] = d * glu_act(gq[BUF][vq][q], gelu);
-            }
-            *reinterpret_cast<f32x4*>(dst + o) = dg;
-            *reinterpret_cast<f32x4*>(dst + o + F * OES) = du;
-          }
-          GMOE_SCHED_FENCE();
-        });
-        continue;
-      }
-#pragma unroll
-      for (int i = 0; i < WTM; ++i) {
-        const int64_t m = (int64_t)mt * BM + wm * (BM / 2) + i * 32 + (lane & 31);
-        if (m >= n_e) continue;
-#pragma unroll
-        for (int j = 0; j < WTN; ++j) {
-#pragma unroll
-          for (int vq = 0; vq < 4; ++vq) {
-            const int64_t n = (int64_t)nt * BN + wn * (BN / 2) + j * 32 + 8 * vq + 4 * (lane >> 5);
-            if (n >= F) continue;
-            const int64_t og = (m * 2 * F + n) * OES, ou = (m * 2 * F + F + n) * OES;
-            const f32x4 gv = *reinterpret_cast<const f32x4*>(fc1 + og);
-            const f32x4 uv = *reinterpret_cast<const f32x4*>(fc1 + ou);
-            f32x4 dg, du;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              const float d = acc[i][j][4 * vq + q];
-              dg[q] = d * glu_act_grad(gv[q], gelu) * uv[q];
-              du[q] = d * glu_act(gv[q], gelu);
-            }
-            *reinterpret_cast<f32x4*>(dfc1 + og) = dg;
-            *reinterpret_cast<f32x4*>(dfc1 + ou) = du;
-          }
+        for (int q = 0; q < 8; ++q) {
+          dg[q] = d[q] * glu_act_grad(g[q], gelu) * u[q];
+          du[q] = d[q] * glu_act(g[q], gelu);
         }
+        st16(dfc1 + og, Vec16<DT>::pack(dg));
+        st16(dfc1 + ou, Vec16<DT>::pack(du));
       }
+      __syncthreads();  // the next tile's prologue writes stage 0
       continue;
     }
     unsigned char* c_base;
@@ -1302,10 +1231,15 @@ static inline bool gmm_use_remainder(const GmmParams& p) {
 // Whether a 128x128-tile NN / NT launch is worth a split reduction, from the host-side sizes (an expert
 // has at least one row tile, and its last one is half full on average); the kernels decide again from the
 // tiles there are.
+//
+// fp32: the alternative is gmm_f32.hip, which needs no workspace and is ahead from 144 tiles on (us, K x M,
+// experts, rows: 65 split against 63, 1024 x 512, 8, 4096); with a few dozen tiles it leaves CUs idle (20
+// against 30, 512 x 128, 4, 400; 46 against 162, 3584 x 896, 4, 130).  Hence at least four pieces.
 static inline bool gmm_split_pays(const GmmParams& p, int dtype) {
   const int es = dtype == GMOE_F32 ? 4 : 2;
   const int64_t least = p.N < p.E ? p.N : p.E, average = (p.N + 127) / 128 + p.E / 2;
   const int64_t tiles = (average > least ? average : least) * ((p.M + 127) / 128);
+  if (dtype == GMOE_F32 && tiles * 4 > kSplitSlots) return false;
   return split_pieces(split_us_per_k_tile(es), (p.K * es + 127) / 128, tiles, kSplitSlots,
                       weight_stream_us(p.E, p.K, p.M, es)) > 1;
 }
@@ -1346,23 +1280,21 @@ static int launch_gmm_remainder(const GmmParams& p, hipStream_t st) {
 //             twice); optionally with the gated activation in the epilogue;
 //   TN 16-bit both operands [k][outer]: LDS-DMA copies of 512-byte rows, 4 stages (1.5 % faster than
 //             the register-staged form);
-//   fp32      register-staged, 4x4 blocks transposed in registers where needed.
 // Small groups: 128x128 tiles, two workgroups per CU.
+// fp32: three bf16 planes per operand on the bf16 matrix cores (gmm_f32.hip), 1.3-1.9 times as fast as the fp32
+// MFMA with a smaller error; the fp32 MFMA kernels serve split reductions and dW of operands beyond 2 GiB.
 template <int DT, int ODT, int MODE, int EPI>
-static int launch_gmm_mode(const GmmParams& p, int dtype, int out_dtype, hipStream_t st) {
-  constexpr bool half = Elem<DT>::bytes == 2;
+static int launch_gmm_16bit(const GmmParams& p, int dtype, int out_dtype, hipStream_t st) {
   constexpr bool glu_fwd = EPI == EPI_GLU_FWD_SILU || EPI == EPI_GLU_FWD_GELU;
-  if constexpr (half && MODE == MODE_TN) {
+  if constexpr (MODE == MODE_TN) {
     if (gmm_tn_short_pays(p)) return launch_gmm_tn_short(p, dtype, out_dtype, st);
-  }
-  if constexpr (half && MODE != MODE_TN) {
+  } else {
     if (gmm_rows_pays(p, MODE, EPI)) return launch_gmm_rows(p, MODE, dtype, out_dtype, EPI, st);
   }
   if (gmm_large_tiles(p, MODE)) {
-    if constexpr (MODE == MODE_TN && half) {
-      (void)dtype;
+    if constexpr (MODE == MODE_TN) {
       return launch_gmm_dtl_tn(p, dtype, out_dtype, st);
-    } else if constexpr (MODE == MODE_NN && half && EPI == EPI_NONE) {
+    } else if constexpr (MODE == MODE_NN && EPI == EPI_NONE) {
       // the short last row tiles pay off as a launch of their own only when it can be split
       if (p.ws == nullptr || p.ws_floats < 2 * 128 * 128 || !gmm_use_remainder(p))
         return launch_gmm_cfg<DT, ODT, MODE_NN, 256, 256, EPI_NONE, false, true>(p, st);
@@ -1371,16 +1303,16 @@ static int launch_gmm_mode(const GmmParams& p, int dtype, int out_dtype, hipStre
       m.main_grid = gmm_grid(1);
       const int rc = launch_gmm_cfg<DT, ODT, MODE_NN, 256, 256, EPI_NONE, false, true>(m, st);
       return rc != GMOE_OK ? rc : launch_gmm_remainder<DT, ODT, MODE_NN>(m, st);
-    } else if constexpr (MODE == MODE_NN && half) {
+    } else if constexpr (MODE == MODE_NN) {
       return launch_gmm_cfg<DT, ODT, MODE_NN, 256, 256, EPI, false, true>(p, st);
-    } else if constexpr (MODE == MODE_NT && EPI == EPI_NONE) {
+    } else if constexpr (EPI == EPI_NONE) {
       if (!gmm_use_remainder(p)) return launch_gmm_cfg<DT, ODT, MODE_NT, 256, 256, EPI_NONE>(p, st);
       GmmParams m = p;
       m.row_part = ROWS_AUTO_MAIN;
       m.main_grid = gmm_grid(1);
       const int rc = launch_gmm_cfg<DT, ODT, MODE_NT, 256, 256, EPI_NONE>(m, st);
       return rc != GMOE_OK ? rc : launch_gmm_remainder<DT, ODT, MODE_NT>(m, st);
-    } else if constexpr (!glu_fwd) {
+    } else {
       return launch_gmm_cfg<DT, ODT, MODE, 256, 256, EPI>(p, st);
     }
   }
@@ -1393,6 +1325,27 @@ static int launch_gmm_mode(const GmmParams& p, int dtype, int out_dtype, hipStre
     }
     return launch_gmm_cfg<DT, ODT, MODE, 128, 128, EPI>(p, st, 2);
   }
+}
+
+template <int MODE, int EPI>
+static int launch_gmm_fp32(const GmmParams& p, hipStream_t st) {
+  if constexpr (MODE == MODE_TN) {
+    // a buffer resource of gmm_f32.hip spans all rows of an expert, of which the host knows the bound N only
+    if (p.N * (p.K > p.M ? p.K : p.M) * 4 >= (1ll << 31)) {
+      if (gmm_large_tiles(p, MODE)) return launch_gmm_cfg<GMOE_F32, GMOE_F32, MODE, 256, 256, EPI>(p, st);
+      return launch_gmm_cfg<GMOE_F32, GMOE_F32, MODE, 128, 128, EPI>(p, st, 2);
+    }
+  } else if constexpr (EPI == EPI_NONE) {
+    if (p.ws != nullptr && p.ws_floats >= 2 * 128 * 128 && gmm_split_pays(p, GMOE_F32))
+      return launch_gmm_split<GMOE_F32, GMOE_F32, MODE>(p, st);
+  }
+  return launch_gmm_f32(p, MODE, EPI, st);
+}
+
+template <int DT, int ODT, int MODE, int EPI>
+static int launch_gmm_mode(const GmmParams& p, int dtype, int out_dtype, hipStream_t st) {
+  if constexpr (DT == GMOE_F32) return launch_gmm_fp32<MODE, EPI>(p, st);
+  else return launch_gmm_16bit<DT, ODT, MODE, EPI>(p, dtype, out_dtype, st);
 }
 
 template <int DT, int ODT>
@@ -1485,7 +1438,8 @@ int64_t gmm_dense_workspace_floats(int64_t N, int64_t K, int64_t M, int mode, in
   p.N = N;
   p.K = K;
   p.M = M;
-  const bool split = (gmm_large_tiles(p, mode) && gmm_use_remainder(p)) || gmm_split_pays(p, dtype);
+  const bool split =
+      (dtype != GMOE_F32 && gmm_large_tiles(p, mode) && gmm_use_remainder(p)) || gmm_split_pays(p, dtype);
   return split ? (int64_t)kSplitSlots * 128 * 128 : 0;
 }
 
@@ -1510,7 +1464,8 @@ extern "C" int64_t gmoe_gmm_workspace_bytes(int E, int64_t N, int64_t K, int64_t
   p.K = K;
   p.M = M;
   const int mode = trans_b ? MODE_NT : MODE_NN;
-  const bool split = (gmm_large_tiles(p, mode) && gmm_use_remainder(p)) || gmm_split_pays(p, dtype);
+  const bool split =
+      (dtype != GMOE_F32 && gmm_large_tiles(p, mode) && gmm_use_remainder(p)) || gmm_split_pays(p, dtype);
   return split ? (int64_t)kSplitSlots * 128 * 128 * 4 : 0;
 }
 

@@ -244,6 +244,9 @@ int launch_gmm_tn_short(const GmmParams& p, int dtype, int out_dtype, hipStream_
 // Launches the row-adaptive kernel (gmm_rows.hip) for 16-bit operands.
 int launch_gmm_rows(const GmmParams& p, int mode, int dtype, int out_dtype, int epi, hipStream_t st);
 
+// Launches the fp32 kernel on split operands (gmm_f32.hip).
+int launch_gmm_f32(const GmmParams& p, int mode, int epi, hipStream_t st);
+
 // Launches the weight-stationary kernel for fp8 weights and few rows per expert (gmm_fp8s.hip);
 // whether it applies: gmm_fp8_skinny_applies.
 int launch_gmm_fp8_skinny(const GmmParams& p, bool trans_b, hipStream_t st);
