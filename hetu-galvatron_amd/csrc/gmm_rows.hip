@@ -39,7 +39,7 @@ struct Stages {
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 
-// Row chunks of an expert with n rows: units of 32 rows dealt as evenly as possible to
+// Row chunks of an expert with n rows: units of kUnit rows dealt as evenly as possible to
 // ceil(units / 4) chunks.
 __device__ __forceinline__ int chunk_count(long long n) {
   const long long units = (n + kUnit - 1) / kUnit;
