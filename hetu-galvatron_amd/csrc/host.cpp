@@ -263,7 +263,8 @@ struct RmsNormResidual : Function<RmsNormResidual> {
     auto [y, rstd] = rmsnorm_fwd(x, weight, eps);
     ctx->save_for_backward({x, weight, rstd});
     ctx->set_materialize_grads(false);
-    return {y, x.detach()};
+    // a view, so that autograd refuses to have it written in place: that would change the caller's x
+    return {y, x.view_as(x)};
   }
   static variable_list backward(AutogradContext* ctx, variable_list g) {
     if (!g[0].defined()) return {g[1], Tensor(), Tensor()};

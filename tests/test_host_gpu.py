@@ -1,5 +1,5 @@
-"""Argument forms of the native autograd nodes: what the tensor-level checks refuse, and the slot of the
-loss tracker that a layer index names."""
+"""Argument forms of the native autograd nodes: what the tensor-level checks refuse, the slot of the loss
+tracker that a layer index names, and writes in place on what a node returned."""
 import pytest
 import torch
 
@@ -45,3 +45,18 @@ def test_tracker_slot(pkg, dev, layer_idx, slot):
     expected = torch.zeros(3)
     expected[slot] = router.last_aux_loss.item() / 0.01
     torch.testing.assert_close(values.cpu(), expected, rtol=1e-6, atol=0)
+
+
+@pytest.mark.parametrize("transposed", [False, True])
+def test_residual_is_not_written_in_place(pkg, dev, transposed):
+    """The second output of PreRouterNorm is the input: writing it would change what the caller holds."""
+    cfg = pkg.MoEConfig(hidden_size=64, num_moe_experts=4, moe_ffn_hidden_size=64, params_dtype=torch.float32)
+    norm = pkg.PreRouterNorm(cfg, device=dev)
+    x = torch.randn(4, 2, 64, generator=torch.Generator().manual_seed(1)).to(dev).requires_grad_(True)
+    before = x.detach().clone()
+    out, residual = norm(x.transpose(0, 1) if transposed else x)
+    with pytest.raises(RuntimeError, match="modified inplace"):
+        residual.add_(1.0)
+    assert torch.equal(x.detach(), before)
+    (out.sum() + (2 * residual).sum()).backward()
+    assert x.grad is not None
