@@ -9,8 +9,15 @@
 //     in fp32.  (One accumulator for everything would be rounded 12 times per block inside the MFMA.)
 //     Error against float64, 2-norm, normal operands, this kernel and the fp32 MFMA kernel it replaces:
 //     K 512 0.9e-7 / 4.1e-7, K 2048 1.6e-7 / 8.1e-7, K 4096 2.2e-7 / 11e-7, K 4 3.2e-8 / 4.4e-8.
-//   * An infinity (also a value that bf16 rounds to one) leaves NaN as its remainder, so every result that
-//     depends on an infinity or NaN is NaN.  A tile that holds a NaN is computed again on the fp32 MFMA.
+//   * Three planes hold an fp32 value exactly from 2^-110 on: its last bit is then no smaller than the smallest
+//     bf16 number (the matrix cores take subnormal ones as they are).  An infinity (also a value that bf16
+//     rounds to one) leaves NaN as its remainder, so every result that depends on an infinity or NaN is NaN.
+//     A tile that met a smaller operand, other than zero, or that holds a NaN is computed again on the fp32
+//     MFMA.  The look at the operands costs 1-2 % of a launch, 2-4 % on 64-row tiles (4146 x 2048 x 512 over 8
+//     experts NN 109 -> 111 us, NT 99 -> 103; 8192 x 2048 x 2048 over 8 NN 378 -> 385, NT 370 -> 377, TN 371 ->
+//     379): a minimum over the stage, and only where that finds a zero or a small value, the exact look
+//     (operands with a seventh of zero rows: 1-5 % more); always exact, 8 %.  A launch computed again as a
+//     whole takes 2 to 6 times as long.
 //   * Tiles of RF*64 rows (RF = 1, 2: an expert's rows are shared out in 64-row units) x 128 columns, 2x2
 //     wavefronts of (RF*32) x 64, two workgroups per CU: one splits operands while the other multiplies.  With
 //     at most one tile per CU the tiles are cut to 64 rows (4096 x 1024 x 512 over 8 experts 75 -> 62 us).
@@ -56,6 +63,8 @@ __device__ __forceinline__ void split8(const float (&x)[8], u32x4& hi, u32x4& mi
   }
 }
 
+constexpr float kSplitMin = 0x1p-110f;  // smallest magnitude that three planes hold exactly
+
 // One operand's path to LDS: U units of 64 outer indices, an item = 8 reduction elements of one of them,
 // U items per thread and stage.  KC: the reduction index is the contiguous one.
 template <bool KC, int U>
@@ -67,8 +76,10 @@ struct Loader {
   int oct[U];
   float x[U][8];
 
-  // src: outer index 0, reduction element 0 of the tile; bytes: what may be read from there
-  __device__ __forceinline__ void init(const unsigned char* src, int64_t ld, int64_t bytes, int tid) {
+  // src: outer index 0, reduction element 0 of the tile; bytes: what may be read from there; outers: indices
+  // that exist (k contiguous: the last one is read for those that do not, which are never stored: zeros would
+  // take every stage through holds_small)
+  __device__ __forceinline__ void init(const unsigned char* src, int64_t ld, int64_t bytes, int64_t outers, int tid) {
     rsrc = make_rsrc(src, bytes);
     k_bytes = (uint32_t)(KC ? 4 : ld * 4);
 #pragma unroll
@@ -77,7 +88,8 @@ struct Loader {
       // k contiguous: 4 lanes read the 128 bytes of a row; otherwise a wavefront reads 64 columns
       const int outer = KC ? id >> 2 : id & (U * kUnit - 1);
       oct[i] = KC ? id & 3 : id / (U * kUnit);
-      voff[i] = KC ? (uint32_t)(outer * ld * 4 + oct[i] * 32) : (uint32_t)(oct[i] * 8 * ld * 4 + outer * 4);
+      const int64_t from = outer < outers ? outer : outers - 1;
+      voff[i] = KC ? (uint32_t)(from * ld * 4 + oct[i] * 32) : (uint32_t)(oct[i] * 8 * ld * 4 + outer * 4);
       lds[i] = (uint32_t)(oct[i] * OCTET + outer * 16);
     }
   }
@@ -112,6 +124,27 @@ struct Loader {
       *reinterpret_cast<u32x4*>(stage + 2 * PLANE + lds[i]) = lo;
     }
   }
+  // Smallest magnitude of the stage and `m`, zeros included; a NaN may hide the others, or be the result.
+  __device__ __forceinline__ float smallest(float m) const {
+#pragma unroll
+    for (int i = 0; i < U; ++i)
+#pragma unroll
+      for (int q = 0; q < 8; q += 2)
+        asm("v_min3_f32 %0, |%1|, |%2|, %3" : "=v"(m) : "v"(x[i][q]), "v"(x[i][q + 1]), "v"(m));
+    return m;
+  }
+  // Whether the stage holds a value below kSplitMin that is not zero.
+  __device__ __forceinline__ bool holds_small() const {
+    uint32_t least = 0xffffffffu;  // of twice the bits, less one: zero wraps to the top
+#pragma unroll
+    for (int i = 0; i < U; ++i)
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const uint32_t v = __float_as_uint(x[i][q]) * 2u - 1u;
+        least = v < least ? v : least;
+      }
+    return least < __float_as_uint(kSplitMin) * 2u - 1u;
+  }
   // element (outer, k) for the fp32 MFMA; past the end of either reads as zero
   __device__ __forceinline__ float one(int outer, int64_t k, int64_t K, int64_t ld) const {
     const uint32_t off = KC ? (uint32_t)((outer * ld + k) * 4) : (uint32_t)((k * ld + outer) * 4);
@@ -139,14 +172,14 @@ __device__ __forceinline__ void run_tile(const GmmParams& p, const Item& it, uns
   Loader<MODE == MODE_NT, 2> lb;
   const int64_t ld_a = p.K, ld_b = MODE == MODE_NT ? p.K : M;
   if constexpr (MODE == MODE_TN) {
-    la.init(p.a + (it.row0 * p.K + it.first) * 4, ld_a, (it.n * p.K - it.first) * 4, tid);
-    lb.init(p.b + (it.row0 * M + col0) * 4, ld_b, (it.n * M - col0) * 4, tid);
+    la.init(p.a + (it.row0 * p.K + it.first) * 4, ld_a, (it.n * p.K - it.first) * 4, it.cnt, tid);
+    lb.init(p.b + (it.row0 * M + col0) * 4, ld_b, (it.n * M - col0) * 4, M - col0, tid);
   } else {
-    la.init(p.a + (it.row0 + it.first) * p.K * 4, ld_a, it.cnt * p.K * 4, tid);
+    la.init(p.a + (it.row0 + it.first) * p.K * 4, ld_a, it.cnt * p.K * 4, it.cnt, tid);
     if constexpr (MODE == MODE_NT)
-      lb.init(p.b + ((int64_t)it.e * M + col0) * p.K * 4, ld_b, (M - col0) * p.K * 4, tid);
+      lb.init(p.b + ((int64_t)it.e * M + col0) * p.K * 4, ld_b, (M - col0) * p.K * 4, M - col0, tid);
     else
-      lb.init(p.b + ((int64_t)it.e * p.K * M + col0) * 4, ld_b, (p.K * M - col0) * 4, tid);
+      lb.init(p.b + ((int64_t)it.e * p.K * M + col0) * 4, ld_b, (p.K * M - col0) * 4, M - col0, tid);
   }
 
   f32x16 sum[RF][2];
@@ -165,9 +198,12 @@ __device__ __forceinline__ void run_tile(const GmmParams& p, const Item& it, uns
     la.load(0, red);
     lb.load(0, red);
   }
+  uint64_t small = 0;  // lanes
   for (int s = 0; s < stages; ++s) {
     la.store(lds);
     lb.store(lds + OPERAND);
+    if (__ballot(!(la.smallest(lb.smallest(kSplitMin)) >= kSplitMin)) != 0)
+      small |= __ballot(la.holds_small() || lb.holds_small());
     __syncthreads();
     if (s + 1 < stages) {
       la.load((int64_t)(s + 1) * BKT, red);
@@ -221,32 +257,38 @@ __device__ __forceinline__ void run_tile(const GmmParams& p, const Item& it, uns
     __syncthreads();
   }
 
-  // an infinity or NaN among the operands: the tile again on the fp32 MFMA
-  int nan = 0;
+  // a small operand, an infinity or a NaN: the tile again on the fp32 MFMA
+  int redo = small != 0;
 #pragma unroll
   for (int i = 0; i < RF; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) nan |= sum[i][j][v] != sum[i][j][v];
-  if (__builtin_expect(__syncthreads_or(nan), 0)) {
+      for (int v = 0; v < 16; ++v) redo |= sum[i][j][v] != sum[i][j][v];
+  if (__builtin_expect(__syncthreads_or(redo), 0)) {
 #pragma unroll
     for (int i = 0; i < RF; ++i)
 #pragma unroll
       for (int j = 0; j < 2; ++j) sum[i][j] = f32x16{};
+    constexpr int kAhead = 2;  // pairs of reduction elements requested together
 #pragma unroll 1
-    for (int64_t k0 = 0; k0 < red; k0 += 2) {
-      const int64_t k = k0 + (lane >> 5);
-      float av[RF], bv[2];
+    for (int64_t k0 = 0; k0 < red; k0 += 2 * kAhead) {
+      float av[kAhead][RF], bv[kAhead][2];
 #pragma unroll
-      for (int i = 0; i < RF; ++i) av[i] = la.one(wm * RF * 32 + i * 32 + (lane & 31), k, red, ld_a);
+      for (int q = 0; q < kAhead; ++q) {
+        const int64_t k = k0 + 2 * q + (lane >> 5);
 #pragma unroll
-      for (int j = 0; j < 2; ++j) bv[j] = lb.one(wn * 64 + j * 32 + (lane & 31), k, red, ld_b);
+        for (int i = 0; i < RF; ++i) av[q][i] = la.one(wm * RF * 32 + i * 32 + (lane & 31), k, red, ld_a);
 #pragma unroll
-      for (int i = 0; i < RF; ++i)
+        for (int j = 0; j < 2; ++j) bv[q][j] = lb.one(wn * 64 + j * 32 + (lane & 31), k, red, ld_b);
+      }
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
-          sum[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(bv[j], av[i], sum[i][j], 0, 0, 0);
+      for (int q = 0; q < kAhead; ++q)
+#pragma unroll
+        for (int i = 0; i < RF; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+            sum[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(bv[q][j], av[q][i], sum[i][j], 0, 0, 0);
     }
   }
 

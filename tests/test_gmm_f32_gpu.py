@@ -1,5 +1,5 @@
 """fp32 grouped GEMMs on split operands: tile edges, remainders, empty experts, and operands with
-infinities, NaN and values at the end of the range, against float64."""
+infinities, NaN and values at either end of the range, against float64."""
 import pytest
 import torch
 
@@ -66,3 +66,40 @@ def test_non_finite_operands(pkg, dev, mode, value, other):
     # 200 sequential additions at most (the fp32 MFMA's order), each within 2^-24 of the absolute sum
     mag = reference(mode, a, b, counts, torch.abs)
     assert ((got - ref).abs()[finite] <= 2.0 ** -24 * 200 * mag[finite]).all()
+
+
+@pytest.mark.parametrize("mode", MODES)
+@pytest.mark.parametrize("log2_a, log2_b", [(-103, 100), (-118, 100), (100, -118), (-124, 110), (110, -130),
+                                            (-100, -20), (-20, -125), (-60, -80)])
+def test_small_operands(pkg, dev, mode, log2_a, log2_b):
+    """Magnitudes at which the planes of the split run out of exponent, opposite ordinary and large ones, and
+    products that do: no less precise than fp32 products."""
+    counts, K, M = [70, 150, 33], 72, 200
+    off = torch.tensor([0] + counts, device=dev).cumsum(0)
+    a, b = operands(mode, sum(counts), K, M, 3, "cpu", 12)
+    a, b = (a * 2.0 ** log2_a).to(dev), (b * 2.0 ** log2_b).to(dev)
+    a[90:120] = 0.0
+    got, ref = product(pkg, mode, a, b, off).double().cpu(), reference(mode, a, b, counts)
+    # one product after the other (the fp32 MFMA's order): the rounding of addition i has a variance of a third
+    # of (2^-24)^2 times that of i products, together 2^-24 * sqrt(red / 6) of the result's norm; four times
+    # that, and half the spacing of the subnormal numbers per addition
+    red = max(counts) if mode == "TN" else K
+    bound = 4 * 2.0 ** -24 * (red / 6) ** 0.5 * ref.norm() + red * 2.0 ** -150 * ref.numel() ** 0.5
+    assert (got - ref).norm() <= bound, ((got - ref).norm() / bound).item()
+
+
+@pytest.mark.parametrize("mode", MODES)
+def test_one_small_element(pkg, dev, mode):
+    """A single small element in a, the only one of its row (NN, NT) or column (TN) that is not zero."""
+    counts, K, M = [70, 150], 72, 200
+    off = torch.tensor([0] + counts, device=dev).cumsum(0)
+    a, b = operands(mode, sum(counts), K, M, 2, dev, 13)
+    if mode == "TN":
+        a[:, 41] = 0.0
+    else:
+        a[170] = 0.0
+    a[170, 41] = 1.2345678 * 2.0 ** -118
+    got, ref = product(pkg, mode, a, b, off).double().cpu(), reference(mode, a, b, counts)
+    got, ref = (got[1, 41], ref[1, 41]) if mode == "TN" else (got[170], ref[170])
+    # one product, rounded once, and zeros
+    assert ((got - ref).abs() <= 2.0 ** -24 * ref.abs() + 2.0 ** -149).all(), ((got - ref) / ref).abs().max().item()
