@@ -528,34 +528,11 @@ __device__ __forceinline__ void build_tile_cum(const GmmParams& p, int part, int
   __syncthreads();
 }
 
-// Pieces the reduction of every tile of a 128x128 launch is cut into, 1 for none: a K tile of a tile that
-// has its CU to itself costs `us_per_k_tile`, a split launch 6 us for the second kernel and 0.026 us per
-// piece for the 128 KiB of partial sums written and read again; it cannot end before the weights have been
-// streamed (`stream_us`).  Measured on both sides of the line: 128 tiles of 44 K tiles 27 unsplit against
-// 32 us in four pieces, 64 tiles of 16 K tiles 13 against 21, 96 tiles of 64 K tiles 45 against 32, fp32
-// 4 tiles of 16 K tiles 36 against 14; 256 tiles of 224 K tiles (940 MB of weights) 159 against 193.
-__host__ __device__ inline int split_pieces(float us_per_k_tile, long long k_tiles, long long tiles, long long slots,
-                                            float stream_us) {
-  if (tiles <= 0) return 1;
-  long long most = slots / tiles;
-  if (most > kMaxSplit) most = kMaxSplit;
-  if (most > k_tiles) most = k_tiles;
-  if (most < 2) return 1;
-  const float whole = us_per_k_tile * (float)k_tiles, per_piece = 0.026f * (float)tiles;
-  long long s = (long long)(sqrtf(whole / per_piece) + 0.5f);
-  s = s < 2 ? 2 : (s > most ? most : s);
-  const float split = whole / (float)s > stream_us ? whole / (float)s : stream_us;
-  return whole - split > 6.f + per_piece * (float)s ? (int)s : 1;
-}
-__host__ __device__ inline float weight_stream_us(int64_t E, int64_t K, int64_t M, int elem_bytes) {
-  return (float)(E * K * M * elem_bytes) / 6.5e6f;  // 6.5 TB/s
-}
-__host__ __device__ constexpr float split_us_per_k_tile(int elem_bytes) { return elem_bytes == 2 ? 0.42f : 2.1f; }
 // What both kernels of a split launch use: depends on launch parameters and the tile count only.
-__device__ __forceinline__ int split_count(const GmmParams& p, float us_per_k_tile, long long total_tiles,
+__device__ __forceinline__ int split_count(const GmmParams& p, int elem_bytes, long long total_tiles,
                                            long long k_tiles, long long tile_elems) {
   if (p.split_slots == 0) return 1;
-  const int s = split_pieces(us_per_k_tile, k_tiles, total_tiles, p.split_slots, p.stream_us);
+  const int s = split_pieces(split_ns_per_k_tile(elem_bytes), k_tiles, total_tiles, p.split_slots, p.stream_ns);
   return (long long)s * total_tiles * tile_elems <= p.ws_floats ? s : 1;
 }
 
@@ -691,7 +668,7 @@ __global__ __launch_bounds__(kGemmThreads, (BM == 128 && BN == 128) ? 2 : 1) voi
   // gmm_split_reduce_kernel adds the S partial tiles in order.
   constexpr bool CAN_SPLIT = MODE != MODE_TN && EPI == EPI_NONE && !BQ && SMALL;
   constexpr long long TILE_ELEMS = (long long)BM * BN;
-  const int S = CAN_SPLIT ? split_count(p, split_us_per_k_tile(ES), total_tiles, (K + BK - 1) / BK, TILE_ELEMS) : 1;
+  const int S = CAN_SPLIT ? split_count(p, ES, total_tiles, (K + BK - 1) / BK, TILE_ELEMS) : 1;
   const long long total_work = total_tiles * S;
 
   // Workgroup w runs on XCD w%8.  Give XCD x the consecutive positions [x*G/8, (x+1)*G/8) of
@@ -1099,7 +1076,7 @@ __global__ __launch_bounds__(kGemmThreads) void gmm_split_reduce_kernel(GmmParam
   if (part == ROWS_NONE) return;
   build_tile_cum<MODE, BM>(p, part, nt_cnt, 0, tile_cum);
   const long long total_tiles = tile_cum[p.E];
-  const int S = split_count(p, split_us_per_k_tile(Elem<DT>::bytes), total_tiles, k_tiles, TILE_ELEMS);
+  const int S = split_count(p, Elem<DT>::bytes, total_tiles, k_tiles, TILE_ELEMS);
   if (S == 1) return;  // the first launch did everything
   int e = 0;
   for (long long item = blockIdx.x; item < total_tiles * 4; item += gridDim.x) {
@@ -1240,8 +1217,8 @@ static inline bool gmm_split_pays(const GmmParams& p, int dtype) {
   const int64_t least = p.N < p.E ? p.N : p.E, average = (p.N + 127) / 128 + p.E / 2;
   const int64_t tiles = (average > least ? average : least) * ((p.M + 127) / 128);
   if (dtype == GMOE_F32 && tiles * 4 > kSplitSlots) return false;
-  return split_pieces(split_us_per_k_tile(es), (p.K * es + 127) / 128, tiles, kSplitSlots,
-                      weight_stream_us(p.E, p.K, p.M, es)) > 1;
+  return split_pieces(split_ns_per_k_tile(es), (p.K * es + 127) / 128, tiles, kSplitSlots,
+                      weight_stream_ns(p.E, p.K, p.M, es)) > 1;
 }
 
 // A split launch with 128x128 tiles: the pieces, then their sums.
@@ -1251,7 +1228,7 @@ static int launch_gmm_split(const GmmParams& p, hipStream_t st) {
   const int64_t slots = p.ws_floats / (128 * 128);
   r.split_slots = (int)(slots < kSplitSlots ? slots : kSplitSlots);
   // the rows left to a remainder launch belong to some of the experts only: no bound from their weights
-  r.stream_us = p.row_part == ROWS_ALL ? weight_stream_us(p.E, p.K, p.M, Elem<DT>::bytes) : 0.f;
+  r.stream_ns = p.row_part == ROWS_ALL ? weight_stream_ns(p.E, p.K, p.M, Elem<DT>::bytes) : 0;
   const int rc = launch_gmm_cfg<DT, ODT, MODE, 128, 128, EPI_NONE>(r, st, 2);
   if (rc != GMOE_OK) return rc;
   // at most split_slots / 2 tiles are split, four quarters each
@@ -1413,7 +1390,7 @@ static int gmm_check(GmmParams& p, const void* a, const void* b, void* c, const 
   p.ws = nullptr;
   p.ws_floats = 0;
   p.split_slots = 0;
-  p.stream_us = 0.f;
+  p.stream_ns = 0;
   p.main_grid = 0;
   return GMOE_OK;
 }

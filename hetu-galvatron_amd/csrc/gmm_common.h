@@ -4,6 +4,7 @@
 #include <type_traits>
 
 #include "gmoe_common.h"
+#include "split_rule.h"
 
 namespace gmoe {
 
@@ -72,11 +73,11 @@ struct GmmParams {
   const unsigned char* a_scale;  // fp8 activations: power-of-two row scales, dwords [K/128][N]
   int row_part;              // NN / NT: which rows of every expert this launch covers (ROWS_*)
   int64_t F;
-  // split reduction of a launch with few tiles (see split_count in gmm.hip): fp32 partial tiles
+  // split reduction of a launch with few tiles (split_rule.h, split_count in gmm.hip): fp32 partial tiles
   float* ws;
   int64_t ws_floats;
   int split_slots;           // tiles x splits this launch may spread over; 0 = never split
-  float stream_us;           // time the weights take to stream: a split launch cannot be faster
+  int64_t stream_ns;         // time the weights take to stream: a split launch cannot be faster
   int main_grid;             // ROWS_AUTO_*: workgroups of the launch with 256-row tiles
 };
 // First row of group e.  A null offset table means one group holding all N rows (dense GEMM on the
@@ -84,7 +85,6 @@ struct GmmParams {
 __device__ __forceinline__ long long group_begin(const GmmParams& p, int e) {
   return p.offsets ? p.offsets[e] : (e > 0 ? (long long)p.N : 0ll);
 }
-constexpr int kMaxSplit = 8;
 
 // A launch with 256-row tiles leaves an expert's last n % 256 rows, when they are at most kRemRows,
 // to a second launch with 128-row tiles: a tile that is almost empty costs as much as a full one,
@@ -95,8 +95,6 @@ constexpr int kMaxSplit = 8;
 enum { ROWS_ALL = 0, ROWS_MAIN = 1, ROWS_REMAINDER = 2, ROWS_AUTO_MAIN = 3, ROWS_AUTO_REMAINDER = 4,
        ROWS_NONE = 5 };
 constexpr int kRemRows = 128;
-// Workgroups the split remainder launch spreads over: two per CU.
-constexpr int kSplitSlots = 512;
 // rows [begin, begin + count) of an expert with n rows that belong to `part`
 __device__ __forceinline__ void expert_row_part(long long n, int part, long long& begin,
                                                 long long& count) {
