@@ -27,16 +27,16 @@ namespace {
 
 // ---- the library ----------------------------------------------------------------------------------
 #define GMOE_ENTRY_POINTS(X)                                                                          \
-  X(gmoe_status_string) X(gmoe_route_workspace_bytes) X(gmoe_route_topk) X(gmoe_route_topk_bwd)       \
-  X(gmoe_seq_aux_loss) X(gmoe_seq_aux_loss_bwd) X(gmoe_router_bookkeeping) X(gmoe_capacity_select)    \
-  X(gmoe_permute_plan_workspace_bytes) X(gmoe_permute_plan) X(gmoe_expert_offsets)                    \
-  X(gmoe_permute_rows) X(gmoe_unpermute_rows) X(gmoe_unpermute_rows_bwd) X(gmoe_glu_fwd)              \
-  X(gmoe_glu_bwd) X(gmoe_glu_fwd_fp8store) X(gmoe_glu_bwd_fp8in) X(gmoe_gmm_workspace_bytes)          \
-  X(gmoe_gmm) X(gmoe_gmm_glu) X(gmoe_gmm_glu_bwd) X(gmoe_gmm_fp8w) X(gmoe_gmm_fp8a)                   \
-  X(gmoe_quantize_fp8_rows) X(gmoe_glu_fwd_quantize_fp8_rows) X(gmoe_glu_bwd_quantize_fp8_rows)       \
-  X(gmoe_gate_fwd_workspace_bytes) X(gmoe_gate_fwd) X(gmoe_gate_bwd_input_workspace_bytes)            \
-  X(gmoe_gate_bwd_input) X(gmoe_gate_bwd_workspace_rows) X(gmoe_gate_bwd_weight) X(gmoe_rmsnorm_fwd)  \
-  X(gmoe_rmsnorm_bwd_workspace_rows) X(gmoe_rmsnorm_bwd)
+  X(gmoe_abi_version) X(gmoe_status_string) X(gmoe_route_workspace_bytes) X(gmoe_route_topk)          \
+  X(gmoe_route_topk_bwd) X(gmoe_seq_aux_loss) X(gmoe_seq_aux_loss_bwd) X(gmoe_router_bookkeeping)     \
+  X(gmoe_capacity_select) X(gmoe_permute_plan_workspace_bytes) X(gmoe_permute_plan)                   \
+  X(gmoe_expert_offsets) X(gmoe_permute_rows) X(gmoe_unpermute_rows) X(gmoe_unpermute_rows_bwd)       \
+  X(gmoe_glu_fwd) X(gmoe_glu_bwd) X(gmoe_glu_fwd_fp8store) X(gmoe_glu_bwd_fp8in)                      \
+  X(gmoe_gmm_workspace_bytes) X(gmoe_gmm) X(gmoe_gmm_glu) X(gmoe_gmm_glu_bwd) X(gmoe_gmm_fp8w)        \
+  X(gmoe_gmm_fp8a) X(gmoe_quantize_fp8_rows) X(gmoe_glu_fwd_quantize_fp8_rows)                        \
+  X(gmoe_glu_bwd_quantize_fp8_rows) X(gmoe_gate_fwd_workspace_bytes) X(gmoe_gate_fwd)                 \
+  X(gmoe_gate_bwd_input_workspace_bytes) X(gmoe_gate_bwd_input) X(gmoe_gate_bwd_workspace_rows)       \
+  X(gmoe_gate_bwd_weight) X(gmoe_rmsnorm_fwd) X(gmoe_rmsnorm_bwd_workspace_rows) X(gmoe_rmsnorm_bwd)
 
 struct Library {
 #define X(name) decltype(&::name) name = nullptr;
@@ -57,6 +57,11 @@ void bind_library(const std::string& path, const py::object& loss_scale_reader) 
   if (lib.name == nullptr) throw std::runtime_error(path + " does not export " #name);
   GMOE_ENTRY_POINTS(X)
 #undef X
+  // names resolve in a library of any age; the arguments are those of the header this file was compiled with
+  const int abi = lib.gmoe_abi_version();
+  if (abi != GMOE_ABI_VERSION)
+    throw std::runtime_error(path + " has ABI version " + std::to_string(abi) + ", the host module was built for " +
+                             std::to_string(GMOE_ABI_VERSION) + ": build both again");
   L = lib;
   read_loss_scale = new py::object(loss_scale_reader);
 }

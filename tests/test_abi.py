@@ -2,6 +2,8 @@
 import ctypes
 import os
 import re
+import shutil
+import subprocess
 
 import pytest
 
@@ -49,6 +51,19 @@ def test_abi_version_and_status_strings(pkg):
     # pure host-side helpers, no device needed
     assert lib.gmoe_route_workspace_bytes(1024, 8) > 0
     assert lib.gmoe_permute_plan_workspace_bytes(1024, 8) >= 2 * 8 * 4 * 4
+
+
+@pytest.mark.skipif(shutil.which("gcc") is None, reason="needs gcc")
+@pytest.mark.parametrize("newer", [-1, 1])
+def test_host_module_refuses_a_library_of_another_abi(pkg, tmp_path, newer):
+    """Every name resolves, the version differs: its calls would pass arguments the library does not expect."""
+    source = tmp_path / "other.c"
+    source.write_text("".join("int %s(void) { return %d; }\n" % (name, pkg._C.ABI_VERSION + newer)
+                              for name in declared_functions()))
+    library = str(tmp_path / "other.so")
+    subprocess.check_call(["gcc", "-shared", "-fPIC", str(source), "-o", library])
+    with pytest.raises(RuntimeError, match="ABI"):
+        pkg._C.host().bind_library(library, lambda: None)
 
 
 def test_argument_checks_reject_bad_calls_without_a_gpu(pkg):
