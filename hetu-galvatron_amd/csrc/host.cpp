@@ -286,6 +286,7 @@ struct RmsNormResidual : Function<RmsNormResidual> {
 // count is padded to a multiple of 8 with zero rows of the weight.
 int64_t padded_experts(int64_t E) { return E <= 16 ? E : (E + 7) / 8 * 8; }
 Tensor pad_dim(const Tensor& t, int64_t dim, int64_t n) {
+  at::NoGradGuard copy_only;  // for a launch: the gradient is the node's, no graph of the copy
   auto shape = t.sizes().vec();
   shape[dim] = n;
   Tensor out = at::zeros(shape, t.options());

@@ -60,3 +60,19 @@ def test_residual_is_not_written_in_place(pkg, dev, transposed):
     assert torch.equal(x.detach(), before)
     (out.sum() + (2 * residual).sum()).backward()
     assert x.grad is not None
+
+
+@pytest.mark.parametrize("E", [16, 20, 24, 61])
+def test_gate_records_one_node(pkg, dev, E):
+    """Padding the router weight (20, 61 experts) is part of the launch: autograd records the projection and
+    nothing else."""
+    x = torch.randn(8, 64, device=dev, requires_grad=True)
+    weight = torch.randn(E, 64, device=dev, requires_grad=True)
+    before = (x * 1).grad_fn._sequence_nr()
+    logits = pkg.router._GateProjection.apply(x, weight, torch.float32)
+    after = (x * 1).grad_fn._sequence_nr()
+    assert logits.grad_fn._sequence_nr() == before + 1 and after == before + 2
+    (2 * logits).sum().backward()
+    # sums of 8 and of at most 61 fp32 values of a few units, in another order
+    torch.testing.assert_close(weight.grad, (2 * x.detach().sum(0)).expand(E, 64), rtol=1e-5, atol=1e-5)
+    torch.testing.assert_close(x.grad, (2 * weight.detach().sum(0)).expand(8, 64), rtol=1e-5, atol=1e-4)
