@@ -443,9 +443,10 @@ struct Fp8Loader<R, true, DEPTH> : Fp8TransposeLoader<R, DEPTH> {};
 // ROWS_AUTO_MAIN / ROWS_AUTO_REMAINDER -> ROWS_MAIN / ROWS_REMAINDER when leaving the experts' short
 // last row tiles to their own launch saves more time in the launch with 256-row tiles (whole rounds
 // of its persistent grid) than the second launch takes, else ROWS_ALL / ROWS_NONE.  Both launches
-// evaluate the same counts and the same model, so they agree.  Times in microseconds per 128-byte
-// K tile, measured on the Mixtral shape: 1.3 in a 256x256 tile; in a 128x128 tile 2.5 with two
-// workgroups per CU walking whole reductions, 1.9 when the reduction is split.
+// evaluate the same counts and the same model in whole numbers, so they agree.  Times in nanoseconds per
+// 128-byte K tile, measured on the Mixtral shape: 1300 in a 256x256 tile; in a 128x128 tile 2500 with two
+// workgroups per CU walking whole reductions, 1900 when the reduction is split (16-bit operands only).  Over
+// 108 launches of 9 shapes with 2000 to 8000 rows per expert the choice costs 0.24 % against the better of both.
 __device__ inline int resolve_row_part(const GmmParams& p, int k_tiles, int* counts) {
   if (p.row_part != ROWS_AUTO_MAIN && p.row_part != ROWS_AUTO_REMAINDER) return p.row_part;
   const int tid = threadIdx.x;
@@ -469,16 +470,12 @@ __device__ inline int resolve_row_part(const GmmParams& p, int k_tiles, int* cou
   const long long tiles_all = counts[0] * nt256, tiles_main = counts[1] * nt256, tiles_rem = counts[2] * nt128;
   const long long g = p.main_grid > 0 ? p.main_grid : 256;
   const long long rounds_saved = (tiles_all + g - 1) / g - (tiles_main + g - 1) / g;
-  long long s = 1;
-  if (tiles_rem > 0 && p.ws != nullptr) {
-    s = kSplitSlots / tiles_rem;
-    if (s > kMaxSplit) s = kMaxSplit;
-    if (s > k_tiles) s = k_tiles;
-    if (s < 2 || s * tiles_rem * 128 * 128 > p.ws_floats) s = 1;
-  }
-  const float saved = 1.3f * (float)(rounds_saved * k_tiles);
-  const float cost = s > 1 ? 1.9f * (float)(k_tiles / s) + 24.f
-                           : 2.5f * (float)(((tiles_rem + kSplitSlots - 1) / kSplitSlots) * k_tiles) + 8.f;
+  // the pieces launch_gmm_remainder's launch comes to
+  const long long slots = p.ws == nullptr ? 0 : p.ws_floats / (128 * 128);
+  const int s = split_pieces(split_ns_per_k_tile(2), k_tiles, tiles_rem, slots < kSplitSlots ? slots : kSplitSlots, 0);
+  const long long saved = 1300 * rounds_saved * k_tiles;
+  const long long cost = s > 1 ? 1900ll * (k_tiles / s) + kSplitReduceNs + kSplitNsPerPiece * tiles_rem * s
+                               : 2500 * ((tiles_rem + kSplitSlots - 1) / kSplitSlots) * k_tiles + 8000;
   const bool use = tiles_rem > 0 && saved > cost;
   __syncthreads();  // the caller reuses counts
   if (p.row_part == ROWS_AUTO_MAIN) return use ? ROWS_MAIN : ROWS_ALL;
