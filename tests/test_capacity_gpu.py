@@ -1,5 +1,5 @@
 """Capacity selection against a stable sort on the CPU, at the edges of its blocks of 1024 tokens and of
-the 16384 tokens whose keys stay in registers.  Bit for bit: it moves values and computes none."""
+the 16384 tokens (kCapKeys * kCapThreads) whose keys stay in LDS.  Bit for bit: it moves values and computes none."""
 import pytest
 import torch
 

@@ -103,3 +103,21 @@ def test_one_small_element(pkg, dev, mode):
     got, ref = (got[1, 41], ref[1, 41]) if mode == "TN" else (got[170], ref[170])
     # one product, rounded once, and zeros
     assert ((got - ref).abs() <= 2.0 ** -24 * ref.abs() + 2.0 ** -149).all(), ((got - ref) / ref).abs().max().item()
+
+
+@pytest.mark.parametrize("E, M", [(5, 264), (3, 40)])
+def test_dw_beyond_2gib(pkg, dev, E, M):
+    """dW of operands of 2 GiB and more on the fp32 MFMA kernels (256x256 and 128x128 tiles), one expert's rows
+    longer than a buffer resource."""
+    counts, K = [0, 135000, 1, 4000, 77][:E], 4096
+    off = torch.tensor([0] + counts, device=dev).cumsum(0)
+    g = torch.Generator(device=dev).manual_seed(M)
+    a = torch.empty(sum(counts), K, device=dev).normal_(generator=g)
+    b = torch.empty(sum(counts), M, device=dev).normal_(generator=g)
+    assert a.numel() * 4 >= 1 << 31
+    got, lo = product(pkg, "TN", a, b, off), 0
+    for e, n in enumerate(counts):
+        ref = a[lo:lo + n].double().t().contiguous() @ b[lo:lo + n].double()
+        lo += n
+        # as in test_small_operands
+        assert (got[e].double() - ref).norm() <= 4 * 2.0 ** -24 * (n / 6 + 1) ** 0.5 * ref.norm()

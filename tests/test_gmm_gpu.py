@@ -183,9 +183,8 @@ FUSED_SHAPES = [(4096, 512, 1024, 8, ()), (8192, 1024, 1024, 8, ()), (8300, 1024
 
 
 def fused_cases():
-    """Every (dtype, activation, shape); fp32 beyond 4096 rows only once: the one case whose d(act)
-    product has enough 256x256 tiles to take the large-tile kernel with the fused activation backward
-    working from the accumulators (the smaller fp32 cases cover the rest)."""
+    """Every (dtype, activation, shape); fp32 beyond 4096 rows only once: one kernel serves fp32 of any size
+    (the smaller cases cover it), there with several tiles per workgroup."""
     out = []
     for dtype in (torch.bfloat16, torch.float32, torch.float16):
         for act in ("silu", "gelu"):
