@@ -1162,7 +1162,8 @@ constexpr int64_t kRemainderMinRows = 2048;  // see gmm_use_remainder
 //   * from 512 rows on the 256x256 tiles are the alternative.  NN gains 1-10 % as long as the
 //     reduction is long enough to carry its prologue (n 1024: 1730 -> 1681, K 7168; but 223 -> 238 at
 //     K 1024); NT loses 4-10 % (its 64-byte pieces of two operands against 128-byte ones there:
-//     1632 -> 1727, K 4096), so it stays.  From 2048 rows on the remainder launches take over.
+//     1632 -> 1727, K 4096), so it stays.  From 2048 rows on the remainder launches take over.  These
+//     limits hold also where there are too few 256x256 tiles and 128x128 ones follow, which was not measured.
 //   * with less than three quarters of a round of tiles, or a last round that leaves more than 30 % of
 //     all rounds idle, the smaller tiles spread better (K 2816, M 1024, 16 experts, 64 tiles: 27 -> 43).
 //   * the activation backward (NT) around 256 rows: half the experts take a second chunk of two units,
