@@ -13,11 +13,13 @@
 //     bf16 number (the matrix cores take subnormal ones as they are).  An infinity (also a value that bf16
 //     rounds to one) leaves NaN as its remainder, so every result that depends on an infinity or NaN is NaN.
 //     A tile that met a smaller operand, other than zero, or that holds a NaN is computed again on the fp32
-//     MFMA.  The look at the operands costs 1-2 % of a launch, 2-4 % on 64-row tiles (4146 x 2048 x 512 over 8
-//     experts NN 109 -> 111 us, NT 99 -> 103; 8192 x 2048 x 2048 over 8 NN 378 -> 385, NT 370 -> 377, TN 371 ->
-//     379): a minimum over the stage, and only where that finds a zero or a small value, the exact look
-//     (operands with a seventh of zero rows: 1-5 % more); always exact, 8 %.  A launch computed again as a
-//     whole takes 2 to 6 times as long.
+//     MFMA.  The look at the operands costs 1-2 % of a launch, 2-4 % on 64-row tiles: a minimum over the stage,
+//     and only where that finds a zero or a small value, the exact look (operands with a seventh of zero rows:
+//     1-5 % more; always exact: 8 % of a launch).  A launch computed again as a whole takes 2 to 6 times as
+//     long.
+//   * Buffer resources are made uniform by hand: the rows' addresses come from the offset table, and the
+//     compiler repeated every load of the K loop for each value a lane might hold (4146 x 2048 x 512 over 8
+//     experts NN 111 -> 100 us, NT 103 -> 97; 8192 x 2048 x 2048 over 8 NN 398 -> 388, NT 392 -> 384).
 //   * Tiles of RF*64 rows (RF = 1, 2: an expert's rows are shared out in 64-row units) x 128 columns, 2x2
 //     wavefronts of (RF*32) x 64, two workgroups per CU: one splits operands while the other multiplies.  With
 //     at most one tile per CU the tiles are cut to 64 rows (4096 x 1024 x 512 over 8 experts 75 -> 62 us).
@@ -47,8 +49,13 @@ constexpr int OPERAND = 3 * PLANE;
 constexpr int LDS_BYTES = 2 * OPERAND;
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, int64_t bytes) {
+  // the same in every lane, which the compiler cannot see: it would repeat each load for every distinct value
+  const uint64_t p = (uint64_t)(uintptr_t)base;
+  const uint64_t u = (uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(p >> 32)) << 32 |
+                     (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)p);
   const uint32_t n = bytes <= 0 ? 0u : (bytes > 0x7fffffffll ? 0x7fffffffu : (uint32_t)bytes);
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)n, 0x00020000);
+  return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(u), 0, __builtin_amdgcn_readfirstlane((int)n),
+                                           0x00020000);
 }
 
 // Eight fp32 values as three planes of eight bf16, each rounded to nearest.
@@ -127,10 +134,12 @@ struct Loader {
   // Smallest magnitude of the stage and `m`, zeros included; a NaN may hide the others, or be the result.
   __device__ __forceinline__ float smallest(float m) const {
 #pragma unroll
-    for (int i = 0; i < U; ++i)
-#pragma unroll
-      for (int q = 0; q < 8; q += 2)
-        asm("v_min3_f32 %0, |%1|, |%2|, %3" : "=v"(m) : "v"(x[i][q]), "v"(x[i][q + 1]), "v"(m));
+    for (int i = 0; i < U; ++i)  // in one piece: the compiler pads every asm statement with a no-op
+      asm("v_min3_f32 %0, |%2|, |%3|, %1\n\tv_min3_f32 %0, |%4|, |%5|, %0\n\t"
+          "v_min3_f32 %0, |%6|, |%7|, %0\n\tv_min3_f32 %0, |%8|, |%9|, %0"
+          : "=&v"(m)
+          : "v"(m), "v"(x[i][0]), "v"(x[i][1]), "v"(x[i][2]), "v"(x[i][3]), "v"(x[i][4]), "v"(x[i][5]), "v"(x[i][6]),
+            "v"(x[i][7]));
     return m;
   }
   // Whether the stage holds a value below kSplitMin that is not zero.
