@@ -1180,20 +1180,30 @@ static inline bool gmm_rows_pays(const GmmParams& p, int mode, int epi) {
   return n >= 128 && n < 512;
 }
 
-// dW of 16-bit operands with a short reduction and few output tiles (gmm_tn.hip: 128x256 tiles, two
-// workgroups per CU) against the 256x256 LDS-DMA kernel, or 128x128 tiles where that one does not apply;
-// n = rows per expert, us on both sides.  From one round of 256x256 tiles on that kernel, whose tiles run
-// into each other, is the faster one at any n: n 383: 911 against 999 (4096 x 28672, 8 experts), n 256:
-// 213 against 240 (2048 x 4096, 32), n 640: 65 against 65 (2816 x 1024, 16).  Below that, and where its rows
+// dW of 16-bit operands with a short reduction (gmm_tn.hip: 128x256 tiles, two workgroups per CU) against the
+// 256x256 LDS-DMA kernel, or 128x128 tiles where that one does not apply; n = rows per expert, us on both
+// sides.  From one round of 256x256 tiles on that kernel, whose tiles run into each other, is the
+// faster one at n 128 and more (n 128: 454 against 462, n 190: 495 against 550, n 383: 779 against 837, 4096 x 28672,
+// 8 experts); fewer rows come here (n 64: 410 -> 366; 64 experts of 2048 x 2816, n 64: 168 -> 144, n 20: 149 -> 136).  With less than a round of them, and where its rows
 // would be padding (K under 512), the smaller tiles spread better: 128 tiles of 256x256, 20 -> 15
 // (1024 x 1024, 8), 240: 16.3 -> 15.1 (640 x 1280, 16), 384 x 4096 over 64 experts 120 -> 110.  More than
 // 768 rows are left to the 256x256 tiles (n 1024: 1884 against 1935), fewer than three quarters of a tile
 // per CU to 128x128 ones (128 tiles of 1024 x 512: 13 against 15).
+constexpr int64_t kTnFewRows = 112;
 static inline bool gmm_tn_short_pays(const GmmParams& p) {
   const int64_t n = p.N / (p.E > 0 ? p.E : 1), col_tiles = (p.M + 255) / 256;
   if (p.K < 128 || p.M < 256 || p.E * ((p.K + 127) / 128) * col_tiles * 4 < gmm_grid(1) * 3) return false;
-  if (p.K >= 512 && p.E * ((p.K + 255) / 256) * col_tiles >= gmm_grid(1)) return false;
+  if (n >= kTnFewRows && p.K >= 512 && p.E * ((p.K + 255) / 256) * col_tiles >= gmm_grid(1)) return false;
   return n <= 768;
+}
+
+// Whether reading the operands beforehand (warm_operands) pays: they take bytes / 5 TB/s, and the launch has to be
+// one of many more result bytes (us without and with, operands from HBM: 698 -> 497 for n 190 and 914 -> 772 for n 383,
+// 4096 x 28672 over 8 experts, half of either from the nontemporal stores; 438 -> 360 for n 64; 288 -> 255 for n 256 of
+// 2048 x 2816 over 64; but 98 -> 112 for n 383 of 1024 x 5632 over 16, 82 MB of operands for 184 MB of results).
+static inline bool gmm_tn_warm_pays(const GmmParams& p) {
+  const int64_t n = p.N / (p.E > 0 ? p.E : 1), operands = p.N * (p.K + p.M) * 2, result = p.E * p.K * p.M * 2;
+  return operands <= (192ll << 20) && operands * 4 <= result && (gmm_tn_streams(p) || n < kTnFewRows);
 }
 
 // The separate launch for short last row tiles pays off once an expert has many full row tiles:
@@ -1262,14 +1272,15 @@ template <int DT, int ODT, int MODE, int EPI>
 static int launch_gmm_16bit(const GmmParams& p, int dtype, int out_dtype, hipStream_t st) {
   constexpr bool glu_fwd = EPI == EPI_GLU_FWD_SILU || EPI == EPI_GLU_FWD_GELU;
   if constexpr (MODE == MODE_TN) {
-    if (gmm_tn_short_pays(p)) return launch_gmm_tn_short(p, dtype, out_dtype, st);
+    GmmParams q = p;
+    q.warm = gmm_tn_warm_pays(p);
+    if (gmm_tn_short_pays(p)) return launch_gmm_tn_short(q, dtype, out_dtype, st);
+    if (gmm_large_tiles(p, MODE)) return launch_gmm_dtl_tn(q, dtype, out_dtype, st);
   } else {
     if (gmm_rows_pays(p, MODE, EPI)) return launch_gmm_rows(p, MODE, dtype, out_dtype, EPI, st);
   }
-  if (gmm_large_tiles(p, MODE)) {
-    if constexpr (MODE == MODE_TN) {
-      return launch_gmm_dtl_tn(p, dtype, out_dtype, st);
-    } else if constexpr (MODE == MODE_NN && EPI == EPI_NONE) {
+  if (MODE != MODE_TN && gmm_large_tiles(p, MODE)) {
+    if constexpr (MODE == MODE_NN && EPI == EPI_NONE) {
       // the short last row tiles pay off as a launch of their own only when it can be split
       if (p.ws == nullptr || p.ws_floats < 2 * 128 * 128 || !gmm_use_remainder(p))
         return launch_gmm_cfg<DT, ODT, MODE_NN, 256, 256, EPI_NONE, false, true>(p, st);
@@ -1280,14 +1291,14 @@ static int launch_gmm_16bit(const GmmParams& p, int dtype, int out_dtype, hipStr
       return rc != GMOE_OK ? rc : launch_gmm_remainder<DT, ODT, MODE_NN>(m, st);
     } else if constexpr (MODE == MODE_NN) {
       return launch_gmm_cfg<DT, ODT, MODE_NN, 256, 256, EPI, false, true>(p, st);
-    } else if constexpr (EPI == EPI_NONE) {
+    } else if constexpr (MODE == MODE_NT && EPI == EPI_NONE) {
       if (!gmm_use_remainder(p)) return launch_gmm_cfg<DT, ODT, MODE_NT, 256, 256, EPI_NONE>(p, st);
       GmmParams m = p;
       m.row_part = ROWS_AUTO_MAIN;
       m.main_grid = gmm_grid(1);
       const int rc = launch_gmm_cfg<DT, ODT, MODE_NT, 256, 256, EPI_NONE>(m, st);
       return rc != GMOE_OK ? rc : launch_gmm_remainder<DT, ODT, MODE_NT>(m, st);
-    } else {
+    } else if constexpr (MODE != MODE_TN) {
       return launch_gmm_cfg<DT, ODT, MODE, 256, 256, EPI>(p, st);
     }
   }
@@ -1390,6 +1401,7 @@ static int gmm_check(GmmParams& p, const void* a, const void* b, void* c, const 
   p.split_slots = 0;
   p.stream_ns = 0;
   p.main_grid = 0;
+  p.warm = false;
   return GMOE_OK;
 }
 

@@ -79,6 +79,7 @@ struct GmmParams {
   int split_slots;           // tiles x splits this launch may spread over; 0 = never split
   int64_t stream_ns;         // time the weights take to stream: a split launch cannot be faster
   int main_grid;             // ROWS_AUTO_*: workgroups of the launch with 256-row tiles
+  bool warm;                 // TN: read both operands once before the first tile (warm_operands)
 };
 // First row of group e.  A null offset table means one group holding all N rows (dense GEMM on the
 // grouped kernels: the gate projection of large expert counts).
@@ -110,6 +111,33 @@ __host__ __device__ __forceinline__ int64_t tn_segment_rows(int64_t K, int64_t M
   const int64_t pitch = (K > M ? K : M) * es;
   const int64_t rows = (0x7fffffffll - 1024) / pitch;
   return rows < 64 ? 64 : rows / 64 * 64;
+}
+
+// TN: a result that does not fit the memory-side cache (256 MB) beside the operands.
+static inline bool gmm_tn_streams(const GmmParams& p) { return p.E * p.K * p.M * 2 >= (256ll << 20); }
+
+// TN of few rows per expert: the results are most of the traffic, and copies of operands that come from
+// HBM queue behind the stores, a latency that the few K tiles of an output tile cannot hide.  One pass over
+// both operands by all workgroups, at the rate of a plain read, leaves them in the memory-side cache.
+__device__ __forceinline__ void warm_bytes(const unsigned char* base, int64_t bytes) {
+  constexpr int DEPTH = 8;
+  const int64_t step = (int64_t)gridDim.x * kGemmThreads * 16;
+  int64_t o = ((int64_t)blockIdx.x * kGemmThreads + threadIdx.x) * 16;
+  u32x4 v[DEPTH];
+  for (; o + (DEPTH - 1) * step < bytes; o += DEPTH * step) {
+#pragma unroll
+    for (int i = 0; i < DEPTH; ++i) v[i] = *reinterpret_cast<const u32x4*>(base + o + i * step);
+#pragma unroll
+    for (int i = 0; i < DEPTH; ++i) asm volatile("" ::"v"(v[i]));
+  }
+  for (; o < bytes; o += step) {
+    v[0] = *reinterpret_cast<const u32x4*>(base + o);
+    asm volatile("" ::"v"(v[0]));
+  }
+}
+__device__ __forceinline__ void warm_operands(const GmmParams& p) {
+  warm_bytes(p.a, p.N * p.K * 2);
+  warm_bytes(p.b, p.N * p.M * 2);
 }
 
 enum { EPI_NONE = 0, EPI_GLU_FWD_SILU = 1, EPI_GLU_FWD_GELU = 2, EPI_GLU_BWD_SILU = 3, EPI_GLU_BWD_GELU = 4 };
@@ -187,6 +215,12 @@ typedef __attribute__((address_space(3))) unsigned char lds_byte;
 
 __device__ __forceinline__ uint32_t lds_offset_of(const void* p) {
   return (uint32_t)(uintptr_t)(lds_byte*)(p);
+}
+
+// ... and back: the object of type T at an LDS offset
+template <typename T>
+__device__ __forceinline__ __attribute__((address_space(3))) T* lds_at(uint32_t offset) {
+  return (__attribute__((address_space(3))) T*)(uintptr_t)offset;
 }
 
 // One LDS-DMA instruction: lane L copies 16 bytes from rsrc[voff + soff] to LDS[lds_base + 16*L].

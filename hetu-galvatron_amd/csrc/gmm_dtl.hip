@@ -16,10 +16,15 @@
 //     LDS reads.
 //   * The K tiles of all of a workgroup's output tiles form one sequence: the last three of a tile
 //     request the first three of the next, and the stores of a tile are left in flight under the next
-//     tile's MFMAs.  Before, each tile waited for its first copies and for its stores with idle matrix
-//     cores, about 10 us of 36 at 1024 rows per expert: dW of 7168 x 4096 over 32 experts 1930 -> 1752 us
-//     (1098 TFLOP/s), 2048 x 2816 over 64 786 -> 707, 1408 x 2048 over 64 433 -> 393; with 4096 rows per
-//     expert the launches are bound by the chip's power and unchanged (6050 us).
+//     tile's MFMAs.
+//   * Long reductions (STORE_SPREAD): a 16-bit result is rounded into half the registers while the next tile's
+//     first MFMAs overwrite the accumulators, and stored piece by piece under the MFMAs after those, so that
+//     the matrix cores see no epilogue (5 us of 33 per tile at 1024 rows per expert).  1024 rows: 7168 x 4096 over
+//     32 experts 1730 -> 1660 us, 2048 x 2816 over 64 750 -> 725; 4096 rows of 4096 x 28672 over 8 6050 -> 5940,
+//     where the chip's power is the bound.
+//   * Large results are stored past the L2s' reusable lines (nontemporal), and few rows per expert read both
+//     operands once beforehand (warm_operands): the launch is then bound by its writes.  4096 x 28672 over 8
+//     experts, operands from HBM: 190 rows each 698 -> 497 us (3.8 TB/s of results), 383 rows 914 -> 772.
 //   * Both operands have the reduction index (the token) as the slow dimension in memory; they are
 //     stored in LDS as they are in memory, [k][outer], and the MFMA fragments are read with the
 //     transposing LDS load ds_read_b64_tr_b16: a group of 16 lanes reads a 4(k) x 16(outer) block
@@ -40,6 +45,8 @@ constexpr int NST = 4;                  // LDS stages
 constexpr int OPER_BYTES = 256 * BKT * 2;  // one operand tile: 16 KiB
 constexpr int STAGE_BYTES = 2 * OPER_BYTES;
 constexpr int LOADS_PER_TILE = 8;       // LDS-DMA instructions per wavefront per K tile (4 per operand)
+
+constexpr int kNontemporal = 2;         // cache policy operand of a buffer store
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 // ---- operand stored outer-contiguous: LDS tile [32 k][256 outer], 512 bytes per k row ----------
@@ -106,12 +113,15 @@ __device__ __forceinline__ float acc_read(float a) {
 // carried across).
 struct Work {
   u32x4 ra, rb;  // the operands' rows, from the tile's first column on
-  int kt_cnt;    // K tiles, at least NST - 1: the copies reach one stretch ahead, never two
+  int kt_cnt;    // K tiles, at least MIN_KT (whole ones past the last row read as zero)
   int e, mt, nt; // e < 0: none left
   bool last;     // the tile's last stretch
 };
 
-template <int DT, int ODT>
+// How a tile's result is stored (the rule is in launch_cfg): after its last K tile, with ordinary or with
+// nontemporal stores, or nontemporally in four K tiles spread over the next tile.
+enum { STORE_NOW, STORE_NOW_STREAM, STORE_SPREAD };
+template <int DT, int ODT, int STORE>
 __global__ __launch_bounds__(kGemmThreads) void gmm_dtl_kernel(GmmParams p) {
   typedef TransOperand OpA;
   typedef TransOperand OpB;
@@ -120,7 +130,11 @@ __global__ __launch_bounds__(kGemmThreads) void gmm_dtl_kernel(GmmParams p) {
   constexpr int NM = 16;  // MFMAs per K step
   constexpr int RA = OpA::READS_PER_FRAG, RB = OpB::READS_PER_FRAG;
   constexpr int NREAD = WT * RA + WT * RB;  // LDS reads per K step
-  constexpr int STORES = ODT == GMOE_F32 ? 0 : 32;  // result stores of a tile left in flight, per wavefront
+  static_assert(ODT != GMOE_F32 || STORE == STORE_NOW, "32-bit results are stored from the accumulators");
+  constexpr bool SPREAD = STORE == STORE_SPREAD;
+  constexpr int STORES = 8;  // stores per wavefront and fragment row of a 16-bit result
+  // the copies reach one stretch ahead, never two; the result of the tile before takes nine
+  constexpr int MIN_KT = SPREAD ? 9 : NST - 1;
   static_assert(NREAD == NM && LOADS_PER_TILE == NM / 2, "one read per MFMA, a copy after every fourth");
 
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
@@ -178,7 +192,7 @@ __global__ __launch_bounds__(kGemmThreads) void gmm_dtl_kernel(GmmParams p) {
     w.ra = make_raw_rsrc(p.a + ((row0 + seg0) * K + (int64_t)w.mt * BM) * 2, (k_lim * K - (int64_t)w.mt * BM) * 2);
     w.rb = make_raw_rsrc(p.b + ((row0 + seg0) * M + (int64_t)w.nt * BN) * 2, (k_lim * M - (int64_t)w.nt * BN) * 2);
     const int kt = (int)((k_lim + BKT - 1) / BKT);
-    w.kt_cnt = kt < NST - 1 ? NST - 1 : kt;
+    w.kt_cnt = kt < MIN_KT ? MIN_KT : kt;
     w.last = left <= seg_rows;
     if (w.last) {
       s = s >= whole ? -1 : (s + G < whole ? s + G : tail_tile());
@@ -209,6 +223,7 @@ __global__ __launch_bounds__(kGemmThreads) void gmm_dtl_kernel(GmmParams p) {
     }
   };
 
+  if (p.warm) warm_operands(p);
   Work cur;
   fetch(cur);
   if (cur.e < 0) return;
@@ -225,109 +240,165 @@ __global__ __launch_bounds__(kGemmThreads) void gmm_dtl_kernel(GmmParams p) {
     frag_read(r, std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{}, lds);
   });
 
+  // ---- the result of a tile: lane holds row (lane%32), columns 8*(v/4) + 4*(lane/32) + v%4 of each 32x32 ----
+  // 16-bit results are rounded into `pk` (half the registers) and go to memory 32 rows x 128 columns at a time,
+  // through 8 KiB of LDS of the wavefront's own: the 16-byte piece c of row r sits in slot c ^ (r & 15).  The
+  // buffer stores carry no condition (rows and columns that do not exist are out of the resource), so each
+  // fragment row leaves STORES of them in flight.
+  constexpr int OES = Elem<ODT>::bytes;
+  u32x2 pk[WT][WT][4];
+  u32x4 sv[4];  // pieces on their way from LDS to memory
+  const uint32_t mine = lds0 + NST * STAGE_BYTES + wave * 8192;
+  // a lane's 8 bytes of slot 0 of its fragment row; its 16 bytes of rows 0..3
+  uint32_t put = mine + (lane & 31) * 256 + (lane & 15) * 16 + 8 * (lane >> 5);
+  uint32_t get = mine + (lane >> 4) * 256 + ((lane & 15) ^ (lane >> 4)) * 16;
+  __amdgpu_buffer_rsrc_t rc;
+  uint32_t vo = 0;
+  const uint32_t four_rows = (uint32_t)(4 * M * OES);
+  auto take = [&](auto i_c, auto j_c) {  // accumulator (i, j) -> pk
+    constexpr int i = decltype(i_c)::value, j = decltype(j_c)::value;
+#pragma unroll
+    for (int vq = 0; vq < 4; ++vq) {
+      pk[i][j][vq] = pack4<ODT>(acc_read(acc[i][j][4 * vq]), acc_read(acc[i][j][4 * vq + 1]),
+                                acc_read(acc[i][j][4 * vq + 2]), acc_read(acc[i][j][4 * vq + 3]));
+      asm volatile("" : "+v"(pk[i][j][vq]));  // rounded here: sunk to its use, the fp32 values spill
+    }
+  };
+  auto stage_put = [&](auto i_c, auto m_c) {  // 4 columns of every row of fragment row i
+    constexpr int i = decltype(i_c)::value, m = decltype(m_c)::value;
+    *lds_at<u32x2>(put ^ (m * 16)) = pk[i][m / 4][m % 4];
+  };
+  auto stage_get = [&](auto t_c) {  // rows 4t .. 4t+3, 256 bytes each
+    constexpr int t = decltype(t_c)::value;
+    sv[t % 4] = *lds_at<const u32x4>((get ^ (t % 4 * 64)) + t * 1024);
+  };
+  auto stage_store = [&](auto t_c) {
+    __builtin_amdgcn_raw_buffer_store_b128(sv[decltype(t_c)::value % 4], rc, (int)vo, 0, STORE == STORE_NOW ? 0 : kNontemporal);
+    vo += four_rows;
+  };
+  auto locate = [&](const Work& w) {  // where the tile's result goes
+    const int64_t c_rows = K - (int64_t)w.mt * BM, n = (int64_t)w.nt * BN + wn * 128 + (lane & 15) * 8;
+    rc = __builtin_amdgcn_make_buffer_rsrc(p.c + ((int64_t)w.e * K + (int64_t)w.mt * BM) * M * OES, 0,
+                                           (int)((c_rows < BM ? c_rows : BM) * M * OES), 0x00020000);
+    vo = n < M ? (uint32_t)(((wm * 128 + (lane >> 4)) * M + n) * OES) : kOob;
+  };
+
   // The K tiles of all stretches form one sequence through the NST stages: the last three of a stretch
   // request the first three of the next, so that neither the first copies of a tile nor the stores of the
   // tile before are waited for with idle matrix cores.
-  bool stored = false;  // the tile before left its STORES in flight
-  int g = 0;            // K tiles done, all stretches
-  for (;;) {
-    Work nx;
-    clear();
-    for (;;) {
-      fetch(nx);
-      for (int kt = 0; kt < cur.kt_cnt; ++kt, ++g) {
-        const unsigned char* here = lds + (g & (NST - 1)) * STAGE_BYTES;
-        const unsigned char* nxt = lds + ((g + 1) & (NST - 1)) * STAGE_BYTES;
-        const uint32_t st3 = lds0 + (uint32_t)(((g + 3) & (NST - 1)) * STAGE_BYTES);
-        const bool own = kt + 3 < cur.kt_cnt;
-        const int kt3 = own ? kt + 3 : kt + 3 - cur.kt_cnt;
-        const u32x4 ra = own ? cur.ra : nx.ra, rb = own ? cur.rb : nx.rb;
-        const uint32_t offa = oa.offset(ra, kt3), offb = ob.offset(rb, kt3);
-        // ---- K step 0: MFMAs on buffer 0; read step 1 into buffer 1; request a of tile kt+3 ---
-        // One fragment read per MFMA and a copy after every fourth: the stage of tile kt-1 is free for
-        // both steps, and copies spread over both are 1-2 % faster than all eight at the end of this
-        // one (dW of fc1 on the Mixtral shape 6.20 -> 6.14 ms, 1.09 -> 1.06 ms for 8192 x 2048 x 11264).
-        static_for<0, NM>([&](auto m_c) {
-          constexpr int m = decltype(m_c)::value;
-          // boustrophedon order over the fragments: one operand changes per MFMA
-          constexpr int mi = m / WT, mj = (mi & 1) ? WT - 1 - m % WT : m % WT;
-          Mma<DT>::run(fa[0][mi], fb[0][mj], acc[mi][mj]);
-          GMOE_SCHED_FENCE();
-          frag_read(m_c, std::integral_constant<int, 1>{}, std::integral_constant<int, 1>{}, here);
-          if constexpr (m % 4 == 2) oa.template issue<m / 4>(ra, offa, st3, wave);
-          GMOE_SCHED_FENCE();
-        });
-        // tile kt+1 must have landed (kt+2 and the half of kt+3 may still be in flight, and for the first
-        // two tiles of a stretch the stores issued between their requests); the barrier also tells everyone
-        // that this tile's stage has been read for the last time
-        if (stored && kt < 2) wait_dma_outstanding<LOADS_PER_TILE + 4 + STORES>();
-        else wait_dma_outstanding<LOADS_PER_TILE + 4>();
-        __syncthreads();
+  int g = 0;  // K tiles done, all stretches
+  Work nx;
+  // One K tile.  kind PLAIN: MFMAs, fragment reads, copies; TAKE: also the result of the tile before out of
+  // the accumulators; 0..3: also fragment row `kind` of it to memory.  `stores`: how many may be in flight
+  // behind the copies of tile kt+1.
+  constexpr int PLAIN = -1, TAKE = -2;
+  auto k_tile = [&](auto kind_c, auto stores_c, int kt) __attribute__((always_inline)) {
+    constexpr int kind = decltype(kind_c)::value;
+    const unsigned char* here = lds + (g & (NST - 1)) * STAGE_BYTES;
+    const unsigned char* nxt = lds + ((g + 1) & (NST - 1)) * STAGE_BYTES;
+    const uint32_t st3 = lds0 + (uint32_t)(((g + 3) & (NST - 1)) * STAGE_BYTES);
+    const bool own = kt + 3 < cur.kt_cnt;
+    const int kt3 = own ? kt + 3 : kt + 3 - cur.kt_cnt;
+    const u32x4 ra = own ? cur.ra : nx.ra, rb = own ? cur.rb : nx.rb;
+    const uint32_t offa = oa.offset(ra, kt3), offb = ob.offset(rb, kt3);
+    if constexpr (kind >= 0) asm volatile("" : "+v"(put), "+v"(get));  // the addresses made of them are not kept
+    // ---- K step 0: MFMAs on buffer 0; read step 1 into buffer 1; request a of tile kt+3 ---
+    // One fragment read per MFMA and a copy after every fourth: the stage of tile kt-1 is free for
+    // both steps, and copies spread over both are 1-2 % faster than all eight at the end of this
+    // one (dW of fc1 on the Mixtral shape 6.20 -> 6.14 ms, 1.09 -> 1.06 ms for 8192 x 2048 x 11264).
+    static_for<0, NM>([&](auto m_c) {
+      constexpr int m = decltype(m_c)::value;
+      // boustrophedon order over the fragments: one operand changes per MFMA
+      constexpr int mi = m / WT, mj = (mi & 1) ? WT - 1 - m % WT : m % WT;
+      if constexpr (kind == TAKE) {
+        // written 16 MFMAs ago, so complete
+        take(std::integral_constant<int, mi>{}, std::integral_constant<int, mj>{});
         GMOE_SCHED_FENCE();
-        // ---- K step 1: MFMAs on buffer 1; read step 0 of tile kt+1 into buffer 0; request b of kt+3
-        static_for<0, NM>([&](auto m_c) {
-          constexpr int m = decltype(m_c)::value;
-          // boustrophedon order over the fragments: one operand changes per MFMA
-          constexpr int mi = m / WT, mj = (mi & 1) ? WT - 1 - m % WT : m % WT;
-          Mma<DT>::run(fa[1][mi], fb[1][mj], acc[mi][mj]);
-          GMOE_SCHED_FENCE();
-          frag_read(m_c, std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{}, nxt);
-          if constexpr (m % 4 == 2) ob.template issue<m / 4>(rb, offb, st3 + OPER_BYTES, wave);
-          GMOE_SCHED_FENCE();
-        });
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[mi][mj][v] = 0.f;
       }
-      if (cur.last) break;
-      stored = false;
-      cur = nx;
-    }
-    stored = STORES > 0;
-
-    // ---- epilogue: lane holds row (lane%32), columns 8*(v/4) + 4*(lane/32) + v%4 of each 32x32 ----
-    constexpr int OES = Elem<ODT>::bytes;
-    unsigned char* c_tile = p.c + ((int64_t)cur.e * K + (int64_t)cur.mt * BM) * M * OES;
-    const int64_t c_rows = K - (int64_t)cur.mt * BM;
-    if constexpr (ODT != GMOE_F32) {
-      // 32 rows x 128 columns at a time through the wavefront's own 2 x 4 KiB of the stage that was read
-      // last: the pieces its own copies fill next, so no barrier is needed.  The 16-byte piece c of row r
-      // sits in slot c ^ (r & 15).  The buffer stores carry no condition (rows and columns that do not
-      // exist are out of the resource), so STORES of them are in flight.
-      unsigned char* mine = lds + ((g - 1) & (NST - 1)) * STAGE_BYTES + wave * 4096;
-      const auto rc = __builtin_amdgcn_make_buffer_rsrc(
-          c_tile, 0, (int)((c_rows < BM ? c_rows : BM) * M * OES), 0x00020000);
-      asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // the last MFMA's result, read by acc_read
+      Mma<DT>::run(fa[0][mi], fb[0][mj], acc[mi][mj]);
       GMOE_SCHED_FENCE();
-      int ln = lane;
-      asm volatile("" : "+v"(ln));  // the addresses below are computed here, not kept through the main loop
-      const int64_t n = (int64_t)cur.nt * BN + wn * 128 + (ln & 15) * 8;
-      uint32_t vo = n < M ? (uint32_t)(((wm * 128 + (ln >> 4)) * M + n) * OES) : kOob;
-      const uint32_t four_rows = (uint32_t)(4 * M * OES);
-      const int r = ln & 31;
-      unsigned char* w = mine + (r >> 4) * OPER_BYTES + (r & 15) * 256 + 8 * (ln >> 5);
-#pragma unroll
-      for (int i = 0; i < WT; ++i) {
-#pragma unroll
-        for (int j = 0; j < WT; ++j)
-#pragma unroll
-          for (int vq = 0; vq < 4; ++vq)
-            *reinterpret_cast<u32x2*>(w + ((j * 4 + vq) ^ (r & 15)) * 16) =
-                pack4<ODT>(acc_read(acc[i][j][4 * vq]), acc_read(acc[i][j][4 * vq + 1]),
-                           acc_read(acc[i][j][4 * vq + 2]), acc_read(acc[i][j][4 * vq + 3]));
-        GMOE_SCHED_FENCE();
-        u32x4 v[8];
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-          const int row = t * 4 + (ln >> 4);
-          v[t] = *reinterpret_cast<const u32x4*>(mine + (row >> 4) * OPER_BYTES + (row & 15) * 256 +
-                                                 (((ln & 15) ^ (row & 15)) * 16));
-        }
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-          __builtin_amdgcn_raw_buffer_store_b128(v[t], rc, (int)vo, 0, 0);
-          vo += four_rows;
-        }
-        GMOE_SCHED_FENCE();
+      frag_read(m_c, std::integral_constant<int, 1>{}, std::integral_constant<int, 1>{}, here);
+      if constexpr (kind >= 0) stage_put(kind_c, m_c);
+      if constexpr (m % 4 == 2) oa.template issue<m / 4>(ra, offa, st3, wave);
+      GMOE_SCHED_FENCE();
+    });
+    // tile kt+1 must have landed (kt+2, the half of kt+3 and stores issued since may still be in flight);
+    // the barrier also tells everyone that this tile's stage has been read for the last time
+    wait_dma_outstanding<LOADS_PER_TILE + 4 + decltype(stores_c)::value>();
+    __syncthreads();
+    GMOE_SCHED_FENCE();
+    // ---- K step 1: MFMAs on buffer 1; read step 0 of tile kt+1 into buffer 0; request b of kt+3
+    static_for<0, NM>([&](auto m_c) {
+      constexpr int m = decltype(m_c)::value;
+      constexpr int mi = m / WT, mj = (mi & 1) ? WT - 1 - m % WT : m % WT;
+      Mma<DT>::run(fa[1][mi], fb[1][mj], acc[mi][mj]);
+      GMOE_SCHED_FENCE();
+      if constexpr (kind >= 0) {
+        if constexpr (m >= 4 && m < 12) stage_store(std::integral_constant<int, m - 4>{});
+        if constexpr (m < 8) stage_get(m_c);
+      }
+      frag_read(m_c, std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{}, nxt);
+      if constexpr (m % 4 == 2) ob.template issue<m / 4>(rb, offb, st3 + OPER_BYTES, wave);
+      GMOE_SCHED_FENCE();
+    });
+    ++g;
+  };
+  constexpr std::integral_constant<int, PLAIN> plain{};
+  constexpr std::integral_constant<int, 0> none{};
+  constexpr std::integral_constant<int, STORES> some{};
+  constexpr std::integral_constant<int, WT * STORES> all{};
+  // fragment row i at once, with no MFMAs beside it
+  auto store_row = [&](auto i_c) {
+    GMOE_SCHED_FENCE();
+    static_for<0, WT>([&](auto j_c) { take(i_c, j_c); });
+    static_for<0, 16>([&](auto m_c) { stage_put(i_c, m_c); });
+    static_for<0, 2>([&](auto h_c) {
+      constexpr int h = decltype(h_c)::value;
+      static_for<4 * h, 4 * h + 4>(stage_get);
+      static_for<4 * h, 4 * h + 4>(stage_store);
+    });
+    GMOE_SCHED_FENCE();
+  };
+
+  bool pending = false;  // there is a tile before, its result in the accumulators (SPREAD) or on its way
+  for (;;) {
+    fetch(nx);
+    int kt = 0;
+    if (SPREAD && pending) {
+      const int stride = (cur.kt_cnt - 1) / WT;
+      k_tile(std::integral_constant<int, TAKE>{}, none, kt++);
+      static_for<0, WT>([&](auto i_c) __attribute__((always_inline)) {
+        k_tile(i_c, none, kt++);
+        k_tile(plain, some, kt++);
+        if constexpr (decltype(i_c)::value + 1 < WT)
+          for (int r = 2; r < stride; ++r) k_tile(plain, none, kt++);
+      });
+    } else {
+      clear();
+      // the copies of the first two tiles were requested before the stores
+      if (ODT != GMOE_F32 && pending)
+        for (; kt < 2; ++kt) k_tile(plain, all, kt);
+    }
+    for (;;) {
+      for (; kt < cur.kt_cnt; ++kt) k_tile(plain, none, kt);
+      if (cur.last) break;
+      cur = nx;
+      fetch(nx);
+      kt = 0;
+    }
+    pending = true;
+    if constexpr (ODT != GMOE_F32) {
+      locate(cur);
+      if constexpr (!SPREAD) {
+        asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // the last MFMA's result, read by acc_read
+        asm volatile("" : "+v"(put), "+v"(get));
+        static_for<0, WT>(store_row);
       }
     } else {
+      unsigned char* c_tile = p.c + ((int64_t)cur.e * K + (int64_t)cur.mt * BM) * M * OES;
+      const int64_t c_rows = K - (int64_t)cur.mt * BM;
 #pragma unroll
       for (int i = 0; i < WT; ++i) {
         const int64_t m = wm * 128 + i * 32 + (lane & 31);
@@ -347,13 +418,17 @@ __global__ __launch_bounds__(kGemmThreads) void gmm_dtl_kernel(GmmParams p) {
     if (nx.e < 0) break;
     cur = nx;
   }
+  if constexpr (SPREAD) {
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // the last MFMA's result, read by acc_read
+    static_for<0, WT>(store_row);
+  }
   wait_dma_outstanding<0>();  // nothing may land in LDS after the workgroup has ended
 }
 
-template <int DT, int ODT>
-static int launch_cfg(const GmmParams& p, hipStream_t st) {
-  constexpr size_t smem = (size_t)NST * STAGE_BYTES;
-  auto kern = gmm_dtl_kernel<DT, ODT>;
+template <int DT, int ODT, int STORE>
+static int launch_kernel(const GmmParams& p, hipStream_t st) {
+  constexpr size_t smem = (size_t)NST * STAGE_BYTES + (ODT == GMOE_F32 ? 0 : 4 * 8192)  /* a wavefront's staging */;
+  auto kern = gmm_dtl_kernel<DT, ODT, STORE>;
   static std::atomic<uint64_t> done_mask{0};
   if (!gmoe_once_per_device(done_mask, [&] {
         return hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
@@ -364,6 +439,24 @@ static int launch_cfg(const GmmParams& p, hipStream_t st) {
   if (grid < 8) grid = 8;
   hipLaunchKernelGGL(kern, dim3(grid), dim3(kGemmThreads), smem, st, p);
   return gmoe_launch_status();
+}
+
+// n = rows per expert, us, operands not in a cache:
+//   * n 1024: stores spread over the next tile 1658 against 1711 after the tile (7168 x 4096, 32 experts), 677
+//     against 688 (2048 x 2816, 64), 1741 against 1699 (4096 x 28672, 8).  At 640 the copies wait behind the spread
+//     stores (1278 against 1141, 4096 x 28672).
+//   * nontemporal against ordinary stores: 895 against 924 (n 448, 4096 x 28672, 8), 388 against 399 (n 512, 2048 x 2816,
+//     64), 304 against 347 (n 256, 14336 x 4096, 8).  Results that the memory-side cache holds are better left there
+//     (n 256, 8 experts of 1024 x 4096, 64 MB: 30 against 39).
+template <int DT, int ODT>
+static int launch_cfg(const GmmParams& p, hipStream_t st) {
+  if constexpr (ODT == GMOE_F32) {
+    return launch_kernel<DT, ODT, STORE_NOW>(p, st);
+  } else {
+    if (p.N / (p.E > 0 ? p.E : 1) >= 900) return launch_kernel<DT, ODT, STORE_SPREAD>(p, st);
+    if (gmm_tn_streams(p)) return launch_kernel<DT, ODT, STORE_NOW_STREAM>(p, st);
+    return launch_kernel<DT, ODT, STORE_NOW>(p, st);
+  }
 }
 
 }  // namespace dtl

@@ -107,3 +107,26 @@ def test_long_reduction_edges(pkg, dev, dtype, K, M):
         # as above; the sums of a long reduction stay within a few sqrt(n)
         assert (got32[e].double() - want).abs().max().item() <= 2.0 ** -24 * 25 * min(n, 100 * n ** 0.5) * 4
         s += n
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("K,M", [(1160, 1096), (520, 4104)])
+def test_medium_reduction_edges(pkg, dev, dtype, K, M):
+    """dW on 256x256 tiles that are stored in the next tile's first six K tiles (of 32 rows): fewer rows
+    than that, one more or less, empty experts in turn, and more; output edges inside a tile."""
+    rows = [0, 1, 33, 159, 160, 161, 0, 191, 192, 193, 223, 225, 0, 900, 64, 700]
+    E, N = len(rows), sum(rows)
+    g = torch.Generator(device=dev).manual_seed(K + M)
+    print("case", dtype, K, M, flush=True)
+    off = torch.tensor([0] + rows, device=dev).cumsum(0)
+    a = torch.empty(N, K, device=dev).normal_(generator=g).to(dtype)
+    b = torch.empty(N, M, device=dev).normal_(generator=g).to(dtype)
+    got32 = on_kernel("gmm_dtl_kernel", lambda: pkg.ops.gmm(a, b, off, trans_a=True, out_dtype=torch.float32))
+    got = on_kernel("gmm_dtl_kernel", lambda: pkg.ops.gmm(a, b, off, trans_a=True))
+    assert torch.equal(got, got32.to(dtype))
+    s = 0
+    for e, n in enumerate(rows):
+        want = a[s:s + n].double().t().contiguous() @ b[s:s + n].double()
+        # as in test_long_reduction_edges
+        assert (got32[e].double() - want).abs().max().item() <= 2.0 ** -24 * 25 * min(n, 100 * n ** 0.5) * 4
+        s += n
