@@ -6,6 +6,8 @@
 //   plan_count  per 256-token chunk and expert: number of routed tokens (wavefront ballots)
 //   plan_scan   one exclusive scan over the (expert-major) chunk counts
 //   plan_fill   rank inside the chunk from the ballots + chunk base -> destination rows
+// Up to 8192 chunk counts plan_fill adds up what it needs of them itself, and of a map of up to 16384 entries it
+// counts that too: two launches or one.
 // The plan is kept token-major (dst_map [T,E] int32) so that the row kernels, which run one
 // wavefront per token, find all destinations of a token in one coalesced load.
 //
@@ -13,6 +15,7 @@
 // instruction), with streaming (nontemporal) hints on data that is touched once: scatter (permute), gather-reduce in fp32 (unpermute; also permute's backward) and
 // the backward of the weighted unpermute including the gate gradients.
 #include <mutex>
+#include <type_traits>
 
 #include "gmoe_common.h"
 
@@ -120,34 +123,161 @@ __global__ __launch_bounds__(kScanThreads) void plan_scan_kernel(const int* coun
   }
 }
 
+// Where plan_fill has its bases from: the scan's prefixes, the chunk counts or the routing map itself.  A launch
+// of this size is all latency (5 us each under the profiler), so the fewest that the size allows are taken: with
+// few counts every workgroup adds up the ones before its own, with a small map it counts the map
+// (permute_plan_launch has the limits).
+enum { BASE_SCANNED, BASE_COUNTS, BASE_MAP };
+
+constexpr int kFillExperts = 8;
+
+// Bytes of w that are not zero, as 0x01 each.
+__device__ __forceinline__ uint32_t nonzero_bytes(uint32_t w) {
+  return ((((w & 0x7f7f7f7fu) + 0x7f7f7f7fu) | w) >> 7) & 0x01010101u;
+}
+
+// The map's bytes of token t for the slice's experts, zero past the last token or expert.
+__device__ __forceinline__ uint64_t slice_bits(const uint8_t* map, int64_t t, int64_t T, int E, int vec8, int e_begin,
+                                               int e_cnt) {
+  if (t >= T) return 0ull;
+  const uint8_t* row = map + t * E + e_begin;
+  if (vec8) return *reinterpret_cast<const uint64_t*>(row);  // E % 8 == 0 and an 8-byte aligned map
+  uint64_t bits = 0;
+#pragma unroll
+  for (int j = 0; j < kFillExperts; ++j)
+    if (j < e_cnt) bits |= (uint64_t)row[j] << (8 * j);
+  return bits;
+}
+
+// For the workgroup's slice of experts: s_before = tokens of all experts before the slice, s_total[j] = tokens of
+// its expert j, s_chunk[j] = those of them before this chunk.  Ends with a barrier.
+template <int BASE>
+__device__ __forceinline__ void slice_base(const uint8_t* map, const int* counts, int64_t T, int E, int NC, int vec8, int vec4,
+                                           int e_begin, int e_cnt, int& s_before, int* s_total, int* s_chunk) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  if (tid < kFillExperts) s_total[tid] = s_chunk[tid] = 0;
+  if (tid == kFillExperts) s_before = 0;
+  __syncthreads();
+  int before = 0;
+  if constexpr (BASE == BASE_COUNTS) {
+    const int own = e_begin * NC, end = own + e_cnt * NC;
+    for (int i0 = tid; i0 < own; i0 += 8 * kChunkTokens) {
+      int v[8];  // eight loads in flight: one at a time, their latency is the launch
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const int i = i0 + q * kChunkTokens;
+        v[q] = i < own ? counts[i] : 0;
+      }
+#pragma unroll
+      for (int q = 0; q < 8; ++q) before += v[q];
+    }
+    for (int i = own + tid; i < end; i += kChunkTokens) {
+      const int j = (i - own) / NC, c = i - own - j * NC, v = counts[i];
+      if (v == 0) continue;
+      atomicAdd(&s_total[j], v);
+      if (c < (int)blockIdx.x) atomicAdd(&s_chunk[j], v);
+    }
+  } else {
+    // the slice's own experts by ballots, four chunks' loads in flight
+    int tot[kFillExperts] = {}, part[kFillExperts] = {};
+    for (int c0 = 0; c0 < NC; c0 += 4) {
+      uint64_t bits[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int64_t t = (int64_t)(c0 + q) * kChunkTokens + tid;
+        bits[q] = slice_bits(map, t, T, E, vec8, e_begin, e_cnt);
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int j = 0; j < kFillExperts; ++j) {
+          const int n = __popcll(__ballot(((bits[q] >> (8 * j)) & 0xffull) != 0));
+          tot[j] += n;
+          part[j] += c0 + q < (int)blockIdx.x ? n : 0;
+        }
+    }
+    if (lane == 0) {
+#pragma unroll
+      for (int j = 0; j < kFillExperts; ++j) {
+        atomicAdd(&s_total[j], tot[j]);
+        atomicAdd(&s_chunk[j], part[j]);
+      }
+    }
+    // the columns before them
+    if (vec4) {
+      const uint32_t words = e_begin / 4, all = (uint32_t)T * words;
+      for (uint32_t i0 = tid; i0 < all; i0 += 8 * kChunkTokens) {
+        uint32_t v[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+          const uint32_t i = i0 + q * kChunkTokens, t = i / words;
+          v[q] = i < all ? *reinterpret_cast<const uint32_t*>(map + (int64_t)t * E + (i - t * words) * 4) : 0u;
+        }
+#pragma unroll
+        for (int q = 0; q < 8; ++q) before += __popc(nonzero_bytes(v[q]));
+      }
+    } else {
+      const uint32_t cols = e_begin, all = (uint32_t)T * cols;
+      for (uint32_t i0 = tid; i0 < all; i0 += 8 * kChunkTokens) {
+        uint8_t v[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+          const uint32_t i = i0 + q * kChunkTokens, t = i / cols;
+          v[q] = i < all ? map[(int64_t)t * E + (i - t * cols)] : 0;
+        }
+#pragma unroll
+        for (int q = 0; q < 8; ++q) before += v[q] != 0;
+      }
+    }
+  }
+  if (e_begin > 0) {
+    const int sum = (int)wave_sum_f32((float)before);  // exact: below 2^24
+    if (lane == 0) atomicAdd(&s_before, sum);
+  }
+  __syncthreads();
+}
+
 // Workgroup (chunk, slice): the destination rows of 256 tokens for kFillExperts consecutive experts.
 // Slicing the experts keeps the grid at chunks x E / 8 workgroups (a 64-expert router over 8192
 // tokens has only 32 chunks) and lets a lane write its token's 8 destinations as two 16-byte stores.
-constexpr int kFillExperts = 8;
-
+// Unless the bases are scanned already, the first chunk's workgroups also write the experts' totals and offsets.
+template <int BASE>
 __global__ __launch_bounds__(kChunkTokens) void plan_fill_kernel(
-    const uint8_t* map, int64_t T, int E, int NC, int vec8, int64_t capacity, const int* base,
-    int32_t* dst_map, long long* sorted_indices, int64_t sorted_cap, long long* row_id_map) {
+    const uint8_t* map, int64_t T, int E, int NC, int vec8, int vec4, int64_t capacity, const int* base,
+    int32_t* dst_map, long long* sorted_indices, int64_t sorted_cap, long long* row_id_map,
+    long long* tokens_per_expert, long long* expert_offsets) {
   __shared__ unsigned long long bal[kChunkTokens / 64][kFillExperts];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int64_t t = (int64_t)blockIdx.x * kChunkTokens + tid;
   const bool valid = t < T;
   const int e_begin = blockIdx.y * kFillExperts;
   const int e_cnt = E - e_begin < kFillExperts ? E - e_begin : kFillExperts;
-  const uint8_t* row = map + (valid ? t : 0) * (int64_t)E + e_begin;
-  if (vec8) {  // E % 8 == 0 and an 8-byte aligned map: one load covers the slice
-    const uint64_t bits = valid ? *reinterpret_cast<const uint64_t*>(row) : 0ull;
+  int expert_base[kFillExperts];  // of the first token of this chunk
+  if constexpr (BASE != BASE_SCANNED) {
+    __shared__ int s_before, s_total[kFillExperts], s_chunk[kFillExperts];
+    slice_base<BASE>(map, base, T, E, NC, vec8, vec4, e_begin, e_cnt, s_before, s_total, s_chunk);
+    int run = s_before;
 #pragma unroll
     for (int j = 0; j < kFillExperts; ++j) {
-      const uint64_t b = __ballot(((bits >> (8 * j)) & 0xffull) != 0);
-      if (lane == 0) bal[wave][j] = b;
+      expert_base[j] = s_chunk[j] + (capacity > 0 ? 0 : run);
+      if (blockIdx.x == 0 && tid == j && j < e_cnt) {
+        tokens_per_expert[e_begin + j] = capacity > 0 ? capacity : s_total[j];
+        expert_offsets[e_begin + j] = capacity > 0 ? (e_begin + j) * capacity : run;
+      }
+      run += s_total[j];
     }
+    if (blockIdx.x == 0 && tid == 0 && e_begin + e_cnt == E)
+      expert_offsets[E] = capacity > 0 ? (long long)E * capacity : run;
   } else {
 #pragma unroll
-    for (int j = 0; j < kFillExperts; ++j) {
-      const uint64_t b = __ballot(valid && j < e_cnt && row[j] != 0);
-      if (lane == 0) bal[wave][j] = b;
-    }
+    for (int j = 0; j < kFillExperts; ++j)
+      expert_base[j] = j < e_cnt ? base[(int64_t)(e_begin + j) * NC + blockIdx.x] : 0;
+  }
+  const uint64_t bits = slice_bits(map, t, T, E, vec8, e_begin, e_cnt);
+#pragma unroll
+  for (int j = 0; j < kFillExperts; ++j) {
+    const uint64_t b = __ballot(((bits >> (8 * j)) & 0xffull) != 0);
+    if (lane == 0) bal[wave][j] = b;
   }
   __syncthreads();
   const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
@@ -161,7 +291,7 @@ __global__ __launch_bounds__(kChunkTokens) void plan_fill_kernel(
     for (int w = 0; w < wave; ++w) before += __popcll(bal[w][j]);
     const uint64_t b = bal[wave][j];
     const bool pred = (b >> lane) & 1ull;
-    int64_t rank = (int64_t)base[(int64_t)e * NC + blockIdx.x] + before + __popcll(b & lt);
+    int64_t rank = (int64_t)expert_base[j] + before + __popcll(b & lt);
     int64_t dst;
     if (capacity > 0)
       dst = rank < capacity ? (int64_t)e * capacity + rank : -1;
@@ -642,6 +772,12 @@ static inline int dtype_bytes(int dt) {
     default: return 0;
   }
 }
+// Largest map that every workgroup of plan_fill counts by itself, and most chunk counts that every one adds up.
+// Times of a plan in a graph's replay, us: from the map 5.8 against 7.5 with three launches (128 x 4), 7.9 against 9.5
+// (1531 x 8), but 16.3 against 9.2 at 65536 entries (16384 x 4); from the counts 11.9 against 14.8 (8192 x 64, 2048
+// counts), 14.2 against 18.3 (4096 counts), 42.5 against 39.3 at 16384 counts.  Issued one by one, each launch less
+// is 4 to 5 us of host time as well.
+constexpr int64_t kMapEntries = 16 * 1024, kCountEntries = 8 * 1024;
 static inline bool prob_dtype_ok(int dt) { return dt == GMOE_F32 || dt == GMOE_BF16 || dt == GMOE_F16; }
 
 }  // namespace gmoe
@@ -685,24 +821,36 @@ extern "C" int64_t gmoe_permute_plan_workspace_bytes(int64_t T, int E) {
   return 2 * (int64_t)E * (NC > 0 ? NC : 1) * (int64_t)sizeof(int);
 }
 
-// Argument checks and the three plan launches; counts / base are E * max(NC, 1) ints each.
+// The plan launches; counts / base are E * max(NC, 1) ints each.
 static int permute_plan_launch(const uint8_t* routing_map, int64_t T, int E, int64_t capacity,
                                int32_t* dst_map, int64_t* sorted_indices, int64_t sorted_cap,
                                int64_t* row_id_map, int64_t* tokens_per_expert,
                                int64_t* expert_offsets, int* counts, int* base, hipStream_t st) {
   const int NC = (int)((T + kChunkTokens - 1) / kChunkTokens);
   const int vec8 = ((E & 7) == 0 && gmoe_aligned(routing_map, 8)) ? 1 : 0;
+  const int vec4 = ((E & 3) == 0 && gmoe_aligned(routing_map, 4)) ? 1 : 0;
+  auto fill = [&](auto base_c, const int* table) {
+    hipLaunchKernelGGL(plan_fill_kernel<decltype(base_c)::value>, dim3(NC, (E + kFillExperts - 1) / kFillExperts),
+                       dim3(kChunkTokens), 0, st, routing_map, T, E, NC, vec8, vec4, capacity, table, dst_map,
+                       reinterpret_cast<long long*>(sorted_indices), sorted_cap,
+                       reinterpret_cast<long long*>(row_id_map), reinterpret_cast<long long*>(tokens_per_expert),
+                       reinterpret_cast<long long*>(expert_offsets));
+  };
+  if (NC > 0 && T * E <= kMapEntries) {
+    fill(std::integral_constant<int, BASE_MAP>{}, nullptr);
+    return gmoe_launch_status();
+  }
   if (NC > 0)
     hipLaunchKernelGGL(plan_count_kernel, dim3(NC), dim3(kChunkTokens), (size_t)E * 4 * sizeof(int),
                        st, routing_map, T, E, NC, vec8, counts);
+  if (NC > 0 && (int64_t)E * NC <= kCountEntries) {
+    fill(std::integral_constant<int, BASE_COUNTS>{}, counts);
+    return gmoe_launch_status();
+  }
   hipLaunchKernelGGL(plan_scan_kernel, dim3(1), dim3(kScanThreads), 0, st, counts, E, NC, capacity,
                      base, reinterpret_cast<long long*>(tokens_per_expert),
                      reinterpret_cast<long long*>(expert_offsets));
-  if (NC > 0)
-    hipLaunchKernelGGL(plan_fill_kernel, dim3(NC, (E + kFillExperts - 1) / kFillExperts),
-                       dim3(kChunkTokens), 0, st, routing_map, T, E, NC,
-                       vec8, capacity, base, dst_map, reinterpret_cast<long long*>(sorted_indices),
-                       sorted_cap, reinterpret_cast<long long*>(row_id_map));
+  if (NC > 0) fill(std::integral_constant<int, BASE_SCANNED>{}, base);
   return gmoe_launch_status();
 }
 

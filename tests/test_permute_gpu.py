@@ -263,3 +263,30 @@ def test_unpermute_with_residual_equals_unpermute_then_add(pkg, dev, dtype, T, E
         plain.backward(go.to(dev))
         assert fused.dtype == dtype and torch.equal(fused, plain)
         assert torch.equal(rg.grad, go.to(dev)) and torch.equal(yg.grad, y2.grad)
+
+
+@pytest.mark.parametrize("capacity", [0, 37])
+@pytest.mark.parametrize("T,E", [(1, 1), (255, 3), (256, 4), (257, 12), (2048, 8), (2049, 8), (4096, 4), (273, 60), (274, 60),
+                                 (1024, 16), (1025, 16), (32768, 64), (32769, 64)])
+def test_plan_at_the_limits_of_its_launches(pkg, dev, T, E, capacity):
+    """One launch up to 16384 map entries, two up to 8192 chunk counts, three beyond; a last slice of fewer than
+    eight experts; an expert without tokens and one with all of them."""
+    g = torch.Generator().manual_seed(T + E)
+    m = torch.rand(T, E, generator=g) < 0.3
+    m[:, -1] = True
+    m[:, E // 2] = False
+    counts = m.sum(0)
+    rank = m.long().cumsum(0) - 1
+    if capacity:
+        base, kept = torch.arange(E + 1) * capacity, m & (rank < capacity)
+        want_counts, n = torch.full((E,), capacity), E * capacity
+    else:
+        base, kept = torch.cat([torch.zeros(1, dtype=torch.long), counts.cumsum(0)]), m
+        want_counts, n = counts, int(counts.sum())
+    want = torch.where(kept, rank + base[:-1], torch.full_like(rank, -1))
+    print("case", T, E, capacity, flush=True)
+    dst, order, row_ids, got_counts, offsets = pkg._C.host().permute_plan(m.to(dev), n, capacity, True, True)
+    assert torch.equal(dst.cpu().long(), want) and torch.equal(row_ids.cpu(), want.t())
+    assert torch.equal(got_counts.cpu(), want_counts) and torch.equal(offsets.cpu(), base)
+    tokens = torch.arange(T)[:, None].expand(T, E)
+    assert torch.equal(order.cpu()[want[kept]], tokens[kept])
