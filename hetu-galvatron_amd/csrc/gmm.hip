@@ -1216,17 +1216,20 @@ static inline bool gmm_use_remainder(const GmmParams& p) {
 // Whether a 128x128-tile NN / NT launch is worth a split reduction, from the host-side sizes (an expert
 // has at least one row tile, and its last one is half full on average); the kernels decide again from the
 // tiles there are.
-//
-// fp32: the alternative is gmm_f32.hip, which needs no workspace and is ahead from 144 tiles on (us, K x M,
-// experts, rows: 65 split against 63, 1024 x 512, 8, 4096); with a few dozen tiles it leaves CUs idle (20
-// against 30, 512 x 128, 4, 400; 46 against 162, 3584 x 896, 4, 130).  Hence at least four pieces.
-static inline bool gmm_split_pays(const GmmParams& p, int dtype) {
-  const int es = dtype == GMOE_F32 ? 4 : 2;
+static inline bool gmm_split_pays(const GmmParams& p) {
   const int64_t least = p.N < p.E ? p.N : p.E, average = (p.N + 127) / 128 + p.E / 2;
   const int64_t tiles = (average > least ? average : least) * ((p.M + 127) / 128);
-  if (dtype == GMOE_F32 && tiles * 4 > kSplitSlots) return false;
-  return split_pieces(split_ns_per_k_tile(es), (p.K * es + 127) / 128, tiles, kSplitSlots,
-                      weight_stream_ns(p.E, p.K, p.M, es)) > 1;
+  return split_pieces(split_ns_per_k_tile(2), (p.K * 2 + 127) / 128, tiles, kSplitSlots,
+                      weight_stream_ns(p.E, p.K, p.M, 2)) > 1;
+}
+
+// fp32 values of workspace that an NN / NT launch can use.
+static inline int64_t gmm_workspace_floats(const GmmParams& p, int mode, int dtype) {
+  if (dtype == GMOE_F32) {
+    const int pieces = gmm_f32_pieces(p.E, p.N, p.K, p.M);
+    return pieces > 1 ? pieces * p.N * p.M : 0;
+  }
+  return (gmm_large_tiles(p, mode) && gmm_use_remainder(p)) || gmm_split_pays(p) ? (int64_t)kSplitSlots * 128 * 128 : 0;
 }
 
 // A split launch with 128x128 tiles: the pieces, then their sums.
@@ -1267,7 +1270,7 @@ static int launch_gmm_remainder(const GmmParams& p, hipStream_t st) {
 //             the register-staged form);
 // Small groups: 128x128 tiles, two workgroups per CU.
 // fp32: three bf16 planes per operand on the bf16 matrix cores (gmm_f32.hip), 1.3-1.9 times as fast as the fp32
-// MFMA with a smaller error; the fp32 MFMA kernels serve split reductions and dW of operands beyond 2 GiB.
+// MFMA with a smaller error; the fp32 MFMA kernels serve dW of operands beyond 2 GiB.
 template <int DT, int ODT, int MODE, int EPI>
 static int launch_gmm_16bit(const GmmParams& p, int dtype, int out_dtype, hipStream_t st) {
   constexpr bool glu_fwd = EPI == EPI_GLU_FWD_SILU || EPI == EPI_GLU_FWD_GELU;
@@ -1306,7 +1309,7 @@ static int launch_gmm_16bit(const GmmParams& p, int dtype, int out_dtype, hipStr
     return GMOE_ERR_UNSUPPORTED;  // the caller runs the GEMM and the activation kernel instead
   } else {
     if constexpr (MODE != MODE_TN && EPI == EPI_NONE) {
-      if (p.ws != nullptr && p.ws_floats >= 2 * 128 * 128 && gmm_split_pays(p, dtype))
+      if (p.ws != nullptr && p.ws_floats >= 2 * 128 * 128 && gmm_split_pays(p))
         return launch_gmm_split<DT, ODT, MODE>(p, st);
     }
     return launch_gmm_cfg<DT, ODT, MODE, 128, 128, EPI>(p, st, 2);
@@ -1322,8 +1325,11 @@ static int launch_gmm_fp32(const GmmParams& p, hipStream_t st) {
       return launch_gmm_cfg<GMOE_F32, GMOE_F32, MODE, 128, 128, EPI>(p, st, 2);
     }
   } else if constexpr (EPI == EPI_NONE) {
-    if (p.ws != nullptr && p.ws_floats >= 2 * 128 * 128 && gmm_split_pays(p, GMOE_F32))
-      return launch_gmm_split<GMOE_F32, GMOE_F32, MODE>(p, st);
+    GmmParams q = p;
+    q.pieces = gmm_f32_pieces(p.E, p.N, p.K, p.M);
+    const int64_t room = p.ws != nullptr ? p.ws_floats / (p.N * p.M) : 0;
+    if (q.pieces > room) q.pieces = room < 2 ? 1 : (int)room;
+    return launch_gmm_f32(q, MODE, EPI, st);
   }
   return launch_gmm_f32(p, MODE, EPI, st);
 }
@@ -1401,6 +1407,7 @@ static int gmm_check(GmmParams& p, const void* a, const void* b, void* c, const 
   p.split_slots = 0;
   p.stream_ns = 0;
   p.main_grid = 0;
+  p.pieces = 1;
   p.warm = false;
   return GMOE_OK;
 }
@@ -1425,9 +1432,7 @@ int64_t gmm_dense_workspace_floats(int64_t N, int64_t K, int64_t M, int mode, in
   p.N = N;
   p.K = K;
   p.M = M;
-  const bool split =
-      (dtype != GMOE_F32 && gmm_large_tiles(p, mode) && gmm_use_remainder(p)) || gmm_split_pays(p, dtype);
-  return split ? (int64_t)kSplitSlots * 128 * 128 : 0;
+  return gmm_workspace_floats(p, mode, dtype);
 }
 
 int gmm_grouped_tn(const void* a, const void* b, void* c, const int64_t* offsets, int groups, int64_t N,
@@ -1450,10 +1455,7 @@ extern "C" int64_t gmoe_gmm_workspace_bytes(int E, int64_t N, int64_t K, int64_t
   p.N = N;
   p.K = K;
   p.M = M;
-  const int mode = trans_b ? MODE_NT : MODE_NN;
-  const bool split =
-      (dtype != GMOE_F32 && gmm_large_tiles(p, mode) && gmm_use_remainder(p)) || gmm_split_pays(p, dtype);
-  return split ? (int64_t)kSplitSlots * 128 * 128 * 4 : 0;
+  return gmm_workspace_floats(p, trans_b ? MODE_NT : MODE_NN, dtype) * 4;
 }
 
 extern "C" int gmoe_gmm(const void* a, const void* b, void* c, const int64_t* expert_offsets, int E,

@@ -79,6 +79,7 @@ struct GmmParams {
   int split_slots;           // tiles x splits this launch may spread over; 0 = never split
   int64_t stream_ns;         // time the weights take to stream: a split launch cannot be faster
   int main_grid;             // ROWS_AUTO_*: workgroups of the launch with 256-row tiles
+  int pieces;                // fp32 NN / NT: pieces of the reduction, from the host (gmm_f32.hip); 1 = whole
   bool warm;                 // TN: read both operands once before the first tile (warm_operands)
 };
 // First row of group e.  A null offset table means one group holding all N rows (dense GEMM on the

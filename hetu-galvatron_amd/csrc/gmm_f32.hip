@@ -23,6 +23,10 @@
 //   * Tiles of RF*64 rows (RF = 1, 2: an expert's rows are shared out in 64-row units) x 128 columns, 2x2
 //     wavefronts of (RF*32) x 64, two workgroups per CU: one splits operands while the other multiplies.  With
 //     at most one tile per CU the tiles are cut to 64 rows (4096 x 1024 x 512 over 8 experts 75 -> 62 us).
+//   * NN / NT launches that leave CUs idle cut their reduction into pieces (gmm_f32_pieces in split_rule.h).  A
+//     piece's results go to the workspace as a matrix of their own, and a second launch adds the matrices, bound by
+//     that traffic: dX of 4096 x 2048 x 512 over 8 experts 102 -> 70 us, 2000 x 5632 x 1024 267 -> 163, 130 x
+//     3584 x 896 over 4 44 -> 24 (there against the fp32 MFMA in pieces).
 //   * Operands go through registers (the split) into one LDS stage of 32 reduction elements:
 //     [operand][plane][octet of k][row][8], so that the fragment reads of 32 rows are contiguous; octets lie
 //     32 bytes off a multiple of 128, which takes the bank conflicts out of the writes of 4 octets x 2 rows
@@ -167,6 +171,7 @@ struct Item {
   long long row0;      // first row of the expert
   int64_t n;           // rows of the expert
   int64_t first, cnt;  // output rows of the tile: [first, first + cnt) of the expert's (TN: of K)
+  int piece;           // of the reduction, of p.pieces
 };
 
 template <int MODE, int EPI, int RF>
@@ -202,13 +207,20 @@ __device__ __forceinline__ void run_tile(const GmmParams& p, const Item& it, uns
   const uint32_t frag = (uint32_t)((lane >> 5) * OCTET + (lane & 31) * 16);
   const unsigned char* fa = lds + frag + wm * RF * 32 * 16;
   const unsigned char* fb = lds + OPERAND + frag + wn * 64 * 16;
-  const int stages = (int)((red + BKT - 1) / BKT);
-  if (stages > 0) {
-    la.load(0, red);
-    lb.load(0, red);
+  // the stages of this tile's piece of the reduction
+  constexpr bool CAN_SPLIT = MODE != MODE_TN && EPI == EPI_NONE;
+  const int all_stages = (int)((red + BKT - 1) / BKT);
+  int from = 0, stages = all_stages;
+  if constexpr (CAN_SPLIT) {
+    from = all_stages * it.piece / p.pieces;
+    stages = all_stages * (it.piece + 1) / p.pieces;
+  }
+  if (stages > from) {
+    la.load((int64_t)from * BKT, red);
+    lb.load((int64_t)from * BKT, red);
   }
   uint64_t small = 0;  // lanes
-  for (int s = 0; s < stages; ++s) {
+  for (int s = from; s < stages; ++s) {
     la.store(lds);
     lb.store(lds + OPERAND);
     if (__ballot(!(la.smallest(lb.smallest(kSplitMin)) >= kSplitMin)) != 0)
@@ -280,16 +292,17 @@ __device__ __forceinline__ void run_tile(const GmmParams& p, const Item& it, uns
 #pragma unroll
       for (int j = 0; j < 2; ++j) sum[i][j] = f32x16{};
     constexpr int kAhead = 2;  // pairs of reduction elements requested together
+    const int64_t end = (int64_t)stages * BKT < red ? (int64_t)stages * BKT : red;
 #pragma unroll 1
-    for (int64_t k0 = 0; k0 < red; k0 += 2 * kAhead) {
+    for (int64_t k0 = (int64_t)from * BKT; k0 < end; k0 += 2 * kAhead) {
       float av[kAhead][RF], bv[kAhead][2];
 #pragma unroll
       for (int q = 0; q < kAhead; ++q) {
         const int64_t k = k0 + 2 * q + (lane >> 5);
 #pragma unroll
-        for (int i = 0; i < RF; ++i) av[q][i] = la.one(wm * RF * 32 + i * 32 + (lane & 31), k, red, ld_a);
+        for (int i = 0; i < RF; ++i) av[q][i] = la.one(wm * RF * 32 + i * 32 + (lane & 31), k, end, ld_a);
 #pragma unroll
-        for (int j = 0; j < 2; ++j) bv[q][j] = lb.one(wn * 64 + j * 32 + (lane & 31), k, red, ld_b);
+        for (int j = 0; j < 2; ++j) bv[q][j] = lb.one(wn * 64 + j * 32 + (lane & 31), k, end, ld_b);
       }
 #pragma unroll
       for (int q = 0; q < kAhead; ++q)
@@ -334,11 +347,15 @@ __device__ __forceinline__ void run_tile(const GmmParams& p, const Item& it, uns
       }
     } else {
       const int64_t row = MODE == MODE_TN ? (int64_t)it.e * p.K + it.first + m : it.row0 + it.first + m;
+      unsigned char* out = p.c;
+      if constexpr (CAN_SPLIT) {
+        if (p.pieces > 1) out = reinterpret_cast<unsigned char*>(p.ws + it.piece * p.N * M);
+      }
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
         if (n0 + q * 8 >= M) continue;
         const f32x16& v = sum[i][q / 4];
-        *reinterpret_cast<f32x4*>(p.c + (row * M + n0 + q * 8) * 4) =
+        *reinterpret_cast<f32x4*>(out + (row * M + n0 + q * 8) * 4) =
             f32x4{v[q % 4 * 4], v[q % 4 * 4 + 1], v[q % 4 * 4 + 2], v[q % 4 * 4 + 3]};
       }
     }
@@ -391,11 +408,11 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gmm_f32_kernel(GmmParams p) {
   };
   int max_units = kMaxUnits;
   count_tiles(max_units);
-  if (tile_cum[E] <= (int)gridDim.x / 2) {
+  if ((int64_t)tile_cum[E] * p.pieces <= (int)gridDim.x / 2) {
     max_units = 1;
     count_tiles(max_units);
   }
-  const int total = tile_cum[E];
+  const int tiles_all = tile_cum[E], total = tiles_all * p.pieces;  // a piece's tiles are neighbours
 
   // XCD x takes the positions [x*G/8, (x+1)*G/8) of every whole round of G tiles; the last, partial
   // round is dealt to the XCDs in equal consecutive shares
@@ -409,8 +426,11 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gmm_f32_kernel(GmmParams p) {
       v = base + xcd * share + slot;
       if (slot >= share || v >= total) break;
     }
-    while (tile_cum[e + 1] <= v) ++e;
     Item it;
+    it.piece = __builtin_amdgcn_readfirstlane(v / tiles_all);
+    v -= it.piece * tiles_all;
+    if (v < tile_cum[e]) e = 0;
+    while (tile_cum[e + 1] <= v) ++e;
     it.e = __builtin_amdgcn_readfirstlane(e);
     it.row0 = group_begin(p, it.e);
     it.n = group_begin(p, it.e + 1) - it.row0;
@@ -427,6 +447,19 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gmm_f32_kernel(GmmParams p) {
   }
 }
 
+// c = the sum of the pieces' results, which lie behind one another in the workspace, in ascending order.
+__global__ __launch_bounds__(256) void f32_pieces_sum_kernel(GmmParams p) {
+  const int64_t quads = group_begin(p, p.E) * p.M / 4, step = p.N * p.M / 4;
+  const f32x4* ws = reinterpret_cast<const f32x4*>(p.ws);
+  f32x4* out = reinterpret_cast<f32x4*>(p.c);
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < quads; i += (int64_t)gridDim.x * 256) {
+    f32x4 sum = ws[i];
+#pragma unroll 4
+    for (int s = 1; s < p.pieces; ++s) sum += ws[s * step + i];
+    out[i] = sum;
+  }
+}
+
 template <int MODE, int EPI>
 static int launch_cfg(const GmmParams& p, hipStream_t st) {
   auto kern = gmm_f32_kernel<MODE, EPI>;
@@ -439,6 +472,11 @@ static int launch_cfg(const GmmParams& p, hipStream_t st) {
   int grid = (gmoe_cu_count() / 8) * 8 * 2;
   if (grid < 8) grid = 8;
   hipLaunchKernelGGL(kern, dim3(grid), dim3(kGemmThreads), LDS_BYTES, st, p);
+  if (p.pieces > 1) {
+    const int64_t blocks = (p.N * p.M / 4 + 255) / 256;
+    hipLaunchKernelGGL(f32_pieces_sum_kernel, dim3((unsigned)(blocks < 4 * grid ? blocks : 4 * grid)), dim3(256), 0, st,
+                       p);
+  }
   return gmoe_launch_status();
 }
 

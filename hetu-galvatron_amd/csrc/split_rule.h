@@ -40,4 +40,42 @@ __host__ __device__ inline int split_pieces(int64_t ns_per_k_tile, int64_t k_til
   return whole - split > kSplitReduceNs + per_piece * s ? (int)s : 1;
 }
 
+// Pieces of the reduction of an fp32 NN / NT launch (gmm_f32.hip), each a result of its own in the workspace; only
+// the host asks.  Times in ns per stage of 32 reduction elements, measured: 2600 for two 128-row tiles of a CU,
+// 2000 for a lone one, 1700 and 1300 for 64-row tiles, 5000 around a tile, 4000 and the traffic for the sums.
+// A round of 512 tiles ends with its slowest, so three pieces of 144 tiles beat two and four (us in 1, 2, 3, 4, 6
+// pieces, 4096 x 2048 x 512 over 8 experts: 110, 93, 73, 88, 84; 2000 x 5632 x 1024: 269, 214, 170, 204, 187;
+// 130 x 3584 x 896 over 4, in 1, 4, 8, 16: 153, 48, 30, 24).  A launch with a full round stays whole (4096 x
+// 512 x 2048: 81, in two pieces 87).
+constexpr int kF32MaxPieces = 16;
+
+inline int gmm_f32_pieces(int64_t E, int64_t N, int64_t K, int64_t M) {
+  if (N < 1) return 1;
+  const int64_t cols = (M + 127) / 128, busy = N < E ? N : E, stages = (K + 31) / 32;
+  // the last tile of an expert is half full on average
+  int64_t tiles128 = (N + 127) / 128 + E / 2, tiles64 = (N + 63) / 64 + E / 2;
+  if (tiles128 < busy) tiles128 = busy;
+  if (tiles64 < busy) tiles64 = busy;
+  const int64_t stream_ns = weight_stream_ns(E, K, M, 4);
+  int best = 1;
+  int64_t best_ns = 0;
+  for (int s = 1; s <= kF32MaxPieces && s <= stages; ++s) {
+    if (s > 1 && s * N * M > (int64_t)kSplitSlots * 128 * 128) break;
+    const bool small = tiles128 * cols * s <= kSplitSlots / 2;  // the kernel's own rule
+    int64_t tiles = (small ? tiles64 : tiles128) * cols * s;
+    tiles += tiles / 16;  // loads are uneven
+    const int64_t rounds = tiles / kSplitSlots, rest = tiles % kSplitSlots, per_piece = (stages + s - 1) / s;
+    const int64_t pair = per_piece * (small || tiles64 == tiles128 ? 1700 : 2600) + 5000;
+    const int64_t lone = per_piece * (small || tiles64 == tiles128 ? 1300 : 2000) + 5000;
+    int64_t ns = rounds * pair + (rest == 0 ? 0 : (rest <= kSplitSlots / 2 ? lone : pair));
+    if (ns < stream_ns) ns = stream_ns;
+    if (s > 1) ns += 4000 + (s + 1) * N * M / 1000;  // 4 bytes at 4 TB/s
+    if (s == 1 || ns < best_ns) {
+      best = s;
+      best_ns = ns;
+    }
+  }
+  return best;
+}
+
 }  // namespace gmoe

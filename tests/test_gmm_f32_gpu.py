@@ -44,6 +44,28 @@ def test_edges(pkg, dev, mode, K, M):
     assert ((got - reference(mode, a, b, COUNTS)).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("mode", ["NN", "NT"])
+@pytest.mark.parametrize("counts, K, M", [([130], 3584, 128), ([0, 65, 0, 3], 1000, 136), ([520, 500, 490, 538], 2048, 512),
+                                          ([1], 648, 8), ([37, 30, 41, 0], 1416, 2048)])
+def test_pieces(pkg, dev, mode, counts, K, M):
+    """Reductions cut into pieces, the last of them shorter, with a small element in the first piece and one in
+    the last, in different rows; the same bits again."""
+    E, N = len(counts), sum(counts)
+    need = pkg._C.lib().gmoe_gmm_workspace_bytes(E, N, K, M, 0, mode == "NT", 0)
+    assert need % (N * M * 4) == 0 and need >= 2 * N * M * 4
+    off = torch.tensor([0] + counts, device=dev).cumsum(0)
+    a, b = operands(mode, N, K, M, E, dev, K + M)
+    a[0, 0] = a[N - 1, K - 1] = 2.0 ** -120
+    got = product(pkg, mode, a, b, off)
+    # as in test_edges, one more addition per piece; the pieces with a small element are products added one after
+    # the other: 2^-24 of the absolute sum each
+    pieces = need // (N * M * 4)
+    bound = 2.0 ** -24 * (1 + 12 + (K + 31) // 32 + pieces + (K + pieces - 1) // pieces)
+    ref, mag = reference(mode, a, b, counts), reference(mode, a, b, counts, torch.abs)
+    assert ((got.double().cpu() - ref).abs() <= bound * mag).all()
+    assert torch.equal(got, product(pkg, mode, a, b, off))
+
+
 @pytest.mark.parametrize("mode", MODES)
 @pytest.mark.parametrize("value, other", [(float("inf"), 1.0), (float("-inf"), 0.0), (float("nan"), 1.0),
                                           (torch.finfo(torch.float32).max, 2.0 ** -20)])
