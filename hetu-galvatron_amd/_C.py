@@ -14,7 +14,7 @@ import threading
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # GALVATRON_MOE_LIB selects another build of the same ABI (e.g. a tuning variant)
 LIB_PATH = os.environ.get("GALVATRON_MOE_LIB") or os.path.join(_HERE, "_lib", "libgalvatron_moe.so")
-ABI_VERSION = 11
+ABI_VERSION = 12
 
 GMOE_F32, GMOE_BF16, GMOE_F16, GMOE_F8E4M3 = 0, 1, 2, 3
 SCORE_SOFTMAX, SCORE_SIGMOID, SCORE_IDENTITY = 0, 1, 2
@@ -33,6 +33,8 @@ PROTOTYPES = {
     "gmoe_route_topk": (_int, [_vp, _int, _i64, _int, _int, _int, _int, _f32, _vp, _vp, _int, _int,
                                _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "gmoe_seq_aux_loss": (_int, [_vp, _int, _vp, _i64, _int, _int, _int, _int, _f32, _vp, _vp, _vp, _vp]),
+    "gmoe_seq_aux_loss_workspace_bytes": (_i64, [_i64, _int, _int]),
+    "gmoe_seq_aux_loss_ws": (_int, [_vp, _int, _vp, _i64, _int, _int, _int, _int, _f32, _vp, _vp, _vp, _vp, _i64, _vp]),
     "gmoe_seq_aux_loss_bwd": (_int, [_vp, _int, _i64, _int, _int, _int, _int, _vp, _f32, _vp, _vp, _vp]),
     "gmoe_score_stats": (_int, [_vp, _int, _i64, _int, _int, _int, _vp, _vp, _vp]),
     "gmoe_score_stats_bwd": (_int, [_vp, _int, _i64, _int, _int, _int, _vp, _f32, _f32, _vp, _vp, _vp]),

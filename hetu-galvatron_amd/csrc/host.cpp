@@ -28,7 +28,7 @@ namespace {
 // ---- the library ----------------------------------------------------------------------------------
 #define GMOE_ENTRY_POINTS(X)                                                                          \
   X(gmoe_abi_version) X(gmoe_status_string) X(gmoe_route_workspace_bytes) X(gmoe_route_topk)          \
-  X(gmoe_route_topk_bwd) X(gmoe_seq_aux_loss) X(gmoe_seq_aux_loss_bwd) X(gmoe_router_bookkeeping)     \
+  X(gmoe_route_topk_bwd) X(gmoe_seq_aux_loss_workspace_bytes) X(gmoe_seq_aux_loss_ws) X(gmoe_seq_aux_loss_bwd) X(gmoe_router_bookkeeping)     \
   X(gmoe_capacity_select) X(gmoe_permute_plan_workspace_bytes) X(gmoe_permute_plan)                   \
   X(gmoe_expert_offsets) X(gmoe_permute_rows) X(gmoe_unpermute_rows) X(gmoe_unpermute_rows_bwd)       \
   X(gmoe_glu_fwd) X(gmoe_glu_bwd) X(gmoe_glu_fwd_fp8store) X(gmoe_glu_bwd_fp8in)                      \
@@ -502,10 +502,12 @@ struct SeqAuxLoss : Function<SeqAuxLoss> {
     c10::DeviceGuard on(x.device());
     Tensor counts = empty_of(x, {B, E}, at::kFloat), scores = empty_of(x, {B, E}, at::kFloat),
            loss = empty_of(x, {}, at::kFloat);
-    check(L.gmoe_seq_aux_loss(ptr(x), dt(x), ptr_as<uint8_t>(rmap), S, (int)B, (int)E, (int)k, (int)score_fn,
-                              (float)coeff, ptr_as<float>(counts), ptr_as<float>(scores), ptr_as<float>(loss),
-                              stream_of(x)),
-          "gmoe_seq_aux_loss");
+    const int64_t nbytes = L.gmoe_seq_aux_loss_workspace_bytes(S, (int)B, (int)E);
+    const Tensor ws = bytes_of(x, nbytes);
+    check(L.gmoe_seq_aux_loss_ws(ptr(x), dt(x), ptr_as<uint8_t>(rmap), S, (int)B, (int)E, (int)k, (int)score_fn,
+                                 (float)coeff, ptr_as<float>(counts), ptr_as<float>(scores), ptr_as<float>(loss),
+                                 ptr(ws), nbytes, stream_of(x)),
+          "gmoe_seq_aux_loss_ws");
     ctx->save_for_backward({x, counts});
     ctx->saved_data["S"] = S;
     ctx->saved_data["k"] = k;

@@ -54,14 +54,25 @@ __device__ __forceinline__ void routing_scores(const float (&logit)[kVpt], const
 }
 
 // ---- sequence-level load-balancing loss ------------------------------------------------------------
-// One workgroup per sequence b: token (s, b) is row s * B + b.  counts[b,e] = number of tokens of the
-// sequence routed to e, scores[b,e] = sum_s score(s,b,e).
+// Token (s, b) is row s * B + b.  counts[b,e] = number of tokens of sequence b routed to e, scores[b,e] =
+// sum_s score(s,b,e).  A workgroup's loop is a chain of loads, exponentials and shuffles, 2-3 us per 4
+// wavefronts of tokens, so a sequence is shared out to as many workgroups as it has such steps (P of them, up to
+// 64): their partial counts and scores go to the workspace [P][B][counts, scores][E] and the second kernel, which
+// was there, adds them in order.
 constexpr int kSeqThreads = 256;
+constexpr int kSeqParts = 64;
+
+// Workgroups per sequence: one per step, not more than two per CU in all.
+static int seq_parts(int64_t S, int B, int G) {
+  const int64_t step = (GMOE_WAVE / G) * (kSeqThreads / GMOE_WAVE), steps = (S + step - 1) / step, most = 512 / B;
+  const int64_t parts = steps < kSeqParts ? steps : kSeqParts;
+  return (int)(parts < most ? parts : (most < 1 ? 1 : most));
+}
 
 template <int DT, int G>
 __global__ __launch_bounds__(kSeqThreads) void seq_aux_stats_kernel(
     const void* logits, const uint8_t* map, int64_t S, int B, int E, int k, int score_fn,
-    float* seq_counts, float* seq_scores) {
+    float* seq_counts, float* seq_scores, int64_t part_stride) {
   typedef Elem<DT> El;
   constexpr int TPW = GMOE_WAVE / G;
   constexpr int NW = kSeqThreads / GMOE_WAVE;
@@ -76,7 +87,7 @@ __global__ __launch_bounds__(kSeqThreads) void seq_aux_stats_kernel(
     accP[v] = accC[v] = 0.f;
     evalid[v] = (e0 + v) < E;
   }
-  for (int64_t q0 = 0; q0 < S; q0 += NW * TPW) {
+  for (int64_t q0 = (int64_t)blockIdx.y * (NW * TPW); q0 < S; q0 += (int64_t)gridDim.y * (NW * TPW)) {
     const int64_t q = q0 + wave * TPW + lane / G;
     const bool tvalid = q < S;
     const int64_t row = ((tvalid ? q : 0) * B + b) * (int64_t)E;
@@ -109,24 +120,52 @@ __global__ __launch_bounds__(kSeqThreads) void seq_aux_stats_kernel(
       p += red[w][0][e];
       c += red[w][1][e];
     }
-    seq_scores[(int64_t)b * E + e] = p;
-    seq_counts[(int64_t)b * E + e] = c;
+    seq_scores[blockIdx.y * part_stride + (int64_t)b * E + e] = p;
+    seq_counts[blockIdx.y * part_stride + (int64_t)b * E + e] = c;
   }
 }
 
-// loss = scale * sum_b sum_e counts[b,e] * scores[b,e], summed per sequence by one wavefront each in
-// lane-strided order, the sequences added in ascending order.
-__global__ __launch_bounds__(64) void seq_aux_finish_kernel(const float* seq_counts,
-                                                            const float* seq_scores, int B, int E,
-                                                            float scale, float* loss) {
-  const int lane = threadIdx.x;
+// loss = scale * sum_b sum_e counts[b,e] * scores[b,e].  A sequence's sum is one wavefront's, in lane-strided
+// order; a wavefront adds its sequences in ascending order, and the wavefronts' totals are added in order.
+// parts > 1: first the partial counts and scores of `ws`, again in order.
+constexpr int kSeqFinishThreads = 512;
+
+__global__ __launch_bounds__(kSeqFinishThreads) void seq_aux_finish_kernel(float* seq_counts, float* seq_scores,
+                                                                           const float* ws, int parts, int B, int E,
+                                                                           float scale, float* loss) {
+  constexpr int NW = kSeqFinishThreads / GMOE_WAVE;
+  __shared__ float wave_total[NW];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t BE = (int64_t)B * E;
   float total = 0.f;
-  for (int b = 0; b < B; ++b) {
+  for (int b = wave; b < B; b += NW) {
     float a = 0.f;
-    for (int e = lane; e < E; e += 64) a += seq_counts[(int64_t)b * E + e] * seq_scores[(int64_t)b * E + e];
+    for (int e = lane; e < E; e += 64) {
+      const int64_t at = (int64_t)b * E + e;
+      float c = 0.f, s = 0.f;
+      if (parts > 1) {
+#pragma unroll 16
+        for (int p = 0; p < parts; ++p) {
+          c += ws[p * 2 * BE + at];
+          s += ws[p * 2 * BE + BE + at];
+        }
+        seq_counts[at] = c;
+        seq_scores[at] = s;
+      } else {
+        c = seq_counts[at];
+        s = seq_scores[at];
+      }
+      a += c * s;
+    }
     total += wave_sum_f32(a);
   }
-  if (lane == 0) loss[0] = total * scale;
+  if (lane == 0) wave_total[wave] = total;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    float sum = wave_total[0];
+    for (int w = 1; w < NW; ++w) sum += wave_total[w];
+    loss[0] = sum * scale;
+  }
 }
 
 // ---- sinkhorn ----------------------------------------------------------------------------------------
@@ -381,11 +420,12 @@ static int launch_score_stats(int G, int grid, const void* x, int64_t T, int E, 
 
 template <int DT>
 static int launch_seq_stats(int G, const void* logits, const uint8_t* map, int64_t S, int B, int E,
-                            int k, int score_fn, float* counts, float* scores, hipStream_t st) {
-#define GMOE_CASE(g)                                                                              \
-  case g:                                                                                         \
-    hipLaunchKernelGGL((seq_aux_stats_kernel<DT, g>), dim3(B), dim3(kSeqThreads), 0, st, logits, \
-                       map, S, B, E, k, score_fn, counts, scores);                                 \
+                            int k, int score_fn, float* counts, float* scores, int parts, hipStream_t st) {
+  const int64_t stride = 2 * (int64_t)B * E;
+#define GMOE_CASE(g)                                                                                     \
+  case g:                                                                                                \
+    hipLaunchKernelGGL((seq_aux_stats_kernel<DT, g>), dim3(B, parts), dim3(kSeqThreads), 0, st, logits, \
+                       map, S, B, E, k, score_fn, counts, scores, stride);                               \
     break;
   switch (G) {
     GMOE_CASE(1) GMOE_CASE(2) GMOE_CASE(4) GMOE_CASE(8) GMOE_CASE(16) GMOE_CASE(32) GMOE_CASE(64)
@@ -419,6 +459,20 @@ extern "C" int gmoe_seq_aux_loss(const void* logits, int dtype, const uint8_t* r
                                  int64_t seq_length, int batch_size, int E, int k, int score_fn,
                                  float coeff, float* seq_counts, float* seq_scores, float* loss,
                                  void* stream) {
+  return gmoe_seq_aux_loss_ws(logits, dtype, routing_map, seq_length, batch_size, E, k, score_fn, coeff, seq_counts,
+                              seq_scores, loss, nullptr, 0, stream);
+}
+
+extern "C" int64_t gmoe_seq_aux_loss_workspace_bytes(int64_t seq_length, int batch_size, int E) {
+  if (seq_length < 1 || batch_size < 1 || E < 1 || E > kVpt * GMOE_WAVE) return 0;
+  const int parts = seq_parts(seq_length, batch_size, route_group_lanes(E, 0));
+  return parts > 1 ? (int64_t)parts * 2 * batch_size * E * 4 : 0;
+}
+
+extern "C" int gmoe_seq_aux_loss_ws(const void* logits, int dtype, const uint8_t* routing_map, int64_t seq_length,
+                                    int batch_size, int E, int k, int score_fn, float coeff, float* seq_counts,
+                                    float* seq_scores, float* loss, void* workspace, int64_t workspace_bytes,
+                                    void* stream) {
   GMOE_CHECK_ARG(seq_length >= 1 && batch_size >= 1 && E >= 1 && k >= 1 && k <= E);
   GMOE_CHECK_ARG(score_fn == GMOE_SCORE_SOFTMAX || score_fn == GMOE_SCORE_SIGMOID ||
                  score_fn == GMOE_SCORE_IDENTITY);
@@ -427,18 +481,25 @@ extern "C" int gmoe_seq_aux_loss(const void* logits, int dtype, const uint8_t* r
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int G = route_group_lanes(E, 0);
   const int sig = score_fn;
+  const int64_t BE = (int64_t)batch_size * E;
+  float* ws = static_cast<float*>(workspace);
+  int parts = seq_parts(seq_length, batch_size, G);
+  const int64_t room = ws != nullptr && gmoe_aligned(ws, 4) ? workspace_bytes / (2 * BE * 4) : 0;
+  if (parts > room) parts = room < 2 ? 1 : (int)room;
+  float* counts = parts > 1 ? ws : seq_counts;
+  float* scores = parts > 1 ? ws + BE : seq_scores;
   int rc;
   switch (dtype) {
-    case GMOE_F32: rc = launch_seq_stats<GMOE_F32>(G, logits, routing_map, seq_length, batch_size, E, k, sig, seq_counts, seq_scores, st); break;
-    case GMOE_BF16: rc = launch_seq_stats<GMOE_BF16>(G, logits, routing_map, seq_length, batch_size, E, k, sig, seq_counts, seq_scores, st); break;
-    case GMOE_F16: rc = launch_seq_stats<GMOE_F16>(G, logits, routing_map, seq_length, batch_size, E, k, sig, seq_counts, seq_scores, st); break;
+    case GMOE_F32: rc = launch_seq_stats<GMOE_F32>(G, logits, routing_map, seq_length, batch_size, E, k, sig, counts, scores, parts, st); break;
+    case GMOE_BF16: rc = launch_seq_stats<GMOE_BF16>(G, logits, routing_map, seq_length, batch_size, E, k, sig, counts, scores, parts, st); break;
+    case GMOE_F16: rc = launch_seq_stats<GMOE_F16>(G, logits, routing_map, seq_length, batch_size, E, k, sig, counts, scores, parts, st); break;
     default: return GMOE_ERR_UNSUPPORTED;
   }
   if (rc != GMOE_OK) return rc;
   // cost_coeff = counts * E / (S k), mean over s of the scores, sum over e, mean over b, times coeff
   const float scale = coeff * (float)E /
                       ((float)batch_size * (float)seq_length * (float)seq_length * (float)k);
-  hipLaunchKernelGGL(seq_aux_finish_kernel, dim3(1), dim3(64), 0, st, seq_counts, seq_scores,
+  hipLaunchKernelGGL(seq_aux_finish_kernel, dim3(1), dim3(kSeqFinishThreads), 0, st, seq_counts, seq_scores, ws, parts,
                      batch_size, E, scale, loss);
   return gmoe_launch_status();
 }

@@ -139,11 +139,13 @@ def seq_aux_loss(logits: torch.Tensor, routing_map: torch.Tensor, batch_size: in
     counts = torch.empty((batch_size, E), dtype=torch.float32, device=dev)
     scores = torch.empty((batch_size, E), dtype=torch.float32, device=dev)
     loss = torch.empty((), dtype=torch.float32, device=dev)
+    L = _C.lib()
+    ws = torch.empty((L.gmoe_seq_aux_loss_workspace_bytes(seq_length, batch_size, E),), dtype=torch.uint8, device=dev)
     with _on(dev):
-        st = _C.lib().gmoe_seq_aux_loss(_ptr(logits), _dt(logits), _ptr(routing_map), seq_length,
-                                        batch_size, E, k, _score_fn(score_fn), float(coeff),
-                                        _ptr(counts), _ptr(scores), _ptr(loss), _stream(dev))
-    _C.check(st, "gmoe_seq_aux_loss")
+        st = L.gmoe_seq_aux_loss_ws(_ptr(logits), _dt(logits), _ptr(routing_map), seq_length,
+                                    batch_size, E, k, _score_fn(score_fn), float(coeff),
+                                    _ptr(counts), _ptr(scores), _ptr(loss), _ptr(ws), ws.numel(), _stream(dev))
+    _C.check(st, "gmoe_seq_aux_loss_ws")
     return loss, counts, scores
 
 

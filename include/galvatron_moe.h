@@ -22,7 +22,7 @@
 extern "C" {
 #endif
 
-#define GMOE_ABI_VERSION 11
+#define GMOE_ABI_VERSION 12
 
 typedef enum {
   GMOE_F32 = 0,
@@ -102,6 +102,14 @@ int gmoe_route_topk_bwd(const void* logits, int dtype, int64_t T, int E, int k, 
 int gmoe_seq_aux_loss(const void* logits, int dtype, const uint8_t* routing_map, int64_t seq_length,
                       int batch_size, int E, int k, int score_fn, float coeff, float* seq_counts,
                       float* seq_scores, float* loss, void* stream);
+
+/* The same with a workspace of gmoe_seq_aux_loss_workspace_bytes (0: none is used), in which several
+ * workgroups share a sequence; a smaller one, or NULL, is used as far as it goes. */
+int64_t gmoe_seq_aux_loss_workspace_bytes(int64_t seq_length, int batch_size, int E);
+int gmoe_seq_aux_loss_ws(const void* logits, int dtype, const uint8_t* routing_map, int64_t seq_length,
+                         int batch_size, int E, int k, int score_fn, float coeff, float* seq_counts,
+                         float* seq_scores, float* loss, void* workspace, int64_t workspace_bytes,
+                         void* stream);
 
 /* Its gradient: dlogits[t,:] = scale * grad_loss[0] * J_t^T seq_counts[t % batch_size, :], J_t the
  * Jacobian of token t's scores; scale = coeff * E / (B S^2 k) for the loss above.  grad_loss

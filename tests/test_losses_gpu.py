@@ -25,7 +25,7 @@ def oracle_scores(logits, score_fn, k):
 
 @pytest.mark.parametrize("score_fn", ["softmax", "sigmoid"])
 @pytest.mark.parametrize("S,B,E,k", [(64, 4, 8, 2), (33, 5, 64, 8), (17, 3, 60, 6), (16, 2, 256, 8),
-                                     (1, 7, 8, 1), (300, 1, 16, 1)])
+                                     (1, 7, 8, 1), (300, 1, 16, 1), (33, 1, 60, 4), (2500, 1, 64, 8), (70, 300, 64, 2)])
 def test_seq_aux_loss_kernel(pkg, orc, dev, score_fn, S, B, E, k):
     print("case", score_fn, S, B, E, k, flush=True)
     coeff = 0.03
