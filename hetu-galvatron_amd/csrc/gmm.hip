@@ -1159,25 +1159,34 @@ constexpr int64_t kRemainderMinRows = 2048;  // see gmm_use_remainder
 //   * up to 512 rows the 128x128 kernel multiplies padding and moves twice the operands per product:
 //     n 384: 996 -> 731 (4096 x 28672, 8), 436 -> 338 (2048 x 2816, 64), NT 974 -> 765 (7168 x 4096, 32);
 //     n 160: 654 -> 380 (7168 x 4096, 32).
-//   * from 512 rows on the 256x256 tiles are the alternative.  NN gains 1-10 % as long as the
-//     reduction is long enough to carry its prologue (n 1024: 1730 -> 1681, K 7168; but 223 -> 238 at
-//     K 1024); NT loses 4-10 % (its 64-byte pieces of two operands against 128-byte ones there:
-//     1632 -> 1727, K 4096), so it stays.  From 2048 rows on the remainder launches take over.  These
-//     limits hold also where there are too few 256x256 tiles and 128x128 ones follow, which was not measured.
-//   * with less than three quarters of a round of tiles, or a last round that leaves more than 30 % of
-//     all rounds idle, the smaller tiles spread better (K 2816, M 1024, 16 experts, 64 tiles: 27 -> 43).
+//   * from 512 rows on the 256x256 tiles are the alternative, or 128x128 where those are too few.  NN gains
+//     1-17 % (n 1024: 1730 -> 1681, K 7168; 894: 119 -> 113, 1440 x 9632, 4; 1264: 126 -> 115, 544 x 2816, 24;
+//     against 128x128 tiles n 835: 47 -> 40, 1280 x 2048, 8).  NT gains up to K 896 (n 667: 76 -> 71, 672 x 1952,
+//     32; 824: 35 -> 30, 896 x 1728, 8) and loses 4-10 % beyond (its 64-byte pieces of two operands against
+//     128-byte ones there: 1632 -> 1727, K 4096).  From 2048 rows on the remainder launches take over.
+//   * the activation backward against 256x256 tiles gains from 512 rows on, whatever the last round holds, as
+//     both have the same rounds: n 619: 110 -> 85 (1088 x 4032, 8), 1004: 126 -> 119 (2112 x 1888, 8), 1578: 96 ->
+//     75 (736 x 704, 16), 4096 x 2944 225 -> 211; no gain at K 6016.
+//   * otherwise, with less than three quarters of a round of tiles, or a last round that leaves more than 30 %
+//     of all rounds idle, the smaller tiles spread better (K 2816, M 1024, 16 experts, 64 tiles: 27 -> 43).
+//   * K 512 and less: prologue and epilogue weigh as much as the reduction (n 119: 47 -> 50, 512 x 7776, 24; but
+//     n 215: 130 -> 103, 576 x 7968, 32, with the activation n 135: 166 -> 126, 608 x 9728, 32).
 //   * the activation backward (NT) around 256 rows: half the experts take a second chunk of two units,
-//     whose epilogue does not overlap anything (361 -> 408 at K 7168); 128x128 tiles there.
+//     whose epilogue does not overlap anything (361 -> 408 at K 7168); 128x128 tiles there, and for K under
+//     1024 from 400 to 511 rows too (n 466: 39 -> 42, 768 x 576, 32; 354: 53 -> 47, 864 x 1984, 16).
 static inline bool gmm_rows_pays(const GmmParams& p, int mode, int epi) {
   const int64_t n = p.N / (p.E > 0 ? p.E : 1);
   const bool glu = epi == EPI_GLU_FWD_SILU || epi == EPI_GLU_FWD_GELU;
   const int64_t cols = glu ? (p.F + 127) / 128 : (p.M + 255) / 256;
   const int64_t tiles = p.E * ((n + 16 + 255) / 256) * cols;
   const int64_t cus = gmm_grid(1), rounds = (tiles + cus - 1) / cus;
-  if (p.K < 1024 || tiles * 4 < cus * 3 || tiles * 10 < rounds * cus * 7) return false;
-  if (mode == MODE_NN) return n >= 96 && n < kRemainderMinRows && (n < 512 || p.K >= 1536);
-  if (epi != EPI_NONE && n >= 240 && n < 288) return false;
-  return n >= 128 && n < 512;
+  if (p.K <= 512 || n >= kRemainderMinRows) return false;
+  if (mode == MODE_NT && epi != EPI_NONE && n >= 512) return p.K <= 4096 && gmm_large_tiles(p, mode);
+  if (tiles * 4 < cus * 3 || tiles * 10 < rounds * cus * 7) return false;
+  if (mode == MODE_NN) return n >= 96;
+  if (n >= 512) return p.K <= 896;
+  if (epi != EPI_NONE && ((n >= 240 && n < 288) || (p.K < 1024 && n >= 400))) return false;
+  return n >= 128;
 }
 
 // dW of 16-bit operands with a short reduction (gmm_tn.hip: 128x256 tiles, two workgroups per CU) against the

@@ -27,7 +27,7 @@ def on_kernel(kernel, call):
 
 @pytest.mark.parametrize("act", ["silu", "gelu"])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("K,F", [(1024, 1024), (1160, 904), (1544, 1096)])
+@pytest.mark.parametrize("K,F", [(1024, 1024), (1160, 904), (1544, 1096), (520, 1024)])
 def test_chunk_edges(pkg, dev, dtype, K, F, act):
     E, N, M = len(ROWS), sum(ROWS), 2 * F
     g = torch.Generator(device=dev).manual_seed(K + F)
@@ -130,3 +130,21 @@ def test_medium_reduction_edges(pkg, dev, dtype, K, M):
         # as in test_long_reduction_edges
         assert (got32[e].double() - want).abs().max().item() <= 2.0 ** -24 * 25 * min(n, 100 * n ** 0.5) * 4
         s += n
+
+
+@pytest.mark.parametrize("K,F", [(520, 4104), (896, 4096), (2056, 4104)])
+def test_activation_backward_of_many_rows(pkg, dev, K, F):
+    """512 rows per expert and more, where 256x256 tiles could be had: the fused backward is the backward of the
+    separate product, to the bit, whichever kernel that is on."""
+    counts = [513, 767, 1025, 640, 0, 1, 1300, 560]
+    off = torch.tensor([0] + counts, device=dev).cumsum(0)
+    g = torch.Generator(device=dev).manual_seed(K)
+
+    def rnd(*s, std=1.0):
+        return torch.empty(*s, device=dev).normal_(0.0, std, generator=g).bfloat16()
+
+    a, wt, fc1 = rnd(sum(counts), K), rnd(len(counts), F, K, std=K ** -0.5), rnd(sum(counts), 2 * F)
+    got = on_kernel("gmm_rows_kernel", lambda: pkg.ops.gmm_glu_bwd(a, wt, fc1, off, "silu"))
+    product = lambda: pkg.ops.gmm(a, wt, off, trans_b=True)
+    d = on_kernel("gmm_rows_kernel", product) if K <= 896 else product()
+    assert torch.equal(got, pkg.ops.glu_bwd(d, fc1, "silu"))
