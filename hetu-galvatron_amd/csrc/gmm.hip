@@ -1153,7 +1153,7 @@ constexpr int64_t kRemainderMinRows = 2048;  // see gmm_use_remainder
 // Row-adaptive tiles (gmm_rows.hip) for 16-bit NN / NT: tiles of 64 to 256 rows x 256 columns that
 // share an expert's rows evenly, one workgroup per CU.  Measured against the 128x128 and 256x256 tiles
 // in the same process, n = rows per expert, times of both sides in us (K x M, experts):
-//   * n below 96 (NT: 128): an expert is one 128-row tile either way and its weights bound the launch;
+//   * n below 112 (NT: 128, with the activation 96): an expert is one 128-row tile either way and its weights bound the launch;
 //     the 128x128 kernel with two workgroups per CU streams them a little faster
 //     (n 64: 375 against 399 for 4096 x 28672, 8 experts).
 //   * up to 512 rows the 128x128 kernel multiplies padding and moves twice the operands per product:
@@ -1167,13 +1167,16 @@ constexpr int64_t kRemainderMinRows = 2048;  // see gmm_use_remainder
 //   * the activation backward against 256x256 tiles gains from 512 rows on, whatever the last round holds, as
 //     both have the same rounds: n 619: 110 -> 85 (1088 x 4032, 8), 1004: 126 -> 119 (2112 x 1888, 8), 1578: 96 ->
 //     75 (736 x 704, 16), 4096 x 2944 225 -> 211; no gain at K 6016.
-//   * otherwise, with less than three quarters of a round of tiles, or a last round that leaves more than 30 %
-//     of all rounds idle, the smaller tiles spread better (K 2816, M 1024, 16 experts, 64 tiles: 27 -> 43).
+//   * the smaller tiles spread better over the CUs with few tiles (K 2112, M 928, 8 experts, 64 tiles: 25 -> 33)
+//     and, backward, with a last round that leaves more than 30 % of all rounds idle.  As the chunks adapt
+//     to the rounds, NN is ahead from half a round on (144 tiles of 736 x 2144: 26 -> 24, 96 of 3808 x 1440: 59 ->
+//     52, but 112 of 576 x 1600: 17 -> 18), with the activation from a third (100 tiles of 768 x 5120: 25 -> 23,
+//     72 of 2496 x 768: 44 -> 39), NT of 512 rows and more between 0.6 and two rounds (192 tiles of 5632 x 1024: 149
+//     -> 130, 168 of 3552 x 3392: 90 -> 75; 144 of 1504 x 1472: 33 -> 36).
 //   * K 512 and less: prologue and epilogue weigh as much as the reduction (n 119: 47 -> 50, 512 x 7776, 24; but
 //     n 215: 130 -> 103, 576 x 7968, 32, with the activation n 135: 166 -> 126, 608 x 9728, 32).
 //   * the activation backward (NT) around 256 rows: half the experts take a second chunk of two units,
-//     whose epilogue does not overlap anything (361 -> 408 at K 7168); 128x128 tiles there, and for K under
-//     1024 from 400 to 511 rows too (n 466: 39 -> 42, 768 x 576, 32; 354: 53 -> 47, 864 x 1984, 16).
+//     whose epilogue does not overlap anything (361 -> 408 at K 7168); 128x128 tiles there.
 static inline bool gmm_rows_pays(const GmmParams& p, int mode, int epi) {
   const int64_t n = p.N / (p.E > 0 ? p.E : 1);
   const bool glu = epi == EPI_GLU_FWD_SILU || epi == EPI_GLU_FWD_GELU;
@@ -1181,12 +1184,17 @@ static inline bool gmm_rows_pays(const GmmParams& p, int mode, int epi) {
   const int64_t tiles = p.E * ((n + 16 + 255) / 256) * cols;
   const int64_t cus = gmm_grid(1), rounds = (tiles + cus - 1) / cus;
   if (p.K <= 512 || n >= kRemainderMinRows) return false;
-  if (mode == MODE_NT && epi != EPI_NONE && n >= 512) return p.K <= 4096 && gmm_large_tiles(p, mode);
-  if (tiles * 4 < cus * 3 || tiles * 10 < rounds * cus * 7) return false;
-  if (mode == MODE_NN) return n >= 96;
-  if (n >= 512) return p.K <= 896;
-  if (epi != EPI_NONE && ((n >= 240 && n < 288) || (p.K < 1024 && n >= 400))) return false;
-  return n >= 128;
+  const bool full = tiles * 4 >= cus * 3 && tiles * 10 >= rounds * cus * 7;
+  // narrower results pad the 256 columns
+  const bool wide = p.M >= 512;
+  if (mode == MODE_NN)
+    return (full && n >= (glu ? 96 : 112)) || (wide && n >= 128 && tiles * 10 >= cus * (glu ? 3 : 5));
+  if (epi != EPI_NONE) {
+    if (n >= 512) return gmm_large_tiles(p, mode) ? p.K <= 4096 : full;
+    return full && n >= 128 && !(n >= 240 && n < 288);
+  }
+  if (n >= 512) return (wide && tiles <= 2 * cus && tiles * 10 >= cus * 6) || (full && p.K <= 896);
+  return full && n >= 128;
 }
 
 // dW of 16-bit operands with a short reduction (gmm_tn.hip: 128x256 tiles, two workgroups per CU) against the

@@ -3,8 +3,8 @@
 // per expert (the rule with both sides' times is gmm_rows_pays in gmm.hip).
 //
 //   * A tile is RF*64 rows (RF = 1..4, chosen per tile) x 256 columns of C.  An expert's rows are cut
-//     into chunks of up to 256 that are as equal as 64-row steps allow, so at most 63 rows per expert
-//     are padding: a fixed 128- or 256-row tile multiplies a third of its rows for nothing at 380 rows
+//     into chunks of up to 256 (192, 128 where those fill the rounds better: best_max_units) that are as
+//     equal as 64-row steps allow, so at most 63 rows per expert are padding: a fixed 128- or 256-row tile multiplies a third of its rows for nothing at 380 rows
 //     per expert, and its operand stream is the larger the smaller the tile.
 //   * 2x2 wavefronts of (RF*32) x 128, one workgroup per CU.
 //   * Operands go global -> LDS without staging registers (buffer_load ... lds) in stages of 32
@@ -40,10 +40,44 @@ struct Stages {
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 
 // Row chunks of an expert with n rows: units of kUnit rows dealt as evenly as possible to
-// ceil(units / 4) chunks.
-__device__ __forceinline__ int chunk_count(long long n) {
-  const long long units = (n + kUnit - 1) / kUnit;
-  return (int)((units + kMaxUnits - 1) / kMaxUnits);
+// ceil(units / max_units) chunks.
+__device__ __forceinline__ int unit_count(long long n) { return (int)((n + kUnit - 1) / kUnit); }
+__device__ __forceinline__ int chunk_count(long long n, int max_units) {
+  return (unit_count(n) + max_units - 1) / max_units;
+}
+// The chunk size that ends first.  A stage of a tile of u units takes as long as its operands stream, 16 + 4 u KiB
+// at 42 GB/s; prologue and epilogue take as long as 250 KiB.  Where the largest chunks leave a round part empty,
+// smaller ones fill it (us with chunks of up to 256 rows and with these: NT 640 rows, 5632 x 1024, 16 experts 143 ->
+// 130; NN 370, 3808 x 1440, 8 61 -> 52; with the activation 258, 3392 x 6400, 4 82 -> 60).  units, chunks: of this thread's experts, summed over the workgroup here.
+__device__ __forceinline__ int best_max_units(int units, const int (&chunks)[kMaxUnits + 1], int nt_cnt, int grid,
+                                              int64_t K, int (*sums)[kMaxUnits + 1], int lane, int wave) {
+  int v[kMaxUnits + 1] = {units, 0, chunks[2], chunks[3], chunks[4]};
+#pragma unroll
+  for (int i = 0; i <= kMaxUnits; ++i) {
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) v[i] += __shfl_xor(v[i], d);
+    if (lane == 0) sums[wave][i] = v[i];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i <= kMaxUnits; ++i) {
+    v[i] = 0;
+#pragma unroll
+    for (int w = 0; w < kGemmThreads / 64; ++w) v[i] += sums[w][i];
+  }
+  const float fixed = 16.f + 250.f / (float)((K + BKT - 1) / BKT);
+  int best = kMaxUnits;
+  float least = 0.f;
+#pragma unroll
+  for (int u = kMaxUnits; u >= 2; --u) {
+    const int rounds = (int)(((long long)v[u] * nt_cnt + grid - 1) / grid);
+    const float cost = (float)rounds * (fixed + 4.f * (float)v[0] / (float)(v[u] > 0 ? v[u] : 1));
+    if (u == kMaxUnits || cost < 0.95f * least) {
+      best = u;
+      least = cost;
+    }
+  }
+  return best;
 }
 // first unit and unit count of chunk c of cnt
 __device__ __forceinline__ void chunk_units(long long n, int cnt, int c, int& first, int& units) {
@@ -384,20 +418,32 @@ __global__ __launch_bounds__(kGemmThreads, 1) void gmm_rows_kernel(GmmParams p) 
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
   __shared__ int tile_cum[kMaxGroupsLds + 1];
   __shared__ int wave_tot[kGemmThreads / 64];
+  __shared__ int sums[kGemmThreads / 64][kMaxUnits + 1];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t lds0 = lds_offset_of(lds);
   const int E = p.E;
   const int nt_cnt = GLU ? (int)((p.F + 127) / 128) : (int)((p.M + BN - 1) / BN);
 
+  int max_units = kMaxUnits;
   {
     // tiles per expert -> exclusive prefix (a thread owns kPer consecutive experts)
     constexpr int kPer = kMaxGroupsLds / kGemmThreads;
-    int cnt[kPer], local = 0;
+    long long rows_of[kPer];
+    int units = 0, chunks[kMaxUnits + 1] = {};
 #pragma unroll
     for (int j = 0; j < kPer; ++j) {
       const int e = tid * kPer + j;
-      cnt[j] = e >= E ? 0 : nt_cnt * chunk_count(group_begin(p, e + 1) - group_begin(p, e));
+      rows_of[j] = e >= E ? 0 : group_begin(p, e + 1) - group_begin(p, e);
+      units += unit_count(rows_of[j]);
+#pragma unroll
+      for (int u = 2; u <= kMaxUnits; ++u) chunks[u] += chunk_count(rows_of[j], u);
+    }
+    max_units = best_max_units(units, chunks, nt_cnt, (int)gridDim.x, p.K, sums, lane, wave);
+    int cnt[kPer], local = 0;
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      cnt[j] = nt_cnt * chunk_count(rows_of[j], max_units);
       local += cnt[j];
     }
     int incl = local;
@@ -437,7 +483,7 @@ __global__ __launch_bounds__(kGemmThreads, 1) void gmm_rows_kernel(GmmParams p) 
     Item it;
     it.e = __builtin_amdgcn_readfirstlane(e);
     const long long row0 = group_begin(p, e), n_e = group_begin(p, e + 1) - row0;
-    const int chunks = chunk_count(n_e);
+    const int chunks = chunk_count(n_e, max_units);
     int c, first, units;
     strip_order(v - tile_cum[e], chunks, nt_cnt, c, it.nt);
     chunk_units(n_e, chunks, c, first, units);
