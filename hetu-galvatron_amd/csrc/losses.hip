@@ -526,7 +526,8 @@ extern "C" int gmoe_score_stats(const void* x, int dtype, int64_t T, int E, int 
     if (rc != GMOE_OK) return rc;
   }
   hipLaunchKernelGGL(route_stats_reduce_kernel, dim3(E + 1), dim3(GMOE_WAVE), 0, st,
-                     static_cast<const float*>(stats_ws), T > 0 ? grid : 0, E, stats);
+                     static_cast<const float*>(stats_ws), T > 0 ? grid : 0, E, stats, (const int*)nullptr,
+                     (unsigned long long*)nullptr);
   return gmoe_launch_status();
 }
 

@@ -31,6 +31,7 @@ struct RouteParams {
   int32_t* topk_idx;
   unsigned long long* counts;
   float* stats_ws;  // [gridDim.x][E+1]
+  int* counts_ws;   // [gridDim.x][E] behind it, with statistics and several workgroups
 };
 
 template <int DT, int G>
@@ -255,9 +256,14 @@ __global__ __launch_bounds__(kRouteThreads) void route_topk_kernel(RouteParams p
   }
 
   __syncthreads();
+  // A lone workgroup's histogram is the result.  With statistics, which a second launch adds up anyway, that one
+  // adds the histograms too.  Only otherwise the counts are cleared beforehand and added to: the clearing was a
+  // launch of 1.5-5 us in every call.
   for (int i = tid; i < E; i += kRouteThreads) {
     const int c = hist[i];
-    if (c) atomicAdd(&p.counts[i], (unsigned long long)c);
+    if (p.counts_ws) p.counts_ws[(int64_t)blockIdx.x * E + i] = c;
+    else if (gridDim.x == 1) p.counts[i] = (unsigned long long)c;
+    else if (c) atomicAdd(&p.counts[i], (unsigned long long)c);
   }
 
   if (want_stats) {
@@ -509,7 +515,7 @@ using namespace gmoe;
 
 extern "C" int64_t gmoe_route_workspace_bytes(int64_t T, int E) {
   (void)T;
-  return (int64_t)kRouteMaxBlocks * (E + 1) * (int64_t)sizeof(float);
+  return (int64_t)kRouteMaxBlocks * ((E + 1) * (int64_t)sizeof(float) + E * (int64_t)sizeof(int));
 }
 
 extern "C" int gmoe_route_topk(const void* logits, int dtype, int64_t T, int E, int k, int score_fn,
@@ -533,10 +539,14 @@ extern "C" int gmoe_route_topk(const void* logits, int dtype, int64_t T, int E, 
     group_topk = 0;
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
-  hipLaunchKernelGGL(fill_u64_kernel, dim3((E + 255) / 256), dim3(256), 0, st,
-                     reinterpret_cast<unsigned long long*>(tokens_per_expert), E, 0ull);
+  unsigned long long* counts = reinterpret_cast<unsigned long long*>(tokens_per_expert);
   const int G = route_group_lanes(E, num_groups);
   const int grid = route_grid(T, G);
+  int* counts_ws = stats && grid > 1
+                       ? reinterpret_cast<int*>(static_cast<float*>(stats_ws) + (int64_t)kRouteMaxBlocks * (E + 1))
+                       : nullptr;
+  if (T == 0 || (grid > 1 && counts_ws == nullptr))
+    hipLaunchKernelGGL(fill_u64_kernel, dim3((E + 255) / 256), dim3(256), 0, st, counts, E, 0ull);
   if (T > 0) {
     RouteParams p;
     p.logits = logits;
@@ -552,7 +562,8 @@ extern "C" int gmoe_route_topk(const void* logits, int dtype, int64_t T, int E, 
     p.probs = probs;
     p.map = routing_map;
     p.topk_idx = topk_idx;
-    p.counts = reinterpret_cast<unsigned long long*>(tokens_per_expert);
+    p.counts = counts;
+    p.counts_ws = counts_ws;
     p.stats_ws = stats ? static_cast<float*>(stats_ws) : nullptr;
     const size_t smem = ((E * 4 + 15) / 16) * 16 + (size_t)kRouteThreads * (kVpt + 1) * 4;
     int rc;
@@ -565,8 +576,8 @@ extern "C" int gmoe_route_topk(const void* logits, int dtype, int64_t T, int E, 
     if (rc != GMOE_OK) return rc;
   }
   if (stats) {
-    hipLaunchKernelGGL(route_stats_reduce_kernel, dim3(E + 1), dim3(GMOE_WAVE), 0, st,
-                       static_cast<const float*>(stats_ws), T > 0 ? grid : 0, E, stats);
+    hipLaunchKernelGGL(route_stats_reduce_kernel, dim3(E + 1 + (counts_ws ? E : 0)), dim3(GMOE_WAVE), 0, st,
+                       static_cast<const float*>(stats_ws), T > 0 ? grid : 0, E, stats, counts_ws, counts);
   }
   return gmoe_launch_status();
 }

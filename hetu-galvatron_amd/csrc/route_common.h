@@ -35,9 +35,20 @@ static inline int route_group_lanes(int E, int num_groups) {
 // One wavefront per statistic: lane l adds the partials of workgroups l, l + 64, ... in order, then
 // the 64 lane sums meet in a fixed butterfly, so the result depends only on the launch's grid.  (One
 // thread per statistic walking all workgroups took 63 us at 64 experts: 2048 dependent loads.)
-static __global__ __launch_bounds__(GMOE_WAVE) void route_stats_reduce_kernel(const float* ws, int nblocks,
-                                                                       int E, float* stats) {
+// Workgroups beyond the E + 1 of the statistics add up the workgroups' token counts, one expert each.
+static __global__ __launch_bounds__(GMOE_WAVE) void route_stats_reduce_kernel(const float* ws, int nblocks, int E,
+                                                                       float* stats, const int* counts_ws,
+                                                                       unsigned long long* counts) {
   const int e = blockIdx.x;
+  if (e > E) {
+    const int c = e - E - 1;
+    unsigned long long n = 0;
+    for (int b = threadIdx.x; b < nblocks; b += GMOE_WAVE) n += (unsigned long long)counts_ws[(int64_t)b * E + c];
+#pragma unroll
+    for (int d = 1; d < GMOE_WAVE; d <<= 1) n += __shfl_xor(n, d);
+    if (threadIdx.x == 0) counts[c] = n;
+    return;
+  }
   float a = 0.f;
   for (int b = threadIdx.x; b < nblocks; b += GMOE_WAVE) a += ws[(int64_t)b * (E + 1) + e];
   a = wave_sum_f32(a);

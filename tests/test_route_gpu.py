@@ -266,3 +266,17 @@ def test_router_module_aux_and_z_loss_gradients(pkg, orc, dev, score_fn):
     if score_fn == "softmax":
         aux = orc.switch_load_balancing_loss(torch.softmax(lg, -1), o_map.sum(0), k, 0.01)
         torch.testing.assert_close(router.router.last_aux_loss.cpu(), aux, rtol=1e-5, atol=1e-9)
+
+
+@pytest.mark.parametrize("want_stats", [False, True])
+@pytest.mark.parametrize("T,E,k", [(1, 8, 2), (256, 8, 2), (257, 8, 2), (32, 64, 8), (33, 64, 8), (5000, 60, 4),
+                                   (140000, 8, 1), (3, 512, 8)])
+def test_token_counts(pkg, dev, T, E, k, want_stats):
+    """One workgroup, several, more tiles than workgroups: the counts are the map's column sums, also into memory
+    that held others."""
+    logits = torch.randn(T, E, generator=torch.Generator().manual_seed(T + E)).to(dev)
+    for _ in range(2):
+        _, rmap, counts, stats, _ = pkg.ops.route_topk(logits, k, want_stats=want_stats)
+        assert torch.equal(counts, rmap.sum(0)) and (stats is not None) == want_stats
+        counts.fill_(-7)
+        del counts
