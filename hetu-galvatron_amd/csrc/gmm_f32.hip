@@ -27,6 +27,7 @@
 //     piece's results go to the workspace as a matrix of their own, and a second launch adds the matrices, bound by
 //     that traffic: dX of 4096 x 2048 x 512 over 8 experts 102 -> 70 us, 2000 x 5632 x 1024 267 -> 163, 130 x
 //     3584 x 896 over 4 44 -> 24 (there against the fp32 MFMA in pieces).
+//     Error against float64, whole and in pieces: 1.6e-7 / 1.1e-7, 2.6e-7 / 1.7e-7 and 2.1e-7 / 1.2e-7.
 //   * Operands go through registers (the split) into one LDS stage of 32 reduction elements:
 //     [operand][plane][octet of k][row][8], so that the fragment reads of 32 rows are contiguous; octets lie
 //     32 bytes off a multiple of 128, which takes the bank conflicts out of the writes of 4 octets x 2 rows
