@@ -448,12 +448,13 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gmm_f32_kernel(GmmParams p) {
   }
 }
 
-// c = the sum of the pieces' results, which lie behind one another in the workspace, in ascending order.
+// c = the sum of the pieces' results, which lie behind one another in the workspace, in ascending order.  Rows
+// outside the groups have no pieces, and c keeps them.
 __global__ __launch_bounds__(256) void f32_pieces_sum_kernel(GmmParams p) {
-  const int64_t quads = group_begin(p, p.E) * p.M / 4, step = p.N * p.M / 4;
+  const int64_t first = group_begin(p, 0) * p.M / 4, quads = group_begin(p, p.E) * p.M / 4, step = p.N * p.M / 4;
   const f32x4* ws = reinterpret_cast<const f32x4*>(p.ws);
   f32x4* out = reinterpret_cast<f32x4*>(p.c);
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < quads; i += (int64_t)gridDim.x * 256) {
+  for (int64_t i = first + (int64_t)blockIdx.x * 256 + threadIdx.x; i < quads; i += (int64_t)gridDim.x * 256) {
     f32x4 sum = ws[i];
 #pragma unroll 4
     for (int s = 1; s < p.pieces; ++s) sum += ws[s * step + i];

@@ -66,6 +66,26 @@ def test_pieces(pkg, dev, mode, counts, K, M):
     assert torch.equal(got, product(pkg, mode, a, b, off))
 
 
+@pytest.mark.parametrize("mode", ["NN", "NT"])
+def test_pieces_leave_rows_outside_the_groups(pkg, dev, mode):
+    """An offset table over rows 40..170 of 300, as for some of the experts of a larger buffer: the other rows of
+    the result stay as they were."""
+    N, K, M, first, last = 300, 3584, 128, 40, 170
+    L, nt = pkg._C.lib(), int(mode == "NT")
+    a, b = operands(mode, N, K, M, 2, dev, 5)
+    need = L.gmoe_gmm_workspace_bytes(2, N, K, M, 0, nt, 0)
+    assert need >= 2 * N * M * 4
+    off = torch.tensor([first, 100, last], device=dev)
+    ws, c = torch.full((need // 4,), 1e30, device=dev), torch.full((N, M), 7.0, device=dev)
+    assert L.gmoe_gmm(a.data_ptr(), b.data_ptr(), c.data_ptr(), off.data_ptr(), 2, N, K, M, 0, nt, 0, 0, ws.data_ptr(),
+                      need, torch.cuda.current_stream().cuda_stream) == 0
+    assert (c[:first] == 7.0).all() and (c[last:] == 7.0).all()
+    want = pkg.ops.gmm(a[first:last].contiguous(), b, off - first, trans_b=bool(nt))
+    # two orders of the same sums: 2^-24 of the absolute sum per addition, as in test_pieces, on either side
+    mag = reference(mode, a[first:last], b, [60, 70], torch.abs)
+    assert ((c[first:last] - want).double().cpu().abs() <= 2 * 2.0 ** -24 * (13 + 112 + 16) * mag).all()
+
+
 @pytest.mark.parametrize("mode", MODES)
 @pytest.mark.parametrize("value, other", [(float("inf"), 1.0), (float("-inf"), 0.0), (float("nan"), 1.0),
                                           (torch.finfo(torch.float32).max, 2.0 ** -20)])
