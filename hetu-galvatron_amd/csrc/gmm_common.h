@@ -4,6 +4,7 @@
 #include <type_traits>
 
 #include "gmoe_common.h"
+#include "copy_range.h"
 #include "split_rule.h"
 
 namespace gmoe {

@@ -80,8 +80,7 @@ struct TransOperand {
   }
   // Offset of K tile kt inside the resource, clamped to its end: whole K tiles past the last row read as zero.
   __device__ __forceinline__ uint32_t offset(const u32x4& rsrc, int kt) const {
-    const uint64_t o = (uint64_t)(uint32_t)kt * stage_bytes;
-    return o < rsrc[2] ? (uint32_t)o : rsrc[2];
+    return stage_offset(rsrc[2], (uint32_t)kt, stage_bytes);
   }
   template <int q>
   __device__ __forceinline__ void issue(const u32x4& rsrc, uint32_t off, uint32_t lds_tile, int wave) const {

@@ -119,10 +119,11 @@ struct KContig {
     frag[0] = (uint32_t)((frag_row0 + r) * 64 + ((g ^ ((r >> 2) & 3)) * 16));
     frag[1] = frag[0] ^ 32u;
   }
+  __device__ __forceinline__ uint32_t offset(int kt) const { return stage_offset(rsrc[2], (uint32_t)kt, BKT * 2); }
   template <int q>
-  __device__ __forceinline__ void issue(int kt, uint32_t lds_tile) const {
+  __device__ __forceinline__ void issue(int kt, uint32_t off, uint32_t lds_tile, int) const {
     const bool kok = (int64_t)kt * BKT + kchunk < k_lim;
-    dma16(lds_tile + lds_off + q * 1024, kok ? voff[q] : kOob, rsrc, (uint32_t)(kt * BKT * 2));
+    dma16(lds_tile + lds_off + q * 1024, kok ? voff[q] : kOob, rsrc, off);
   }
   static constexpr int READS = 1;
   template <int j, int ks, int h>
@@ -136,7 +137,7 @@ struct KContig {
 struct OuterContig {
   u32x4 rsrc;
   uint32_t voff[4];
-  uint32_t row_bytes;
+  uint32_t stage_bytes;  // global bytes between consecutive K tiles
   uint32_t frag_k;
   uint32_t frag_seg[4];
 
@@ -146,7 +147,7 @@ struct OuterContig {
   __device__ __forceinline__ void init(const unsigned char* src, int64_t ld, int64_t o0, int64_t k_limit,
                                        int wave, int lane, SegOf&& seg, int64_t gap) {
     rsrc = make_raw_rsrc(src + o0 * 2, k_limit * ld * 2 - o0 * 2);
-    row_bytes = (uint32_t)(ld * 2);
+    stage_bytes = (uint32_t)(ld * 2 * BKT);
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const int krow = (wave * 4 + q) * 2 + (lane >> 5);
@@ -162,9 +163,10 @@ struct OuterContig {
 #pragma unroll
     for (int j = 0; j < 4; ++j) frag_seg[j] = (uint32_t)(((seg(j) ^ f) * 64) + half * 32 + (s & 3) * 8);
   }
+  __device__ __forceinline__ uint32_t offset(int kt) const { return stage_offset(rsrc[2], (uint32_t)kt, stage_bytes); }
   template <int q>
-  __device__ __forceinline__ void issue(int kt, uint32_t lds_tile, int wave) const {
-    dma16(lds_tile + (uint32_t)((wave * 4 + q) * 1024), voff[q], rsrc, (uint32_t)(kt * BKT) * row_bytes);
+  __device__ __forceinline__ void issue(int, uint32_t off, uint32_t lds_tile, int wave) const {
+    dma16(lds_tile + (uint32_t)((wave * 4 + q) * 1024), voff[q], rsrc, off);
   }
   static constexpr int READS = 2;
   template <int j, int ks, int h>
@@ -279,14 +281,10 @@ __device__ __forceinline__ void run_tile(const GmmParams& p, const Item& it, uns
   const int kt_cnt = (int)((K + BKT - 1) / BKT);
   u32x4 fa[2][RF], fb[2][4];
 
-  auto issue = [&](auto op_c, int kt, uint32_t st) {
+  auto issue = [&](auto op_c, int kt, uint32_t offa, uint32_t offb, uint32_t st) {
     constexpr int op = decltype(op_c)::value;
-    if constexpr (op < RF) {
-      oa.template issue<op>(kt, st);
-    } else {
-      if constexpr (MODE == MODE_NT) ob.template issue<op - RF>(kt, st + A_BYTES);
-      else ob.template issue<op - RF>(kt, st + A_BYTES, wave);
-    }
+    if constexpr (op < RF) oa.template issue<op>(kt, offa, st, wave);
+    else ob.template issue<op - RF>(kt, offb, st + A_BYTES, wave);
   };
   auto frag_read = [&](auto r_c, auto ks_c, auto buf_c, const unsigned char* stage) {
     constexpr int r = decltype(r_c)::value, ks = decltype(ks_c)::value, buf = decltype(buf_c)::value;
@@ -313,7 +311,8 @@ __device__ __forceinline__ void run_tile(const GmmParams& p, const Item& it, uns
 
   static_for<0, NST - 1>([&](auto t_c) {
     constexpr int t = decltype(t_c)::value;
-    static_for<0, NLOAD>([&](auto q) { issue(q, t, lds0 + t * STAGE_BYTES); });
+    const uint32_t offa = oa.offset(t), offb = ob.offset(t);
+    static_for<0, NLOAD>([&](auto q) { issue(q, t, offa, offb, lds0 + t * STAGE_BYTES); });
   });
   wait_dma_outstanding<(NST - 2) * NLOAD>();
   __syncthreads();
@@ -327,16 +326,20 @@ __device__ __forceinline__ void run_tile(const GmmParams& p, const Item& it, uns
     const unsigned char* cur = lds + s0 * STAGE_BYTES;
     const unsigned char* nxt = lds + s1 * STAGE_BYTES;
     const uint32_t stl = lds0 + (uint32_t)(sl * STAGE_BYTES);
+    const int ktl = kt + NST - 1;
+    const uint32_t offa = oa.offset(ktl), offb = ob.offset(ktl);
     // step 0: read step 1's fragments; request half of the tile kt+NST-1 into the stage tile kt-1 left
     k_step(c0, std::integral_constant<int, NLOAD / 2>{}, [&](auto r_c) { frag_read(r_c, c1, c1, cur); },
-           [&](auto q_c) { issue(q_c, kt + NST - 1, stl); });
+           [&](auto q_c) { issue(q_c, ktl, offa, offb, stl); });
     // tile kt+1 has landed (the later ones may be in flight); every wavefront has read this stage
     wait_dma_outstanding<(NST - 3) * NLOAD + NLOAD / 2>();
     __syncthreads();
     GMOE_SCHED_FENCE();
     // step 1: read step 0's fragments of tile kt+1; request the other half
     k_step(c1, std::integral_constant<int, NLOAD - NLOAD / 2>{}, [&](auto r_c) { frag_read(r_c, c0, c0, nxt); },
-           [&](auto q_c) { issue(std::integral_constant<int, NLOAD / 2 + decltype(q_c)::value>{}, kt + NST - 1, stl); });
+           [&](auto q_c) {
+             issue(std::integral_constant<int, NLOAD / 2 + decltype(q_c)::value>{}, ktl, offa, offb, stl);
+           });
     sl = s0;
     s0 = s1;
   }

@@ -27,12 +27,12 @@ typedef short s16x4 __attribute__((ext_vector_type(4)));
 struct Outer128 {
   u32x4 rsrc;
   uint32_t voff[2];
-  uint32_t row_bytes;
+  uint32_t stage_bytes;  // global bytes between consecutive K tiles
   uint32_t frag[4];
   __device__ __forceinline__ void init(const unsigned char* src, int64_t ld, int64_t o0, int64_t k_limit,
                                        int wave, int lane) {
     rsrc = make_raw_rsrc(src + o0 * 2, k_limit * ld * 2 - o0 * 2);
-    row_bytes = (uint32_t)(ld * 2);
+    stage_bytes = (uint32_t)(ld * 2 * BKT);
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
       const int krow = (wave * 2 + q) * 4 + (lane >> 4);
@@ -45,9 +45,10 @@ struct Outer128 {
     for (int j = 0; j < 4; ++j)
       frag[j] = (uint32_t)((8 * g + (s >> 2)) * 256 + ((j ^ (s >> 2)) * 64) + half * 32 + (s & 3) * 8);
   }
+  __device__ __forceinline__ uint32_t offset(int kt) const { return stage_offset(rsrc[2], (uint32_t)kt, stage_bytes); }
   template <int q>
-  __device__ __forceinline__ void issue(int kt, uint32_t lds_tile, int wave) const {
-    dma16(lds_tile + (uint32_t)((wave * 2 + q) * 1024), voff[q], rsrc, (uint32_t)(kt * BKT) * row_bytes);
+  __device__ __forceinline__ void issue(uint32_t off, uint32_t lds_tile, int wave) const {
+    dma16(lds_tile + (uint32_t)((wave * 2 + q) * 1024), voff[q], rsrc, off);
   }
   static constexpr int READS = 2;
   template <int j, int ks, int h>
@@ -65,14 +66,14 @@ struct Outer128 {
 struct Outer256 {
   u32x4 rsrc;
   uint32_t voff[4];
-  uint32_t row_bytes;
+  uint32_t stage_bytes;  // global bytes between consecutive K tiles
   uint32_t frag_k;
   uint32_t frag_seg[2];
 
   __device__ __forceinline__ void init(const unsigned char* src, int64_t ld, int64_t o0, int64_t k_limit,
                                        int wave, int lane) {
     rsrc = make_raw_rsrc(src + o0 * 2, k_limit * ld * 2 - o0 * 2);
-    row_bytes = (uint32_t)(ld * 2);
+    stage_bytes = (uint32_t)(ld * 2 * BKT);
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const int krow = (wave * 4 + q) * 2 + (lane >> 5);
@@ -87,9 +88,10 @@ struct Outer256 {
     frag_seg[0] = (uint32_t)((((2 * wave) ^ f) * 64) + half * 32 + (s & 3) * 8);
     frag_seg[1] = (uint32_t)((((2 * wave + 1) ^ f) * 64) + half * 32 + (s & 3) * 8);
   }
+  __device__ __forceinline__ uint32_t offset(int kt) const { return stage_offset(rsrc[2], (uint32_t)kt, stage_bytes); }
   template <int q>
-  __device__ __forceinline__ void issue(int kt, uint32_t lds_tile, int wave) const {
-    dma16(lds_tile + (uint32_t)((wave * 4 + q) * 1024), voff[q], rsrc, (uint32_t)(kt * BKT) * row_bytes);
+  __device__ __forceinline__ void issue(uint32_t off, uint32_t lds_tile, int wave) const {
+    dma16(lds_tile + (uint32_t)((wave * 4 + q) * 1024), voff[q], rsrc, off);
   }
   static constexpr int READS = 2;
   template <int j, int ks, int h>
@@ -151,10 +153,10 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gmm_tn_kernel(GmmParams p) {
       ob.init(p.b + (row0 + seg0) * M * 2, M, (int64_t)nt * BN, k_lim, wave, lane);
       const int kt_cnt = (int)((k_lim + BKT - 1) / BKT);
       u32x4 fa[2][WM], fb[2][WN];
-      auto issue = [&](auto op_c, int kt, uint32_t st) {
+      auto issue = [&](auto op_c, uint32_t offa, uint32_t offb, uint32_t st) {
         constexpr int op = decltype(op_c)::value;
-        if constexpr (op < 2) oa.template issue<op>(kt, st, wave);
-        else ob.template issue<op - 2>(kt, st + A_BYTES, wave);
+        if constexpr (op < 2) oa.template issue<op>(offa, st, wave);
+        else ob.template issue<op - 2>(offb, st + A_BYTES, wave);
       };
       auto frag_read = [&](auto r_c, auto ks_c, auto buf_c, const unsigned char* stage) {
         constexpr int r = decltype(r_c)::value, ks = decltype(ks_c)::value, buf = decltype(buf_c)::value;
@@ -176,8 +178,8 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gmm_tn_kernel(GmmParams p) {
       constexpr std::integral_constant<int, 0> c0{};
       constexpr std::integral_constant<int, 1> c1{};
 
-      static_for<0, NLOAD>([&](auto q) { issue(q, 0, lds0); });
-      static_for<0, NLOAD>([&](auto q) { issue(q, 1, lds0 + STAGE_BYTES); });
+      static_for<0, NLOAD>([&](auto q) { issue(q, 0u, 0u, lds0); });
+      static_for<0, NLOAD>([&](auto q) { issue(q, oa.offset(1), ob.offset(1), lds0 + STAGE_BYTES); });
       wait_dma_outstanding<NLOAD>();
       __syncthreads();
       static_for<0, NREAD>([&](auto r) { frag_read(r, c0, c0, lds); });
@@ -187,11 +189,12 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gmm_tn_kernel(GmmParams p) {
         const unsigned char* cur = lds + s0 * STAGE_BYTES;
         const unsigned char* nxt = lds + s1 * STAGE_BYTES;
         const uint32_t st2 = lds0 + (uint32_t)(s2 * STAGE_BYTES);
+        const uint32_t offa = oa.offset(kt + 2), offb = ob.offset(kt + 2);
         // step 0: read step 1's fragments, request tile kt+2 into the stage tile kt-1 has left
         k_step(c0, [&](auto op_c) {
           constexpr int op = decltype(op_c)::value;
           if constexpr (op < NREAD) frag_read(op_c, c1, c1, cur);
-          else issue(std::integral_constant<int, op - NREAD>{}, kt + 2, st2);
+          else issue(std::integral_constant<int, op - NREAD>{}, offa, offb, st2);
         }, std::integral_constant<int, NREAD + NLOAD>{});
         // tile kt+1 has landed (kt+2 may be in flight) and every wavefront has read this stage
         wait_dma_outstanding<NLOAD>();
