@@ -118,7 +118,8 @@ struct Work {
 };
 
 // How a tile's result is stored (the rule is in launch_cfg): after its last K tile, with ordinary or with
-// nontemporal stores, or nontemporally in four K tiles spread over the next tile.
+// nontemporal stores, or nontemporally in four K tiles spread over the next tile.  A next tile of fewer than nine
+// K tiles (an empty expert, or one of 256 rows and less) has no room for that: then at once.
 enum { STORE_NOW, STORE_NOW_STREAM, STORE_SPREAD };
 template <int DT, int ODT, int STORE>
 __global__ __launch_bounds__(kGemmThreads) void gmm_dtl_kernel(GmmParams p) {
@@ -132,8 +133,8 @@ __global__ __launch_bounds__(kGemmThreads) void gmm_dtl_kernel(GmmParams p) {
   static_assert(ODT != GMOE_F32 || STORE == STORE_NOW, "32-bit results are stored from the accumulators");
   constexpr bool SPREAD = STORE == STORE_SPREAD;
   constexpr int STORES = 8;  // stores per wavefront and fragment row of a 16-bit result
-  // the copies reach one stretch ahead, never two; the result of the tile before takes nine
-  constexpr int MIN_KT = SPREAD ? 9 : NST - 1;
+  constexpr int MIN_KT = NST - 1;  // the copies reach one stretch ahead, never two
+  constexpr int SPREAD_KT = 1 + 2 * WT;  // K tiles that the result of the tile before takes
   static_assert(NREAD == NM && LOADS_PER_TILE == NM / 2, "one read per MFMA, a copy after every fourth");
 
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
@@ -176,6 +177,7 @@ __global__ __launch_bounds__(kGemmThreads) void gmm_dtl_kernel(GmmParams p) {
     if (s < 0) {
       w.ra = w.rb = make_raw_rsrc(p.a, 0);
       w.e = -1;
+      w.kt_cnt = 0;
       return;
     }
     const int e = s / per_expert;
@@ -361,11 +363,32 @@ __global__ __launch_bounds__(kGemmThreads) void gmm_dtl_kernel(GmmParams p) {
     GMOE_SCHED_FENCE();
   };
 
-  bool pending = false;  // there is a tile before, its result in the accumulators (SPREAD) or on its way
+  // The K tiles of `cur` from kt on, its further stretches included.
+  auto finish = [&](int kt) __attribute__((always_inline)) {
+    for (;;) {
+      for (; kt < cur.kt_cnt; ++kt) k_tile(plain, none, kt);
+      if (cur.last) break;
+      cur = nx;
+      fetch(nx);
+      kt = 0;
+    }
+  };
+
+  bool stored = false;  // the stores of a tile before are in flight
   for (;;) {
     fetch(nx);
     int kt = 0;
-    if (SPREAD && pending) {
+    clear();
+    // the copies of the first two tiles were requested before the stores
+    if (ODT != GMOE_F32 && stored)
+      for (; kt < 2; ++kt) k_tile(plain, all, kt);
+    finish(kt);
+    // a loop of its own: the accumulators must not meet those of another path, of which there is no copy
+    while (SPREAD && nx.kt_cnt >= SPREAD_KT) {
+      locate(cur);
+      cur = nx;
+      fetch(nx);
+      kt = 0;
       const int stride = (cur.kt_cnt - 1) / WT;
       k_tile(std::integral_constant<int, TAKE>{}, none, kt++);
       static_for<0, WT>([&](auto i_c) __attribute__((always_inline)) {
@@ -374,27 +397,14 @@ __global__ __launch_bounds__(kGemmThreads) void gmm_dtl_kernel(GmmParams p) {
         if constexpr (decltype(i_c)::value + 1 < WT)
           for (int r = 2; r < stride; ++r) k_tile(plain, none, kt++);
       });
-    } else {
-      clear();
-      // the copies of the first two tiles were requested before the stores
-      if (ODT != GMOE_F32 && pending)
-        for (; kt < 2; ++kt) k_tile(plain, all, kt);
+      finish(kt);
     }
-    for (;;) {
-      for (; kt < cur.kt_cnt; ++kt) k_tile(plain, none, kt);
-      if (cur.last) break;
-      cur = nx;
-      fetch(nx);
-      kt = 0;
-    }
-    pending = true;
     if constexpr (ODT != GMOE_F32) {
       locate(cur);
-      if constexpr (!SPREAD) {
-        asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // the last MFMA's result, read by acc_read
-        asm volatile("" : "+v"(put), "+v"(get));
-        static_for<0, WT>(store_row);
-      }
+      asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // the last MFMA's result, read by acc_read
+      asm volatile("" : "+v"(put), "+v"(get));
+      static_for<0, WT>(store_row);
+      stored = true;
     } else {
       unsigned char* c_tile = p.c + ((int64_t)cur.e * K + (int64_t)cur.mt * BM) * M * OES;
       const int64_t c_rows = K - (int64_t)cur.mt * BM;
@@ -416,10 +426,6 @@ __global__ __launch_bounds__(kGemmThreads) void gmm_dtl_kernel(GmmParams p) {
     }
     if (nx.e < 0) break;
     cur = nx;
-  }
-  if constexpr (SPREAD) {
-    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // the last MFMA's result, read by acc_read
-    static_for<0, WT>(store_row);
   }
   wait_dma_outstanding<0>();  // nothing may land in LDS after the workgroup has ended
 }

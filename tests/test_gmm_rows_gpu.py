@@ -12,16 +12,16 @@ pytestmark = pytest.mark.gpu
 ROWS = [0, 1, 63, 64, 65, 127, 128, 129, 191, 193, 255, 256, 257, 320, 511, 513] * 3
 
 
-def on_kernel(kernel, call):
-    """call(), with the only GEMM that it launches being `kernel` (nothing is asked where the profiler sees no
-    launch at all, as beside another profiler)."""
+def on_kernel(kernel, call, form=""):
+    """call(), with the only GEMM that it launches being `kernel`, its last template argument `form` (nothing is
+    asked where the profiler sees no launch at all, as beside another profiler)."""
     from torch.profiler import ProfilerActivity, profile
 
     with profile(activities=[ProfilerActivity.CUDA]) as trace:
         out = call()
         torch.cuda.synchronize()
     names = [e.name for e in trace.events() if "gmoe::" in e.name and "gmm" in e.name]
-    assert not names or (len(names) == 1 and "::%s<" % kernel in names[0]), names
+    assert not names or (len(names) == 1 and "::%s<" % kernel in names[0] and form + ">(" in names[0]), names
     return out
 
 
@@ -86,50 +86,47 @@ def test_short_reduction_edges(pkg, dev, dtype, K, M):
         s += n
 
 
-@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("K,M", [(1160, 904), (520, 4104)])
-def test_long_reduction_edges(pkg, dev, dtype, K, M):
-    """dW on 256x256 tiles, whose copies run ahead into the next tile: experts with no rows, with less
-    than the copies' three stages (96 rows) and with many, in turn; output edges inside a tile."""
-    rows = [0, 1, 31, 3000, 32, 33, 95, 96, 97, 0, 0, 4097, 7, 2500, 65, 5000]
+STORE_NOW, STORE_NOW_STREAM, STORE_SPREAD = ", 0", ", 1", ", 2"  # how gmm_dtl_kernel stores a tile
+
+
+def check_dw(pkg, dev, dtype, rows, K, M, form):
     E, N = len(rows), sum(rows)
     g = torch.Generator(device=dev).manual_seed(K + M)
     print("case", dtype, K, M, flush=True)
     off = torch.tensor([0] + rows, device=dev).cumsum(0)
     a = torch.empty(N, K, device=dev).normal_(generator=g).to(dtype)
     b = torch.empty(N, M, device=dev).normal_(generator=g).to(dtype)
-    got32 = on_kernel("gmm_dtl_kernel", lambda: pkg.ops.gmm(a, b, off, trans_a=True, out_dtype=torch.float32))
-    got = on_kernel("gmm_dtl_kernel", lambda: pkg.ops.gmm(a, b, off, trans_a=True))
+    got32 = on_kernel("gmm_dtl_kernel", lambda: pkg.ops.gmm(a, b, off, trans_a=True, out_dtype=torch.float32), STORE_NOW)
+    got = on_kernel("gmm_dtl_kernel", lambda: pkg.ops.gmm(a, b, off, trans_a=True), form)
     assert torch.equal(got, got32.to(dtype))
     s = 0
     for e, n in enumerate(rows):
         want = a[s:s + n].double().t().contiguous() @ b[s:s + n].double()
-        # as above; the sums of a long reduction stay within a few sqrt(n)
+        # exact products of values up to about 5 x 5, n fp32 additions: 2^-24 * 25 * n bounds each sum; those of a
+        # long reduction stay within a few sqrt(n)
         assert (got32[e].double() - want).abs().max().item() <= 2.0 ** -24 * 25 * min(n, 100 * n ** 0.5) * 4
         s += n
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("K,M", [(1160, 904), (520, 4104)])
+@pytest.mark.parametrize("rows", [[0, 1, 31, 3000, 32, 33, 95, 96, 97, 0, 0, 4097, 7, 2500, 65, 5000],
+                                  [3000, 0, 287, 256, 288, 289, 257, 3500, 320, 384, 385, 0, 416, 417, 1, 5500]])
+def test_long_reduction_edges(pkg, dev, dtype, rows, K, M):
+    """dW on 256x256 tiles, whose copies run ahead into the next tile and whose results are stored under its MFMAs:
+    experts with no rows, with less than the copies' three stages (96 rows), around the nine K tiles (of 32 rows)
+    that the stores take and the fourths of the next tile that they are spread over, and with many, in turn;
+    output edges inside a tile."""
+    check_dw(pkg, dev, dtype, rows, K, M, STORE_SPREAD)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("K,M", [(1160, 1096), (520, 4104)])
 def test_medium_reduction_edges(pkg, dev, dtype, K, M):
-    """dW on 256x256 tiles that are stored in the next tile's first six K tiles (of 32 rows): fewer rows
-    than that, one more or less, empty experts in turn, and more; output edges inside a tile."""
+    """dW on 256x256 tiles that are stored before the next one: around the copies' three stages (96 rows) and
+    whole K tiles (32), empty experts in turn, and many rows; output edges inside a tile."""
     rows = [0, 1, 33, 159, 160, 161, 0, 191, 192, 193, 223, 225, 0, 900, 64, 700]
-    E, N = len(rows), sum(rows)
-    g = torch.Generator(device=dev).manual_seed(K + M)
-    print("case", dtype, K, M, flush=True)
-    off = torch.tensor([0] + rows, device=dev).cumsum(0)
-    a = torch.empty(N, K, device=dev).normal_(generator=g).to(dtype)
-    b = torch.empty(N, M, device=dev).normal_(generator=g).to(dtype)
-    got32 = on_kernel("gmm_dtl_kernel", lambda: pkg.ops.gmm(a, b, off, trans_a=True, out_dtype=torch.float32))
-    got = on_kernel("gmm_dtl_kernel", lambda: pkg.ops.gmm(a, b, off, trans_a=True))
-    assert torch.equal(got, got32.to(dtype))
-    s = 0
-    for e, n in enumerate(rows):
-        want = a[s:s + n].double().t().contiguous() @ b[s:s + n].double()
-        # as in test_long_reduction_edges
-        assert (got32[e].double() - want).abs().max().item() <= 2.0 ** -24 * 25 * min(n, 100 * n ** 0.5) * 4
-        s += n
+    check_dw(pkg, dev, dtype, rows, K, M, STORE_NOW)
 
 
 @pytest.mark.parametrize("K,F", [(520, 4104), (896, 4096), (2056, 4104)])
