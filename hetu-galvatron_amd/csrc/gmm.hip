@@ -1153,9 +1153,9 @@ constexpr int64_t kRemainderMinRows = 2048;  // see gmm_use_remainder
 // Row-adaptive tiles (gmm_rows.hip) for 16-bit NN / NT: tiles of 64 to 256 rows x 256 columns that
 // share an expert's rows evenly, one workgroup per CU.  Measured against the 128x128 and 256x256 tiles
 // in the same process, n = rows per expert, times of both sides in us (K x M, experts):
-//   * n below 112 (NT: 128, with the activation 96): an expert is one 128-row tile either way and its weights bound the launch;
-//     the 128x128 kernel with two workgroups per CU streams them a little faster
-//     (n 64: 375 against 399 for 4096 x 28672, 8 experts).
+//   * n below 112 (NT: 128, with the activation 96): an expert is one 128-row tile either way and its weights bound
+//     the launch; the 128x128 kernel with two workgroups per CU streams them a little faster (n 64: 375 against 399
+//     for 4096 x 28672, 8 experts).
 //   * up to 512 rows the 128x128 kernel multiplies padding and moves twice the operands per product:
 //     n 384: 996 -> 731 (4096 x 28672, 8), 436 -> 338 (2048 x 2816, 64), NT 974 -> 765 (7168 x 4096, 32);
 //     n 160: 654 -> 380 (7168 x 4096, 32).
@@ -1198,19 +1198,22 @@ static inline bool gmm_rows_pays(const GmmParams& p, int mode, int epi) {
 }
 
 // dW of 16-bit operands with a short reduction (gmm_tn.hip: 128x256 tiles, two workgroups per CU) against the
-// 256x256 LDS-DMA kernel, or 128x128 tiles where that one does not apply; n = rows per expert, us on both
-// sides.  From one round of 256x256 tiles on that kernel, whose tiles run into each other, is the
-// faster one at n 128 and more (n 128: 454 against 462, n 190: 495 against 550, n 383: 779 against 837, 4096 x 28672,
-// 8 experts); fewer rows come here (n 64: 410 -> 366; 64 experts of 2048 x 2816, n 64: 168 -> 144, n 20: 149 -> 136).  With less than a round of them, and where its rows
-// would be padding (K under 512), the smaller tiles spread better: 128 tiles of 256x256, 20 -> 15
-// (1024 x 1024, 8), 240: 16.3 -> 15.1 (640 x 1280, 16), 384 x 4096 over 64 experts 120 -> 110.  More than
-// 768 rows are left to the 256x256 tiles (n 1024: 1884 against 1935), fewer than three quarters of a tile
-// per CU to 128x128 ones (128 tiles of 1024 x 512: 13 against 15).
-constexpr int64_t kTnFewRows = 112;
+// 256x256 LDS-DMA kernel, or 128x128 tiles where that one does not apply; n = rows per expert, us of that kernel /
+// of this one.  From one round of 256x256 tiles on that kernel, whose tiles run into each other, is the faster one
+// except for few rows: n 24, 8 experts of 6144 x 16384 291 / 266, n 48 291 / 297, n 96 299 / 368; 14336 x 4096, 8 n
+// 24 161 / 159, n 48 161 / 177, n 96 174 / 205.  A result under 256 MB has the ordinary stores there and
+// nontemporal ones here, which moves the line: 1024 x 5632, 16 n 24 44 / 41, n 64 45 / 44, n 96 49 / 47; 1024 x
+// 1024, 64 n 64 33 / 34, n 96 37 / 36; 2048 x 1184, 32 n 64 40 / 40, n 96 42 / 43.  With less than a round of
+// 256x256 tiles, and where its rows would be padding (K under 512), the smaller tiles spread better: 128 tiles of
+// 256x256, 20 / 15 (1024 x 1024, 8), 240: 16.3 / 15.1 (640 x 1280, 16), 384 x 4096 over 64 experts 120 / 110.  More
+// than 768 rows are left to the 256x256 tiles (n 1024: 1884 against 1935), fewer than three quarters of a tile per
+// CU to 128x128 ones (128 tiles of 1024 x 512: 13 against 15).
+constexpr int64_t kTnFewRows = 112, kTnFewRowsStreamed = 32;
 static inline bool gmm_tn_short_pays(const GmmParams& p) {
   const int64_t n = p.N / (p.E > 0 ? p.E : 1), col_tiles = (p.M + 255) / 256;
   if (p.K < 128 || p.M < 256 || p.E * ((p.K + 127) / 128) * col_tiles * 4 < gmm_grid(1) * 3) return false;
-  if (n >= kTnFewRows && p.K >= 512 && p.E * ((p.K + 255) / 256) * col_tiles >= gmm_grid(1)) return false;
+  const bool few = n < (gmm_tn_streams(p) ? kTnFewRowsStreamed : kTnFewRows);
+  if (!few && p.K >= 512 && p.E * ((p.K + 255) / 256) * col_tiles >= gmm_grid(1)) return false;
   return n <= 768;
 }
 
