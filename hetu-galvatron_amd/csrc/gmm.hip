@@ -1218,12 +1218,14 @@ static inline bool gmm_tn_short_pays(const GmmParams& p) {
 }
 
 // Whether reading the operands beforehand (warm_operands) pays: they take bytes / 5 TB/s, and the launch has to be
-// one of many more result bytes (us without and with, operands from HBM: 698 -> 497 for n 190 and 914 -> 772 for n 383,
-// 4096 x 28672 over 8 experts, half of either from the nontemporal stores; 438 -> 360 for n 64; 288 -> 255 for n 256 of
-// 2048 x 2816 over 64; but 98 -> 112 for n 383 of 1024 x 5632 over 16, 82 MB of operands for 184 MB of results).
+// one of many more result bytes.  us without / with, operands from HBM, result bytes over operand bytes in
+// parentheses: 4096 x 28672 over 8 experts n 192 544 / 483 (19), n 384 788 / 740 (9); 7168 x 4096 over 32 n 192 500
+// / 466 (14), n 384 757 / 799 (7); 14336 x 4096 over 8 n 448 420 / 407 (7), n 512 462 / 475 (6); 2048 x 2816 over
+// 64 n 128 175 / 158 (9), n 256 246 / 263 (5).  Smaller results gain nothing: 1024 x 5632 over 16 n 96 47 / 50,
+// 1024 x 1024 over 64 36 / 40.
 static inline bool gmm_tn_warm_pays(const GmmParams& p) {
-  const int64_t n = p.N / (p.E > 0 ? p.E : 1), operands = p.N * (p.K + p.M) * 2, result = p.E * p.K * p.M * 2;
-  return operands <= (192ll << 20) && operands * 4 <= result && (gmm_tn_streams(p) || n < kTnFewRows);
+  const int64_t operands = p.N * (p.K + p.M) * 2, result = p.E * p.K * p.M * 2;
+  return operands <= (192ll << 20) && operands * 7 <= result && gmm_tn_streams(p);
 }
 
 // The separate launch for short last row tiles pays off once an expert has many full row tiles:

@@ -129,6 +129,14 @@ def test_medium_reduction_edges(pkg, dev, dtype, K, M):
     check_dw(pkg, dev, dtype, rows, K, M, STORE_NOW)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_streamed_result_edges(pkg, dev, dtype):
+    """dW on 256x256 tiles with a result of 290 MiB, stored past the caches, and operands of a twelfth of it, read
+    beforehand: 85 rows per expert on average, empty experts in turn; output edges inside a tile."""
+    rows = [0, 1, 33, 95, 96, 97, 0, 127, 160, 161, 64, 65, 0, 300, 31, 130]
+    check_dw(pkg, dev, dtype, rows, 1160, 8200, STORE_NOW_STREAM)
+
+
 @pytest.mark.parametrize("K,F", [(520, 4104), (896, 4096), (2056, 4104)])
 def test_activation_backward_of_many_rows(pkg, dev, K, F):
     """512 rows per expert and more, where 256x256 tiles could be had: the fused backward is the backward of the
