@@ -2,11 +2,15 @@
 //   c[e] = a[rows_e]^T @ b[rows_e],  a [N,K], b [N,M], c [E,K,M]: the contract of gmm_dtl.hip.
 //
 // For outputs of less than a round of 256x256 tiles, whose CUs then have nothing to hide a tile's prologue
-// and epilogue under, and for a few dozen rows per expert, where a launch is all prologue and epilogue.  Here a tile is 128x256 and two workgroups share a CU (72 KiB of LDS, at most
-// 256 registers each): one multiplies while the other copies its first stages or writes its result.
-// Results are stored nontemporally (64 experts of 384 x 4096, 384 rows each: 123 -> 108 us).
-// The price is half again as much operand traffic per product, so long reductions and large outputs
-// stay with gmm_dtl.hip (the rule with both sides' times is gmm_tn_short_pays in gmm.hip).
+// and epilogue under, and for a few dozen rows per expert, where a launch is all prologue and epilogue.  Here a tile
+// is 128x256 and two workgroups share a CU (72 KiB of LDS, at most 256 registers each): one multiplies while the
+// other copies its first stages or writes its result.
+// Results are stored nontemporally, whatever their size (us with ordinary stores / so: 7 MB of them 9.5 / 8.7, 31 MB
+// 15.4 / 13.7, 64 MB 22.4 / 22.0, 192 MB 73 / 71, 350 MB 117 / 99).  A launch that reads a result of 30 to 250 MB
+// next loses as much as is gained here (with a pass over it: 51 MB 36 / 38, 128 MB 82 / 85), beyond that it gains
+// too (552 MB 375 / 330); weight gradients are not read before the backward has ended. The price is half again as
+// much operand traffic per product, so long reductions and large outputs stay with gmm_dtl.hip (the rule with both
+// sides' times is gmm_tn_short_pays in gmm.hip).
 #include "gmm_common.h"
 
 namespace gmoe {
