@@ -19,12 +19,11 @@
 //     tile's MFMAs.
 //   * Long reductions (STORE_SPREAD): a 16-bit result is rounded into half the registers while the next tile's
 //     first MFMAs overwrite the accumulators, and stored piece by piece under the MFMAs after those, so that
-//     the matrix cores see no epilogue (5 us of 33 per tile at 1024 rows per expert).  1024 rows: 7168 x 4096 over
-//     32 experts 1730 -> 1660 us, 2048 x 2816 over 64 750 -> 725; 4096 rows of 4096 x 28672 over 8 6050 -> 5940,
-//     where the chip's power is the bound.
+//     the matrix cores see no epilogue (2-4 % at 1024 rows per expert, nothing at 4096, where the chip's power is
+//     the bound; figures at launch_cfg).
 //   * Large results are stored past the L2s' reusable lines (nontemporal), and few rows per expert read both
 //     operands once beforehand (warm_operands): the launch is then bound by its writes.  4096 x 28672 over 8
-//     experts, operands from HBM: 190 rows each 698 -> 497 us (3.8 TB/s of results), 383 rows 914 -> 772.
+//     experts, operands from HBM: 192 rows each 663 -> 483 us (3.9 TB/s of results), 384 rows 882 -> 740.
 //   * Both operands have the reduction index (the token) as the slow dimension in memory; they are
 //     stored in LDS as they are in memory, [k][outer], and the MFMA fragments are read with the
 //     transposing LDS load ds_read_b64_tr_b16: a group of 16 lanes reads a 4(k) x 16(outer) block
@@ -446,19 +445,26 @@ static int launch_kernel(const GmmParams& p, hipStream_t st) {
   return gmoe_launch_status();
 }
 
-// n = rows per expert, us, operands not in a cache:
-//   * n 1024: stores spread over the next tile 1658 against 1711 after the tile (7168 x 4096, 32 experts), 677
-//     against 688 (2048 x 2816, 64), 1741 against 1699 (4096 x 28672, 8).  At 640 the copies wait behind the spread
-//     stores (1278 against 1141, 4096 x 28672).
-//   * nontemporal against ordinary stores: 895 against 924 (n 448, 4096 x 28672, 8), 388 against 399 (n 512, 2048 x 2816,
-//     64), 304 against 347 (n 256, 14336 x 4096, 8).  Results that the memory-side cache holds are better left there
-//     (n 256, 8 experts of 1024 x 4096, 64 MB: 30 against 39).
+// n = rows per expert, us, operands from HBM and a result buffer of its own for every launch (into one buffer, the
+// part of it that the memory-side cache still holds favours ordinary stores):
+//   * stores after the tile / spread over the next one: n 1024 811 / 789 (14336 x 4096, 8 experts), 1621 / 1581
+//     (7168 x 4096, 32), 662 / 653 (2048 x 2816, 64), 185 / 175 (1024 x 5632, 16); n 900 326 / 308 (1408 x 2048,
+//     64).  At n 640 as often behind as ahead (457 / 465, 252 / 245, 124 / 126).  A store covers four rows, and
+//     where those lie 14 KB and more apart, the copies wait behind the spread ones until a tile is long: n 1024
+//     1596 / 1656, n 1408 2100 / 2112, n 1600 2352 / 2339 (4096 x 28672, 8); n 1024 1347 / 1380, n 1408 1773 / 1770
+//     (6144 x 16384, 8); n 1024 820 / 827, n 1408 1072 / 1067 (2048 x 7168, 32).
+//   * ordinary / nontemporal stores after the tile: n 256 742 / 634, n 448 897 / 851 (4096 x 28672, 8), n 256 264 /
+//     246, n 512 387 / 394 (2048 x 2816, 64), n 256 99 / 84 (4096 x 4096, 8, 256 MB); smaller results either way: n
+//     256 74 / 71 (1024 x 5632, 16), 53 / 57 (1024 x 1024, 64), n 1152 100 / 112 (2816 x 1024, 16).
+constexpr int64_t kSpreadRows = 900, kSpreadRowsWide = 1408, kSpreadWide = 7168;
+
 template <int DT, int ODT>
 static int launch_cfg(const GmmParams& p, hipStream_t st) {
   if constexpr (ODT == GMOE_F32) {
     return launch_kernel<DT, ODT, STORE_NOW>(p, st);
   } else {
-    if (p.N / (p.E > 0 ? p.E : 1) >= 900) return launch_kernel<DT, ODT, STORE_SPREAD>(p, st);
+    if (p.N / (p.E > 0 ? p.E : 1) >= (p.M >= kSpreadWide ? kSpreadRowsWide : kSpreadRows))
+      return launch_kernel<DT, ODT, STORE_SPREAD>(p, st);
     if (gmm_tn_streams(p)) return launch_kernel<DT, ODT, STORE_NOW_STREAM>(p, st);
     return launch_kernel<DT, ODT, STORE_NOW>(p, st);
   }
