@@ -1133,68 +1133,23 @@ static int launch_gmm_cfg(const GmmParams& p, hipStream_t st, int blocks_per_cu 
   return gmoe_launch_status();
 }
 
-// Large tiles once an expert's share of rows (NN/NT) or the output itself (TN) can fill them and
+// Large tiles once an expert's share of rows (NN/NT, nn_large_tiles) or the output itself (TN) can fill them and
 // there are enough of them for every CU; smaller problems spread over more, smaller tiles.
 static inline bool gmm_large_tiles(const GmmParams& p, int mode) {
   const int64_t experts = p.E > 0 ? p.E : 1;
-  const int64_t rows_per_expert = mode == MODE_TN ? p.K : p.N / experts;
-  if (rows_per_expert < 512 || p.M < 256) return false;
-  const int64_t col_tiles = (p.M + 255) / 256;
-  const int64_t tiles = mode == MODE_TN ? experts * ((p.K + 255) / 256) * col_tiles
-                                        : ((p.N + 255) / 256) * col_tiles;
+  if (mode != MODE_TN) return nn_large_tiles(experts, p.N, p.M);
   // TN: the 128x128 kernel runs at about 0.4 of the large one's rate per FLOP, so the large tiles win
   // as soon as the small ones need a second round of their 512 slots (C3's shared experts, 176 large
   // tiles: 0.29 -> 0.22 ms)
-  return tiles >= (mode == MODE_TN ? 129 : 256);
+  return p.K >= 512 && p.M >= 256 && experts * ((p.K + 255) / 256) * ((p.M + 255) / 256) >= 129;
 }
 
-constexpr int64_t kRemainderMinRows = 2048;  // see gmm_use_remainder
-
-// Row-adaptive tiles (gmm_rows.hip) for 16-bit NN / NT: tiles of 64 to 256 rows x 256 columns that
-// share an expert's rows evenly, one workgroup per CU.  Measured against the 128x128 and 256x256 tiles
-// in the same process, n = rows per expert, times of both sides in us (K x M, experts):
-//   * n below 112 (NT: 128, with the activation 96): an expert is one 128-row tile either way and its weights bound
-//     the launch; the 128x128 kernel with two workgroups per CU streams them a little faster (n 64: 375 against 399
-//     for 4096 x 28672, 8 experts).
-//   * up to 512 rows the 128x128 kernel multiplies padding and moves twice the operands per product:
-//     n 384: 996 -> 731 (4096 x 28672, 8), 436 -> 338 (2048 x 2816, 64), NT 974 -> 765 (7168 x 4096, 32);
-//     n 160: 654 -> 380 (7168 x 4096, 32).
-//   * from 512 rows on the 256x256 tiles are the alternative, or 128x128 where those are too few.  NN gains
-//     1-17 % (n 1024: 1730 -> 1681, K 7168; 894: 119 -> 113, 1440 x 9632, 4; 1264: 126 -> 115, 544 x 2816, 24;
-//     against 128x128 tiles n 835: 47 -> 40, 1280 x 2048, 8).  NT gains up to K 896 (n 667: 76 -> 71, 672 x 1952,
-//     32; 824: 35 -> 30, 896 x 1728, 8) and loses 4-10 % beyond (its 64-byte pieces of two operands against
-//     128-byte ones there: 1632 -> 1727, K 4096).  From 2048 rows on the remainder launches take over.
-//   * the activation backward against 256x256 tiles gains from 512 rows on, whatever the last round holds, as
-//     both have the same rounds: n 619: 110 -> 85 (1088 x 4032, 8), 1004: 126 -> 119 (2112 x 1888, 8), 1578: 96 ->
-//     75 (736 x 704, 16), 4096 x 2944 225 -> 211; no gain at K 6016.
-//   * the smaller tiles spread better over the CUs with few tiles (K 2112, M 928, 8 experts, 64 tiles: 25 -> 33)
-//     and, backward, with a last round that leaves more than 30 % of all rounds idle.  As the chunks adapt
-//     to the rounds, NN is ahead from half a round on (144 tiles of 736 x 2144: 26 -> 24, 96 of 3808 x 1440: 59 ->
-//     52, but 112 of 576 x 1600: 17 -> 18), with the activation from a third (100 tiles of 768 x 5120: 25 -> 23,
-//     72 of 2496 x 768: 44 -> 39), NT of 512 rows and more between 0.6 and two rounds (192 tiles of 5632 x 1024: 149
-//     -> 130, 168 of 3552 x 3392: 90 -> 75; 144 of 1504 x 1472: 33 -> 36).
-//   * K 512 and less: prologue and epilogue weigh as much as the reduction (n 119: 47 -> 50, 512 x 7776, 24; but
-//     n 215: 130 -> 103, 576 x 7968, 32, with the activation n 135: 166 -> 126, 608 x 9728, 32).
-//   * the activation backward (NT) around 256 rows: half the experts take a second chunk of two units,
-//     whose epilogue does not overlap anything (361 -> 408 at K 7168); 128x128 tiles there.
+// Row-adaptive tiles (gmm_rows.hip) for 16-bit NN / NT: tiles of 64 to 256 rows x 256 columns that share an
+// expert's rows evenly, one workgroup per CU.  The rule, with both sides' times, is in rows_rule.h.
 static inline bool gmm_rows_pays(const GmmParams& p, int mode, int epi) {
-  const int64_t n = p.N / (p.E > 0 ? p.E : 1);
-  const bool glu = epi == EPI_GLU_FWD_SILU || epi == EPI_GLU_FWD_GELU;
-  const int64_t cols = glu ? (p.F + 127) / 128 : (p.M + 255) / 256;
-  const int64_t tiles = p.E * ((n + 16 + 255) / 256) * cols;
-  const int64_t cus = gmm_grid(1), rounds = (tiles + cus - 1) / cus;
-  if (p.K <= 512 || n >= kRemainderMinRows) return false;
-  const bool full = tiles * 4 >= cus * 3 && tiles * 10 >= rounds * cus * 7;
-  // narrower results pad the 256 columns
-  const bool wide = p.M >= 512;
-  if (mode == MODE_NN)
-    return (full && n >= (glu ? 96 : 112)) || (wide && n >= 128 && tiles * 10 >= cus * (glu ? 3 : 5));
-  if (epi != EPI_NONE) {
-    if (n >= 512) return gmm_large_tiles(p, mode) ? p.K <= 4096 : full;
-    return full && n >= 128 && !(n >= 240 && n < 288);
-  }
-  if (n >= 512) return (wide && tiles <= 2 * cus && tiles * 10 >= cus * 6) || (full && p.K <= 896);
-  return full && n >= 128;
+  const RowsKind kind = mode == MODE_NN ? (epi == EPI_NONE ? ROWS_NN : ROWS_NN_GLU)
+                                        : (epi == EPI_NONE ? ROWS_NT : ROWS_NT_GLU_BWD);
+  return rows_pays(kind, p.E, p.N, p.K, p.M, gmm_grid(1));
 }
 
 // dW of 16-bit operands with a short reduction (gmm_tn.hip: 128x256 tiles, two workgroups per CU) against the
@@ -1232,18 +1187,11 @@ static inline bool gmm_tn_warm_pays(const GmmParams& p) {
 // at 4096 rows per expert (Mixtral shape) it saves 4-7 % of a GEMM, at 1024 rows per expert (64 or 32
 // experts) the main kernel with its partial tiles is 5-10 % faster than the two launches.
 static inline bool gmm_use_remainder(const GmmParams& p) {
-  return p.N / (p.E > 0 ? p.E : 1) >= kRemainderMinRows;
+  return p.N / (p.E > 0 ? p.E : 1) >= kNnRemainderRows;
 }
 
-// Whether a 128x128-tile NN / NT launch is worth a split reduction, from the host-side sizes (an expert
-// has at least one row tile, and its last one is half full on average); the kernels decide again from the
-// tiles there are.
-static inline bool gmm_split_pays(const GmmParams& p) {
-  const int64_t least = p.N < p.E ? p.N : p.E, average = (p.N + 127) / 128 + p.E / 2;
-  const int64_t tiles = (average > least ? average : least) * ((p.M + 127) / 128);
-  return split_pieces(split_ns_per_k_tile(2), (p.K * 2 + 127) / 128, tiles, kSplitSlots,
-                      weight_stream_ns(p.E, p.K, p.M, 2)) > 1;
-}
+// Whether a 128x128-tile NN / NT launch is worth a split reduction; the kernels decide again from the tiles there are.
+static inline bool gmm_split_pays(const GmmParams& p) { return nn_split_pieces(p.E, p.N, p.K, p.M) > 1; }
 
 // fp32 values of workspace that an NN / NT launch can use.
 static inline int64_t gmm_workspace_floats(const GmmParams& p, int mode, int dtype) {

@@ -5,6 +5,7 @@
 
 #include "gmoe_common.h"
 #include "copy_range.h"
+#include "rows_rule.h"
 #include "split_rule.h"
 
 namespace gmoe {

@@ -1,11 +1,12 @@
 // Grouped GEMM with row-adaptive tiles for 16-bit operands (bf16 / fp16) on gfx950: NN and NT of
 // gmm.hip's contract, with the fused gated-activation epilogues, for a few dozen to a few hundred rows
-// per expert (the rule with both sides' times is gmm_rows_pays in gmm.hip).
+// per expert (the rule with both sides' times is rows_rule.h).
 //
 //   * A tile is RF*64 rows (RF = 1..4, chosen per tile) x 256 columns of C.  An expert's rows are cut
 //     into chunks of up to 256 (192, 128 where those fill the rounds better: best_max_units) that are as
-//     equal as 64-row steps allow, so at most 63 rows per expert are padding: a fixed 128- or 256-row tile multiplies a third of its rows for nothing at 380 rows
-//     per expert, and its operand stream is the larger the smaller the tile.
+//     equal as 64-row steps allow, so at most 63 rows per expert are padding: a fixed 128- or 256-row tile
+//     multiplies a third of its rows for nothing at 380 rows per expert, and its operand stream is the larger the
+//     smaller the tile.
 //   * 2x2 wavefronts of (RF*32) x 128, one workgroup per CU.
 //   * Operands go global -> LDS without staging registers (buffer_load ... lds) in stages of 32
 //     reduction elements, 4 stages for 256 rows up to 7 for 64 rows; one barrier per stage.
@@ -48,7 +49,8 @@ __device__ __forceinline__ int chunk_count(long long n, int max_units) {
 // The chunk size that ends first.  A stage of a tile of u units takes as long as its operands stream, 16 + 4 u KiB
 // at 42 GB/s; prologue and epilogue take as long as 250 KiB.  Where the largest chunks leave a round part empty,
 // smaller ones fill it (us with chunks of up to 256 rows and with these: NT 640 rows, 5632 x 1024, 16 experts 143 ->
-// 130; NN 370, 3808 x 1440, 8 61 -> 52; with the activation 258, 3392 x 6400, 4 82 -> 60).  units, chunks: of this thread's experts, summed over the workgroup here.
+// 130; NN 370, 3808 x 1440, 8 61 -> 52; with the activation 258, 3392 x 6400, 4 82 -> 60).  units, chunks: of this
+// thread's experts, summed over the workgroup here.
 __device__ __forceinline__ int best_max_units(int units, const int (&chunks)[kMaxUnits + 1], int nt_cnt, int grid,
                                               int64_t K, int (*sums)[kMaxUnits + 1], int lane, int wave) {
   int v[kMaxUnits + 1] = {units, 0, chunks[2], chunks[3], chunks[4]};
