@@ -6,14 +6,15 @@
 //   plan_count  per 256-token chunk and expert: number of routed tokens (wavefront ballots)
 //   plan_scan   one exclusive scan over the (expert-major) chunk counts
 //   plan_fill   rank inside the chunk from the ballots + chunk base -> destination rows
-// Up to 8192 chunk counts plan_fill adds up what it needs of them itself, and of a map of up to 16384 entries it
+// Up to 8192 chunk counts plan_fill adds up what it needs of them itself, and of a small map (kMapEntries) it
 // counts that too: two launches or one.
 // The plan is kept token-major (dst_map [T,E] int32) so that the row kernels, which run one
 // wavefront per token, find all destinations of a token in one coalesced load.
 //
 // Row kernels move whole rows with 16-byte accesses per lane (a wavefront covers 1 KiB per
-// instruction), with streaming (nontemporal) hints on data that is touched once: scatter (permute), gather-reduce in fp32 (unpermute; also permute's backward) and
-// the backward of the weighted unpermute including the gate gradients.
+// instruction), with streaming (nontemporal) hints on data that is touched once: scatter (permute), gather-reduce
+// in fp32 (unpermute; also permute's backward) and the backward of the weighted unpermute including the gate
+// gradients.
 #include <mutex>
 #include <type_traits>
 
@@ -773,11 +774,14 @@ static inline int dtype_bytes(int dt) {
   }
 }
 // Largest map that every workgroup of plan_fill counts by itself, and most chunk counts that every one adds up.
-// Times of a plan in a graph's replay, us: from the map 5.8 against 7.5 with three launches (128 x 4), 7.9 against 9.5
-// (1531 x 8), but 16.3 against 9.2 at 65536 entries (16384 x 4); from the counts 11.9 against 14.8 (8192 x 64, 2048
-// counts), 14.2 against 18.3 (4096 counts), 42.5 against 39.3 at 16384 counts.  Issued one by one, each launch less
-// is 4 to 5 us of host time as well.
-constexpr int64_t kMapEntries = 16 * 1024, kCountEntries = 8 * 1024;
+// Times of a plan in a graph's replay, us, one launch / two / three (tokens x experts): from the map 7.0 / 7.1 /
+// 8.9 (512 x 4), 8.2 / 8.2 / 10.7 (2048 x 8), 8.9 / 10.3 / 11.7 (256 x 64), but 13.3 / 10.6 / 12.4 at 65536 entries
+// (1024 x 64).  A workgroup walks all tokens, four chunks at a time, and without the 8-byte loads byte by byte, so
+// that there are limits on those too: 9.1 / 8.2 / 11.3 (3072 x 8), 8.9 / 8.5 / 10.5 (768 x 7), 12.8 / 9.5 / 11.9
+// (1024 x 13), 10.1 / 7.2 / 9.4 (2048 x 4), 33 / 6 / 8 (16384 x 1).  From the counts 11.9 against 14.8 (8192 x 64,
+// 2048 counts), 14.2 against 18.3 (4096 counts), 42.5 against 39.3 at 16384 counts.  Issued one by one, each launch
+// less is 4 to 5 us of host time as well.
+constexpr int64_t kMapEntries = 16 * 1024, kMapTokens = 2048, kMapTokensBytes = 768, kCountEntries = 8 * 1024;
 static inline bool prob_dtype_ok(int dt) { return dt == GMOE_F32 || dt == GMOE_BF16 || dt == GMOE_F16; }
 
 }  // namespace gmoe
@@ -836,7 +840,7 @@ static int permute_plan_launch(const uint8_t* routing_map, int64_t T, int E, int
                        reinterpret_cast<long long*>(row_id_map), reinterpret_cast<long long*>(tokens_per_expert),
                        reinterpret_cast<long long*>(expert_offsets));
   };
-  if (NC > 0 && T * E <= kMapEntries) {
+  if (NC > 0 && T * E <= kMapEntries && T <= (vec8 ? kMapTokens : kMapTokensBytes)) {
     fill(std::integral_constant<int, BASE_MAP>{}, nullptr);
     return gmoe_launch_status();
   }

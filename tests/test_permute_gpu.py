@@ -267,10 +267,11 @@ def test_unpermute_with_residual_equals_unpermute_then_add(pkg, dev, dtype, T, E
 
 @pytest.mark.parametrize("capacity", [0, 37])
 @pytest.mark.parametrize("T,E", [(1, 1), (255, 3), (256, 4), (257, 12), (2048, 8), (2049, 8), (4096, 4), (273, 60), (274, 60),
-                                 (1024, 16), (1025, 16), (32768, 64), (32769, 64)])
+                                 (1024, 16), (1025, 16), (32768, 64), (32769, 64), (768, 13), (769, 13), (5661, 1)])
 def test_plan_at_the_limits_of_its_launches(pkg, dev, T, E, capacity):
-    """One launch up to 16384 map entries, two up to 8192 chunk counts, three beyond; a last slice of fewer than
-    eight experts; an expert without tokens and one with all of them."""
+    """One launch up to 16384 map entries of up to 2048 tokens (768 where the experts are no multiple of eight), two
+    up to 8192 chunk counts, three beyond; a last slice of fewer than eight experts; an expert without tokens and
+    one with all of them."""
     g = torch.Generator().manual_seed(T + E)
     m = torch.rand(T, E, generator=g) < 0.3
     m[:, -1] = True
