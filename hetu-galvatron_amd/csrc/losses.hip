@@ -128,12 +128,11 @@ __global__ __launch_bounds__(kSeqThreads) void seq_aux_stats_kernel(
 // loss = scale * sum_b sum_e counts[b,e] * scores[b,e].  A sequence's sum is one wavefront's, in lane-strided
 // order; a wavefront adds its sequences in ascending order, and the wavefronts' totals are added in order.
 // parts > 1: first the partial counts and scores of `ws`, again in order.
-constexpr int kSeqFinishThreads = 512;
-
-__global__ __launch_bounds__(kSeqFinishThreads) void seq_aux_finish_kernel(float* seq_counts, float* seq_scores,
-                                                                           const float* ws, int parts, int B, int E,
-                                                                           float scale, float* loss) {
-  constexpr int NW = kSeqFinishThreads / GMOE_WAVE;
+// NW: wavefronts; PARTS: several partial counts and scores.  One sequence whole: 0.5 us less of 7 than the general form.
+template <int NW, bool PARTS>
+__global__ __launch_bounds__(NW * GMOE_WAVE) void seq_aux_finish_kernel(float* seq_counts, float* seq_scores,
+                                                                        const float* ws, int parts, int B, int E,
+                                                                        float scale, float* loss) {
   __shared__ float wave_total[NW];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t BE = (int64_t)B * E;
@@ -143,7 +142,7 @@ __global__ __launch_bounds__(kSeqFinishThreads) void seq_aux_finish_kernel(float
     for (int e = lane; e < E; e += 64) {
       const int64_t at = (int64_t)b * E + e;
       float c = 0.f, s = 0.f;
-      if (parts > 1) {
+      if constexpr (PARTS) {
 #pragma unroll 16
         for (int p = 0; p < parts; ++p) {
           c += ws[p * 2 * BE + at];
@@ -159,13 +158,13 @@ __global__ __launch_bounds__(kSeqFinishThreads) void seq_aux_finish_kernel(float
     }
     total += wave_sum_f32(a);
   }
-  if (lane == 0) wave_total[wave] = total;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    float sum = wave_total[0];
-    for (int w = 1; w < NW; ++w) sum += wave_total[w];
-    loss[0] = sum * scale;
+  if constexpr (NW > 1) {
+    if (lane == 0) wave_total[wave] = total;
+    __syncthreads();
+    total = wave_total[0];
+    for (int w = 1; w < NW; ++w) total += wave_total[w];
   }
+  if (threadIdx.x == 0) loss[0] = total * scale;
 }
 
 // ---- sinkhorn ----------------------------------------------------------------------------------------
@@ -499,8 +498,15 @@ extern "C" int gmoe_seq_aux_loss_ws(const void* logits, int dtype, const uint8_t
   // cost_coeff = counts * E / (S k), mean over s of the scores, sum over e, mean over b, times coeff
   const float scale = coeff * (float)E /
                       ((float)batch_size * (float)seq_length * (float)seq_length * (float)k);
-  hipLaunchKernelGGL(seq_aux_finish_kernel, dim3(1), dim3(kSeqFinishThreads), 0, st, seq_counts, seq_scores, ws, parts,
-                     batch_size, E, scale, loss);
+  auto finish = [&](auto waves_c, auto parts_c) {
+    constexpr int NW = decltype(waves_c)::value;
+    hipLaunchKernelGGL((seq_aux_finish_kernel<NW, decltype(parts_c)::value>), dim3(1), dim3(NW * GMOE_WAVE), 0, st,
+                       seq_counts, seq_scores, ws, parts, batch_size, E, scale, loss);
+  };
+  constexpr std::integral_constant<int, 1> one{};
+  constexpr std::integral_constant<int, 8> eight{};
+  if (batch_size > 1) parts > 1 ? finish(eight, std::true_type{}) : finish(eight, std::false_type{});
+  else parts > 1 ? finish(one, std::true_type{}) : finish(one, std::false_type{});
   return gmoe_launch_status();
 }
 
