@@ -213,8 +213,10 @@ __device__ __forceinline__ void run_tile(const GmmParams& p, const Item& it, uns
   const int all_stages = (int)((red + BKT - 1) / BKT);
   int from = 0, stages = all_stages;
   if constexpr (CAN_SPLIT) {
-    from = all_stages * it.piece / p.pieces;
-    stages = all_stages * (it.piece + 1) / p.pieces;
+    if (p.pieces > 1) {
+      from = all_stages * it.piece / p.pieces;
+      stages = all_stages * (it.piece + 1) / p.pieces;
+    }
   }
   if (stages > from) {
     la.load((int64_t)from * BKT, red);
@@ -428,9 +430,12 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gmm_f32_kernel(GmmParams p) {
       if (slot >= share || v >= total) break;
     }
     Item it;
-    it.piece = __builtin_amdgcn_readfirstlane(v / tiles_all);
-    v -= it.piece * tiles_all;
-    if (v < tile_cum[e]) e = 0;
+    it.piece = 0;
+    if (p.pieces > 1) {
+      it.piece = __builtin_amdgcn_readfirstlane(v / tiles_all);
+      v -= it.piece * tiles_all;
+      if (v < tile_cum[e]) e = 0;
+    }
     while (tile_cum[e + 1] <= v) ++e;
     it.e = __builtin_amdgcn_readfirstlane(e);
     it.row0 = group_begin(p, it.e);
