@@ -18,7 +18,6 @@
 //    columns are cut into slabs of 256 * NV vectors (blockIdx.y) so the registers do not grow with H.
 //  * weight gradient dW = dlogits^T @ x: the same ownership with the accumulators in registers; one
 //    fp32 partial [E,H] per workgroup, summed in a fixed order by sum_partial_rows.
-#include <atomic>
 #include <type_traits>
 
 #include "gmm_common.h"

@@ -472,7 +472,7 @@ __device__ inline int resolve_row_part(const GmmParams& p, int k_tiles, int* cou
   const long long rounds_saved = (tiles_all + g - 1) / g - (tiles_main + g - 1) / g;
   // the pieces launch_gmm_remainder's launch comes to
   const long long slots = p.ws == nullptr ? 0 : p.ws_floats / (128 * 128);
-  const int s = split_pieces(split_ns_per_k_tile(2), k_tiles, tiles_rem, slots < kSplitSlots ? slots : kSplitSlots, 0);
+  const int s = split_pieces(k_tiles, tiles_rem, slots < kSplitSlots ? slots : kSplitSlots, 0);
   const long long saved = 1300 * rounds_saved * k_tiles;
   const long long cost = s > 1 ? 1900ll * (k_tiles / s) + kSplitReduceNs + kSplitNsPerPiece * tiles_rem * s
                                : 2500 * ((tiles_rem + kSplitSlots - 1) / kSplitSlots) * k_tiles + 8000;
@@ -526,10 +526,10 @@ __device__ __forceinline__ void build_tile_cum(const GmmParams& p, int part, int
 }
 
 // What both kernels of a split launch use: depends on launch parameters and the tile count only.
-__device__ __forceinline__ int split_count(const GmmParams& p, int elem_bytes, long long total_tiles,
-                                           long long k_tiles, long long tile_elems) {
+__device__ __forceinline__ int split_count(const GmmParams& p, long long total_tiles, long long k_tiles,
+                                           long long tile_elems) {
   if (p.split_slots == 0) return 1;
-  const int s = split_pieces(split_ns_per_k_tile(elem_bytes), k_tiles, total_tiles, p.split_slots, p.stream_ns);
+  const int s = split_pieces(k_tiles, total_tiles, p.split_slots, p.stream_ns);
   return (long long)s * total_tiles * tile_elems <= p.ws_floats ? s : 1;
 }
 
@@ -665,7 +665,7 @@ __global__ __launch_bounds__(kGemmThreads, (BM == 128 && BN == 128) ? 2 : 1) voi
   // gmm_split_reduce_kernel adds the S partial tiles in order.
   constexpr bool CAN_SPLIT = MODE != MODE_TN && EPI == EPI_NONE && !BQ && SMALL;
   constexpr long long TILE_ELEMS = (long long)BM * BN;
-  const int S = CAN_SPLIT ? split_count(p, ES, total_tiles, (K + BK - 1) / BK, TILE_ELEMS) : 1;
+  const int S = CAN_SPLIT ? split_count(p, total_tiles, (K + BK - 1) / BK, TILE_ELEMS) : 1;
   const long long total_work = total_tiles * S;
 
   // Workgroup w runs on XCD w%8.  Give XCD x the consecutive positions [x*G/8, (x+1)*G/8) of
@@ -1073,7 +1073,7 @@ __global__ __launch_bounds__(kGemmThreads) void gmm_split_reduce_kernel(GmmParam
   if (part == ROWS_NONE) return;
   build_tile_cum<MODE, BM>(p, part, nt_cnt, 0, tile_cum);
   const long long total_tiles = tile_cum[p.E];
-  const int S = split_count(p, Elem<DT>::bytes, total_tiles, k_tiles, TILE_ELEMS);
+  const int S = split_count(p, total_tiles, k_tiles, TILE_ELEMS);
   if (S == 1) return;  // the first launch did everything
   int e = 0;
   for (long long item = blockIdx.x; item < total_tiles * 4; item += gridDim.x) {

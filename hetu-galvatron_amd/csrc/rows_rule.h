@@ -56,7 +56,7 @@ inline bool nn_large_tiles(int64_t E, int64_t N, int64_t M) {
 inline int nn_split_pieces(int64_t E, int64_t N, int64_t K, int64_t M) {
   const int64_t least = N < E ? N : E, average = (N + 127) / 128 + E / 2;
   const int64_t tiles = (average > least ? average : least) * ((M + 127) / 128);
-  return split_pieces(split_ns_per_k_tile(2), (K * 2 + 127) / 128, tiles, kSplitSlots, weight_stream_ns(E, K, M, 2));
+  return split_pieces((K * 2 + 127) / 128, tiles, kSplitSlots, weight_stream_ns(E, K, M, 2));
 }
 
 // Five times the mean of f(rows of an expert), for loads that differ by up to 14 %.
