@@ -27,7 +27,7 @@ constexpr int BN = 256;
 constexpr int BKT = 32;  // reduction elements per stage
 constexpr int B_BYTES = BN * BKT * 2;
 constexpr int kUnit = 64;     // rows per unit: 32 for each of the two wavefront rows
-constexpr int kMaxUnits = 4;  // units per tile
+constexpr int kMaxUnits = kRowsMaxUnits;  // units per tile
 
 // LDS stages of a tile of RF units: as many as fit 144 KiB
 template <int RF>
@@ -46,11 +46,7 @@ __device__ __forceinline__ int unit_count(long long n) { return (int)((n + kUnit
 __device__ __forceinline__ int chunk_count(long long n, int max_units) {
   return (unit_count(n) + max_units - 1) / max_units;
 }
-// The chunk size that ends first.  A stage of a tile of u units takes as long as its operands stream, 16 + 4 u KiB
-// at 42 GB/s; prologue and epilogue take as long as 250 KiB.  Where the largest chunks leave a round part empty,
-// smaller ones fill it (us with chunks of up to 256 rows and with these: NT 640 rows, 5632 x 1024, 16 experts 143 ->
-// 130; NN 370, 3808 x 1440, 8 61 -> 52; with the activation 258, 3392 x 6400, 4 82 -> 60).  units, chunks: of this
-// thread's experts, summed over the workgroup here.
+// rows_chunk_units for the launch; units, chunks: of this thread's experts, summed over the workgroup here.
 __device__ __forceinline__ int best_max_units(int units, const int (&chunks)[kMaxUnits + 1], int nt_cnt, int grid,
                                               int64_t K, int (*sums)[kMaxUnits + 1], int lane, int wave) {
   int v[kMaxUnits + 1] = {units, 0, chunks[2], chunks[3], chunks[4]};
@@ -67,19 +63,7 @@ __device__ __forceinline__ int best_max_units(int units, const int (&chunks)[kMa
 #pragma unroll
     for (int w = 0; w < kGemmThreads / 64; ++w) v[i] += sums[w][i];
   }
-  const float fixed = 16.f + 250.f / (float)((K + BKT - 1) / BKT);
-  int best = kMaxUnits;
-  float least = 0.f;
-#pragma unroll
-  for (int u = kMaxUnits; u >= 2; --u) {
-    const int rounds = (int)(((long long)v[u] * nt_cnt + grid - 1) / grid);
-    const float cost = (float)rounds * (fixed + 4.f * (float)v[0] / (float)(v[u] > 0 ? v[u] : 1));
-    if (u == kMaxUnits || cost < 0.95f * least) {
-      best = u;
-      least = cost;
-    }
-  }
-  return best;
+  return rows_chunk_units(v, nt_cnt, grid, K);
 }
 // first unit and unit count of chunk c of cnt
 __device__ __forceinline__ void chunk_units(long long n, int cnt, int c, int& first, int& units) {

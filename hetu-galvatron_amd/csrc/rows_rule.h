@@ -1,5 +1,6 @@
 // Whether a 16-bit NN / NT launch goes to the row-adaptive tiles (gmm_rows.hip): what it takes there against what
-// it takes on the 256x256 tiles, or on 128x128 ones where those are too few.  Only the host asks.
+// it takes on the 256x256 tiles, or on 128x128 ones where those are too few (only the
+// host asks); and into which chunks the kernel cuts an expert's rows.
 //
 // Both sides were measured for 3400 shapes (E 1-64, 72-2040 rows per expert, K 256-28672, M 128-28672, 3e8 to 4e12
 // operations, weights from HBM, loads that differ by 7 %), and the constants are fitted to them.  us of the other
@@ -21,6 +22,29 @@
 #include "split_rule.h"
 
 namespace gmoe {
+
+// Rows of a chunk, in units of 64: the size, of 4, 3 and 2, that ends first.  v[0]: units of all experts, v[2..4]:
+// their chunks of up to so many units.  A stage of a tile of u units takes as long as its operands stream, 16 + 4 u
+// KiB at 42 GB/s; prologue and epilogue take as long as 250 KiB.  Where the largest chunks leave a round part
+// empty, smaller ones fill it (us with chunks of up to 256 rows / with these, rows per expert: NT 640, 5632 x 1024,
+// 16 experts 146 / 137; NN 640, 2816 x 1024, 16 75 / 69; with the activation 817, 6432 x 4832, 8 468 / 428).  Asked
+// by the kernel.
+constexpr int kRowsMaxUnits = 4;
+__host__ __device__ inline int rows_chunk_units(const int (&v)[kRowsMaxUnits + 1], int col_tiles, int grid, int64_t K) {
+  const float fixed = 16.f + 250.f / (float)((K + 31) / 32);
+  int best = kRowsMaxUnits;
+  float least = 0.f;
+#pragma unroll
+  for (int u = kRowsMaxUnits; u >= 2; --u) {
+    const int rounds = (int)(((long long)v[u] * col_tiles + grid - 1) / grid);
+    const float cost = (float)rounds * (fixed + 4.f * (float)v[0] / (float)(v[u] > 0 ? v[u] : 1));
+    if (u == kRowsMaxUnits || cost < 0.95f * least) {
+      best = u;
+      least = cost;
+    }
+  }
+  return best;
+}
 
 enum RowsKind { ROWS_NN, ROWS_NN_GLU, ROWS_NT, ROWS_NT_GLU_BWD };
 

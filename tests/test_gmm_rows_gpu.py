@@ -8,6 +8,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 ROWS = [0, 1, 63, 64, 65, 127, 128, 129, 191, 193, 255, 256, 257, 320, 511, 513]
+EDGES = [(1024, 1024, 4), (1160, 904, 4), (1544, 1096, 3), (520, 1024, 4)]  # K, F, times that ROWS are repeated
 
 
 def on_kernel(kernel, call, form=""):
@@ -25,7 +26,7 @@ def on_kernel(kernel, call, form=""):
 
 @pytest.mark.parametrize("act", ["silu", "gelu"])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("K,F,times", [(1024, 1024, 4), (1160, 904, 4), (1544, 1096, 3), (520, 1024, 4)])
+@pytest.mark.parametrize("K,F,times", EDGES)
 def test_chunk_edges(pkg, dev, dtype, K, F, times, act):
     """Every size of expert `times` times: as often as it takes for F columns to be most of a round of tiles, short
     of which the launches go to smaller ones (48 experts, 1024 x 1024, us there and here: NT 41 / 44, backward 55 / 60)."""

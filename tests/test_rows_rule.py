@@ -1,10 +1,12 @@
 """The choice between the row-adaptive tiles and the others (csrc/rows_rule.h) where both were measured and one is
-clearly ahead, and at the limits of what it looks at."""
+clearly ahead, and at the limits of what it looks at; and the chunks that the row-adaptive tiles cut rows into."""
 import os
 import shutil
 import subprocess
 
 import pytest
+
+from test_gmm_rows_gpu import EDGES, ROWS
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "hetu-galvatron_amd", "csrc")
 PROGRAM = """
@@ -13,9 +15,13 @@ PROGRAM = """
 #include "rows_rule.h"
 #include <cstdio>
 int main() {
-  long long kind, E, N, K, M;
-  while (std::scanf("%lld %lld %lld %lld %lld", &kind, &E, &N, &K, &M) == 5)
-    std::printf("%d\\n", gmoe::rows_pays((gmoe::RowsKind)kind, E, N, K, M, 256));
+  long long v, a, b, c, d, e;
+  while (std::scanf("%lld %lld %lld %lld %lld %lld", &v, &a, &b, &c, &d, &e) == 6) {
+    const int units[5] = {(int)a, 0, (int)b, (int)c, (int)d};
+    const int col_tiles = (int)(e >> 32);
+    std::printf("%d\\n", v < 0 ? gmoe::rows_chunk_units(units, col_tiles, 256, e & 0xffffffff)
+                               : gmoe::rows_pays((gmoe::RowsKind)v, a, b, c, d, e));
+  }
 }
 """
 NN, GLU, NT, GLU_BWD = range(4)
@@ -35,22 +41,55 @@ MEASURED = [
 ]
 
 
-@pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
-def test_choice(tmp_path):
-    (tmp_path / "rule.cpp").write_text(PROGRAM)
-    exe = str(tmp_path / "rule")
-    subprocess.check_call(["g++", "-O2", "-std=c++17", "-I" + CSRC, str(tmp_path / "rule.cpp"), "-o", exe])
+@pytest.fixture(scope="module")
+def evaluate(tmp_path_factory):
+    if shutil.which("g++") is None:
+        pytest.skip("needs g++")
+    folder = tmp_path_factory.mktemp("rule")
+    (folder / "rule.cpp").write_text(PROGRAM)
+    exe = str(folder / "rule")
+    subprocess.check_call(["g++", "-O2", "-std=c++17", "-Wno-unknown-pragmas", "-I" + CSRC, str(folder / "rule.cpp"), "-o", exe])
 
-    def choices(cases):
-        text = "\n".join("%d %d %d %d %d" % c for c in cases)
-        return [int(v) for v in subprocess.run([exe], input=text, text=True, capture_output=True, check=True).stdout.split()]
+    def run(cases):
+        text = "\n".join("%d %d %d %d %d %d" % c for c in cases)
+        out = subprocess.run([exe], input=text, text=True, capture_output=True, check=True).stdout.split()
+        assert len(out) == len(cases)
+        return [int(v) for v in out]
 
-    got = choices([(kind, E, n * E, K, M) for kind, E, n, K, M, _, _ in MEASURED])
+    return run
+
+
+def test_choice(evaluate):
+    got = evaluate([(kind, E, n * E, K, M, 256) for kind, E, n, K, M, _, _ in MEASURED])
     wrong = [c for c, v in zip(MEASURED, got) if v != (c[6] < c[5])]
     assert not wrong, wrong
     # no rows, fewer than 96, reductions of up to 512, 2048 rows and more: never; one expert and a thousand: an answer
     shapes = [(E, n, K, M) for E in (1, 8, 1024) for n in (0, 1, 95, 96, 2047, 2048) for K in (8, 512, 520, 4096)
               for M in (8, 128, 4096)]
     for kind in (NN, GLU, NT, GLU_BWD):
-        for (E, n, K, M), v in zip(shapes, choices([(kind, E, n * E, K, M) for E, n, K, M in shapes])):
+        for (E, n, K, M), v in zip(shapes, evaluate([(kind, E, n * E, K, M, 256) for E, n, K, M in shapes])):
             assert v in (0, 1) and not (v and (n < 96 or n >= 2048 or K <= 512)), (kind, E, n, K, M)
+
+
+def test_chunks(evaluate):
+    """Chunks of up to 256, 192 and 128 rows against the rule in Python, for the edge test on the GPU, which reaches all
+    three; no rows at all; one tile."""
+    def units(rows):
+        u = [-(-r // 64) for r in rows]
+        return [sum(u)] + [sum(-(-x // size) for x in u) for size in (2, 3, 4)]
+
+    def model(counts, col_tiles, K):
+        best, least = 4, None
+        for size in (4, 3, 2):
+            chunks = counts[size - 1]
+            cost = -(-chunks * col_tiles // 256) * (16 + 250 / -(-K // 32) + 4 * counts[0] / max(chunks, 1))
+            if least is None or cost < 0.95 * least:
+                best, least = size, cost
+        return best
+
+    edges = [(units(ROWS * times), cols, K) for K, F, times in EDGES for cols in (-(-F // 128), -(-F // 256))]
+    other = [(units(rows), cols, K) for rows in ([0, 0], [1], [640] * 16, [256] * 64, [370] * 8) for cols in (1, 4, 6, 25)
+             for K in (520, 1024, 5632)]
+    got = evaluate([(-1, *counts, cols << 32 | K) for counts, cols, K in edges + other])
+    assert got == [model(*c) for c in edges + other]
+    assert set(got[:len(edges)]) == {2, 3, 4}
