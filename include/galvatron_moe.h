@@ -104,7 +104,8 @@ int gmoe_seq_aux_loss(const void* logits, int dtype, const uint8_t* routing_map,
                       float* seq_scores, float* loss, void* stream);
 
 /* The same with a workspace of gmoe_seq_aux_loss_workspace_bytes (0: none is used), in which several
- * workgroups share a sequence; a smaller one, or NULL, is used as far as it goes. */
+ * workgroups share a sequence; a smaller one, or NULL, is used as far as it goes.  How many share one, and with
+ * that the order of the additions and the last bits of scores and loss, depend on the workspace's size. */
 int64_t gmoe_seq_aux_loss_workspace_bytes(int64_t seq_length, int batch_size, int E);
 int gmoe_seq_aux_loss_ws(const void* logits, int dtype, const uint8_t* routing_map, int64_t seq_length,
                          int batch_size, int E, int k, int score_fn, float coeff, float* seq_counts,
@@ -313,11 +314,11 @@ int gmoe_bias_rows_bwd(const void* grad, int dtype, int64_t N, int64_t M,
  * a, b in `dtype` (GMOE_BF16, GMOE_F16 or GMOE_F32), fp32 accumulation, c in `out_dtype`.
  * K and M must be multiples of 8 (16-byte rows).  One persistent kernel walks a device-side tile
  * list built from expert_offsets; no host synchronisation.
- * workspace (optional, 16-byte aligned, workspace_bytes long): scratch for fp32 partial tiles.  With
- * gmoe_gmm_workspace_bytes(...) bytes, the launch for the experts' short last row tiles (trans_b
- * with large groups) splits its reduction over otherwise idle CUs; without, it runs unsplit.  The
- * result does not depend on the contents of the workspace, only (in the last bits: another order of
- * the same fp32 additions) on whether one is given.
+ * workspace (optional, 16-byte aligned, workspace_bytes long): scratch for fp32 partial results.  With
+ * gmoe_gmm_workspace_bytes(...) bytes, launches of few tiles, and the one for the experts' short last
+ * row tiles with large groups, split their reduction over otherwise idle CUs; a smaller one is used as
+ * far as it goes, without one they run unsplit.  The result does not depend on the contents of the
+ * workspace, only (in the last bits: another order of the same fp32 additions) on its size.
  */
 int64_t gmoe_gmm_workspace_bytes(int E, int64_t N, int64_t K, int64_t M, int trans_a, int trans_b,
                                  int dtype);

@@ -86,6 +86,30 @@ def test_pieces_leave_rows_outside_the_groups(pkg, dev, mode):
     assert ((c[first:last] - want).double().cpu().abs() <= 2 * 2.0 ** -24 * (13 + 112 + 16) * mag).all()
 
 
+@pytest.mark.parametrize("mode", ["NN", "NT"])
+@pytest.mark.parametrize("room", [0, 0.5, 1, 2, 3.7, None])
+def test_smaller_workspaces(pkg, dev, mode, room):
+    """NULL, less than a piece, one, fewer pieces than wanted, all: as many as fit, and nothing is written behind."""
+    counts, K, M = [37, 30, 41, 0], 1416, 2048
+    E, N, L, nt = len(counts), sum(counts), pkg._C.lib(), int(mode == "NT")
+    off = torch.tensor([0] + counts, device=dev).cumsum(0)
+    a, b = operands(mode, N, K, M, E, dev, 3)
+    piece, need = N * M * 4, L.gmoe_gmm_workspace_bytes(E, N, K, M, 0, nt, 0)
+    assert need >= 4 * piece
+    size = need if room is None else int(room * piece) // 4 * 4
+    ws, c = torch.full((need // 4 + 1024,), 5.0, device=dev), torch.empty(N, M, device=dev)
+    assert L.gmoe_gmm(a.data_ptr(), b.data_ptr(), c.data_ptr(), off.data_ptr(), E, N, K, M, 0, nt, 0, 0,
+                      ws.data_ptr() if room != 0 else None, size, torch.cuda.current_stream().cuda_stream) == 0
+    # what is used are whole pieces, two or more
+    pieces = size // piece
+    used = (ws != 5.0).nonzero()
+    assert (len(used) == 0 and pieces < 2) or piece // 4 < int(used[-1]) + 1 <= pieces * piece // 4, (pieces, int(used[-1]))
+    # as in test_pieces
+    bound = 2.0 ** -24 * (1 + 12 + (K + 31) // 32 + 16)
+    ref, mag = reference(mode, a, b, counts), reference(mode, a, b, counts, torch.abs)
+    assert ((c.double().cpu() - ref).abs() <= bound * mag).all()
+
+
 @pytest.mark.parametrize("mode", MODES)
 @pytest.mark.parametrize("value, other", [(float("inf"), 1.0), (float("-inf"), 0.0), (float("nan"), 1.0),
                                           (torch.finfo(torch.float32).max, 2.0 ** -20)])

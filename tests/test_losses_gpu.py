@@ -48,6 +48,37 @@ def test_seq_aux_loss_kernel(pkg, orc, dev, score_fn, S, B, E, k):
     assert torch.equal(loss, loss2) and torch.equal(scores, scores2)
 
 
+@pytest.mark.parametrize("batch", [1, 3])
+@pytest.mark.parametrize("room", [None, 0, 0.5, 1, 2, 3.7])
+def test_seq_aux_loss_smaller_workspaces(pkg, orc, dev, batch, room):
+    """The entry point without a workspace, a workspace of NULL, of less than a part, of one, of fewer parts than
+    wanted: the same loss, and nothing is written behind the parts that fit."""
+    S, E, k, coeff, L = 2500, 64, 8, 0.03, pkg._C.lib()
+    logits = make_logits(S * batch, E, torch.float32, seed=batch)
+    _, rmap, _ = orc.topk_softmax_with_capacity(logits, k)
+    want = orc.sequence_load_balancing_loss(oracle_scores(logits, "softmax", k), rmap, batch, S, k, coeff)
+    part, need = 2 * batch * E * 4, L.gmoe_seq_aux_loss_workspace_bytes(S, batch, E)
+    assert need >= 4 * part
+    x, m = logits.to(dev), rmap.to(dev)
+    counts, scores = (torch.empty(batch, E, device=dev) for _ in range(2))
+    loss, ws = torch.empty((), device=dev), torch.full((need // 4,), -1.0, device=dev)
+    st = torch.cuda.current_stream().cuda_stream
+    args = (x.data_ptr(), 0, m.data_ptr(), S, batch, E, k, pkg._C.SCORE_SOFTMAX, coeff, counts.data_ptr(), scores.data_ptr(),
+            loss.data_ptr())
+    size = int((room or 0) * part) // 4 * 4
+    if room is None:
+        assert L.gmoe_seq_aux_loss(*args, st) == 0
+    else:
+        assert L.gmoe_seq_aux_loss_ws(*args, ws.data_ptr() if room else None, size, st) == 0
+    parts = size // part
+    written = int((ws != -1.0).sum()) * 4  # counts and scores are not negative
+    assert written == (parts * part if parts > 1 else 0)
+    assert torch.equal(counts.cpu(), rmap.view(S, batch, E).sum(0).float())
+    torch.testing.assert_close(scores.cpu(), oracle_scores(logits, "softmax", k).view(S, batch, E).sum(0), rtol=1e-5,
+                               atol=1e-6)
+    torch.testing.assert_close(loss.cpu(), want, rtol=1e-5, atol=1e-9)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_seq_aux_loss_16bit_logits(pkg, orc, dev, dtype):
     S, B, E, k, coeff = 128, 4, 8, 2, 0.01
