@@ -273,7 +273,8 @@ __global__ __launch_bounds__(kGemmThreads) void gmm_dtl_kernel(GmmParams p) {
     sv[t % 4] = *lds_at<const u32x4>((get ^ (t % 4 * 64)) + t * 1024);
   };
   auto stage_store = [&](auto t_c) {
-    __builtin_amdgcn_raw_buffer_store_b128(sv[decltype(t_c)::value % 4], rc, (int)vo, 0, STORE == STORE_NOW ? 0 : kNontemporal);
+    __builtin_amdgcn_raw_buffer_store_b128(sv[decltype(t_c)::value % 4], rc, (int)vo, 0,
+                                           STORE == STORE_NOW ? 0 : kNontemporal);
     vo += four_rows;
   };
   auto locate = [&](const Work& w) {  // where the tile's result goes

@@ -128,7 +128,8 @@ __global__ __launch_bounds__(kSeqThreads) void seq_aux_stats_kernel(
 // loss = scale * sum_b sum_e counts[b,e] * scores[b,e].  A sequence's sum is one wavefront's, in lane-strided
 // order; a wavefront adds its sequences in ascending order, and the wavefronts' totals are added in order.
 // parts > 1: first the partial counts and scores of `ws`, again in order.
-// NW: wavefronts; PARTS: several partial counts and scores.  One sequence whole: 0.5 us less of 7 than the general form.
+// NW: wavefronts; PARTS: several partial counts and scores.  One sequence whole: 0.5 us less of 7 than the general
+// form.
 template <int NW, bool PARTS>
 __global__ __launch_bounds__(NW * GMOE_WAVE) void seq_aux_finish_kernel(float* seq_counts, float* seq_scores,
                                                                         const float* ws, int parts, int B, int E,
@@ -489,9 +490,18 @@ extern "C" int gmoe_seq_aux_loss_ws(const void* logits, int dtype, const uint8_t
   float* scores = parts > 1 ? ws + BE : seq_scores;
   int rc;
   switch (dtype) {
-    case GMOE_F32: rc = launch_seq_stats<GMOE_F32>(G, logits, routing_map, seq_length, batch_size, E, k, sig, counts, scores, parts, st); break;
-    case GMOE_BF16: rc = launch_seq_stats<GMOE_BF16>(G, logits, routing_map, seq_length, batch_size, E, k, sig, counts, scores, parts, st); break;
-    case GMOE_F16: rc = launch_seq_stats<GMOE_F16>(G, logits, routing_map, seq_length, batch_size, E, k, sig, counts, scores, parts, st); break;
+    case GMOE_F32:
+      rc = launch_seq_stats<GMOE_F32>(G, logits, routing_map, seq_length, batch_size, E, k, sig, counts, scores, parts,
+                                       st);
+      break;
+    case GMOE_BF16:
+      rc = launch_seq_stats<GMOE_BF16>(G, logits, routing_map, seq_length, batch_size, E, k, sig, counts, scores, parts,
+                                       st);
+      break;
+    case GMOE_F16:
+      rc = launch_seq_stats<GMOE_F16>(G, logits, routing_map, seq_length, batch_size, E, k, sig, counts, scores, parts,
+                                       st);
+      break;
     default: return GMOE_ERR_UNSUPPORTED;
   }
   if (rc != GMOE_OK) return rc;

@@ -153,8 +153,9 @@ __device__ __forceinline__ uint64_t slice_bits(const uint8_t* map, int64_t t, in
 // For the workgroup's slice of experts: s_before = tokens of all experts before the slice, s_total[j] = tokens of
 // its expert j, s_chunk[j] = those of them before this chunk.  Ends with a barrier.
 template <int BASE>
-__device__ __forceinline__ void slice_base(const uint8_t* map, const int* counts, int64_t T, int E, int NC, int vec8, int vec4,
-                                           int e_begin, int e_cnt, int& s_before, int* s_total, int* s_chunk) {
+__device__ __forceinline__ void slice_base(const uint8_t* map, const int* counts, int64_t T, int E, int NC, int vec8,
+                                           int vec4, int e_begin, int e_cnt, int& s_before, int* s_total,
+                                           int* s_chunk) {
   const int tid = threadIdx.x, lane = tid & 63;
   if (tid < kFillExperts) s_total[tid] = s_chunk[tid] = 0;
   if (tid == kFillExperts) s_before = 0;
