@@ -1174,14 +1174,19 @@ static inline bool gmm_tn_short_pays(const GmmParams& p) {
 }
 
 // Whether reading the operands beforehand (warm_operands) pays: they take bytes / 5 TB/s, and the launch has to be
-// one of many more result bytes.  us without / with, operands from HBM, result bytes over operand bytes in
-// parentheses: 4096 x 28672 over 8 experts n 192 544 / 483 (19), n 384 788 / 740 (9); 7168 x 4096 over 32 n 192 500
-// / 466 (14), n 384 757 / 799 (7); 14336 x 4096 over 8 n 448 420 / 407 (7), n 512 462 / 475 (6); 2048 x 2816 over
-// 64 n 128 175 / 158 (9), n 256 246 / 263 (5).  Smaller results gain nothing: 1024 x 5632 over 16 n 96 47 / 50,
-// 1024 x 1024 over 64 36 / 40.
+// one of several times more result bytes.  In a whole step the operands partly lie in the memory-side cache and the
+// stores of one launch meet the loads of the next, so the line is drawn there (us of a step without / with, result
+// bytes over operand bytes of fc1 in parentheses): 320 tokens of 1536, 16 experts of 3072, top 4 451 / 439 (15);
+// 640 of 1024, 64 of 1024, top 8 450 / 433 (9); 132 of 384, 32 of 10240, top 2 620 / 610 (46); 900 of 2048, 64 of
+// 1408, top 4 884 / 841 (21); 1024 of 7168, 32 of 2048, top 8 3199 / 3163 (10); 512 of 4096, 16 of 4096, top 8 1880 /
+// 1834 (11); 2048 of 2048, 64 of 1408, top 8 1445 / 1429 (5).  A smaller result gains nothing: 640 of 2048, 16 of
+// 1024, top 2 (128 and 64 MB) 247 / 249, 512 of 512, 32 of 2048, top 4 (the same) 258 / 261.  One of 240 MB, which is
+// not streamed, still gains with few rows (the 132 tokens: 632 without it / 627).
+constexpr int64_t kTnWarmFewRowsBytes = 192ll << 20;
 static inline bool gmm_tn_warm_pays(const GmmParams& p) {
   const int64_t operands = p.N * (p.K + p.M) * 2, result = p.E * p.K * p.M * 2;
-  return operands <= (192ll << 20) && operands * 7 <= result && gmm_tn_streams(p);
+  if (operands > (192ll << 20) || operands * 4 > result) return false;
+  return gmm_tn_streams(p) || (p.N < kTnFewRows * p.E && result >= kTnWarmFewRowsBytes);
 }
 
 // The separate launch for short last row tiles pays off once an expert has many full row tiles:
