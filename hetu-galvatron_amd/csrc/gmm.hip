@@ -1156,15 +1156,16 @@ static inline bool gmm_rows_pays(const GmmParams& p, int mode, int epi) {
 // 256x256 LDS-DMA kernel, or 128x128 tiles where that one does not apply; n = rows per expert, us of that kernel /
 // of this one.  From one round of 256x256 tiles on that kernel, whose tiles run into each other, is the faster one
 // (n 128 402 / 484, n 383 784 / 879, n 1024 1671 / 1875, 8 experts of 4096 x 28672) except for few rows: n 24, 8
-// experts of 6144 x 16384 291 / 266, n 48 291 / 297, n 96 299 / 368; 14336 x 4096, 8 n 24 161 / 159, n 48 161 /
-// 177, n 96 174 / 205. A result under 256 MB has the ordinary stores there and nontemporal ones here, which moves
-// the line: 1024 x 5632, 16 n 24 44 / 41, n 64 45 / 44, n 96 49 / 47; 1024 x 1024, 64 n 64 33 / 34, n 96 37 / 36;
-// 2048 x 1184, 32 n 64 40 / 40, n 96 42 / 43.  With less than a round of 256x256 tiles, and where its rows would be
-// padding (K under 512), the smaller tiles spread better: 128 tiles of 256x256 14.0 / 11.1 (n 256, 1024 x 1024, 8),
-// 240 17.8 / 15.4 (n 300, 640 x 1280, 16), n 384 of 384 x 4096 over 64 159 / 117.  That holds beyond the 768 rows
-// up to which it is used (n 1024 of 1024 x 1024 29.4 / 22.5).  Fewer than three quarters of a tile per CU stay with
-// 128x128 ones (128 tiles of 1024 x 512, 8: 10.1 / 9.9).
-constexpr int64_t kTnFewRows = 112, kTnFewRowsStreamed = 32;
+// experts of 6144 x 16384 291 / 266, n 48 291 / 297, n 96 299 / 368; in whole steps n 8 717 / 707, n 32 1662 / 1649,
+// n 45 1693 / 1692, n 56 834 / 846, n 75 1752 / 1824, n 100 1128 / 1182 us. A result under 256 MB has the ordinary
+// stores there and nontemporal ones here, which moves the line: 1024 x 5632, 16 n 24 44 / 41, n 64 45 / 44, n 96 49
+// / 47; 1024 x 1024, 64 n 64 33 / 34, n 96 37 / 36; 2048 x 1184, 32 n 64 40 / 40, n 96 42 / 43.  With less than a
+// round of 256x256 tiles, and where its rows would be padding (K under 512), the smaller tiles spread better: 128
+// tiles of 256x256 14.0 / 11.1 (n 256, 1024 x 1024, 8), 240 17.8 / 15.4 (n 300, 640 x 1280, 16), n 384 of 384 x
+// 4096 over 64 159 / 117.  That holds beyond the 768 rows up to which it is used (n 1024 of 1024 x 1024 29.4 /
+// 22.5).  Fewer than three quarters of a tile per CU stay with 128x128 ones (128 tiles of 1024 x 512, 8: 10.1 /
+// 9.9).
+constexpr int64_t kTnFewRows = 112, kTnFewRowsStreamed = 48;
 static inline bool gmm_tn_short_pays(const GmmParams& p) {
   const int64_t n = p.N / (p.E > 0 ? p.E : 1), col_tiles = (p.M + 255) / 256;
   if (p.K < 128 || p.M < 256 || p.E * ((p.K + 127) / 128) * col_tiles * 4 < gmm_grid(1) * 3) return false;
