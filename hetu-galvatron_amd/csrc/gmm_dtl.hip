@@ -454,6 +454,8 @@ static int launch_kernel(const GmmParams& p, hipStream_t st) {
 //     where those lie 14 KB and more apart, the copies wait behind the spread ones until a tile is long: n 1024
 //     1596 / 1656, n 1408 2100 / 2112, n 1600 2352 / 2339 (4096 x 28672, 8); n 1024 1347 / 1380, n 1408 1773 / 1770
 //     (6144 x 16384, 8); n 1024 820 / 827, n 1408 1072 / 1067 (2048 x 7168, 32).
+//     In whole steps with fc1's result stored after the tile / spread, fc2's spread: 8 experts of 8192, hidden
+//     4096, n 1100 5184 / 5274; of 14336, n 1024 8264 / 8295, n 1300 9843 / 9841.
 //   * ordinary / nontemporal stores after the tile: n 256 742 / 634, n 448 897 / 851 (4096 x 28672, 8), n 256 264 /
 //     246, n 512 387 / 394 (2048 x 2816, 64), n 256 99 / 84 (4096 x 4096, 8, 256 MB); smaller results either way: n
 //     256 74 / 71 (1024 x 5632, 16), 53 / 57 (1024 x 1024, 64), n 1152 100 / 112 (2816 x 1024, 16).
