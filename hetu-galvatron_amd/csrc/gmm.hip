@@ -6,8 +6,8 @@
 //   TN  c[e]       = a[rows_e]^T @ b[rows_e] a [N,K]  b [N,M]    c [E,K,M]  (dW)
 //
 // Structure
-//   * 256 threads = 4 wavefronts in a 2x2 grid; the block owns a BM x BN tile of C (256x256, or
-//     128x128 for small groups), each wavefront a (BM/2) x (BN/2) sub-tile made of 32x32 MFMA
+//   * 256 threads = 4 wavefronts in a 2x2 grid; the block owns a BM x BN tile of C (128x128, or
+//     256x256), each wavefront a (BM/2) x (BN/2) sub-tile made of 32x32 MFMA
 //     accumulators (fp32, in AGPRs).
 //   * Operand tiles go global -> registers -> LDS in 16-byte pieces, two LDS stages of 64 (16-bit)
 //     or 32 (fp32) reduction elements.  Global memory is read with buffer loads whose resource
@@ -17,7 +17,7 @@
 //         16-byte fragment reads of consecutive rows hit disjoint banks (DirectLoader);
 //       - reduction index in the slow dimension, 16-bit: kept as in memory, [k][outer], with an XOR
 //         segment swizzle, fragments read with the transposing LDS load ds_read_b64_tr_b16
-//         (RowMajorLoader for 256-wide, RowMajorSmallLoader for 128-wide tiles);
+//         (RowMajorSmallLoader);
 //       - reduction index in the slow dimension, fp32: 4x4 blocks transposed in registers on the way
 //         to LDS (TransposeLoader);
 //       - fp8 weights with block scales: widened to bf16 on the way to LDS, the block scale applied
@@ -32,7 +32,7 @@
 //     the waitcnts.
 //   * The MFMA is issued with the operands swapped (B fragment as SrcA) so that a lane ends up with
 //     4 consecutive columns of one row of C; 16-bit results are staged through LDS and written as
-//     16-byte row-contiguous pieces, optionally through a fused gated-activation epilogue.
+//     16-byte row-contiguous pieces, optionally through the fused backward of a gated activation.
 //   * Tiles are numbered expert-major, inside an expert in strips of 8 column tiles, and handed to
 //     workgroups so that the 32 workgroups that share an XCD (workgroup id mod 8) work on one
 //     4x8 patch of tiles at a time: the A and B panels they stream are shared in that XCD's L2.
@@ -294,85 +294,12 @@ struct Fp8TransposeLoader {
   }
 };
 
-// Reduction index is the slow dimension (16-bit types, 256 outer indices): element (o, k) at
-// src + k*ld + o.  The tile is kept in LDS as it is in memory, [k][outer] with 512-byte rows, in
-// two blocks of 32 k rows; MFMA fragments are read with the transposing LDS load
-// (ds_read_b64_tr_b16: a group of 16 lanes reads a 4(k) x 16(outer) block and every lane receives
-// the 4 k-values of its own outer index), two reads per fragment and K step.  No register
-// transposition.  Bank conflicts: the 64-byte segment sg of row k sits at segment position
-// sg ^ f(k), f(k) = (k & 3) | ((k >> 1) & 4), so the 8 rows one transposing read touches
-// (k0..k0+3 and k0+8..k0+11) land in 8 different segments.
-// Thread t copies the 16-byte piece t%32 of rows t/32 + 8*i: a wavefront reads two whole 512-byte
-// rows per instruction.
-template <int R>
-struct RowMajorLoader {
-  static_assert(R == 256, "512-byte LDS rows");
-  static constexpr int BK = 64;
-  static constexpr int NPIECE = 8;
-  static constexpr int STAGE_BYTES = BK * R * 2;
-  static constexpr int READS = 2;
-  static constexpr bool STORE_NEEDS_ALL_PIECES = false;
-  typedef short s16x4 __attribute__((ext_vector_type(4)));
-  typedef __attribute__((address_space(3))) unsigned char lds_byte;
-  u32x4 r[NPIECE];
-  uint32_t voff;
-  uint32_t row_bytes;
-  __amdgpu_buffer_rsrc_t rsrc;
-  int lds_off[2];        // store offset of the pieces with even / odd index
-  uint32_t frag_k;       // byte offset of the lane's first k row
-  uint32_t frag_seg[4];  // byte offset of the lane's 8 bytes inside a k row, per fragment
-
-  // glu_gap > 0: tile columns 0..127 are outer indices o0..o0+127 (gate), columns 128..255 are
-  // o0+glu_gap.. (the matching up-projection columns)
-  __device__ __forceinline__ void init(const unsigned char* src, int64_t ld, int64_t o0,
-                                       int64_t o_lim, int64_t k_limit, int tid, int64_t glu_gap = 0) {
-    (void)o_lim;  // outer indices past the operand only feed rows / columns of C that are not stored
-    const int c = tid & 31, t5 = tid >> 5;
-    rsrc = make_rsrc(src + o0 * 2, k_limit * ld * 2 - o0 * 2);
-    row_bytes = (uint32_t)(ld * 2);
-    const int64_t col = (glu_gap > 0 && c >= 16) ? glu_gap + (c - 16) * 8 : c * 8;
-    voff = (uint32_t)(((int64_t)t5 * ld + col) * 2);
-    // piece i holds k row (i%4)*8 + t5 of block i/4; f of that row = (t5 & 3) | ((i & 1) << 2)
-    const int P0 = ((((c >> 2) ^ (t5 & 3)) << 2) | (c & 3));
-    lds_off[0] = t5 * 512 + P0 * 16;
-    lds_off[1] = t5 * 512 + (P0 ^ 16) * 16;
-  }
-  // sub0: first outer index of the wavefront's 128 inside the tile; glu: fragments 0,1 are the
-  // wavefront's 64 gate columns, 2,3 the up columns under them
-  __device__ __forceinline__ void init_frag(int sub0, int lane, bool glu = false) {
-    const int s = lane & 15, g = lane >> 5, half = (lane >> 4) & 1;
-    frag_k = (uint32_t)((8 * g + (s >> 2)) * 512);
-    const int f = (s >> 2) | (g << 2);
-    const int seg0 = sub0 / 32;  // 0 or 4
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int seg = glu ? (j < 2 ? seg0 / 2 + j : 4 + seg0 / 2 + (j - 2)) : seg0 + j;
-      frag_seg[j] = (uint32_t)(((seg ^ f) * 64) + half * 32 + (s & 3) * 8);
-    }
-  }
-  template <int i, int SET = 0>
-  __device__ __forceinline__ void load_piece(int kt) {
-    r[i] = buf_ld16(rsrc, voff, (uint32_t)(kt * BK + i * 8) * row_bytes);
-  }
-  template <int i, int SET = 0>
-  __device__ __forceinline__ void store_piece(unsigned char* stage) const {
-    *reinterpret_cast<u32x4*>(stage + (i / 4) * 16384 + (i % 4) * 4096 + lds_off[i & 1]) = r[i];
-  }
-  // half h (4 of the 8 k values) of fragment j of K step KS (0..3)
-  template <int j, int KS, int h>
-  __device__ __forceinline__ void read(const unsigned char* tile, u32x4& f) const {
-    const s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-        (__attribute__((address_space(3))) s16x4*)(lds_byte*)(tile + (KS / 2) * 16384 + frag_k +
-                                                               frag_seg[j] +
-                                                               ((KS % 2) * 16 + h * 4) * 512));
-    const u32x2 w = __builtin_bit_cast(u32x2, v);
-    f[2 * h] = w[0];
-    f[2 * h + 1] = w[1];
-  }
-};
-
-// The same idea for the 128-wide tiles of the small configuration: [k][outer] rows of 256 bytes,
-// the 64-byte segment sg of row k at segment position sg ^ (k & 3).  Half of a transposing read
+// Reduction index is the slow dimension (16-bit types, 128 outer indices): element (o, k) at
+// src + k*ld + o.  The tile is kept in LDS as it is in memory, [k][outer] with 256-byte rows; MFMA
+// fragments are read with the transposing LDS load (ds_read_b64_tr_b16: a group of 16 lanes reads a
+// 4(k) x 16(outer) block and every lane receives the 4 k-values of its own outer index), two reads per
+// fragment and K step.  No register transposition.  Bank conflicts: the 64-byte segment sg of row k sits
+// at segment position sg ^ (k & 3).  Half of a transposing read
 // (32 lanes) touches 4 consecutive k rows x 2 column halves of one logical segment: after the
 // swizzle 8 different 32-byte pieces, all 64 banks once.  Thread t copies the 16-byte piece t%16 of
 // rows t/16 + 16*i.
@@ -440,53 +367,11 @@ struct Fp8Loader : Fp8DirectLoader<R, DEPTH> {};
 template <int R, int DEPTH>
 struct Fp8Loader<R, true, DEPTH> : Fp8TransposeLoader<R, DEPTH> {};
 
-// ROWS_AUTO_MAIN / ROWS_AUTO_REMAINDER -> ROWS_MAIN / ROWS_REMAINDER when leaving the experts' short
-// last row tiles to their own launch saves more time in the launch with 256-row tiles (whole rounds
-// of its persistent grid) than the second launch takes, else ROWS_ALL / ROWS_NONE.  Both launches
-// evaluate the same counts and the same model in whole numbers, so they agree.  Times in nanoseconds per
-// 128-byte K tile, measured on the Mixtral shape: 1300 in a 256x256 tile; in a 128x128 tile 2500 with two
-// workgroups per CU walking whole reductions, 1900 when the reduction is split (16-bit operands only).  Over
-// 108 launches of 9 shapes with 2000 to 8000 rows per expert the choice costs 0.24 % against the better of both.
-__device__ inline int resolve_row_part(const GmmParams& p, int k_tiles, int* counts) {
-  if (p.row_part != ROWS_AUTO_MAIN && p.row_part != ROWS_AUTO_REMAINDER) return p.row_part;
-  const int tid = threadIdx.x;
-  if (tid < 3) counts[tid] = 0;
-  __syncthreads();
-  int all = 0, main = 0, rem = 0;
-  for (int e = tid; e < p.E; e += kGemmThreads) {
-    const long long n = group_begin(p, e + 1) - group_begin(p, e);
-    long long b, c;
-    all += (int)((n + 255) / 256);
-    expert_row_part(n, ROWS_MAIN, b, c);
-    main += (int)((c + 255) / 256);
-    expert_row_part(n, ROWS_REMAINDER, b, c);
-    rem += (int)((c + 127) / 128);
-  }
-  if (all) atomicAdd(&counts[0], all);
-  if (main) atomicAdd(&counts[1], main);
-  if (rem) atomicAdd(&counts[2], rem);
-  __syncthreads();
-  const long long nt256 = (p.M + 255) / 256, nt128 = (p.M + 127) / 128;
-  const long long tiles_all = counts[0] * nt256, tiles_main = counts[1] * nt256, tiles_rem = counts[2] * nt128;
-  const long long g = p.main_grid > 0 ? p.main_grid : 256;
-  const long long rounds_saved = (tiles_all + g - 1) / g - (tiles_main + g - 1) / g;
-  // the pieces launch_gmm_remainder's launch comes to
-  const long long slots = p.ws == nullptr ? 0 : p.ws_floats / (128 * 128);
-  const int s = split_pieces(k_tiles, tiles_rem, slots < kSplitSlots ? slots : kSplitSlots, 0);
-  const long long saved = 1300 * rounds_saved * k_tiles;
-  const long long cost = s > 1 ? 1900ll * (k_tiles / s) + kSplitReduceNs + kSplitNsPerPiece * tiles_rem * s
-                               : 2500 * ((tiles_rem + kSplitSlots - 1) / kSplitSlots) * k_tiles + 8000;
-  const bool use = tiles_rem > 0 && saved > cost;
-  __syncthreads();  // the caller reuses counts
-  if (p.row_part == ROWS_AUTO_MAIN) return use ? ROWS_MAIN : ROWS_ALL;
-  return use ? ROWS_REMAINDER : ROWS_NONE;
-}
-
 // tile_cum[e] = tiles of the experts before e, tile_cum[E] all of them: one pass over the offset table, a
 // thread owns kPer consecutive experts, the per-thread sums are scanned with wavefront shuffles and four
 // wavefront totals in LDS.  Ends with a barrier.
 template <int MODE, int BM>
-__device__ __forceinline__ void build_tile_cum(const GmmParams& p, int part, int nt_cnt, int mt_fixed,
+__device__ __forceinline__ void build_tile_cum(const GmmParams& p, int nt_cnt, int mt_fixed,
                                                int* tile_cum) {
   constexpr int kPer = kMaxGroupsLds / kGemmThreads;
   __shared__ int wave_tot[kGemmThreads / 64];
@@ -497,8 +382,7 @@ __device__ __forceinline__ void build_tile_cum(const GmmParams& p, int part, int
     const int e = tid * kPer + j;
     int c = 0;
     if (e < E) {
-      long long n = group_begin(p, e + 1) - group_begin(p, e), skip;
-      if (MODE != MODE_TN) expert_row_part(n, part, skip, n);
+      const long long n = group_begin(p, e + 1) - group_begin(p, e);
       const long long mt = MODE == MODE_TN ? mt_fixed : (n + BM - 1) / BM;
       c = (int)(mt * nt_cnt);
     }
@@ -596,13 +480,8 @@ __attribute__((noinline)) __device__ void glu_bwd_tile_rows(const unsigned char*
 
 // ---- the kernel -----------------------------------------------------------------------------------
 // BQ: the B operand is fp8 with block scales (p.b_scale), DT is then the type of A and of the MFMA.
-// TR: operands whose reduction index is the slow dimension keep their memory layout in LDS and are
-// read with transposing LDS loads (RowMajorLoader) instead of being transposed in registers.
-template <int DT, int ODT, int MODE, int BM, int BN, int EPI, bool BQ = false, bool TR = false>
+template <int DT, int ODT, int MODE, int BM, int BN, int EPI, bool BQ = false>
 __global__ __launch_bounds__(kGemmThreads, (BM == 128 && BN == 128) ? 2 : 1) void gmm_kernel(GmmParams p) {
-  constexpr bool GLU = (EPI == EPI_GLU_FWD_SILU || EPI == EPI_GLU_FWD_GELU);
-  static_assert(!GLU || (MODE == MODE_NN && TR && DT == ODT), "fused activation: forward GEMM");
-  static_assert(!TR || (Elem<DT>::bytes == 2 && BM == 256 && BN == 256 && !BQ), "TR: 16-bit, 256x256");
   constexpr int ES = Elem<DT>::bytes;
   constexpr int BK = 128 / ES;      // reduction elements per LDS row
   constexpr int WTM = BM / 2 / 32;  // 32x32 accumulators per wavefront, rows
@@ -615,17 +494,13 @@ __global__ __launch_bounds__(kGemmThreads, (BM == 128 && BN == 128) ? 2 : 1) voi
   // weights the second accumulator takes that room and only the weight stream gets the second set.
   constexpr bool SMALL = BM == 128 && BN == 128;
   constexpr int DA = (SMALL && !BQ) ? 2 : 1, DB = SMALL ? 2 : 1;
-  // 16-bit operands whose reduction index is the slow dimension: transposing LDS reads (TR for the
-  // large tiles, always for the small ones); fp32 transposes 4x4 blocks in registers
+  // 16-bit operands whose reduction index is the slow dimension: transposing LDS reads; fp32 transposes
+  // 4x4 blocks in registers
   constexpr bool TRS = SMALL && ES == 2 && !BQ;
-  typedef std::conditional_t<
-      TR && A_T, RowMajorLoader<BM>,
-      std::conditional_t<TRS && A_T, RowMajorSmallLoader<BM, DA>, Loader<BM, ES, A_T, DA>>> LoaderA;
+  typedef std::conditional_t<TRS && A_T, RowMajorSmallLoader<BM, DA>, Loader<BM, ES, A_T, DA>> LoaderA;
   typedef std::conditional_t<
       BQ, Fp8Loader<BN, B_T, DB>,
-      std::conditional_t<TR && B_T, RowMajorLoader<BN>,
-                         std::conditional_t<TRS && B_T, RowMajorSmallLoader<BN, DB>,
-                                            Loader<BN, ES, B_T, DB>>>> LoaderB;
+      std::conditional_t<TRS && B_T, RowMajorSmallLoader<BN, DB>, Loader<BN, ES, B_T, DB>>> LoaderB;
   constexpr int RA = LoaderA::READS, RB = LoaderB::READS;
   constexpr int NF = WTM * RA + WTN * RB;  // LDS fragment reads per K step
   constexpr int A_BYTES = LoaderA::STAGE_BYTES;
@@ -646,22 +521,14 @@ __global__ __launch_bounds__(kGemmThreads, (BM == 128 && BN == 128) ? 2 : 1) voi
   const int E = p.E;
   const int64_t K = p.K, M = p.M;
   // C is rows x M per expert: NN/NT rows = tokens of the expert;  TN rows = K
-  // with the fused activation a column tile is 128 gate + 128 up columns of the [K, 2F] weight
-  const int nt_cnt = GLU ? (int)((p.F + 127) / 128) : (int)((M + BN - 1) / BN);
+  const int nt_cnt = (int)((M + BN - 1) / BN);
   const int mt_fixed = (int)((K + BM - 1) / BM);  // TN only
 
-  int part = ROWS_ALL;
-  if constexpr (MODE != MODE_TN) {
-    part = resolve_row_part(p, (int)((K + BK - 1) / BK), tile_cum);
-    if (part == ROWS_NONE) return;  // the launch with 256-row tiles takes every row
-  }
-
-  build_tile_cum<MODE, BM>(p, part, nt_cnt, mt_fixed, tile_cum);
+  build_tile_cum<MODE, BM>(p, nt_cnt, mt_fixed, tile_cum);
   const long long total_tiles = tile_cum[E];
 
-  // A launch with few tiles and a long reduction (the short last row tiles of the experts) leaves
-  // most CUs idle while each workgroup walks the whole K range.  With a workspace the reduction of
-  // every tile is cut into S pieces, one workgroup each, which store their fp32 accumulators;
+  // A launch with few tiles and a long reduction leaves most CUs idle while each workgroup walks the
+  // whole K range.  With a workspace the reduction of every tile is cut into S pieces, one workgroup each, which store their fp32 accumulators;
   // gmm_split_reduce_kernel adds the S partial tiles in order.
   constexpr bool CAN_SPLIT = MODE != MODE_TN && EPI == EPI_NONE && !BQ && SMALL;
   constexpr long long TILE_ELEMS = (long long)BM * BN;
@@ -688,13 +555,7 @@ __global__ __launch_bounds__(kGemmThreads, (BM == 128 && BN == 128) ? 2 : 1) voi
     const long long s = S > 1 ? v / S : v;
     const int chunk = S > 1 ? (int)(v % S) : 0;
     while (tile_cum[e + 1] <= s) ++e;
-    long long row0 = group_begin(p, e);
-    long long n_e = group_begin(p, e + 1) - row0;
-    if (MODE != MODE_TN) {
-      long long begin;
-      expert_row_part(n_e, part, begin, n_e);
-      row0 += begin;
-    }
+    const long long row0 = group_begin(p, e), n_e = group_begin(p, e + 1) - row0;
     const int mt_cnt = MODE == MODE_TN ? mt_fixed : (int)((n_e + BM - 1) / BM);
     int mt, nt;
     strip_order(s - tile_cum[e], mt_cnt, nt_cnt, mt, nt);
@@ -716,14 +577,9 @@ __global__ __launch_bounds__(kGemmThreads, (BM == 128 && BN == 128) ? 2 : 1) voi
     LoaderA la;
     LoaderB lb;
     la.init_frag(wm * (BM / 2), lane);
-    if constexpr (GLU) lb.init_frag(wn * (BN / 2), lane, true);
-    else lb.init_frag(wn * (BN / 2), lane);
+    lb.init_frag(wn * (BN / 2), lane);
     int64_t k_lim;
-    if constexpr (GLU) {
-      k_lim = K;
-      la.init(p.a + row0 * K * ES, K, (int64_t)mt * BM, n_e, k_lim, tid);
-      lb.init(p.b + (int64_t)e * K * M * ES, M, (int64_t)nt * 128, M, k_lim, tid, p.F);
-    } else if constexpr (BQ) {
+    if constexpr (BQ) {
       // b is [E,K,M] (NN) or [E,M,K] (NT) bytes; its scales [E, ceil(K/128), ceil(M/128)] or
       // [E, ceil(M/128), ceil(K/128)]
       k_lim = K;
@@ -928,40 +784,6 @@ __global__ __launch_bounds__(kGemmThreads, (BM == 128 && BN == 128) ? 2 : 1) voi
 
     // ---- epilogue: lane holds row (lane%32), columns 8*(v/4) + 4*(lane/32) + v%4 of each 32x32 ----
     constexpr int OES = Elem<ODT>::bytes;
-    if constexpr (GLU) {
-      // fragments 0,1 hold gate columns, 2,3 the up columns under them: fc1 = [gate | up] and
-      // act = act_fn(gate) * up, both computed from the values as rounded for fc1.  Staged through
-      // LDS (columns [gate 64 | up 64] per wavefront column half), then written in 16-byte
-      // row-contiguous pieces.
-      constexpr bool gelu = EPI == EPI_GLU_FWD_GELU;
-      const int64_t F = p.F;
-      unsigned char* fc1 = p.c + row0 * M * 2;
-      unsigned char* act = p.c2 + row0 * F * 2;
-      using CT = CTile<BN>;
-      stage_acc_lds<DT, WTM, WTN, BN>(lds, acc, wm * (BM / 2), wn * (BN / 2), lane);
-      __syncthreads();
-      const int cc = tid & 15, r0 = tid >> 4;  // 16 chunks of 8 gate columns per row
-      const int64_t n = (int64_t)nt * 128 + cc * 8;
-      const int lcol = (cc >> 3) * 128 + (cc & 7) * 8;
-#pragma unroll 4
-      for (int it = 0; it < BM / 16; ++it) {
-        const int row = it * 16 + r0;
-        const int64_t m = (int64_t)mt * BM + row;
-        if (m >= n_e || n >= F) continue;
-        const u32x4 gw = ctile_read16(lds + row * CT::pitch + lcol * 2);
-        const u32x4 uw = ctile_read16(lds + row * CT::pitch + (lcol + 64) * 2);
-        float g[8], u[8], o[8];
-        Vec16<DT>::unpack(gw, g);
-        Vec16<DT>::unpack(uw, u);
-#pragma unroll
-        for (int q = 0; q < 8; ++q) o[q] = glu_act(g[q], gelu) * u[q];
-        st16(fc1 + (m * M + n) * 2, gw);
-        st16(fc1 + (m * M + F + n) * 2, uw);
-        st16(act + (m * F + n) * 2, Vec16<DT>::pack(o));
-      }
-      __syncthreads();  // the next tile's prologue writes stage 0
-      continue;
-    }
     if constexpr (EPI == EPI_GLU_BWD_SILU || EPI == EPI_GLU_BWD_GELU) {
       // C = d(act) is not stored: with fc1 = [gate | up] read back, the tile of
       // d(fc1) = [d * act'(gate) * up | d * act(gate)] is written instead (d rounded to the
@@ -1069,9 +891,7 @@ __global__ __launch_bounds__(kGemmThreads) void gmm_split_reduce_kernel(GmmParam
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave >> 1, wn = wave & 1;
   const int64_t M = p.M;
   const int nt_cnt = (int)((M + BN - 1) / BN), k_tiles = (int)((p.K + BK - 1) / BK);
-  const int part = resolve_row_part(p, k_tiles, tile_cum);
-  if (part == ROWS_NONE) return;
-  build_tile_cum<MODE, BM>(p, part, nt_cnt, 0, tile_cum);
+  build_tile_cum<MODE, BM>(p, nt_cnt, 0, tile_cum);
   const long long total_tiles = tile_cum[p.E];
   const int S = split_count(p, total_tiles, k_tiles, TILE_ELEMS);
   if (S == 1) return;  // the first launch did everything
@@ -1080,9 +900,7 @@ __global__ __launch_bounds__(kGemmThreads) void gmm_split_reduce_kernel(GmmParam
     const long long s = item / 4;
     const int i = (int)(item & 3) / WTN, j = (int)(item & 3) % WTN;
     while (tile_cum[e + 1] <= s) ++e;
-    long long row0 = group_begin(p, e), n_e = group_begin(p, e + 1) - row0, begin;
-    expert_row_part(n_e, part, begin, n_e);
-    row0 += begin;
+    const long long row0 = group_begin(p, e), n_e = group_begin(p, e + 1) - row0;
     int mt, nt;
     strip_order(s - tile_cum[e], (int)((n_e + BM - 1) / BM), nt_cnt, mt, nt);
     const float* slot = p.ws + s * S * TILE_ELEMS + (int64_t)(((i * WTN + j) * 4 * kGemmThreads) + tid) * 4;
@@ -1111,15 +929,15 @@ static int gmm_grid(int blocks_per_cu) {
   return grid < 8 ? 8 : grid;
 }
 
-template <int DT, int ODT, int MODE, int BM, int BN, int EPI, bool BQ = false, bool TR = false>
+template <int DT, int ODT, int MODE, int BM, int BN, int EPI, bool BQ = false>
 static int launch_gmm_cfg(const GmmParams& p, hipStream_t st, int blocks_per_cu = 1) {
   // two stages of both operand tiles; the epilogue reuses them as one tile of 16-bit results
   constexpr bool small_tr = BM == 128 && BN == 128 && Elem<DT>::bytes == 2 && !BQ;
-  constexpr size_t a_bytes = MODE != MODE_TN ? BM * kRowPad : ((TR || small_tr) ? 64 * BM * 2 : BM * kRowPad);
-  constexpr size_t b_bytes = MODE == MODE_NT ? BN * kRowPad : ((TR || small_tr) ? 64 * BN * 2 : BN * kRowPad);
+  constexpr size_t a_bytes = MODE != MODE_TN ? BM * kRowPad : (small_tr ? 64 * BM * 2 : BM * kRowPad);
+  constexpr size_t b_bytes = MODE == MODE_NT ? BN * kRowPad : (small_tr ? 64 * BN * 2 : BN * kRowPad);
   constexpr size_t ctile = Elem<ODT>::bytes == 2 ? (size_t)BM * CTile<BN>::pitch : 0;
   constexpr size_t smem = 2 * (a_bytes + b_bytes) > ctile ? 2 * (a_bytes + b_bytes) : ctile;
-  auto kern = gmm_kernel<DT, ODT, MODE, BM, BN, EPI, BQ, TR>;
+  auto kern = gmm_kernel<DT, ODT, MODE, BM, BN, EPI, BQ>;
   if (smem > 48 * 1024) {
     // once per kernel and device (the attribute belongs to the device's copy of the code object)
     static std::atomic<uint64_t> done_mask{0};
@@ -1144,12 +962,23 @@ static inline bool gmm_large_tiles(const GmmParams& p, int mode) {
   return p.K >= 512 && p.M >= 256 && experts * ((p.K + 255) / 256) * ((p.M + 255) / 256) >= 129;
 }
 
-// Row-adaptive tiles (gmm_rows.hip) for 16-bit NN / NT: tiles of 64 to 256 rows x 256 columns that share an
-// expert's rows evenly, one workgroup per CU.  The rule, with both sides' times, is in rows_rule.h.
+// Row-adaptive tiles (gmm_rows.hip) for 16-bit NN / NT: tiles of 64 to 384 rows x 256 columns that share an expert's
+// rows evenly, one workgroup per CU; the rules with both sides' times are in rows_rule.h.  Launches that could fill
+// 256x256 tiles are 12 to 17 % faster here (us there / here, rows per expert, K x M, experts: with activation 4096, 4096
+// x 28672, 8 6211 / 5836; 1024, 7168 x 4096, 32 1661 / 1525; NN 4096, 14336 x 4096, 8 3023 / 2790; activation backward
+// 1024, 7168 x 2048, 32 915 / 838; NT 4096, 28672 x 4096, 8 6010 / 5659; of 3340 such launches 3 % are slower by
+// more than 2 %, where the loads decide whether a round more is needed), so of those only plain NT ones of
+// fewer than 768 rows per expert are left there, where the rules see no gain (600, 2056 x 4104, 8 120 / 123).
+// The kernel's resource of a tile spans 384 rows.
+constexpr int64_t kNtTallRows = 768;
 static inline bool gmm_rows_pays(const GmmParams& p, int mode, int epi) {
   const RowsKind kind = mode == MODE_NN ? (epi == EPI_NONE ? ROWS_NN : ROWS_NN_GLU)
                                         : (epi == EPI_NONE ? ROWS_NT : ROWS_NT_GLU_BWD);
-  return rows_pays(kind, p.E, p.N, p.K, p.M, gmm_grid(1));
+  if (kTallMaxUnits * 64 * p.K * 2 >= (1ll << 31)) return false;
+  const int64_t experts = p.E > 0 ? p.E : 1;
+  if (nn_large_tiles(experts, p.N, p.M))
+    return kind != ROWS_NT || p.N / experts >= kNtTallRows || rows_pays(kind, p.E, p.N, p.K, p.M, gmm_grid(1));
+  return rows_pays(kind, p.E, p.N, p.K, p.M, gmm_grid(1)) || tall_pays(kind, p.E, p.N, p.K, p.M, gmm_grid(1));
 }
 
 // dW of 16-bit operands with a short reduction (gmm_tn.hip: 128x256 tiles, two workgroups per CU) against the
@@ -1190,13 +1019,6 @@ static inline bool gmm_tn_warm_pays(const GmmParams& p) {
   return gmm_tn_streams(p) || (p.N < kTnFewRows * p.E && result >= kTnWarmFewRowsBytes);
 }
 
-// The separate launch for short last row tiles pays off once an expert has many full row tiles:
-// at 4096 rows per expert (Mixtral shape) it saves 4-7 % of a GEMM, at 1024 rows per expert (64 or 32
-// experts) the main kernel with its partial tiles is 5-10 % faster than the two launches.
-static inline bool gmm_use_remainder(const GmmParams& p) {
-  return p.N / (p.E > 0 ? p.E : 1) >= kNnRemainderRows;
-}
-
 // Whether a 128x128-tile NN / NT launch is worth a split reduction; the kernels decide again from the tiles there
 // are.
 static inline bool gmm_split_pays(const GmmParams& p) { return nn_split_pieces(p.E, p.N, p.K, p.M) > 1; }
@@ -1207,7 +1029,7 @@ static inline int64_t gmm_workspace_floats(const GmmParams& p, int mode, int dty
     const int pieces = gmm_f32_pieces(p.E, p.N, p.K, p.M);
     return pieces > 1 ? pieces * p.N * p.M : 0;
   }
-  return (gmm_large_tiles(p, mode) && gmm_use_remainder(p)) || gmm_split_pays(p) ? (int64_t)kSplitSlots * 128 * 128 : 0;
+  return gmm_split_pays(p) ? (int64_t)kSplitSlots * 128 * 128 : 0;
 }
 
 // A split launch with 128x128 tiles: the pieces, then their sums.
@@ -1216,8 +1038,7 @@ static int launch_gmm_split(const GmmParams& p, hipStream_t st) {
   GmmParams r = p;
   const int64_t slots = p.ws_floats / (128 * 128);
   r.split_slots = (int)(slots < kSplitSlots ? slots : kSplitSlots);
-  // the rows left to a remainder launch belong to some of the experts only: no bound from their weights
-  r.stream_ns = p.row_part == ROWS_ALL ? weight_stream_ns(p.E, p.K, p.M, Elem<DT>::bytes) : 0;
+  r.stream_ns = weight_stream_ns(p.E, p.K, p.M, Elem<DT>::bytes);
   const int rc = launch_gmm_cfg<DT, ODT, MODE, 128, 128, EPI_NONE>(r, st, 2);
   if (rc != GMOE_OK) return rc;
   // at most split_slots / 2 tiles are split, four quarters each
@@ -1225,25 +1046,10 @@ static int launch_gmm_split(const GmmParams& p, hipStream_t st) {
   return gmoe_launch_status();
 }
 
-// The launch with 128-row tiles for the rows a ROWS_MAIN launch leaves out.
-template <int DT, int ODT, int MODE>
-static int launch_gmm_remainder(const GmmParams& p, hipStream_t st) {
-  GmmParams r = p;
-  r.row_part = ROWS_AUTO_REMAINDER;
-  if (p.ws == nullptr || p.ws_floats < 2 * 128 * 128)
-    return launch_gmm_cfg<DT, ODT, MODE, 128, 128, EPI_NONE>(r, st, 2);
-  return launch_gmm_split<DT, ODT, MODE>(r, st);  // few tiles, each with the whole reduction
-}
-
 // One kernel per (type, mode, size).  Groups large enough for 256x256 tiles (TFLOP/s measured on the
 // Mixtral shape):
-//   NT        both operands k-contiguous: register-staged, 128-byte row pieces, plain LDS reads;
-//             an expert's short last row tile goes to a second launch with 128-row tiles, which
-//             with a workspace splits its reduction over the idle CUs (-7 % on the dX GEMM of fc1
-//             with ragged groups); plain NN does the same when it has the workspace (-4 % on fc2);
-//   NN 16-bit the same for a, the weight tile kept [k][m] in LDS and read with transposing loads
-//             (6 % faster than LDS-DMA copies, whose 64-byte pieces of a load the address path
-//             twice); optionally with the gated activation in the epilogue;
+//   NN / NT 16-bit  row-adaptive tiles (gmm_rows.hip);
+//   NT 16-bit, short of their rule: both operands k-contiguous, register-staged, 128-byte row pieces, plain LDS reads;
 //   TN 16-bit both operands [k][outer]: LDS-DMA copies of 512-byte rows, 4 stages (1.5 % faster than
 //             the register-staged form);
 // Small groups: 128x128 tiles, two workgroups per CU.
@@ -1261,27 +1067,7 @@ static int launch_gmm_16bit(const GmmParams& p, int dtype, int out_dtype, hipStr
     if (gmm_rows_pays(p, MODE, EPI)) return launch_gmm_rows(p, MODE, dtype, out_dtype, EPI, st);
   }
   if (MODE != MODE_TN && gmm_large_tiles(p, MODE)) {
-    if constexpr (MODE == MODE_NN && EPI == EPI_NONE) {
-      // the short last row tiles pay off as a launch of their own only when it can be split
-      if (p.ws == nullptr || p.ws_floats < 2 * 128 * 128 || !gmm_use_remainder(p))
-        return launch_gmm_cfg<DT, ODT, MODE_NN, 256, 256, EPI_NONE, false, true>(p, st);
-      GmmParams m = p;
-      m.row_part = ROWS_AUTO_MAIN;
-      m.main_grid = gmm_grid(1);
-      const int rc = launch_gmm_cfg<DT, ODT, MODE_NN, 256, 256, EPI_NONE, false, true>(m, st);
-      return rc != GMOE_OK ? rc : launch_gmm_remainder<DT, ODT, MODE_NN>(m, st);
-    } else if constexpr (MODE == MODE_NN) {
-      return launch_gmm_cfg<DT, ODT, MODE_NN, 256, 256, EPI, false, true>(p, st);
-    } else if constexpr (MODE == MODE_NT && EPI == EPI_NONE) {
-      if (!gmm_use_remainder(p)) return launch_gmm_cfg<DT, ODT, MODE_NT, 256, 256, EPI_NONE>(p, st);
-      GmmParams m = p;
-      m.row_part = ROWS_AUTO_MAIN;
-      m.main_grid = gmm_grid(1);
-      const int rc = launch_gmm_cfg<DT, ODT, MODE_NT, 256, 256, EPI_NONE>(m, st);
-      return rc != GMOE_OK ? rc : launch_gmm_remainder<DT, ODT, MODE_NT>(m, st);
-    } else if constexpr (MODE != MODE_TN) {
-      return launch_gmm_cfg<DT, ODT, MODE, 256, 256, EPI>(p, st);
-    }
+    if constexpr (MODE == MODE_NT && EPI == EPI_NONE) return launch_gmm_cfg<DT, ODT, MODE_NT, 256, 256, EPI_NONE>(p, st);
   }
   if constexpr (glu_fwd) {
     return GMOE_ERR_UNSUPPORTED;  // the caller runs the GEMM and the activation kernel instead
@@ -1378,13 +1164,11 @@ static int gmm_check(GmmParams& p, const void* a, const void* b, void* c, const 
   p.aux = nullptr;
   p.b_scale = nullptr;
   p.a_scale = nullptr;
-  p.row_part = ROWS_ALL;
   p.F = 0;
   p.ws = nullptr;
   p.ws_floats = 0;
   p.split_slots = 0;
   p.stream_ns = 0;
-  p.main_grid = 0;
   p.pieces = 1;
   p.warm = false;
   return GMOE_OK;
@@ -1466,8 +1250,7 @@ extern "C" int gmoe_gmm_glu(const void* a, const void* w1, void* fc1, void* act_
   hipStream_t st = static_cast<hipStream_t>(stream);
   p.c2 = static_cast<unsigned char*>(act_out);
   p.F = F;
-  if (dtype != GMOE_F32 && F % 8 == 0 &&
-      (gmm_large_tiles(p, MODE_NN) || gmm_rows_pays(p, MODE_NN, EPI_GLU_FWD_SILU)))
+  if (dtype != GMOE_F32 && F % 8 == 0 && gmm_rows_pays(p, MODE_NN, EPI_GLU_FWD_SILU))
     return gmm_dispatch(p, MODE_NN, dtype, dtype, act == GMOE_ACT_SILU ? EPI_GLU_FWD_SILU : EPI_GLU_FWD_GELU, st);
   // small groups / fp32: the GEMM followed by the activation kernel
   const int rc2 = gmm_dispatch(p, MODE_NN, dtype, dtype, EPI_NONE, st);

@@ -73,14 +73,12 @@ struct GmmParams {
   const unsigned char* aux;  // backward: fc1 [N,2F]
   const unsigned char* b_scale;  // fp8 weights: bf16 block scales
   const unsigned char* a_scale;  // fp8 activations: power-of-two row scales, dwords [K/128][N]
-  int row_part;              // NN / NT: which rows of every expert this launch covers (ROWS_*)
   int64_t F;
   // split reduction of a launch with few tiles (split_rule.h, split_count in gmm.hip): fp32 partial tiles
   float* ws;
   int64_t ws_floats;
   int split_slots;           // tiles x splits this launch may spread over; 0 = never split
   int64_t stream_ns;         // time the weights take to stream: a split launch cannot be faster
-  int main_grid;             // ROWS_AUTO_*: workgroups of the launch with 256-row tiles
   int pieces;                // fp32 NN / NT: pieces of the reduction, from the host (gmm_f32.hip); 1 = whole
   bool warm;                 // TN: read both operands once before the first tile (warm_operands)
 };
@@ -88,24 +86,6 @@ struct GmmParams {
 // grouped kernels: the gate projection of large expert counts).
 __device__ __forceinline__ long long group_begin(const GmmParams& p, int e) {
   return p.offsets ? p.offsets[e] : (e > 0 ? (long long)p.N : 0ll);
-}
-
-// A launch with 256-row tiles leaves an expert's last n % 256 rows, when they are at most kRemRows,
-// to a second launch with 128-row tiles: a tile that is almost empty costs as much as a full one,
-// and with near-uniform routing those tiles alone add a whole round of the persistent grid.
-// ROWS_AUTO_*: the pair of launches decides on the device, from the tile counts, whether the split
-// into ROWS_MAIN + ROWS_REMAINDER pays (resolve_row_part in gmm.hip); if not, the AUTO_MAIN launch
-// takes all rows and the AUTO_REMAINDER launch exits.
-enum { ROWS_ALL = 0, ROWS_MAIN = 1, ROWS_REMAINDER = 2, ROWS_AUTO_MAIN = 3, ROWS_AUTO_REMAINDER = 4,
-       ROWS_NONE = 5 };
-constexpr int kRemRows = 128;
-// rows [begin, begin + count) of an expert with n rows that belong to `part`
-__device__ __forceinline__ void expert_row_part(long long n, int part, long long& begin,
-                                                long long& count) {
-  const long long full = n / 256 * 256, rem = n - full;
-  const bool split = rem > 0 && rem <= kRemRows;
-  begin = (part == ROWS_REMAINDER && split) ? full : 0;
-  count = part == ROWS_ALL ? n : (part == ROWS_MAIN ? (split ? full : n) : (split ? rem : 0));
 }
 
 // TN: rows of an expert one buffer resource may span (both operands, row pitch K and M elements),

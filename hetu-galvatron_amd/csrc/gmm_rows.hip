@@ -1,22 +1,28 @@
 // Grouped GEMM with row-adaptive tiles for 16-bit operands (bf16 / fp16) on gfx950: NN and NT of
-// gmm.hip's contract, with the fused gated-activation epilogues, for a few dozen to a few hundred rows
-// per expert (the rule with both sides' times is rows_rule.h).
+// gmm.hip's contract, with the fused gated-activation epilogues, from 96 rows per expert on (the rules with
+// both sides' times are in rows_rule.h and gmm.hip).
 //
-//   * A tile is RF*64 rows (RF = 1..4, chosen per tile) x 256 columns of C.  An expert's rows are cut
-//     into chunks of up to 256 (192, 128 where those fill the rounds better: best_max_units) that are as
-//     equal as 64-row steps allow, so at most 63 rows per expert are padding: a fixed 128- or 256-row tile
-//     multiplies a third of its rows for nothing at 380 rows per expert, and its operand stream is the larger the
-//     smaller the tile.
-//   * 2x2 wavefronts of (RF*32) x 128, one workgroup per CU.
-//   * Operands go global -> LDS without staging registers (buffer_load ... lds) in stages of 32
-//     reduction elements, 4 stages for 256 rows up to 7 for 64 rows; one barrier per stage.
-//   * What bounds it: the operand stream.  Without the MFMAs the Mixtral-shape fc1 launch still takes
-//     5.5 of 6.5 ms (42 GB/s per CU, whatever the number of stages; 72 GB/s when every stage hits L2),
-//     without the copies 4.3 ms.  Hence the large tile, and the copies spread one by one between the
-//     MFMAs of both K steps (a tile's copies in one burst: 4-9 % slower at full tiles).  Measured
-//     without gain: 64-deep stages (128-byte pieces of the rows), a staggered start of the
-//     workgroups' K walks, 128x256 tiles with two workgroups per CU (their operand stream is half
-//     again as large: 700 instead of 860 TFLOP/s at 383 rows per expert).
+//   * A tile is RF*64 rows (RF = 1..6, chosen per tile) x 256 columns of C.  An expert's rows are cut
+//     into chunks of up to 384 (320 .. 128 where those fill the rounds better: best_max_units) that are as
+//     equal as 64-row steps allow, so at most 63 rows per expert are padding.
+//   * 2x2 wavefronts of (RF*32) x 128, one workgroup per CU.  Up to 24 accumulators of 32x32: 16 in the
+//     256 accumulation registers, the other 8 in architectural ones (mma_vgpr), which leaves 128 of those for
+//     two sets of fragments and the addresses.
+//   * What bounds it: power, and the operand stream where an expert has a few hundred rows (fc1 of the
+//     Mixtral shape at 383 rows per expert: matrix cores 60 % busy at 1.85 GHz; without three fifths of the
+//     MFMAs 575 instead of 663 us at 2.4 GHz).  Both ask for fewer operand bytes per operation.  A 384-row tile
+//     takes 17 % fewer than a 256-row one through L2 and LDS: 4096 rows per expert, 8 experts, us in chunks of up
+//     to 256 / 384 rows, with activation 4096 x 28672 6255 / 5836, NN 14336 x 4096 2953 / 2790, NT 28672 x 4096
+//     5978 / 5727.
+//   * Operands go global -> LDS without staging registers (buffer_load ... lds).  Rows that are contiguous in
+//     the reduction index are copied 64 elements at a time, whole cache lines: copies of 32, half lines, ask L2
+//     one and a half times as often (NT 1024 rows per expert, 2816 x 2048, 64 experts 660 -> 637 us, 28672 x 4096, 8
+//     experts of 383 753 -> 691).  Each operand has a ring of its own as deep as LDS allows; weights whose
+//     reduction index is the slow dimension (NN) move 32 rows of 512 bytes at a time, which lets four to eight of
+//     them be in flight beside two or three tiles of A (one ring of 64-deep tiles for both: with activation 383 rows,
+//     4096 x 28672 734 instead of 686 us).  The copies are spread one by one between the MFMAs.
+//   * Measured without gain: a staggered start of the workgroups' K walks, 128x256 tiles with two workgroups per
+//     CU (their operand stream is half again as large: 700 instead of 860 TFLOP/s at 383 rows per expert).
 #include "gmm_common.h"
 
 namespace gmoe {
@@ -24,18 +30,21 @@ namespace gmoe {
 namespace rows {
 
 constexpr int BN = 256;
-constexpr int BKT = 32;  // reduction elements per stage
-constexpr int B_BYTES = BN * BKT * 2;
-constexpr int kUnit = 64;     // rows per unit: 32 for each of the two wavefront rows
-constexpr int kMaxUnits = kRowsMaxUnits;  // units per tile
+constexpr int BKT = 64;    // reduction elements per round
+constexpr int kUnit = 64;  // rows per unit: 32 for each of the two wavefront rows
+constexpr int kLdsBytes = 160 * 1024;
+constexpr int kMaxUnits = kTallMaxUnits;  // units per tile
 
-// LDS stages of a tile of RF units: as many as fit 144 KiB
-template <int RF>
-struct Stages {
-  static constexpr int a_bytes = RF * kUnit * BKT * 2;
-  static constexpr int bytes = a_bytes + B_BYTES;
-  static constexpr int count = RF == 4 ? 4 : (RF == 3 ? 5 : (RF == 2 ? 6 : 7));
-  static_assert(count * bytes <= 144 * 1024, "LDS");
+// LDS: a ring of 64-deep tiles of A and one of B.  B's are 64 deep where its rows are contiguous in the reduction
+// index (NT), as A's, and 32 deep where they are not (NN).
+template <int MODE, int RF>
+struct Rings {
+  static constexpr bool nt = MODE == MODE_NT;
+  static constexpr int a_bytes = RF * kUnit * BKT * 2, b_bytes = nt ? BN * BKT * 2 : BN * BKT;
+  static constexpr int na = nt ? (RF >= 3 ? 2 : (RF == 2 ? 3 : 4)) : (RF >= 5 ? 2 : 3);
+  static constexpr int nb = nt ? (RF >= 5 ? 2 : (RF >= 2 ? 3 : 4))
+                               : (RF == 6 || RF == 4 ? 4 : (RF == 5 || RF == 3 ? 5 : (RF == 2 ? 7 : 8)));
+  static_assert(na * a_bytes + nb * b_bytes <= kLdsBytes, "LDS");
 };
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
@@ -46,24 +55,23 @@ __device__ __forceinline__ int unit_count(long long n) { return (int)((n + kUnit
 __device__ __forceinline__ int chunk_count(long long n, int max_units) {
   return (unit_count(n) + max_units - 1) / max_units;
 }
-// rows_chunk_units for the launch; units, chunks: of this thread's experts, summed over the workgroup here.
-__device__ __forceinline__ int best_max_units(int units, const int (&chunks)[kMaxUnits + 1], int nt_cnt, int grid,
-                                              int64_t K, int (*sums)[kMaxUnits + 1], int lane, int wave) {
-  int v[kMaxUnits + 1] = {units, 0, chunks[2], chunks[3], chunks[4]};
+// rows_chunk_units for the launch; v: units and chunks of this thread's experts, summed over the workgroup here.
+__device__ __forceinline__ int best_max_units(int (&v)[kMaxUnits + 1], int nt_cnt, int grid, int64_t K, int* sums,
+                                              int lane, int wave) {
 #pragma unroll
   for (int i = 0; i <= kMaxUnits; ++i) {
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) v[i] += __shfl_xor(v[i], d);
-    if (lane == 0) sums[wave][i] = v[i];
+    if (lane == 0) sums[wave * (kMaxUnits + 1) + i] = v[i];
   }
   __syncthreads();
 #pragma unroll
   for (int i = 0; i <= kMaxUnits; ++i) {
     v[i] = 0;
 #pragma unroll
-    for (int w = 0; w < kGemmThreads / 64; ++w) v[i] += sums[w][i];
+    for (int w = 0; w < kGemmThreads / 64; ++w) v[i] += sums[w * (kMaxUnits + 1) + i];
   }
-  return rows_chunk_units(v, nt_cnt, grid, K);
+  return rows_chunk_units(v, nt_cnt, grid, K, 1.f);
 }
 // first unit and unit count of chunk c of cnt
 __device__ __forceinline__ void chunk_units(long long n, int cnt, int c, int& first, int& units) {
@@ -73,19 +81,20 @@ __device__ __forceinline__ void chunk_units(long long n, int cnt, int c, int& fi
   units = base + (c < extra ? 1 : 0);
 }
 
-// Operand with the reduction index contiguous: LDS tile [rows][32 k], 64 bytes per row; the 16-byte
-// piece c of row r sits in slot c ^ ((r >> 2) & 3), so 16 consecutive rows of a fragment read cover
-// all 64 banks.  One copy instruction moves 16 rows.
+// Operand with the reduction index contiguous: LDS tile [rows][64 k], 128 bytes per row; the 16-byte
+// piece c of row r sits in slot c ^ ((r >> 1) & 7), so 16 consecutive rows of a fragment read cover
+// all 64 banks.  One copy instruction moves 8 rows, whole cache lines of them.
 template <int INSTR>  // copy instructions per wavefront and stage
 struct KContig {
   u32x4 rsrc;
-  uint32_t voff[INSTR];
+  uint32_t voff[2];      // even and odd copy instructions, without their rows
+  uint32_t row16_bytes;  // 16 rows of the operand
   uint32_t lds_off;
-  int kchunk;
+  int kchunk[2];
   int64_t k_lim;
-  uint32_t frag[2];  // byte offset of the lane's piece at K step 0 / 1, fragment 0
+  uint32_t frag;  // byte offset of the lane's piece at K step 0, fragment 0
 
-  // row0: first row of the tile; rows past o_lim read as zero
+  // o0: first row of the tile; rows past o_lim read as zero
   __device__ __forceinline__ void init(const unsigned char* src, int64_t ld, int64_t o0, int64_t o_lim,
                                        int rows_max, int64_t k_limit, int wave, int lane,
                                        int frag_row0) {
@@ -93,28 +102,29 @@ struct KContig {
     rows = rows < 0 ? 0 : (rows > rows_max ? rows_max : rows);
     rsrc = make_raw_rsrc(src + o0 * ld * 2, rows * ld * 2);
     k_lim = k_limit;
-    const int chunk = (lane & 3) ^ ((lane >> 4) & 3);
-    kchunk = chunk * 8;
+    row16_bytes = (uint32_t)(16 * ld * 2);
 #pragma unroll
-    for (int q = 0; q < INSTR; ++q) {
-      const int blk = wave * INSTR + q;
-      voff[q] = (uint32_t)(((int64_t)(blk * 16 + (lane >> 2)) * ld + chunk * 8) * 2);
+    for (int q = 0; q < 2; ++q) {
+      const int row = (wave * INSTR + q) * 8 + (lane >> 3);
+      const int chunk = (lane & 7) ^ ((row >> 1) & 7);
+      kchunk[q] = chunk * 8;
+      voff[q] = (uint32_t)((int64_t)row * ld * 2 + chunk * 16);
     }
     lds_off = (uint32_t)(wave * INSTR * 1024);
     const int r = lane & 31, g = lane >> 5;
-    frag[0] = (uint32_t)((frag_row0 + r) * 64 + ((g ^ ((r >> 2) & 3)) * 16));
-    frag[1] = frag[0] ^ 32u;
+    frag = (uint32_t)((frag_row0 + r) * 128 + ((g ^ ((r >> 1) & 7)) * 16));
   }
-  __device__ __forceinline__ uint32_t offset(int kt) const { return stage_offset(rsrc[2], (uint32_t)kt, BKT * 2); }
+  __device__ __forceinline__ uint32_t offset(int kt) const { return (uint32_t)kt * (BKT * 2); }
   template <int q>
   __device__ __forceinline__ void issue(int kt, uint32_t off, uint32_t lds_tile, int) const {
-    const bool kok = (int64_t)kt * BKT + kchunk < k_lim;
-    dma16(lds_tile + lds_off + q * 1024, kok ? voff[q] : kOob, rsrc, off);
+    const bool kok = (int64_t)kt * BKT + kchunk[q & 1] < k_lim;
+    const uint32_t o = off + (q >> 1) * row16_bytes;
+    dma16(lds_tile + lds_off + q * 1024, kok ? voff[q & 1] : kOob, rsrc, o < rsrc[2] ? o : rsrc[2]);
   }
   static constexpr int READS = 1;
   template <int j, int ks, int h>
   __device__ __forceinline__ void read(const unsigned char* tile, u32x4& f) const {
-    f = *reinterpret_cast<const u32x4*>(tile + frag[ks] + j * 32 * 64);
+    f = *reinterpret_cast<const u32x4*>(tile + (frag ^ (ks * 32u)) + j * 32 * 128);
   }
 };
 
@@ -133,7 +143,7 @@ struct OuterContig {
   __device__ __forceinline__ void init(const unsigned char* src, int64_t ld, int64_t o0, int64_t k_limit,
                                        int wave, int lane, SegOf&& seg, int64_t gap) {
     rsrc = make_raw_rsrc(src + o0 * 2, k_limit * ld * 2 - o0 * 2);
-    stage_bytes = (uint32_t)(ld * 2 * BKT);
+    stage_bytes = (uint32_t)(ld * 2 * 32);
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const int krow = (wave * 4 + q) * 2 + (lane >> 5);
@@ -221,6 +231,36 @@ __attribute__((noinline)) __device__ void glu_bwd_rows(const unsigned char* lds,
   });
 }
 
+// acc += b a with the accumulators in architectural registers: the compiler puts those of the builtin into the
+// accumulation registers, which hold 16 fragments.
+template <int DT>
+__device__ __forceinline__ void mma_vgpr(const u32x4& a, const u32x4& b, f32x16& acc) {
+  if constexpr (DT == GMOE_BF16)
+    asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(b), "v"(a));
+  else
+    asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+v"(acc) : "v"(b), "v"(a));
+}
+
+// Before vector instructions read what mma_vgpr wrote: the compiler does not know how long that takes (up to 16 passes
+// and 18 wait states; these are 24).
+__device__ __forceinline__ void mma_settle(f32x16& acc) { asm volatile("s_nop 15\n\ts_nop 7" : "+v"(acc)); }
+
+// Fragments I0 .. I0+IN-1 of both wavefront rows as a tile of 2 * IN * 32 rows.
+template <int ODT, int RF, int I0, int IN>
+__device__ __forceinline__ void stage_acc_part(unsigned char* lds, const f32x16 (&acc)[RF][4], int wm, int wn, int lane) {
+#pragma unroll
+  for (int i = 0; i < IN; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int vq = 0; vq < 4; ++vq) {
+        const int row = wm * IN * 32 + i * 32 + (lane & 31), col = wn * 128 + j * 32 + 8 * vq + 4 * (lane >> 5);
+        const f32x16& v = acc[I0 + i][j];
+        *reinterpret_cast<u32x2*>(lds + row * CTile<BN>::pitch + col * 2) =
+            pack4<ODT>(v[4 * vq], v[4 * vq + 1], v[4 * vq + 2], v[4 * vq + 3]);
+      }
+}
+
 struct Item {
   int e, nt;
   long long row0;   // first row of the chunk, in the whole operand
@@ -231,12 +271,16 @@ struct Item {
 template <int DT, int ODT, int MODE, int EPI, int RF>
 __device__ __forceinline__ void run_tile(const GmmParams& p, const Item& it, unsigned char* lds, uint32_t lds0,
                                          int wave, int lane, int tid) {
+  // what depends on the lane is worked out by each tile size for itself: shared between them it would be spilled
+  asm volatile("" : "+v"(lane), "+v"(tid));
+  asm volatile("" : "+s"(wave), "+s"(lds0));
   constexpr bool GLU = EPI == EPI_GLU_FWD_SILU || EPI == EPI_GLU_FWD_GELU;
   constexpr bool GLU_BWD = EPI == EPI_GLU_BWD_SILU || EPI == EPI_GLU_BWD_GELU;
-  constexpr int A_BYTES = Stages<RF>::a_bytes, STAGE_BYTES = Stages<RF>::bytes, NST = Stages<RF>::count;
-  constexpr int NLOAD = RF + 4;  // copy instructions per wavefront and stage
-  typedef KContig<RF> OpA;
-  typedef std::conditional_t<MODE == MODE_NT, KContig<4>, OuterContig> OpB;
+  typedef Rings<MODE, RF> R;
+  constexpr int NA = R::na, NB = R::nb;
+  constexpr int LA = 2 * RF, LB = R::nt ? 8 : 4;  // copy instructions per wavefront and tile of A / B
+  typedef KContig<2 * RF> OpA;
+  typedef std::conditional_t<MODE == MODE_NT, KContig<8>, OuterContig> OpB;
   constexpr int RB = OpB::READS;
   constexpr int NREAD = RF + 4 * RB;
   constexpr int NM = RF * 4;
@@ -266,26 +310,16 @@ __device__ __forceinline__ void run_tile(const GmmParams& p, const Item& it, uns
 
   const int kt_cnt = (int)((K + BKT - 1) / BKT);
   u32x4 fa[2][RF], fb[2][4];
+  unsigned char* const ring_b = lds + NA * R::a_bytes;
+  const uint32_t lds_b = lds0 + NA * R::a_bytes;
 
-  auto issue = [&](auto op_c, int kt, uint32_t offa, uint32_t offb, uint32_t st) {
-    constexpr int op = decltype(op_c)::value;
-    if constexpr (op < RF) oa.template issue<op>(kt, offa, st, wave);
-    else ob.template issue<op - RF>(kt, offb, st + A_BYTES, wave);
-  };
-  auto frag_read = [&](auto r_c, auto ks_c, auto buf_c, const unsigned char* stage) {
-    constexpr int r = decltype(r_c)::value, ks = decltype(ks_c)::value, buf = decltype(buf_c)::value;
-    if constexpr (r < RF) oa.template read<r, ks, 0>(stage, fa[buf][r]);
-    else ob.template read<(r - RF) / RB, ks, (r - RF) % RB>(stage + A_BYTES, fb[buf][(r - RF) / RB]);
-  };
-
-  // One K step: the MFMAs with NREAD fragment reads and N copy requests spread evenly between them.
-  // Requests issued in a burst (all of a tile's at the end of one step) cost 5-9 % of a large launch.
-  auto k_step = [&](auto ks_c, auto n_c, auto&& read, auto&& request) {
+  auto k_step = [&](auto ks_c, auto n_c, auto&& read, auto&& request) __attribute__((always_inline)) {
     constexpr int ks = decltype(ks_c)::value, N = decltype(n_c)::value;
-    static_for<0, NM>([&](auto m_c) {
+    static_for<0, NM>([&](auto m_c) __attribute__((always_inline)) {
       constexpr int m = decltype(m_c)::value;
       constexpr int mi = m / 4, mj = (mi & 1) ? 3 - m % 4 : m % 4;
-      Mma<DT>::run(fa[ks][mi], fb[ks][mj], acc[mi][mj]);
+      if constexpr (mi < RF - 4) mma_vgpr<DT>(fa[ks & 1][mi], fb[ks & 1][mj], acc[mi][mj]);
+      else Mma<DT>::run(fa[ks & 1][mi], fb[ks & 1][mj], acc[mi][mj]);
       GMOE_SCHED_FENCE();
       static_for<(m * NREAD + NM - 1) / NM, ((m + 1) * NREAD + NM - 1) / NM>(read);
       static_for<(m * N + NM / 2) / NM, ((m + 1) * N + NM / 2) / NM>(request);
@@ -294,42 +328,148 @@ __device__ __forceinline__ void run_tile(const GmmParams& p, const Item& it, uns
   };
   constexpr std::integral_constant<int, 0> c0{};
   constexpr std::integral_constant<int, 1> c1{};
+  constexpr std::integral_constant<int, 2> c2{};
+  constexpr std::integral_constant<int, 3> c3{};
+  auto read_frags = [&](auto ks_c, const unsigned char* ta, const unsigned char* tb) {
+    // reader of the fragments of K step ks, from A's tile ta and B's tile tb
+    return [&, ta, tb](auto r_c) __attribute__((always_inline)) {
+      constexpr int r = decltype(r_c)::value, ks = decltype(ks_c)::value, buf = ks & 1;
+      if constexpr (r < RF) oa.template read<r, ks, 0>(ta, fa[buf][r]);
+      else ob.template read<(r - RF) / RB, R::nt ? ks : (ks & 1), (r - RF) % RB>(tb, fb[buf][(r - RF) / RB]);
+    };
+  };
+  auto next = [](int i, int n) { return i == n - 1 ? 0 : i + 1; };
+  constexpr std::integral_constant<int, 0> none{};
 
-  static_for<0, NST - 1>([&](auto t_c) {
-    constexpr int t = decltype(t_c)::value;
-    const uint32_t offa = oa.offset(t), offb = ob.offset(t);
-    static_for<0, NLOAD>([&](auto q) { issue(q, t, offa, offb, lds0 + t * STAGE_BYTES); });
-  });
-  wait_dma_outstanding<(NST - 2) * NLOAD>();
-  __syncthreads();
-  static_for<0, NREAD>([&](auto r) {
-    frag_read(r, std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{}, lds);
-  });
-  int s0 = 0;        // stage of tile kt
-  int sl = NST - 1;  // stage of tile kt + NST - 1
-  for (int kt = 0; kt < kt_cnt; ++kt) {
-    const int s1 = s0 == NST - 1 ? 0 : s0 + 1;
-    const unsigned char* cur = lds + s0 * STAGE_BYTES;
-    const unsigned char* nxt = lds + s1 * STAGE_BYTES;
-    const uint32_t stl = lds0 + (uint32_t)(sl * STAGE_BYTES);
-    const int ktl = kt + NST - 1;
-    const uint32_t offa = oa.offset(ktl), offb = ob.offset(ktl);
-    // step 0: read step 1's fragments; request half of the tile kt+NST-1 into the stage tile kt-1 left
-    k_step(c0, std::integral_constant<int, NLOAD / 2>{}, [&](auto r_c) { frag_read(r_c, c1, c1, cur); },
-           [&](auto q_c) { issue(q_c, ktl, offa, offb, stl); });
-    // tile kt+1 has landed (the later ones may be in flight); every wavefront has read this stage
-    wait_dma_outstanding<(NST - 3) * NLOAD + NLOAD / 2>();
+  if constexpr (R::nt) {
+    // Order of the copies of round p (64 reduction elements): tile p - 1 + NA of A, then tile p - 1 + NB of B, from
+    // K step 3 of round p - 1 on; where B's ring has two tiles, early enough to land within the round.  Copies land
+    // in order, so what may be in flight when a tile is needed is what was issued after it.
+    constexpr int L = LA + LB;
+    constexpr int N3 = NB == 2 ? L * 3 / 10 : L / 4, N0 = NB == 2 ? L * 4 / 10 : L / 4,
+                  N1 = NB == 2 ? L - N3 - N0 : L / 4, N2 = L - N3 - N0 - N1;
+    constexpr int a_end = (2 - NA) * L + LA, b_end = (3 - NB) * L;
+    constexpr int wait_y = L - (a_end > b_end ? a_end : b_end);
+    // copy op of round p: la, lb the slots of the two tiles
+    auto issue = [&](auto op_c, int p, uint32_t offa, uint32_t offb, int la, int lb) __attribute__((always_inline)) {
+      constexpr int op = decltype(op_c)::value;
+      if constexpr (op < LA) oa.template issue<op>(p - 1 + NA, offa, lds0 + (uint32_t)la * R::a_bytes, wave);
+      else ob.template issue<op - LA>(p - 1 + NB, offb, lds_b + (uint32_t)lb * R::b_bytes, wave);
+    };
+    static_for<0, NB>([&](auto i_c) {
+      constexpr int r = decltype(i_c)::value + 1 - NB;  // rounds 1 - NB .. 0
+      static_for<0, (r == 0 ? N3 : L)>([&](auto q) {
+        if constexpr (decltype(q)::value >= LA || r - 1 + NA >= 0)
+          issue(q, r, oa.offset(r - 1 + NA), ob.offset(r - 1 + NB), r - 1 + NA, r - 1 + NB);
+      });
+    });
+    wait_dma_outstanding<wait_y + N3>();
     __syncthreads();
-    GMOE_SCHED_FENCE();
-    // step 1: read step 0's fragments of tile kt+1; request the other half
-    k_step(c1, std::integral_constant<int, NLOAD - NLOAD / 2>{}, [&](auto r_c) { frag_read(r_c, c0, c0, nxt); },
-           [&](auto q_c) {
-             issue(std::integral_constant<int, NLOAD / 2 + decltype(q_c)::value>{}, ktl, offa, offb, stl);
-           });
-    sl = s0;
-    s0 = s1;
+    static_for<0, NREAD>(read_frags(c0, lds, ring_b));
+    int sa = 0, sb = 0;            // slots of tile kt
+    int la = NA - 1, lb = NB - 1;  // slots of tiles kt - 1 + NA of A and kt - 1 + NB of B
+    for (int kt = 0; kt < kt_cnt; ++kt) {
+      const int sa1 = next(sa, NA), sb1 = next(sb, NB);
+      const unsigned char *ca = lds + sa * R::a_bytes, *cb = ring_b + sb * R::b_bytes;
+      const unsigned char *xa = lds + sa1 * R::a_bytes, *xb = ring_b + sb1 * R::b_bytes;
+      {
+        const uint32_t offa = oa.offset(kt - 1 + NA), offb = ob.offset(kt - 1 + NB);
+        auto request = [&](auto first_c) {
+          return [&](auto q_c) __attribute__((always_inline)) {
+            issue(std::integral_constant<int, decltype(first_c)::value + decltype(q_c)::value>{}, kt, offa, offb, la, lb);
+          };
+        };
+        k_step(c0, std::integral_constant<int, N0>{}, read_frags(c1, ca, cb), request(std::integral_constant<int, N3>{}));
+        k_step(c1, std::integral_constant<int, N1>{}, read_frags(c2, ca, cb), request(std::integral_constant<int, N3 + N0>{}));
+        k_step(c2, std::integral_constant<int, N2>{}, read_frags(c3, ca, cb), request(std::integral_constant<int, N3 + N0 + N1>{}));
+      }
+      // tiles kt + 1 have landed; every wavefront has read tiles kt
+      wait_dma_outstanding<wait_y>();
+      __syncthreads();
+      GMOE_SCHED_FENCE();
+      {
+        const uint32_t offa = oa.offset(kt + NA), offb = ob.offset(kt + NB);
+        k_step(c3, std::integral_constant<int, N3>{}, read_frags(c0, xa, xb),
+               [&](auto q_c) { issue(q_c, kt + 1, offa, offb, sa, sb); });
+      }
+      la = sa;
+      sa = sa1;
+      lb = sb;
+      sb = sb1;
+    }
+  } else {
+    // Order of the copies of round p (64 reduction elements): tile p - 1 + NA of A in K steps 3 of round p - 1
+    // and 0, tiles 2 p - 1 + NB and 2 p + NB of B in K steps 1 and 2.  Copies land in order, so what may be in
+    // flight when a tile is needed is what was issued after it (positions in the order, relative to round 0).
+    constexpr int L = LA + 2 * LB;
+    constexpr auto half = [](int v) { return v < 0 ? -((1 - v) / 2) : v / 2; };
+    constexpr int a_end = (2 - NA) * L + LA;  // tile 1 of A
+    constexpr int b2_end = NB % 2 == 0 ? ((2 - NB) / 2 + 1) * L : half(3 - NB) * L + LA + LB;  // tile 2 of B
+    constexpr int b1_end = NB % 2 == 0 ? half(2 - NB) * L + LA + LB : (half(1 - NB) + 1) * L;  // tile 1 of B
+    constexpr int wait_y = L - (a_end > b2_end ? a_end : b2_end), wait_x = LA - b1_end;
+    constexpr int A3 = LA / 2;
+    auto issue_a = [&](auto q_c, int t, uint32_t off, int slot) __attribute__((always_inline)) {
+      oa.template issue<decltype(q_c)::value>(t, off, lds0 + (uint32_t)slot * R::a_bytes, wave);
+    };
+    auto issue_b = [&](auto q_c, uint32_t off, int slot) __attribute__((always_inline)) {
+      ob.template issue<decltype(q_c)::value>(0, off, lds_b + (uint32_t)slot * R::b_bytes, wave);
+    };
+    static_for<0, NB>([&](auto i_c) {
+      constexpr int r = decltype(i_c)::value - NB;  // rounds -NB .. -1
+      if constexpr (r - 1 + NA >= 0)
+        static_for<0, LA>([&](auto q) { issue_a(q, r - 1 + NA, oa.offset(r - 1 + NA), r - 1 + NA); });
+      if constexpr (2 * r - 1 + NB >= 0)
+        static_for<0, LB>([&](auto q) { issue_b(q, ob.offset(2 * r - 1 + NB), 2 * r - 1 + NB); });
+      if constexpr (2 * r + NB >= 0)
+        static_for<0, LB>([&](auto q) { issue_b(q, ob.offset(2 * r + NB), 2 * r + NB); });
+    });
+    wait_dma_outstanding<wait_y>();
+    __syncthreads();
+    static_for<0, NREAD>(read_frags(c0, lds, ring_b));
+    static_for<0, A3>([&](auto q) { issue_a(q, NA - 1, oa.offset(NA - 1), NA - 1); });
+    int sa = 0, sb = 0;    // slots of tiles p of A and 2 p of B
+    int la = NA - 1, lb = NB - 1;  // slots of tiles p - 1 + NA of A and 2 p - 1 + NB of B
+    for (int p2 = 0; p2 < kt_cnt; ++p2) {
+      const int sb1 = next(sb, NB), sb2 = next(sb1, NB), sa1 = next(sa, NA);
+      const unsigned char *ca = lds + sa * R::a_bytes, *xa = lds + sa1 * R::a_bytes;
+      const unsigned char *b0 = ring_b + sb * R::b_bytes, *b1 = ring_b + sb1 * R::b_bytes, *b2 = ring_b + sb2 * R::b_bytes;
+      {
+        const uint32_t off = oa.offset(p2 - 1 + NA);
+        k_step(c0, std::integral_constant<int, LA - A3>{}, read_frags(c1, ca, b0), [&](auto q_c) {
+          issue_a(std::integral_constant<int, A3 + decltype(q_c)::value>{}, p2 - 1 + NA, off, la);
+        });
+      }
+      // tile 2 p + 1 of B has landed; every wavefront has read tile 2 p
+      wait_dma_outstanding<wait_x>();
+      __syncthreads();
+      GMOE_SCHED_FENCE();
+      {
+        const uint32_t off = ob.offset(2 * p2 - 1 + NB);
+        k_step(c1, std::integral_constant<int, LB>{}, read_frags(c2, ca, b1), [&](auto q_c) { issue_b(q_c, off, lb); });
+      }
+      {
+        const uint32_t off = ob.offset(2 * p2 + NB);
+        k_step(c2, std::integral_constant<int, LB>{}, read_frags(c3, ca, b1), [&](auto q_c) { issue_b(q_c, off, sb); });
+      }
+      // tiles p + 1 of A and 2 p + 2 of B have landed; every wavefront has read A's tile p and B's tile 2 p + 1
+      wait_dma_outstanding<wait_y>();
+      __syncthreads();
+      GMOE_SCHED_FENCE();
+      {
+        const uint32_t off = oa.offset(p2 + NA);
+        k_step(c3, std::integral_constant<int, A3>{}, read_frags(c0, xa, b2),
+               [&](auto q_c) { issue_a(q_c, p2 + NA, off, sa); });
+      }
+      la = sa;
+      sa = sa1;
+      lb = sb1;
+      sb = sb2;
+    }
   }
   wait_dma_outstanding<0>();
+  static_for<0, (RF > 4 ? RF - 4 : 0)>([&](auto i_c) {
+    static_for<0, 4>([&](auto j_c) { mma_settle(acc[decltype(i_c)::value][decltype(j_c)::value]); });
+  });
   __syncthreads();
 
   // ---- epilogue ------------------------------------------------------------------------------
@@ -353,51 +493,66 @@ __device__ __forceinline__ void run_tile(const GmmParams& p, const Item& it, uns
     }
     return;
   } else {
-    stage_acc_lds<ODT, RF, 4, BN>(lds, acc, wm * RF * 32, wn * 128, lane);
-    __syncthreads();
-    if constexpr (GLU) {
-      constexpr bool gelu = EPI == EPI_GLU_FWD_GELU;
-      const int64_t F = p.F;
-      unsigned char* fc1 = p.c + it.row0 * M * 2;
-      unsigned char* act = p.c2 + it.row0 * F * 2;
-      const int cc = tid & 15, r0 = tid >> 4;
-      const int64_t n = (int64_t)it.nt * 128 + cc * 8;
-      const int lcol = (cc >> 3) * 128 + (cc & 7) * 8;
-#pragma unroll 4
-      for (int q = 0; q < RF * 4; ++q) {
-        const int row = q * 16 + r0;
-        if (row >= it.n || n >= F) continue;
-        const u32x4 gw = ctile_read16(lds + row * CT::pitch + lcol * 2);
-        const u32x4 uw = ctile_read16(lds + row * CT::pitch + (lcol + 64) * 2);
-        float g[8], u[8], o[8];
-        Vec16<DT>::unpack(gw, g);
-        Vec16<DT>::unpack(uw, u);
+    // a tile of more than 256 rows is staged in two parts, each of some fragments of both wavefront rows
+    constexpr int PARTS = RF > 4 ? 2 : 1;
+    static_for<0, PARTS>([&](auto part_c) __attribute__((always_inline)) {
+      constexpr int part = decltype(part_c)::value;
+      constexpr int I0 = part * (RF + 1) / 2 * (PARTS - 1), IN = PARTS == 1 ? RF : (part == 0 ? (RF + 1) / 2 : RF / 2);
+      stage_acc_part<ODT, RF, I0, IN>(lds, acc, wm, wn, lane);
+      __syncthreads();
+      constexpr int BLOCKS = PARTS == 1 ? 1 : 2, BROWS = PARTS == 1 ? RF * 64 : IN * 32;
 #pragma unroll
-        for (int t = 0; t < 8; ++t) o[t] = glu_act(g[t], gelu) * u[t];
-        st16(fc1 + (row * M + n) * 2, gw);
-        st16(fc1 + (row * M + F + n) * 2, uw);
-        st16(act + (row * F + n) * 2, Vec16<DT>::pack(o));
-      }
-    } else if constexpr (GLU_BWD) {
-      const int cc = tid & 31, r0 = tid >> 5;
-      const int64_t n = (int64_t)it.nt * BN + cc * 8;
-      constexpr bool gelu = EPI == EPI_GLU_BWD_GELU;
-      const int64_t F = M;
-      const unsigned char* fc1 = p.aux + it.row0 * 2 * F * OES;
-      unsigned char* dfc1 = p.c + it.row0 * 2 * F * OES;
-      if (n < F) glu_bwd_rows<DT, gelu, RF * 8>(lds, fc1, dfc1, F, n, cc, r0, it.n);
-    } else {
-      const int cc = tid & 31, r0 = tid >> 5;
-      const int64_t n = (int64_t)it.nt * BN + cc * 8;
-      unsigned char* c_base = p.c + it.row0 * M * OES;
+      for (int w = 0; w < BLOCKS; ++w) {
+        const int first = w * RF * 32 + I0 * 32;
+        const int64_t rows = it.n - first;
+        if (rows <= 0) continue;
+        const int64_t row0 = it.row0 + first;
+        const unsigned char* tile = lds + w * BROWS * CT::pitch;
+        if constexpr (GLU) {
+          constexpr bool gelu = EPI == EPI_GLU_FWD_GELU;
+          const int64_t F = p.F;
+          unsigned char* fc1 = p.c + row0 * M * 2;
+          unsigned char* act = p.c2 + row0 * F * 2;
+          const int cc = tid & 15, r0 = tid >> 4;
+          const int64_t n = (int64_t)it.nt * 128 + cc * 8;
+          const int lcol = (cc >> 3) * 128 + (cc & 7) * 8;
+#pragma unroll 4
+          for (int q = 0; q < BROWS / 16; ++q) {
+            const int row = q * 16 + r0;
+            if (row >= rows || n >= F) continue;
+            const u32x4 gw = ctile_read16(tile + row * CT::pitch + lcol * 2);
+            const u32x4 uw = ctile_read16(tile + row * CT::pitch + (lcol + 64) * 2);
+            float g[8], u[8], o[8];
+            Vec16<DT>::unpack(gw, g);
+            Vec16<DT>::unpack(uw, u);
+#pragma unroll
+            for (int t = 0; t < 8; ++t) o[t] = glu_act(g[t], gelu) * u[t];
+            st16(fc1 + (row * M + n) * 2, gw);
+            st16(fc1 + (row * M + F + n) * 2, uw);
+            st16(act + (row * F + n) * 2, Vec16<DT>::pack(o));
+          }
+        } else if constexpr (GLU_BWD) {
+          const int cc = tid & 31, r0 = tid >> 5;
+          const int64_t n = (int64_t)it.nt * BN + cc * 8;
+          constexpr bool gelu = EPI == EPI_GLU_BWD_GELU;
+          const int64_t F = M;
+          const unsigned char* fc1 = p.aux + row0 * 2 * F * OES;
+          unsigned char* dfc1 = p.c + row0 * 2 * F * OES;
+          if (n < F) glu_bwd_rows<DT, gelu, BROWS / 8>(tile, fc1, dfc1, F, n, cc, r0, rows);
+        } else {
+          const int cc = tid & 31, r0 = tid >> 5;
+          const int64_t n = (int64_t)it.nt * BN + cc * 8;
+          unsigned char* c_base = p.c + row0 * M * OES;
 #pragma unroll 8
-      for (int q = 0; q < RF * 8; ++q) {
-        const int row = q * 8 + r0;
-        if (row < it.n && n < M)
-          st16(c_base + ((int64_t)row * M + n) * OES, ctile_read16(lds + row * CT::pitch + cc * 16));
+          for (int q = 0; q < BROWS / 8; ++q) {
+            const int row = q * 8 + r0;
+            if (row < rows && n < M)
+              st16(c_base + ((int64_t)row * M + n) * OES, ctile_read16(tile + row * CT::pitch + cc * 16));
+          }
+        }
       }
-    }
-    __syncthreads();
+      __syncthreads();
+    });
   }
 }
 
@@ -405,30 +560,29 @@ template <int DT, int ODT, int MODE, int EPI>
 __global__ __launch_bounds__(kGemmThreads, 1) void gmm_rows_kernel(GmmParams p) {
   constexpr bool GLU = EPI == EPI_GLU_FWD_SILU || EPI == EPI_GLU_FWD_GELU;
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
-  __shared__ int tile_cum[kMaxGroupsLds + 1];
-  __shared__ int wave_tot[kGemmThreads / 64];
-  __shared__ int sums[kGemmThreads / 64][kMaxUnits + 1];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t lds0 = lds_offset_of(lds);
   const int E = p.E;
   const int nt_cnt = GLU ? (int)((p.F + 127) / 128) : (int)((p.M + BN - 1) / BN);
 
-  int max_units = kMaxUnits;
+  // Tiles before and after each of this thread's kPer consecutive experts; the rings and the staged result take all
+  // of the LDS, so the table stays in registers and LDS serves as scratch between tiles.
+  constexpr int kPer = kMaxGroupsLds / kGemmThreads, kWaves = kGemmThreads / 64;
+  int* const scratch = reinterpret_cast<int*>(lds);
+  int tiles_before[kPer + 1], total, max_units;
   {
-    // tiles per expert -> exclusive prefix (a thread owns kPer consecutive experts)
-    constexpr int kPer = kMaxGroupsLds / kGemmThreads;
     long long rows_of[kPer];
-    int units = 0, chunks[kMaxUnits + 1] = {};
+    int v[kMaxUnits + 1] = {};
 #pragma unroll
     for (int j = 0; j < kPer; ++j) {
       const int e = tid * kPer + j;
       rows_of[j] = e >= E ? 0 : group_begin(p, e + 1) - group_begin(p, e);
-      units += unit_count(rows_of[j]);
+      v[0] += unit_count(rows_of[j]);
 #pragma unroll
-      for (int u = 2; u <= kMaxUnits; ++u) chunks[u] += chunk_count(rows_of[j], u);
+      for (int u = 2; u <= kMaxUnits; ++u) v[u] += chunk_count(rows_of[j], u);
     }
-    max_units = best_max_units(units, chunks, nt_cnt, (int)gridDim.x, p.K, sums, lane, wave);
+    max_units = best_max_units(v, nt_cnt, (int)gridDim.x, p.K, scratch + kWaves, lane, wave);
     int cnt[kPer], local = 0;
 #pragma unroll
     for (int j = 0; j < kPer; ++j) {
@@ -441,26 +595,29 @@ __global__ __launch_bounds__(kGemmThreads, 1) void gmm_rows_kernel(GmmParams p) 
       const int o = __shfl_up(incl, d);
       if (lane >= d) incl += o;
     }
-    if (lane == 63) wave_tot[wave] = incl;
+    if (lane == 63) scratch[wave] = incl;
     __syncthreads();
     int run = incl - local;
-    for (int w = 0; w < wave; ++w) run += wave_tot[w];
+    total = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+      if (w < wave) run += scratch[w];
+      total += scratch[w];
+    }
+    total = __builtin_amdgcn_readfirstlane(total);
 #pragma unroll
     for (int j = 0; j < kPer; ++j) {
-      const int e = tid * kPer + j;
-      if (e <= E) tile_cum[e] = run;
+      tiles_before[j] = run;
       run += cnt[j];
     }
-    if (tid == kGemmThreads - 1) tile_cum[E] = run;
+    tiles_before[kPer] = run;
+    __syncthreads();
   }
-  __syncthreads();
-  const int total = tile_cum[E];
 
   // XCD x takes the positions [x*G/8, (x+1)*G/8) of every whole round of G tiles; the last, partial
   // round is dealt to the XCDs in equal consecutive shares
   const int G = gridDim.x, per_xcd = G / 8;
   const int xcd = blockIdx.x % 8, slot = blockIdx.x / 8;
-  int e = 0;
   for (int base = 0; base < total; base += G) {
     int v = base + xcd * per_xcd + slot;
     if (total - base < G) {
@@ -468,13 +625,22 @@ __global__ __launch_bounds__(kGemmThreads, 1) void gmm_rows_kernel(GmmParams p) 
       v = base + xcd * share + slot;
       if (slot >= share || v >= total) break;
     }
-    while (tile_cum[e + 1] <= v) ++e;
+    // the thread whose expert tile v belongs to says so
+#pragma unroll
+    for (int j = 0; j < kPer; ++j)
+      if (v >= tiles_before[j] && v < tiles_before[j + 1]) {
+        scratch[0] = tid * kPer + j;
+        scratch[1] = v - tiles_before[j];
+      }
+    __syncthreads();
     Item it;
-    it.e = __builtin_amdgcn_readfirstlane(e);
-    const long long row0 = group_begin(p, e), n_e = group_begin(p, e + 1) - row0;
+    it.e = __builtin_amdgcn_readfirstlane(scratch[0]);
+    const int place = __builtin_amdgcn_readfirstlane(scratch[1]);
+    __syncthreads();
+    const long long row0 = group_begin(p, it.e), n_e = group_begin(p, it.e + 1) - row0;
     const int chunks = chunk_count(n_e, max_units);
     int c, first, units;
-    strip_order(v - tile_cum[e], chunks, nt_cnt, c, it.nt);
+    strip_order(place, chunks, nt_cnt, c, it.nt);
     chunk_units(n_e, chunks, c, first, units);
     it.row0 = row0 + (long long)first * kUnit;
     it.n = n_e - (long long)first * kUnit;
@@ -483,15 +649,16 @@ __global__ __launch_bounds__(kGemmThreads, 1) void gmm_rows_kernel(GmmParams p) 
       case 1: run_tile<DT, ODT, MODE, EPI, 1>(p, it, lds, lds0, wave, lane, tid); break;
       case 2: run_tile<DT, ODT, MODE, EPI, 2>(p, it, lds, lds0, wave, lane, tid); break;
       case 3: run_tile<DT, ODT, MODE, EPI, 3>(p, it, lds, lds0, wave, lane, tid); break;
-      default: run_tile<DT, ODT, MODE, EPI, 4>(p, it, lds, lds0, wave, lane, tid); break;
+      case 4: run_tile<DT, ODT, MODE, EPI, 4>(p, it, lds, lds0, wave, lane, tid); break;
+      case 5: run_tile<DT, ODT, MODE, EPI, 5>(p, it, lds, lds0, wave, lane, tid); break;
+      default: run_tile<DT, ODT, MODE, EPI, 6>(p, it, lds, lds0, wave, lane, tid); break;
     }
   }
 }
 
 template <int DT, int ODT, int MODE, int EPI>
 static int launch_cfg(const GmmParams& p, hipStream_t st) {
-  constexpr size_t stages = 144 * 1024, ctile = (size_t)256 * CTile<BN>::pitch;
-  constexpr size_t smem = stages > ctile ? stages : ctile;
+  constexpr size_t smem = kLdsBytes;
   auto kern = gmm_rows_kernel<DT, ODT, MODE, EPI>;
   static std::atomic<uint64_t> done_mask{0};
   if (!gmoe_once_per_device(done_mask, [&] {
@@ -504,6 +671,7 @@ static int launch_cfg(const GmmParams& p, hipStream_t st) {
   hipLaunchKernelGGL(kern, dim3(grid), dim3(kGemmThreads), smem, st, p);
   return gmoe_launch_status();
 }
+
 
 template <int DT>
 static int launch_dt(const GmmParams& p, int mode, int out_dtype, int epi, hipStream_t st) {

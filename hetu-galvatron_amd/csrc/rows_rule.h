@@ -1,44 +1,30 @@
-// Whether a 16-bit NN / NT launch goes to the row-adaptive tiles (gmm_rows.hip): what it takes there against what
-// it takes on the 256x256 tiles, or on 128x128 ones where those are too few (only the
-// host asks); and into which chunks the kernel cuts an expert's rows.
-//
-// Both sides were measured for 3400 shapes (E 1-64, 72-2040 rows per expert, K 256-28672, M 128-28672, 3e8 to 4e12
-// operations, weights from HBM, loads that differ by 7 %), and the constants are fitted to them.  us of the other
-// tiles / of these, with the choice (rows per expert, K x M, experts):
-//   * forward with activation: 382, 4096 x 28672, 8 1004 / 724 these; 139, 2048 x 2816, 64 238 / 188 these; 640,
-//     1024 x 5632, 16 162 / 168 others; 1024, 7168 x 4096, 32 1657 / 1624 these.
-//   * NN: 382, 14336 x 4096, 8 537 / 330 these; 1024, 1408 x 2048, 64 374 / 370 these; 267, 576 x 832, 64 34 / 41
-//     others; 921, 1536 x 128, 64 39 / 55 others.
-//   * NT: 382, 28672 x 4096, 8 1074 / 737 these; 640, 5632 x 1024, 16 158 / 137 these; 740, 14336 x 4096, 8 644 / 729
-//     others (here two operands come in 64-byte pieces of a row, there in 128-byte ones); 1000, 640 x 128, 64 29 / 38
-//     others.
-//   * activation backward: 382, 4096 x 14336, 8 525 / 455 these; 640, 1024 x 2816, 16 128 / 119 these; 1000, 4096 x
-//     14336, 8 886 / 945 others; 192, 1024 x 1024, 48 55 / 60 others.
-// It knows the average load only, and where that is close to whole rounds it can be wrong: 376, 576 x 1376, 16 24.5 /
-// 26.6 these; 402, 896 x 1408, 24 with activation 50 / 57 these; 937, 4896 x 1728, 4 77 / 71 others.  In all, the
-// choice costs 1.2 % against the better side of every shape; a limit on each size cost 1.9 %, and these tiles only
-// from 1024 reduction elements and three quarters of a round on 2.7 %.
+// Which 16-bit NN / NT launches go to the row-adaptive tiles (gmm_rows.hip), and into which chunks the kernel cuts an
+// expert's rows.
 #pragma once
 #include "split_rule.h"
 
 namespace gmoe {
 
-// Rows of a chunk, in units of 64: the size, of 4, 3 and 2, that ends first.  v[0]: units of all experts, v[2..4]:
-// their chunks of up to so many units.  A stage of a tile of u units takes as long as its operands stream, 16 + 4 u
-// KiB at 42 GB/s; prologue and epilogue take as long as 250 KiB.  Where the largest chunks leave a round part
-// empty, smaller ones fill it (us with chunks of up to 256 rows / with these, rows per expert: NT 640, 5632 x 1024,
-// 16 experts 146 / 137; NN 640, 2816 x 1024, 16 75 / 69; with the activation 817, 6432 x 4832, 8 468 / 428).  Asked
-// by the kernel.
+// Rows of a chunk, in units of 64: of the sizes SIZES - 1 to 2 the one that ends first.  v[0]: units of all experts,
+// v[u]: their chunks of up to u units.  A stage of a tile of u units takes as long as its operands stream, 16 + 4 u KiB;
+// prologue and epilogue take as long as 250 KiB.  Smaller chunks are taken where they cost less than `ahead` of the
+// best larger ones.  The kernel asks with ahead 1: over 8600 launches of 96 rows per expert and more that costs 1.1 %
+// against the best size of each, 0.95 costs 2.0 % (us in chunks of up to 128 / 192 / 256 / 320 / 384 rows, rows per
+// expert: with activation 383, 4096 x 28672, 8 experts 890 / 776 / 739 / 745 / 686; 640, 1024 x 5632, 16 172 / 152 /
+// 150 / 147 / 135; NN 640, 2816 x 1024, 16 86 / 60 / 67 / 73 / 81; NT 383, 28672 x 4096, 8 817 / 935 / 691 / 700 / 926).
 constexpr int kRowsMaxUnits = 4;
-__host__ __device__ inline int rows_chunk_units(const int (&v)[kRowsMaxUnits + 1], int col_tiles, int grid, int64_t K) {
+constexpr int kTallMaxUnits = 6;
+template <int SIZES>
+__host__ __device__ inline int rows_chunk_units(const int (&v)[SIZES], int col_tiles, int grid, int64_t K,
+                                                float ahead = 0.95f) {
   const float fixed = 16.f + 250.f / (float)((K + 31) / 32);
-  int best = kRowsMaxUnits;
+  int best = SIZES - 1;
   float least = 0.f;
 #pragma unroll
-  for (int u = kRowsMaxUnits; u >= 2; --u) {
+  for (int u = SIZES - 1; u >= 2; --u) {
     const int rounds = (int)(((long long)v[u] * col_tiles + grid - 1) / grid);
     const float cost = (float)rounds * (fixed + 4.f * (float)v[0] / (float)(v[u] > 0 ? v[u] : 1));
-    if (u == kRowsMaxUnits || cost < 0.95f * least) {
+    if (u == SIZES - 1 || cost < ahead * least) {
       best = u;
       least = cost;
     }
@@ -67,8 +53,8 @@ constexpr RowsCosts kRowsCosts[] = {
     {0, 5240, 848, 0.11, 8970, 1.03e6, 22600, 1410, 1.57e6, 1360, 1580, 387, 4680, 15000, 4120}};
 constexpr double kRowsWeights = 6000;
 
-// Rows per expert from which short last row tiles have a launch of their own beside the 256x256 ones.
-constexpr int64_t kNnRemainderRows = 2048;
+// Rows per expert from which rows_pays is not asked (gmm.hip).
+constexpr int64_t kRowsManyRows = 2048;
 
 // 256x256 tiles for NN / NT: an expert's share of rows can fill them and there are enough for every CU.
 inline bool nn_large_tiles(int64_t E, int64_t N, int64_t M) {
@@ -92,12 +78,15 @@ inline int64_t over_loads(int64_t E, int64_t n, F f) {
   return sum;
 }
 
+// The line for chunks of up to 256 rows, with constants fitted to 3400 shapes measured both ways (E 1-64, 72-2040 rows
+// per expert, K 256-28672, M 128-28672) when the kernel had no larger ones and streamed its rows in half cache lines: a
+// launch that paid then pays more now, and tall_pays adds those that pay only now.
 // K, M as in the product (with the activation M = 2F); cus: workgroups of a persistent grid, one per CU.
 inline bool rows_pays(RowsKind kind, int64_t E, int64_t N, int64_t K, int64_t M, int64_t cus) {
   const int64_t n = N / (E > 0 ? E : 1);
   // fewer rows: an expert is one tile either way, and its weights bound the launch; shorter reductions:
-  // prologue and epilogue weigh as much; many rows: the 256x256 tiles have their remainder launches
-  if (n < 96 || n >= kNnRemainderRows || K <= 512) return false;
+  // prologue and epilogue weigh as much
+  if (n < 96 || n >= kRowsManyRows || K <= 512) return false;
   const RowsCosts& c = kRowsCosts[kind];
   const bool glu = kind == ROWS_NN_GLU, large = nn_large_tiles(E, N, M);
   const double weights = (double)E * K * M * 2, ops = 2.0 * N * K * M;
@@ -136,6 +125,65 @@ inline bool rows_pays(RowsKind kind, int64_t E, int64_t N, int64_t K, int64_t M,
   // the activation as a launch of its own
   if (glu && !large) other += 3000 + (double)N * M * 3 / 4000;
   return rows < other;
+}
+
+// Times in ns as above: row-adaptive tiles with chunks of up to 384 rows (a stage is stage + unit_stage per 64 rows),
+// then 128x128 tiles.
+struct TallCosts {
+  double tile, unit, stage, unit_stage, lone_gain, launch, weights, ops;
+  double small_tile, small_pair, small_lone, sums, small_launch, small_weights, small_ops, act;
+};
+constexpr TallCosts kTallCosts[] = {
+    {4620, 960, 217, 141, 0.31, 4200, 4830, 1.48e6, 3760, 1260, 520, 8700, 6300, 4320, 1e6, 0},
+    {4790, 1580, 260, 133, 0.30, 4400, 4540, 1.495e6, 1470, 1200, 490, 20900, 7700, 4530, 0.8e6, 2700},
+    {3840, 1140, 223, 144, 0.30, 4100, 4390, 1.41e6, 2860, 1240, 530, 7400, 6900, 4080, 1e6, 0},
+    {690, 5880, 294, 127, 0.36, 5200, 4080, 1.487e6, 9950, 1350, 560, 0, 3800, 3640, 1e6, 0}};
+
+// Whether a launch that has too few rows or tiles for 256x256 ones is faster in row-adaptive tiles than in 128x128
+// ones.  Fitted to 15000 launches measured both ways (E 1-64, 2-8192 rows per expert, K 128-28672, M 128-28672, 2e8 to
+// 6e12 operations, operands from HBM, loads that differ by 6 or 30 %).  From 96 rows per expert on it costs 0.9 to
+// 2.4 % against the better side of each, all of them in 128x128 tiles 6 to 27 %, rows_pays alone 2 to 22 %.  Below 96
+// rows an expert's weights bound the launch on either side.  us in 128x128 tiles / in these (rows per expert, K x M,
+// experts): NN 137, 2560 x 10240, 24 389 / 264; 656, 1280 x 1280, 2 18.0 / 24.6; with activation 389, 512 x 14336, 64
+// 924 / 562; 121, 7168 x 256, 8 72 / 101; NT 938, 12544 x 2112, 4 280 / 217; 866, 19968 x 1536, 1 97 / 260; activation
+// backward 386, 6272 x 2688, 60 1210 / 956; 599, 304 x 544, 6 15.8 / 26.4.
+inline bool tall_pays(RowsKind kind, int64_t E, int64_t N, int64_t K, int64_t M, int64_t cus) {
+  const int64_t n = N / (E > 0 ? E : 1);
+  if (n < 96) return false;
+  const TallCosts& c = kTallCosts[kind];
+  const bool glu = kind == ROWS_NN_GLU;
+  const double weights = (double)E * K * M * 2, ops = 2.0 * N * K * M;
+  auto cdiv = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
+  auto most = [](double a, double b) { return a > b ? a : b; };
+
+  const int64_t cols = glu ? cdiv(M / 2, 128) : cdiv(M, 256), stages = 2 * cdiv(K, 64);
+  const int64_t units = over_loads(E, n, [&](int64_t r) { return cdiv(r, 64); });
+  double tall = 0;
+  for (int u = kTallMaxUnits; u >= 2; --u) {
+    const int64_t chunks = over_loads(E, n, [&](int64_t r) { return cdiv(cdiv(r, 64), u); });
+    const int64_t tiles = cdiv(E * chunks * cols, 5), rounds = cdiv(tiles, cus), last = tiles - (rounds - 1) * cus;
+    const double average = (double)units / chunks;
+    const double tile = c.tile + c.unit * average + (c.stage + c.unit_stage * average) * stages;
+    const double t = tile * (rounds - c.lone_gain * (1 - (double)last / cus));
+    if (u == kTallMaxUnits || t < tall) tall = t;
+  }
+  tall = most(most(tall, weights / c.weights), ops / c.ops) + c.launch;
+
+  const int64_t steps = cdiv(K, 64), tiles = cdiv(E * over_loads(E, n, [&](int64_t r) { return cdiv(r, 128); }) * cdiv(M, 128), 5);
+  const int pieces = kind == ROWS_NT_GLU_BWD ? 1 : nn_split_pieces(E, N, K, M);
+  double small;
+  if (pieces > 1) {
+    small = (tiles * pieces > cus ? c.small_pair : c.small_lone) * steps / pieces + c.sums +
+            (double)kSplitNsPerPiece * tiles * pieces;
+  } else {
+    const int64_t rounds = tiles / (2 * cus), rest = tiles % (2 * cus);
+    const double pair = c.small_tile + c.small_pair * steps, lone = c.small_tile + c.small_lone * steps;
+    small = rounds * pair;
+    if (rest > 0) small += rest <= cus ? lone : lone + (pair - lone) * (rest - cus) / cus;
+  }
+  small = most(most(small, weights / c.small_weights), ops / c.small_ops) + c.small_launch;
+  if (glu) small += c.act + (double)N * M * 3 / 4000;  // the activation as a launch of its own
+  return tall < 0.97 * small;
 }
 
 }  // namespace gmoe

@@ -1,0 +1,76 @@
+"""The row-adaptive NN / NT tiles of up to 384 rows at their edges: experts of 0 and 1 rows, of one row more or less
+than whole tiles of 320 and 384 rows and of several, reductions that end inside a round (64) and a stage (32) and are
+shorter than the copies run ahead, columns that end inside a tile; plain, fp32 output, and with the activation and its
+backward fused."""
+import pytest
+import torch
+
+from test_gmm_rows_gpu import on_kernel
+
+pytestmark = pytest.mark.gpu
+
+# rows of the experts, K, F: F columns of d(act), 2 F of the forward
+TALL = [
+    ([0, 1, 319, 320, 321, 383, 384, 385, 0, 640, 767, 769, 1153, 1536, 700, 340], 1160, 904),
+    ([384, 383, 0, 1152, 2305, 65, 1, 768, 769, 2000, 1100, 96, 700, 330, 384, 3000], 520, 520),
+    ([1025, 1023, 1500, 0, 1, 2047, 960, 1024], 136, 1096),
+    ([700, 0, 513, 640, 1, 1280, 961, 705], 2088, 2056),
+]
+
+
+@pytest.mark.parametrize("act", ["silu", "gelu"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,K,F", TALL)
+def test_tall_edges(pkg, dev, dtype, rows, K, F, act):
+    E, N, M = len(rows), sum(rows), 2 * F
+    g = torch.Generator(device=dev).manual_seed(K + F)
+    print("case", dtype, K, F, act, flush=True)
+    off = torch.tensor([0] + rows, device=dev).cumsum(0)
+
+    def rnd(*s, std=1.0):
+        return torch.empty(*s, device=dev).normal_(0.0, std, generator=g).to(dtype)
+
+    a, w1 = rnd(N, K), rnd(E, K, M, std=K ** -0.5)
+    wt = rnd(E, F, K, std=K ** -0.5)
+
+    def here(call):
+        return on_kernel("gmm_rows_kernel", call)
+
+    fc1, h = here(lambda: pkg.ops.gmm_glu(a, w1, off, act))
+    plain = here(lambda: pkg.ops.gmm(a, w1, off))
+    plain32 = here(lambda: pkg.ops.gmm(a, w1, off, out_dtype=torch.float32))
+    dfc1 = here(lambda: pkg.ops.gmm_glu_bwd(a, wt, fc1, off, act))
+    # plain NT of fewer than 768 rows per expert may go elsewhere; its sums have the same order there
+    d = pkg.ops.gmm(a, wt, off, trans_b=True)
+    d32 = pkg.ops.gmm(a, wt, off, trans_b=True, out_dtype=torch.float32)
+    assert torch.equal(fc1, plain) and torch.equal(h, pkg.ops.glu_fwd(fc1, act))
+    assert torch.equal(dfc1, pkg.ops.glu_bwd(d, fc1, act))
+    assert torch.equal(plain, plain32.to(dtype)) and torch.equal(d, d32.to(dtype))
+    # products of 16-bit values are exact in fp32; both sides round up to K additions of partial sums
+    # of size about one (rows of a have norm sqrt(K), columns of w norm one): 2^-24 * sqrt(K) per
+    # element typically, eight times that as the bound, and four times that for the tails of a normal sum
+    tol = 8 * 2.0 ** -24 * K ** 0.5 * 4
+    s = 0
+    for e, n in enumerate(rows):
+        x = a[s:s + n].double()
+        for got, want in ((plain32, x @ w1[e].double()), (d32, x @ wt[e].double().t().contiguous())):
+            err = (got[s:s + n].double() - want).abs().max().item() if n else 0.0
+            assert err < tol, (e, n, err)
+        s += n
+
+
+@pytest.mark.parametrize("K,M", [(8, 2056), (72, 2312), (4104, 2056), (1000, 2304)])
+def test_tall_transposed(pkg, dev, K, M):
+    """Plain NT of 768 rows per expert and more, with reductions of a few elements up to many rounds."""
+    rows = [769, 1, 1537, 0, 2200, 384, 1151, 1300]
+    g = torch.Generator(device=dev).manual_seed(K + M)
+    off = torch.tensor([0] + rows, device=dev).cumsum(0)
+    a = torch.empty(sum(rows), K, device=dev).normal_(generator=g).bfloat16()
+    w = torch.empty(len(rows), M, K, device=dev).normal_(0.0, K ** -0.5, generator=g).bfloat16()
+    got = on_kernel("gmm_rows_kernel", lambda: pkg.ops.gmm(a, w, off, trans_b=True, out_dtype=torch.float32))
+    tol = 8 * 2.0 ** -24 * max(K, 64) ** 0.5 * 4  # as above
+    s = 0
+    for e, n in enumerate(rows):
+        want = a[s:s + n].double() @ w[e].double().t().contiguous()
+        assert n == 0 or (got[s:s + n].double() - want).abs().max().item() < tol, (e, n)
+        s += n

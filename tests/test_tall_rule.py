@@ -1,0 +1,95 @@
+"""Which 16-bit NN / NT launches go to the row-adaptive tiles beyond those of rows_pays, where both sides were measured,
+and the chunks of up to 384 rows (csrc/rows_rule.h)."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+from test_gmm_tall_gpu import TALL
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "hetu-galvatron_amd", "csrc")
+PROGRAM = """
+#define __host__
+#define __device__
+#include "rows_rule.h"
+#include <cstdio>
+int main() {
+  long long v, a, b, c, d;
+  while (std::scanf("%lld %lld %lld %lld %lld", &v, &a, &b, &c, &d) == 5) {
+    if (v >= 0) {
+      std::printf("%d\\n", gmoe::tall_pays((gmoe::RowsKind)v, a, b, c, d, 256));
+      continue;
+    }
+    int u[7] = {};
+    for (int i = 0; i < 7; ++i) if (std::scanf("%d", u + i) != 1) return 1;
+    std::printf("%d\\n", gmoe::rows_chunk_units(u, (int)a, (int)b, c, 1.f));
+  }
+}
+"""
+NN, GLU, NT, GLU_BWD = range(4)
+# kind, experts, rows per expert, K, M, us on 128x128 tiles and on the row-adaptive ones
+MEASURED = [
+    (NN, 8, 363, 512, 5120, 35.1, 28.6), (NN, 24, 137, 2560, 10240, 389, 264), (NN, 24, 5374, 2688, 224, 241, 176),
+    (NN, 32, 941, 768, 128, 18.0, 20.4), (NN, 2, 656, 1280, 1280, 18.0, 24.6), (NN, 4, 1701, 10848, 160, 80.4, 130),
+    (GLU, 32, 208, 128, 512, 16.6, 13.8), (GLU, 64, 389, 512, 14336, 924, 562), (GLU, 4, 1318, 1952, 1504, 60.0, 48.4),
+    (GLU, 4, 103, 768, 1024, 15.8, 19.4), (GLU, 8, 121, 7168, 256, 71.9, 101),
+    (NT, 1, 1185, 1792, 7552, 50.9, 38.3), (NT, 4, 938, 12544, 2112, 280, 217), (NT, 32, 203, 1392, 1968, 80.5, 54.8),
+    (NT, 24, 222, 12256, 192, 83.5, 199), (NT, 4, 1769, 1408, 512, 19.7, 25.5), (NT, 1, 866, 19968, 1536, 97.1, 260),
+    (GLU_BWD, 60, 386, 6272, 2688, 1210, 956), (GLU_BWD, 24, 124, 128, 2560, 30.0, 23.3),
+    (GLU_BWD, 2, 1917, 1888, 3936, 95.1, 69.2), (GLU_BWD, 6, 599, 304, 544, 15.8, 26.4),
+    (GLU_BWD, 4, 322, 4992, 1024, 53.6, 72.7),
+]
+
+
+@pytest.fixture(scope="module")
+def evaluate(tmp_path_factory):
+    if shutil.which("g++") is None:
+        pytest.skip("needs g++")
+    folder = tmp_path_factory.mktemp("rule")
+    (folder / "rule.cpp").write_text(PROGRAM)
+    exe = str(folder / "rule")
+    subprocess.check_call(["g++", "-O2", "-std=c++17", "-Wno-unknown-pragmas", "-I" + CSRC, str(folder / "rule.cpp"), "-o", exe])
+
+    def run(cases):
+        text = "\n".join(" ".join(map(str, c)) for c in cases)
+        out = subprocess.run([exe], input=text, text=True, capture_output=True, check=True).stdout.split()
+        assert len(out) == len(cases)
+        return [int(v) for v in out]
+
+    return run
+
+
+def test_choice(evaluate):
+    got = evaluate([(kind, E, n * E, K, M) for kind, E, n, K, M, _, _ in MEASURED])
+    wrong = [c for c, v in zip(MEASURED, got) if v != (c[6] < c[5])]
+    assert not wrong, wrong
+    # no rows and fewer than 96: never; one expert and a thousand, the smallest and long reductions: an answer
+    shapes = [(E, n, K, M) for E in (1, 8, 1024) for n in (0, 1, 95, 96, 2048, 65536) for K in (8, 512, 65536) for M in (8, 4096)]
+    for kind in (NN, GLU, NT, GLU_BWD):
+        for (E, n, K, M), v in zip(shapes, evaluate([(kind, E, n * E, K, M) for E, n, K, M in shapes])):
+            assert v in (0, 1) and not (v and n < 96), (kind, E, n, K, M)
+
+
+def test_chunks(evaluate):
+    """Chunks of up to 384 rows against the rule in Python, for the edge test on the GPU, which reaches tiles of five and
+    six units (of 64 rows); no rows at all; one tile."""
+    def units(rows):
+        u = [-(-r // 64) for r in rows]
+        return [sum(u), 0] + [sum(-(-x // size) for x in u) for size in range(2, 7)]
+
+    def model(counts, col_tiles, K):
+        best, least = 6, None
+        for size in range(6, 1, -1):
+            chunks = counts[size]
+            cost = -(-chunks * col_tiles // 256) * (16 + 250 / -(-K // 32) + 4 * counts[0] / max(chunks, 1))
+            if least is None or cost < least:
+                best, least = size, cost
+        return best
+
+    edges = [(units(rows), cols, K) for rows, K, F in TALL for cols in (-(-F // 128), -(-F // 256))]
+    other = [(units(rows), cols, K) for rows in ([0, 0], [1], [640] * 16, [256] * 64, [370] * 8, [1024] * 64)
+             for cols in (1, 4, 6, 25) for K in (520, 1024, 5632)]
+    got = evaluate([(-1, cols, 256, K, 0, *counts) for counts, cols, K in edges + other])
+    assert got == [model(*c) for c in edges + other]
+    assert {5, 6} <= set(got[:len(edges)])
