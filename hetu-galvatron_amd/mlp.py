@@ -9,6 +9,8 @@ run as one group on the grouped kernels, optionally on its own stream beside the
 """
 from __future__ import annotations
 
+import contextlib
+
 import torch
 import torch.nn.functional as F
 from torch.nn.parameter import Parameter
@@ -291,9 +293,12 @@ class SharedExpertMLP(torch.nn.Module):
     With `config.moe_shared_expert_overlap` the reference's staged interface is available
     (pre_forward_comm, linear_fc1_forward_and_act, linear_fc2_forward, post_forward_comm,
     get_output): the stages enqueue on a stream of the class, so the dense products run beside
-    the dispatch and the routed experts, and get_output makes the current stream wait for them."""
+    the dispatch and the routed experts, and get_output makes the current stream wait for them.
+    Where the layer's work is too little to pay for the second stream (`_stage_stream`), the stages
+    enqueue on the current one."""
 
     stream = None  # shared by all instances, default priority
+    overlap_min_us = 150.0  # see _stage_stream
 
     def __init__(self, config: MoEConfig, gate: bool = False, device=None):
         super().__init__()
@@ -351,27 +356,51 @@ class SharedExpertMLP(torch.nn.Module):
         return out.view(shape)
 
     # -- staged interface (mlp.py:280-400) ----------------------------------------------------------
+    def _stage_stream(self, x):
+        """The stream of the stages: the side stream or the current one.  The second stream costs the host 80 to 150 us
+        in the forward and 80 in the backward (event records, stream switches, waits between the autograd
+        nodes of two streams), and gains 1 to 19 % of the GPU's time.  So it takes a layer whose forward keeps the
+        GPU busy beyond the launches' own time: its weights at 4.5 TB/s or its products at 800 TFLOP/s (fp32: 120),
+        whichever is longer.  us per step with the side stream / without (estimate): 708 tokens of 192, 32 experts
+        of 512, shared 4336 685 / 520 (5); 8345 of 1408, 8 of 384, top 4, shared 384 843 / 1005 (169); 512 of
+        2048, 64 of 1408, top 6, shared 2816 977 / 999 (248); forward alone 512 of 1024, 16 of 2048, shared 4096 216
+        / 162 (50); 16 of 2048, 64 of 1408, top 6, shared 2816 245 / 269 (248)."""
+        cfg, H = self.config, x.shape[-1]
+        tokens = x.numel() // H if H else 0
+        experts, rows = cfg.num_moe_experts or 0, tokens * (cfg.moe_router_topk or 0)
+        routed, shared = cfg.moe_ffn_hidden_size or 0, cfg.moe_shared_expert_intermediate_size
+        weights = 3.0 * x.element_size() * H * (min(experts, rows) * routed + shared)
+        products = 6.0 * H * (rows * routed + tokens * shared)
+        us = max(weights / 4.5e6, products / (1.2e8 if x.dtype == torch.float32 else 8e8))
+        return SharedExpertMLP.stream if us >= self.overlap_min_us else torch.cuda.current_stream()
+
+    def _stage(self):
+        stream = self._staged["stream"]
+        return contextlib.nullcontext() if stream == torch.cuda.current_stream() else torch.cuda.stream(stream)
+
     def pre_forward_comm(self, input):
         assert self.overlap, "stages out of order"
         # a forward that raised between two stages leaves its pieces behind: start afresh
         self._staged = {}
-        side = SharedExpertMLP.stream
-        side.wait_stream(torch.cuda.current_stream())
-        self._staged = {"shape": input.shape}
-        with torch.cuda.stream(side):
+        stream, cur = self._stage_stream(input), torch.cuda.current_stream()
+        if stream != cur:
+            stream.wait_stream(cur)
+        self._staged = {"shape": input.shape, "stream": stream}
+        with self._stage():
             x = input.reshape(-1, input.shape[-1]).contiguous()
-            x.record_stream(side)
+            if stream != cur:
+                x.record_stream(stream)
             self._staged["x"] = x
             self._staged["score"] = self._gate_score(x) if self.use_shared_expert_gate else None
 
     def linear_fc1_forward_and_act(self, overlapped_comm_output=None):
         assert self.overlap and "x" in self._staged, "stages out of order"
-        with torch.cuda.stream(SharedExpertMLP.stream):
+        with self._stage():
             self._staged["act"] = self._fc1_act(self._staged.pop("x"))
 
     def linear_fc2_forward(self, overlapped_comm_output=None):
         assert self.overlap and "act" in self._staged, "stages out of order"
-        with torch.cuda.stream(SharedExpertMLP.stream):
+        with self._stage():
             self._staged["fc2"] = self.linear_fc2(self._staged.pop("act"))
 
     def post_forward_comm(self):
@@ -379,11 +408,11 @@ class SharedExpertMLP(torch.nn.Module):
 
     def get_output(self):
         assert self.overlap and "fc2" in self._staged, "stages out of order"
-        st = self._staged
+        with self._stage():
+            out = self._finish(self._staged["fc2"], self._staged["score"]).view(self._staged["shape"])
+        stream, cur = self._staged["stream"], torch.cuda.current_stream()
         self._staged = {}
-        with torch.cuda.stream(SharedExpertMLP.stream):
-            out = self._finish(st["fc2"], st["score"]).view(st["shape"])
-        cur = torch.cuda.current_stream()
-        cur.wait_stream(SharedExpertMLP.stream)
-        out.record_stream(cur)
+        if stream != cur:
+            cur.wait_stream(stream)
+            out.record_stream(cur)
         return out
