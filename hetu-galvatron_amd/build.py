@@ -15,7 +15,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB_DIR = os.path.join(HERE, "_lib")
 LIB_PATH = os.path.join(LIB_DIR, "libgalvatron_moe.so")
-SOURCES = ["route.hip", "losses.hip", "capacity.hip", "permute.hip", "glu.hip", "bias.hip", "gmm.hip", "gmm_dtl.hip", "gmm_rows.hip", "gmm_tn.hip", "gmm_f32.hip", "gmm_fp8s.hip", "quant.hip", "norm.hip", "gate.hip", "abi.hip"]
+SOURCES = ["route.hip", "losses.hip", "capacity.hip", "permute.hip", "glu.hip", "bias.hip", "gmm.hip", "gmm_dtl.hip", "gmm_rows.hip", "gmm_rows_f16.hip", "gmm_tn.hip", "gmm_f32.hip", "gmm_fp8s.hip", "quant.hip", "norm.hip", "gate.hip", "abi.hip"]
 
 HOST_SOURCE = "host.cpp"  # the native autograd nodes, a torch extension module
 HOST_PATH = os.path.join(LIB_DIR, "_gmoe_host.so")
@@ -34,7 +34,7 @@ HIPCC_FLAGS = [
 # loop headers of the GEMM kernels on 64-byte boundaries: the Mixtral-shape step 0.4 % faster in the
 # same runs (the dW launches 0.9 %), the other shapes unchanged
 SOURCE_FLAGS = {"gmm.hip": ["-falign-loops=64"], "gmm_dtl.hip": ["-falign-loops=64"],
-                "gmm_rows.hip": ["-falign-loops=64"], "gmm_tn.hip": ["-falign-loops=64"]}
+                "gmm_rows.hip": ["-falign-loops=64"], "gmm_rows_f16.hip": ["-falign-loops=64"], "gmm_tn.hip": ["-falign-loops=64"]}
 
 
 def _hipcc() -> str:

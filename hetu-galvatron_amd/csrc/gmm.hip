@@ -962,7 +962,7 @@ static inline bool gmm_large_tiles(const GmmParams& p, int mode) {
   return p.K >= 512 && p.M >= 256 && experts * ((p.K + 255) / 256) * ((p.M + 255) / 256) >= 129;
 }
 
-// Row-adaptive tiles (gmm_rows.hip) for 16-bit NN / NT: tiles of 64 to 384 rows x 256 columns that share an expert's
+// Row-adaptive tiles (gmm_rows_kernel.h) for 16-bit NN / NT: tiles of 64 to 384 rows x 256 columns that share an expert's
 // rows evenly, one workgroup per CU; the rules with both sides' times are in rows_rule.h.  Launches that could fill
 // 256x256 tiles are 12 to 17 % faster here (us there / here, rows per expert, K x M, experts: with activation 4096, 4096
 // x 28672, 8 6211 / 5836; 1024, 7168 x 4096, 32 1661 / 1525; NN 4096, 14336 x 4096, 8 3023 / 2790; activation backward
@@ -1048,7 +1048,7 @@ static int launch_gmm_split(const GmmParams& p, hipStream_t st) {
 
 // One kernel per (type, mode, size).  Groups large enough for 256x256 tiles (TFLOP/s measured on the
 // Mixtral shape):
-//   NN / NT 16-bit  row-adaptive tiles (gmm_rows.hip);
+//   NN / NT 16-bit  row-adaptive tiles (gmm_rows_kernel.h);
 //   NT 16-bit, short of their rule: both operands k-contiguous, register-staged, 128-byte row pieces, plain LDS reads;
 //   TN 16-bit both operands [k][outer]: LDS-DMA copies of 512-byte rows, 4 stages (1.5 % faster than
 //             the register-staged form);

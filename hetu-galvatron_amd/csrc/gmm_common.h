@@ -256,7 +256,7 @@ int launch_gmm_dtl_tn(const GmmParams& p, int dtype, int out_dtype, hipStream_t 
 // Launches the dW kernel for short reductions (gmm_tn.hip) for 16-bit operands.
 int launch_gmm_tn_short(const GmmParams& p, int dtype, int out_dtype, hipStream_t st);
 
-// Launches the row-adaptive kernel (gmm_rows.hip) for 16-bit operands.
+// Launches the row-adaptive kernel (gmm_rows_kernel.h) for 16-bit operands.
 int launch_gmm_rows(const GmmParams& p, int mode, int dtype, int out_dtype, int epi, hipStream_t st);
 
 // Launches the fp32 kernel on split operands (gmm_f32.hip).

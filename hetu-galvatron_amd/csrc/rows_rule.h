@@ -1,4 +1,4 @@
-// Which 16-bit NN / NT launches go to the row-adaptive tiles (gmm_rows.hip), and into which chunks the kernel cuts an
+// Which 16-bit NN / NT launches go to the row-adaptive tiles (gmm_rows_kernel.h), and into which chunks the kernel cuts an
 // expert's rows.
 #pragma once
 #include "split_rule.h"
@@ -135,42 +135,50 @@ struct TallCosts {
 };
 constexpr TallCosts kTallCosts[] = {
     {4620, 960, 217, 141, 0.31, 4200, 4830, 1.48e6, 3760, 1260, 520, 8700, 6300, 4320, 1e6, 0},
-    {4790, 1580, 260, 133, 0.30, 4400, 4540, 1.495e6, 1470, 1200, 490, 20900, 7700, 4530, 0.8e6, 2700},
+    {3130, 1900, 386, 109, 0.38, 5100, 5700, 1.487e6, 2170, 1180, 500, 22300, 6200, 5540, 0.783e6, 3500},
     {3840, 1140, 223, 144, 0.30, 4100, 4390, 1.41e6, 2860, 1240, 530, 7400, 6900, 4080, 1e6, 0},
     {690, 5880, 294, 127, 0.36, 5200, 4080, 1.487e6, 9950, 1350, 560, 0, 3800, 3640, 1e6, 0}};
 
 // Whether a launch that has too few rows or tiles for 256x256 ones is faster in row-adaptive tiles than in 128x128
 // ones.  Fitted to 15000 launches measured both ways (E 1-64, 2-8192 rows per expert, K 128-28672, M 128-28672, 2e8 to
-// 6e12 operations, operands from HBM, loads that differ by 6 or 30 %).  From 96 rows per expert on it costs 0.9 to
-// 2.4 % against the better side of each, all of them in 128x128 tiles 6 to 27 %, rows_pays alone 2 to 22 %.  Below 96
-// rows an expert's weights bound the launch on either side.  us in 128x128 tiles / in these (rows per expert, K x M,
-// experts): NN 137, 2560 x 10240, 24 389 / 264; 656, 1280 x 1280, 2 18.0 / 24.6; with activation 389, 512 x 14336, 64
-// 924 / 562; 121, 7168 x 256, 8 72 / 101; NT 938, 12544 x 2112, 4 280 / 217; 866, 19968 x 1536, 1 97 / 260; activation
+// 6e12 operations, operands from HBM, loads that differ by 6 or 30 %).  From 96 rows per expert on it costs 0.9 to 2.4
+// % against the better side of each, all of them in 128x128 tiles 6 to 27 %, rows_pays alone 2 to 22 %.  Below 96 rows
+// an expert's weights bound the launch on either side; there only the launch with the activation may come here, which
+// is two on the other tiles (1.9 % against the better side, the other tiles 5.4 %, without the host's time for the
+// second launch), and only where those are not split, which spreads the weights' stream evenly over the CUs.  us in
+// 128x128 tiles / in these (rows per expert, K x M, experts): NN 137, 2560 x 10240, 24 389 / 264; 656, 1280 x 1280, 2
+// 18.0 / 24.6; with activation 389, 512 x 14336, 64 924 / 562; 121, 7168 x 256, 8 72 / 101; 3, 4096 x 28672, 8 317 /
+// 346; 3, 4096 x 14336, 8 176 / 172; NT 938, 12544 x 2112, 4 280 / 217; 866, 19968 x 1536, 1 97 / 260; activation
 // backward 386, 6272 x 2688, 60 1210 / 956; 599, 304 x 544, 6 15.8 / 26.4.
 inline bool tall_pays(RowsKind kind, int64_t E, int64_t N, int64_t K, int64_t M, int64_t cus) {
   const int64_t n = N / (E > 0 ? E : 1);
-  if (n < 96) return false;
-  const TallCosts& c = kTallCosts[kind];
   const bool glu = kind == ROWS_NN_GLU;
+  if (n < (glu ? 1 : 96)) return false;
+  const TallCosts& c = kTallCosts[kind];
   const double weights = (double)E * K * M * 2, ops = 2.0 * N * K * M;
   auto cdiv = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
   auto most = [](double a, double b) { return a > b ? a : b; };
 
   const int64_t cols = glu ? cdiv(M / 2, 128) : cdiv(M, 256), stages = 2 * cdiv(K, 64);
   const int64_t units = over_loads(E, n, [&](int64_t r) { return cdiv(r, 64); });
-  double tall = 0;
+  double tall = 0, idle = 0;
   for (int u = kTallMaxUnits; u >= 2; --u) {
     const int64_t chunks = over_loads(E, n, [&](int64_t r) { return cdiv(cdiv(r, 64), u); });
     const int64_t tiles = cdiv(E * chunks * cols, 5), rounds = cdiv(tiles, cus), last = tiles - (rounds - 1) * cus;
     const double average = (double)units / chunks;
     const double tile = c.tile + c.unit * average + (c.stage + c.unit_stage * average) * stages;
     const double t = tile * (rounds - c.lone_gain * (1 - (double)last / cus));
-    if (u == kTallMaxUnits || t < tall) tall = t;
+    if (u == kTallMaxUnits || t < tall) {
+      tall = t;
+      idle = rounds > 0 ? (1 - (double)last / cus) / rounds : 0;
+    }
   }
-  tall = most(most(tall, weights / c.weights), ops / c.ops) + c.launch;
+  // a last round that is part empty does not stream the weights at the whole chip's rate
+  tall = most(most(tall, weights / c.weights * (1 + 0.6 * idle)), ops / c.ops) + c.launch;
 
   const int64_t steps = cdiv(K, 64), tiles = cdiv(E * over_loads(E, n, [&](int64_t r) { return cdiv(r, 128); }) * cdiv(M, 128), 5);
   const int pieces = kind == ROWS_NT_GLU_BWD ? 1 : nn_split_pieces(E, N, K, M);
+  if (n < 96 && pieces > 1) return false;
   double small;
   if (pieces > 1) {
     small = (tiles * pieces > cus ? c.small_pair : c.small_lone) * steps / pieces + c.sums +
@@ -183,7 +191,7 @@ inline bool tall_pays(RowsKind kind, int64_t E, int64_t N, int64_t K, int64_t M,
   }
   small = most(most(small, weights / c.small_weights), ops / c.small_ops) + c.small_launch;
   if (glu) small += c.act + (double)N * M * 3 / 4000;  // the activation as a launch of its own
-  return tall < 0.97 * small;
+  return tall < (glu ? 1.0 : 0.97) * small;
 }
 
 }  // namespace gmoe
