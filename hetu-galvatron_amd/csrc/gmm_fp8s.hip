@@ -9,9 +9,10 @@
 // third of the MFMA work is padding, and the launch is bound by vector instructions and LDS
 // traffic, not by HBM.  Here the weights are stationary in the other sense: a workgroup owns all
 // rows of an expert (up to 192, in 32-row MFMA fragments; more rows are cut into equal chunks) and a
-// strip of 256 columns, and streams that strip's weights from HBM exactly once.
+// strip of 256 columns, and streams that strip's weights from HBM exactly once.  Where strips of 128 columns find a
+// compute unit each, they are that narrow (launch has the figures).
 //
-//   * 8 wavefronts, two per SIMD: 4 column strips of 64 x 2 halves of the row fragments, so a
+//   * 8 wavefronts, two per SIMD: 4 column strips of 64 (32) x 2 halves of the row fragments, so a
 //     wavefront holds at most 3 x 2 accumulators and everything (results, partial sums, fragments)
 //     lives in the 256 architectural registers a wavefront has at that occupancy: the MFMAs write
 //     them directly and the block-scale fold below is one multiply-add per element, without moves
@@ -24,7 +25,7 @@
 //   * The activations of the expert (bf16) are copied by LDS-DMA as well and shared by the column
 //     strips; a fragment read feeds two MFMAs.
 //   * 3 LDS stages of 64 reduction elements (24 KiB of activations + 16 KiB of weights), two stages
-//     in flight while one is multiplied.  One barrier per stage.
+//     in flight while one is multiplied (4 and three with 8 KiB of weights).  One barrier per stage.
 //   * Block scales stay exact: the products of a stage are accumulated unscaled in a second fp32
 //     accumulator (two 32 x 32 sets, alternating), which is multiplied by the block's scale and
 //     added to the result while the next 32 x 32 block is multiplied.  A 128-element scale block is
@@ -40,25 +41,25 @@ namespace gmoe {
 namespace fp8s {
 
 constexpr int THREADS = 512;                     // 8 wavefronts: 2 row halves x 4 column strips
-constexpr int BN = 256;                          // columns per workgroup, 64 per strip
 constexpr int MAXF = 6;                          // 32-row fragments per row chunk, 3 per row half
 constexpr int MAX_ROWS = MAXF * 32;
 constexpr int BKS = 64;                          // reduction elements per stage
-constexpr int B_BYTES = BN * BKS;                // 16 KiB of weights per stage
-constexpr int B_LOADS = B_BYTES / 1024 / 8;      // LDS-DMA instructions per wavefront and stage: 2
 
 // Stage layout.  A8 = false: bf16 activations, [row pairs][256 bytes], 24 KiB, 3 stages.  A8 = true:
 // fp8 activations, [rows][64 bytes] (16 KiB: the copies come in whole KiB per wavefront, rows past
 // 192 are never read), followed by the rows' power-of-two scales as one dword per row (2 KiB), 4
-// stages.
-template <bool A8>
+// stages.  NJ: column fragments of a wavefront; one leaves LDS for one stage more.
+template <bool A8, int NJ>
 struct Cfg {
+  static constexpr int BN = 128 * NJ;                   // columns per workgroup, 32 * NJ per strip
+  static constexpr int B_BYTES = BN * BKS;              // 16 or 8 KiB of weights per stage
+  static constexpr int B_LOADS = B_BYTES / 1024 / 8;    // LDS-DMA instructions per wavefront and stage: 2 or 1
   static constexpr int A_BYTES = A8 ? 16 * 1024 : MAX_ROWS * BKS * 2;
   static constexpr int A_LOADS = A_BYTES / 1024 / 8;  // per wavefront and stage: 3 (bf16) or 2 (fp8)
   static constexpr int S_BYTES = A8 ? 2048 : 0;
   static constexpr int S_LOADS = A8 ? 1 : 0;
   static constexpr int STAGE_BYTES = A_BYTES + B_BYTES + S_BYTES;
-  static constexpr int NST = A8 ? 4 : 3;
+  static constexpr int NST = (A8 ? 4 : 3) + (NJ == 1 ? 1 : 0);
   static constexpr int AHEAD = NST - 1;                // stages requested ahead of the one multiplied
   static constexpr int LOADS_PER_STAGE = A_LOADS + B_LOADS + S_LOADS;
   static constexpr int FRAG_BYTES = A8 ? 32 * 64 : 4096;  // LDS bytes of a 32-row fragment
@@ -75,34 +76,29 @@ __device__ __forceinline__ void dma4(uint32_t lds_base, uint32_t voff, const u32
                : "memory", "m0");
 }
 
-// Timing probes (results are wrong; the library is built without GMOE_FP8S_PROBE): 1 leaves out the
-// fragment reads, conversions, MFMAs and the scale fold (what the copies alone take), 2 the weight
-// copies after the first two stages, 4 the activation copies after the first two stages, 8 the
-// barrier of a stage.
-#ifndef GMOE_FP8S_PROBE
-#define GMOE_FP8S_PROBE 0
-#endif
-constexpr bool kProbeNoCompute = (GMOE_FP8S_PROBE & 1) != 0;
-constexpr bool kProbeNoWeightCopies = (GMOE_FP8S_PROBE & 2) != 0;
-constexpr bool kProbeNoActivationCopies = (GMOE_FP8S_PROBE & 4) != 0;
-constexpr bool kProbeNoBarrier = (GMOE_FP8S_PROBE & 8) != 0;   // with 2 and 4: no barrier per stage
-
 // Row chunks of an expert with n rows: equal parts of at most MAX_ROWS rows, multiples of 32.
 __device__ __forceinline__ int chunks_of(long long n) { return (int)((n + MAX_ROWS - 1) / MAX_ROWS); }
 __device__ __forceinline__ int chunk_rows(long long n, int chunks) {
   return (int)(((n + chunks - 1) / chunks + 31) / 32 * 32);
 }
 
+// NN: where the 32-byte segments of a weight row are swapped to, so that the 8 rows x 32 bytes of one transposing
+// read lie in different banks: a row of 256 bytes covers all of them, one of 128 bytes half.
+template <int NJ>
+__device__ __forceinline__ int seg_swizzle(int krow) {
+  return NJ == 2 ? krow & 7 : (krow >> 1) & 3;
+}
+
 // What a lane needs to issue its copies and read its fragments; set up once per item.
-template <bool NT, bool A8>
+template <bool NT, bool A8, int NJ>
 struct Lane {
   u32x4 rsrc_a, rsrc_b, rsrc_s;
-  uint32_t voff_a[Cfg<A8>::A_LOADS], voff_b[B_LOADS];  // byte offsets of this lane's copies of stage 0
+  uint32_t voff_a[Cfg<A8, NJ>::A_LOADS], voff_b[Cfg<A8, NJ>::B_LOADS];  // byte offsets of this lane's copies of stage 0
   uint32_t voff_s;            // A8: this lane's dword of the activation scales
   uint32_t b_kstep;           // bytes a stage advances in the weight operand
   uint32_t s_kstep;           // A8: bytes a 128-element block advances in the scale table
   uint32_t a_off[4];          // fragment read offsets inside a stage: bf16 per K step; fp8 the two 16-byte halves
-  uint32_t b_off[2];          // NT: per K-step pair (fp8: per half); NN: per column fragment
+  uint32_t b_off[2];          // NT: per K-step pair (fp8: per half); NN: per column fragment of NJ
 };
 
 // The block scales of one item's reduction for this wavefront's column strip, kept in registers: lane
@@ -113,54 +109,91 @@ struct StripScales {
   float r[kScaleRegs];
   __device__ __forceinline__ float at(int kt) const {  // kt: 64-element stage
     const int kb = kt >> 1;
-    float v = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, r[0]), kb & 63));
+    int v = __builtin_amdgcn_readlane(__builtin_bit_cast(int, r[0]), kb & 63);
 #pragma unroll
     for (int q = 1; q < kScaleRegs; ++q) {
-      const float w = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, r[q]), kb & 63));
+      const int w = __builtin_amdgcn_readlane(__builtin_bit_cast(int, r[q]), kb & 63);
       v = (kb >> 6) == q ? w : v;
     }
-    return v;
+    return __builtin_bit_cast(float, v);
   }
 };
 
-// One stage's copies of this wavefront: 3 KiB of activations (rows past the chunk read zeros and
-// cost no memory traffic) and 2 KiB of weights.
 __device__ __forceinline__ u32x4 uniform_rsrc(const u32x4& r) {
   return u32x4{(uint32_t)__builtin_amdgcn_readfirstlane(r[0]), (uint32_t)__builtin_amdgcn_readfirstlane(r[1]),
                (uint32_t)__builtin_amdgcn_readfirstlane(r[2]), (uint32_t)__builtin_amdgcn_readfirstlane(r[3])};
 }
-template <bool NT, bool A8>
-__device__ __forceinline__ void issue_stage(uint32_t lds0, const Lane<NT, A8>& ln, int wave, int kt) {
-  using C = Cfg<A8>;
-  const uint32_t st = lds0 + (uint32_t)((kt % C::NST) * C::STAGE_BYTES);
-  // the resources are wavefront-uniform; the copies take them in scalar registers
-  const u32x4 rsrc_a = uniform_rsrc(ln.rsrc_a), rsrc_b = uniform_rsrc(ln.rsrc_b);
-  const uint32_t b_kstep = __builtin_amdgcn_readfirstlane(ln.b_kstep);
+// bf16 activations: where the next stage's copies go and come from, carried from stage to stage.  Stages past the
+// reduction are requested too: at the resource's end.  (Everything in scalar registers, and computed under the
+// MFMAs: 4096 rows x 7168 x 4096 over 30 experts 335 -> 320 us.  Stages of fp8 activations are shorter and gain
+// nothing; there the copies are placed from the stage's number.)
+template <int NJ>
+struct Ahead {
+  u32x4 rsrc_a, rsrc_b;
+  uint32_t b_kstep;
+  uint32_t stage = 0, off_a = 0, off_b = 0;
+
+  template <bool NT>
+  __device__ __forceinline__ explicit Ahead(const Lane<NT, false, NJ>& ln)
+      : rsrc_a(uniform_rsrc(ln.rsrc_a)), rsrc_b(uniform_rsrc(ln.rsrc_b)),
+        b_kstep(__builtin_amdgcn_readfirstlane(ln.b_kstep)) {}
+  // off and step are below 2 GiB
+  static __device__ __forceinline__ uint32_t further(uint32_t bytes, uint32_t off, uint32_t step) {
+    return off + step < bytes ? off + step : bytes;
+  }
+  __device__ __forceinline__ void advance() {
+    using C = Cfg<false, NJ>;
+    off_a = further(rsrc_a[2], off_a, BKS * 2);
+    off_b = further(rsrc_b[2], off_b, b_kstep);
+    stage = stage == (C::NST - 1) * C::STAGE_BYTES ? 0 : stage + C::STAGE_BYTES;
+  }
+};
+
+// One stage's copies of this wavefront: 3 KiB of activations (rows past the chunk read zeros and
+// cost no memory traffic) and 2 KiB of weights (strips of 256).
+template <bool NT, int NJ>
+__device__ __forceinline__ void issue_stage(uint32_t lds0, const Lane<NT, false, NJ>& ln, int wave, const Ahead<NJ>& at) {
+  using C = Cfg<false, NJ>;
+  const uint32_t st = lds0 + at.stage;
   static_for<0, C::A_LOADS>([&](auto t_c) {
     constexpr int t = decltype(t_c)::value;
-    const uint32_t voff = (kProbeNoActivationCopies && kt > 1) ? kOob : ln.voff_a[t];
-    dma16(st + (uint32_t)((wave * C::A_LOADS + t) * 1024), voff, rsrc_a, (uint32_t)(kt * (A8 ? BKS : BKS * 2)));
+    dma16(st + (uint32_t)((wave * C::A_LOADS + t) * 1024), ln.voff_a[t], at.rsrc_a, at.off_a);
   });
-  static_for<0, B_LOADS>([&](auto t_c) {
+  static_for<0, C::B_LOADS>([&](auto t_c) {
     constexpr int t = decltype(t_c)::value;
-    const uint32_t voff = (kProbeNoWeightCopies && kt > 1) ? kOob : ln.voff_b[t];
-    dma16(st + C::A_BYTES + (uint32_t)((wave * B_LOADS + t) * 1024), voff, rsrc_b, (uint32_t)kt * b_kstep);
+    dma16(st + C::A_BYTES + (uint32_t)((wave * C::B_LOADS + t) * 1024), ln.voff_b[t], at.rsrc_b, at.off_b);
   });
-  if constexpr (A8) {
-    // the scales of the 128-element block the stage belongs to, one dword per row
-    const u32x4 rsrc_s = uniform_rsrc(ln.rsrc_s);
-    const uint32_t s_kstep = __builtin_amdgcn_readfirstlane(ln.s_kstep);
-    dma4(st + C::A_BYTES + B_BYTES + (uint32_t)(wave * 256), ln.voff_s, rsrc_s, (uint32_t)(kt >> 1) * s_kstep);
-  }
+}
+// The same for fp8 activations (2 KiB), and the scales of the 128-element block the stage belongs to, one dword per
+// row.
+template <bool NT, int NJ>
+__device__ __forceinline__ void issue_stage(uint32_t lds0, const Lane<NT, true, NJ>& ln, int wave, int kt) {
+  using C = Cfg<true, NJ>;
+  const uint32_t st = lds0 + (uint32_t)((kt % C::NST) * C::STAGE_BYTES);
+  // the resources are wavefront-uniform; the copies take them in scalar registers
+  const u32x4 rsrc_a = uniform_rsrc(ln.rsrc_a), rsrc_b = uniform_rsrc(ln.rsrc_b), rsrc_s = uniform_rsrc(ln.rsrc_s);
+  const uint32_t b_kstep = __builtin_amdgcn_readfirstlane(ln.b_kstep);
+  const uint32_t s_kstep = __builtin_amdgcn_readfirstlane(ln.s_kstep);
+  const uint32_t off_a = stage_offset(rsrc_a[2], (uint32_t)kt, BKS), off_b = stage_offset(rsrc_b[2], (uint32_t)kt, b_kstep);
+  static_for<0, C::A_LOADS>([&](auto t_c) {
+    constexpr int t = decltype(t_c)::value;
+    dma16(st + (uint32_t)((wave * C::A_LOADS + t) * 1024), ln.voff_a[t], rsrc_a, off_a);
+  });
+  static_for<0, C::B_LOADS>([&](auto t_c) {
+    constexpr int t = decltype(t_c)::value;
+    dma16(st + C::A_BYTES + (uint32_t)((wave * C::B_LOADS + t) * 1024), ln.voff_b[t], rsrc_b, off_b);
+  });
+  dma4(st + C::A_BYTES + C::B_BYTES + (uint32_t)(wave * 256), ln.voff_s, rsrc_s,
+       stage_offset(rsrc_s[2], (uint32_t)(kt >> 1), s_kstep));
 }
 
 // The reduction of one item; its stages 0 and 1 have been requested by the caller.
-template <bool NT, int NF>
-__device__ __forceinline__ void run_item(unsigned char* lds, uint32_t lds0, const Lane<NT, false>& ln,
-                                         const StripScales& scale, int kt_cnt, int wave, int frag0,
-                                         f32x16 (&acc)[NF > 0 ? NF : 1][2]) {
-  constexpr int NST = Cfg<false>::NST, STAGE_BYTES = Cfg<false>::STAGE_BYTES, A_BYTES = Cfg<false>::A_BYTES;
-  constexpr int LOADS_PER_STAGE = Cfg<false>::LOADS_PER_STAGE;
+template <bool NT, int NF, int NJ>
+__device__ __forceinline__ void run_item(unsigned char* lds, uint32_t lds0, const Lane<NT, false, NJ>& ln,
+                                         const StripScales& scale, int kt_cnt, int wave, int frag0, Ahead<NJ>& at,
+                                         f32x16 (&acc)[NF > 0 ? NF : 1][NJ]) {
+  using C = Cfg<false, NJ>;
+  constexpr int A_BYTES = C::A_BYTES;
   const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 
   // Software pipeline of a stage, in program order (pinned with scheduling fences).  The unit of work
@@ -171,22 +204,29 @@ __device__ __forceinline__ void run_item(unsigned char* lds, uint32_t lds0, cons
   // always uses set j.  The weight fragments are widened just before the first blocks need them;
   // the A fragment of a K step is refilled with the next row fragment's as soon as both MFMAs that
   // read it have been issued.
-  u32x4 bf[4][2];
+  u32x4 bf[4][NJ];
   u32x4 fa[4];
   f32x16 accq[2];
   accq[0] = accq[1] = zero;
   float sc_prev = 0.f;  // scale of the pending partial sums (none before the first stage)
 
+  uint32_t here = 0, there = 0;  // the stage's place in LDS, the next one's
+  float sc_next = 0.f;
+  auto prepare = [&](int kt) {  // the next stage's scalar work, under the MFMAs
+    at.advance();
+    there = here == (C::NST - 1) * C::STAGE_BYTES ? 0 : here + C::STAGE_BYTES;
+    sc_next = scale.at(kt + 1);
+  };
   auto stage = [&](int kt, float sc) {
-    const unsigned char* sa = lds + (kt % NST) * STAGE_BYTES + frag0 * 4096;
-    const unsigned char* sb = lds + (kt % NST) * STAGE_BYTES + A_BYTES;
+    const unsigned char* sa = lds + here + frag0 * 4096;
+    const unsigned char* sb = lds + here + A_BYTES;
     // raw weight fragments: NT 16 bytes = K steps 2*kp, 2*kp+1 of column fragment j; NN 8 bytes per
     // (K step, column fragment) through the transposing read
-    u32x4 raw_nt[2][2];
-    i32x2 raw_nn[4][2];
+    u32x4 raw_nt[2][NJ];
+    i32x2 raw_nn[4][NJ];
     auto read_raw = [&](auto part_c) {  // part 0: K steps 0,1; part 1: K steps 2,3
       constexpr int part = decltype(part_c)::value;
-      static_for<0, 2>([&](auto j_c) {
+      static_for<0, NJ>([&](auto j_c) {
         constexpr int j = decltype(j_c)::value;
         if constexpr (NT) {
           raw_nt[part][j] = *reinterpret_cast<const u32x4*>(sb + ln.b_off[part] + j * 2048);
@@ -194,7 +234,7 @@ __device__ __forceinline__ void run_item(unsigned char* lds, uint32_t lds0, cons
           static_for<0, 2>([&](auto q_c) {
             constexpr int ks = 2 * part + decltype(q_c)::value;
             raw_nn[ks][j] = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
-                (__attribute__((address_space(3))) i32x2*)(lds_byte*)(sb + ln.b_off[j] + ks * 4096));
+                (__attribute__((address_space(3))) i32x2*)(lds_byte*)(sb + ln.b_off[j] + ks * 16 * C::BN));
           });
         }
       });
@@ -221,10 +261,14 @@ __device__ __forceinline__ void run_item(unsigned char* lds, uint32_t lds0, cons
     GMOE_SCHED_FENCE();
     static_for<0, NF>([&](auto i_c) {
       constexpr int i = decltype(i_c)::value;
-      static_for<0, 2>([&](auto j_c) {
+      static_for<0, NJ>([&](auto j_c) {
         constexpr int j = decltype(j_c)::value;
-        // the block whose partial sums are pending in set 1 - j
-        constexpr int pi = j == 1 ? i : (i == 0 ? NF - 1 : i - 1), pj = 1 - j;
+        // The block whose partial sums are pending in the other set.  With one column fragment a stage may have an
+        // odd number of blocks: the last one is then folded at the stage's end, and nothing is pending before the
+        // first.
+        constexpr int set = NJ == 2 ? j : i & 1;
+        constexpr int pi = j == 1 ? i : (i == 0 ? NF - 1 : i - 1), pj = NJ - 1 - j;
+        constexpr bool pending = NJ == 2 || i > 0;
         const float fs = (i == 0 && j == 0) ? sc_prev : sc;
         static_for<0, 4>([&](auto ks_c) {
           constexpr int ks = decltype(ks_c)::value;
@@ -234,38 +278,45 @@ __device__ __forceinline__ void run_item(unsigned char* lds, uint32_t lds0, cons
           }
           // the first product of a stage takes C = 0 (an inline constant of the instruction)
           if constexpr (ks == 0)
-            accq[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            accq[set] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
                 __builtin_bit_cast(bf16x8, bf[ks][j]), __builtin_bit_cast(bf16x8, fa[ks]), zero, 0, 0, 0);
           else
-            Mma<GMOE_BF16>::run(fa[ks], bf[ks][j], accq[j]);
+            Mma<GMOE_BF16>::run(fa[ks], bf[ks][j], accq[set]);
           GMOE_SCHED_FENCE();
+          if constexpr (i == 0 && j == 0 && ks == 0) prepare(kt);
+          if constexpr (pending)
 #pragma unroll
-          for (int v = 4 * ks; v < 4 * ks + 4; ++v) acc[pi][pj][v] = fmaf(fs, accq[pj][v], acc[pi][pj][v]);
-          // both MFMAs that read this K step's A fragment have been issued: refill it with the next
+            for (int v = 4 * ks; v < 4 * ks + 4; ++v) acc[pi][pj][v] = fmaf(fs, accq[1 - set][v], acc[pi][pj][v]);
+          // the last MFMA that reads this K step's A fragment has been issued: refill it with the next
           // row fragment's, 4 MFMAs before that is needed
-          if constexpr (j == 1 && i + 1 < NF)
+          if constexpr (j == NJ - 1 && i + 1 < NF)
             fa[ks] = *reinterpret_cast<const u32x4*>(sa + ln.a_off[ks] + (i + 1) * 4096);
           GMOE_SCHED_FENCE();
         });
       });
     });
+    if constexpr (NJ == 1) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[NF - 1][0][v] = fmaf(sc, accq[(NF - 1) & 1][v], acc[NF - 1][0][v]);
+    }
     sc_prev = sc;
   };
 
   float sc = scale.at(0);
   for (int kt = 0; kt < kt_cnt; ++kt) {
-    // stage kt has landed (stage kt+1 may still be in flight); after the barrier every wavefront
+    // stage kt has landed (those after it may still be in flight); after the barrier every wavefront
     // sees it and has finished with stage kt-1, whose buffer the next copies overwrite.  Copies
     // past the reduction read zeros: the count of outstanding copies stays the same to the end.
-    wait_dma_outstanding<LOADS_PER_STAGE>();
-    if constexpr (!kProbeNoBarrier) __syncthreads();
-    issue_stage<NT, false>(lds0, ln, wave, kt + 2);
-    const float sc_next = scale.at(kt + 1);
-    if constexpr (!kProbeNoCompute && NF > 0) stage(kt, sc);
+    wait_dma_outstanding<(C::AHEAD - 1) * C::LOADS_PER_STAGE>();
+    __syncthreads();
+    issue_stage<NT, NJ>(lds0, ln, wave, at);
+    if constexpr (NF > 0) stage(kt, sc);
+    if constexpr (NF == 0) at.advance();
+    here = there;
     sc = sc_next;
   }
   // the last block's partial sums (zero, with scale zero, when the reduction is empty)
-  if constexpr (NF > 0) {
+  if constexpr (NF > 0 && NJ == 2) {
 #pragma unroll
     for (int v = 0; v < 16; ++v) acc[NF - 1][1][v] = fmaf(sc_prev, accq[1][v], acc[NF - 1][1][v]);
   }
@@ -276,11 +327,11 @@ __device__ __forceinline__ void run_item(unsigned char* lds, uint32_t lds0, cons
 // widening), with the rows' power-of-two scales as the instruction's scale operand (exact: an
 // exponent adjustment) and ones for the weights, whose bf16 block scales are applied by the fold as
 // before.  Stages 0 .. 2 have been requested by the caller.
-template <bool NT, int NF>
-__device__ __forceinline__ void run_item(unsigned char* lds, uint32_t lds0, const Lane<NT, true>& ln,
+template <bool NT, int NF, int NJ>
+__device__ __forceinline__ void run_item(unsigned char* lds, uint32_t lds0, const Lane<NT, true, NJ>& ln,
                                          const StripScales& scale, int kt_cnt, int wave, int frag0,
-                                         f32x16 (&acc)[NF > 0 ? NF : 1][2]) {
-  using C = Cfg<true>;
+                                         f32x16 (&acc)[NF > 0 ? NF : 1][NJ]) {
+  using C = Cfg<true, NJ>;
   const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   constexpr int kOnes = 0x7f7f7f7f;  // E8M0 1.0 in every byte
   f32x16 accq[2];
@@ -291,8 +342,8 @@ __device__ __forceinline__ void run_item(unsigned char* lds, uint32_t lds0, cons
     const unsigned char* st = lds + (kt % C::NST) * C::STAGE_BYTES;
     const unsigned char* sa = st + frag0 * C::FRAG_BYTES;
     const unsigned char* sb = st + C::A_BYTES;
-    const int* ss = reinterpret_cast<const int*>(st + C::A_BYTES + B_BYTES) + frag0 * 32 + (threadIdx.x & 31);
-    i32x8 fb[2], fa[2];
+    const int* ss = reinterpret_cast<const int*>(st + C::A_BYTES + C::B_BYTES) + frag0 * 32 + (threadIdx.x & 31);
+    i32x8 fb[NJ], fa[2];
     int sa_e8[NF > 0 ? NF : 1];
     auto read_a = [&](auto i_c) {
       constexpr int i = decltype(i_c)::value;
@@ -300,7 +351,7 @@ __device__ __forceinline__ void run_item(unsigned char* lds, uint32_t lds0, cons
       const u32x4 hi = *reinterpret_cast<const u32x4*>(sa + ln.a_off[1] + i * C::FRAG_BYTES);
       fa[i & 1] = i32x8{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
     };
-    static_for<0, 2>([&](auto j_c) {
+    static_for<0, NJ>([&](auto j_c) {
       constexpr int j = decltype(j_c)::value;
       if constexpr (NT) {
         const u32x4 lo = *reinterpret_cast<const u32x4*>(sb + ln.b_off[0] + j * 2048);
@@ -311,7 +362,7 @@ __device__ __forceinline__ void run_item(unsigned char* lds, uint32_t lds0, cons
         static_for<0, 4>([&](auto q_c) {
           constexpr int qq = decltype(q_c)::value;
           q[qq] = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
-              (__attribute__((address_space(3))) i32x2*)(lds_byte*)(sb + ln.b_off[j] + qq * 2048));
+              (__attribute__((address_space(3))) i32x2*)(lds_byte*)(sb + ln.b_off[j] + qq * 8 * C::BN));
         });
         fb[j] = i32x8{q[0][0], q[0][1], q[1][0], q[1][1], q[2][0], q[2][1], q[3][0], q[3][1]};
       }
@@ -323,20 +374,26 @@ __device__ __forceinline__ void run_item(unsigned char* lds, uint32_t lds0, cons
     static_for<0, NF>([&](auto i_c) {
       constexpr int i = decltype(i_c)::value;
       if constexpr (i + 1 < NF) read_a(std::integral_constant<int, i + 1>{});
-      static_for<0, 2>([&](auto j_c) {
+      static_for<0, NJ>([&](auto j_c) {
         constexpr int j = decltype(j_c)::value;
-        constexpr int pi = j == 1 ? i : (i == 0 ? NF - 1 : i - 1), pj = 1 - j;
+        constexpr int set = NJ == 2 ? j : i & 1;
+        constexpr int pi = j == 1 ? i : (i == 0 ? NF - 1 : i - 1), pj = NJ - 1 - j;
         const float fs = (i == 0 && j == 0) ? sc_prev : sc;
         // first operand: the weights' columns (scale one); second: the rows with their scale, so
         // that a lane ends up with 4 consecutive columns of one row, as in the bf16 kernels
-        accq[j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fb[j], fa[i & 1], zero, 0, 0, 0, kOnes, 0,
+        accq[set] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fb[j], fa[i & 1], zero, 0, 0, 0, kOnes, 0,
                                                                   sa_e8[i]);
         GMOE_SCHED_FENCE();
+        if constexpr (NJ == 2 || i > 0)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) acc[pi][pj][v] = fmaf(fs, accq[pj][v], acc[pi][pj][v]);
+          for (int v = 0; v < 16; ++v) acc[pi][pj][v] = fmaf(fs, accq[1 - set][v], acc[pi][pj][v]);
         GMOE_SCHED_FENCE();
       });
     });
+    if constexpr (NJ == 1) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[NF - 1][0][v] = fmaf(sc, accq[(NF - 1) & 1][v], acc[NF - 1][0][v]);
+    }
     sc_prev = sc;
   };
 
@@ -345,21 +402,22 @@ __device__ __forceinline__ void run_item(unsigned char* lds, uint32_t lds0, cons
     // stage kt has landed (stages kt+1, kt+2 may still be in flight); after the barrier every
     // wavefront has finished with stage kt-1, whose buffer the next copies overwrite
     wait_dma_outstanding<(C::AHEAD - 1) * C::LOADS_PER_STAGE>();
-    if constexpr (!kProbeNoBarrier) __syncthreads();
-    issue_stage<NT, true>(lds0, ln, wave, kt + C::AHEAD);
+    __syncthreads();
+    issue_stage<NT, NJ>(lds0, ln, wave, kt + C::AHEAD);
     const float sc_next = scale.at(kt + 1);
-    if constexpr (!kProbeNoCompute && NF > 0) stage(kt, sc);
+    if constexpr (NF > 0) stage(kt, sc);
     sc = sc_next;
   }
-  if constexpr (NF > 0) {
+  if constexpr (NF > 0 && NJ == 2) {
 #pragma unroll
     for (int v = 0; v < 16; ++v) acc[NF - 1][1][v] = fmaf(sc_prev, accq[1][v], acc[NF - 1][1][v]);
   }
 }
 
-template <bool NT, bool A8>
+template <bool NT, bool A8, int NJ>
 __global__ __launch_bounds__(THREADS, 1) void gmm_fp8_skinny_kernel(GmmParams p) {
-  using C = Cfg<A8>;
+  using C = Cfg<A8, NJ>;
+  constexpr int BN = C::BN, B_LOADS = C::B_LOADS, STRIP = 32 * NJ;
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
   __shared__ int item_cum[kMaxGroupsLds + 1];          // exclusive prefix of items over `order`
   __shared__ unsigned short order[kMaxGroupsLds];      // experts by ascending rows per chunk
@@ -432,10 +490,11 @@ __global__ __launch_bounds__(THREADS, 1) void gmm_fp8_skinny_kernel(GmmParams p)
     if (tid == THREADS - 1) item_cum[E] = run;
   }
   __syncthreads();
-  const long long total = item_cum[E];
+  // (not in a scalar register with fp8 activations: 4 % slower there)
+  const int total = A8 ? item_cum[E] : __builtin_amdgcn_readfirstlane(item_cum[E]);
 
   // Lane geometry that does not depend on the item.
-  Lane<NT, A8> ln;
+  Lane<NT, A8, NJ> ln;
   if constexpr (A8) {
     // fp8 activations [row][64 bytes]: 16-byte unit u of row r at unit u ^ ((r >> 2) & 3); a lane
     // supplies the 32 reduction elements 32*h .. 32*h + 31 of its row (units 2*h, 2*h + 1) to the
@@ -449,13 +508,13 @@ __global__ __launch_bounds__(THREADS, 1) void gmm_fp8_skinny_kernel(GmmParams p)
     if (NT) {
 #pragma unroll
       for (int q = 0; q < 2; ++q)
-        ln.b_off[q] = (uint32_t)((64 * cs + r) * 64 + (((2 * h + q) ^ ((r >> 2) & 3)) << 4));
+        ln.b_off[q] = (uint32_t)((STRIP * cs + r) * 64 + (((2 * h + q) ^ ((r >> 2) & 3)) << 4));
     } else {
       // four transposing reads of 8 k rows each: k rows 32*h + 8*q + t, t = 0 .. 7
       const int i16 = lane & 15, g16 = (lane >> 4) & 1;
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
-        ln.b_off[j] = (uint32_t)((32 * h + (i16 >> 1)) * 256 + (((2 * cs + j) ^ (i16 >> 1)) << 5) +
+      for (int j = 0; j < NJ; ++j)
+        ln.b_off[j] = (uint32_t)((32 * h + (i16 >> 1)) * BN + (((NJ * cs + j) ^ seg_swizzle<NJ>(i16 >> 1)) << 5) +
                                  16 * g16 + 8 * (i16 & 1));
     }
   } else {
@@ -475,14 +534,14 @@ __global__ __launch_bounds__(THREADS, 1) void gmm_fp8_skinny_kernel(GmmParams p)
       const int cl = lane & 31;
 #pragma unroll
       for (int kp = 0; kp < 2; ++kp)
-        ln.b_off[kp] = (uint32_t)((64 * cs + cl) * 64 + (((2 * kp + h) ^ ((cl >> 2) & 3)) << 4));
+        ln.b_off[kp] = (uint32_t)((STRIP * cs + cl) * 64 + (((2 * kp + h) ^ ((cl >> 2) & 3)) << 4));
     } else {
-      // weights [k row][256 bytes]: 32-byte segment sg of row k at segment sg ^ (k & 7); lanes 2t,
+      // weights [k row][BN bytes]: 32-byte segment sg of row k at segment sg ^ seg_swizzle(k); lanes 2t,
       // 2t+1 of a group of 16 address the two halves of k row t of an 8 x 16 block
       const int i16 = lane & 15, g16 = (lane >> 4) & 1;
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
-        ln.b_off[j] = (uint32_t)((8 * h + (i16 >> 1)) * 256 + (((2 * cs + j) ^ (i16 >> 1)) << 5) +
+      for (int j = 0; j < NJ; ++j)
+        ln.b_off[j] = (uint32_t)((8 * h + (i16 >> 1)) * BN + (((NJ * cs + j) ^ seg_swizzle<NJ>(i16 >> 1)) << 5) +
                                  16 * g16 + 8 * (i16 & 1));
     }
   }
@@ -504,16 +563,20 @@ __global__ __launch_bounds__(THREADS, 1) void gmm_fp8_skinny_kernel(GmmParams p)
   // items.  An XCD takes the runs of its workgroups together and deals them round-robin: at any time
   // its workgroups work on consecutive items, the column strips of one or two experts, so its L2
   // holds those experts' activations for all of them and neighbouring weight columns are streamed
-  // together.
-  const long long q_items = total / G, r_items = total % G;
-  auto run_begin = [&](long long w) {
-    return w < r_items ? w * (q_items + 1) : r_items * (q_items + 1) + (w - r_items) * q_items;
-  };
-  const long long first = run_begin((long long)xcd * per_xcd) + slot;
-  const long long last = run_begin((long long)(xcd + 1) * per_xcd);
+  // together.  (The whole rounds first and the rest spread over all XCDs: 4096 rows x 4096 x 7168, 30 experts, NT
+  // 320 -> 346 us.)
+  // Less than a round is spread over all XCDs.  Where one then has several workgroups per (narrow) item, these take
+  // some of the item's row fragments each, side by side, so that the weights come from HBM once.  (In the kernel of
+  // wide strips, where that hardly occurs, the code alone costs 5 % with fp8 activations.)
+  const int q_items = total / G, r_items = total % G;
+  auto run_begin = [&](int w) { return w * q_items + (w < r_items ? w : r_items); };
+  const bool spread = q_items == 0;
+  const int first = spread ? total * xcd / 8 : run_begin(xcd * per_xcd);
+  const int last = spread ? total * (xcd + 1) / 8 : run_begin((xcd + 1) * per_xcd);
+  const int pieces = NJ == 1 && spread && last > first ? per_xcd / (last - first) : 1;  // >= 1: total < G
   int pos = 0;
-  // Item `v` of this workgroup's run: fills the copy addresses and requests the block scales.
-  auto setup = [&](long long v, Item& it) -> bool {
+  // Item `v` of this workgroup's: fills the copy addresses and requests the block scales.
+  auto setup = [&](int v, Item& it) -> bool {
     if (v >= last) return false;
     while (item_cum[pos + 1] <= v) ++pos;
     pos = __builtin_amdgcn_readfirstlane(pos);
@@ -521,11 +584,19 @@ __global__ __launch_bounds__(THREADS, 1) void gmm_fp8_skinny_kernel(GmmParams p)
     const long long row_e = group_begin(p, e);
     const long long n_e = group_begin(p, e + 1) - row_e;
     const int nch = chunks_of(n_e);
-    const int q = (int)(v - item_cum[pos]);
+    const int q = v - item_cum[pos];
     const int ct = q / nch, ch = q % nch;
     const int per = chunk_rows(n_e, nch);
-    const long long r0 = (long long)ch * per;
-    const int rows = (int)(n_e - r0 < per ? n_e - r0 : per);  // >= 1: chunks are never empty
+    long long r0 = (long long)ch * per;
+    int rows = (int)(n_e - r0 < per ? n_e - r0 : per);  // >= 1: chunks are never empty
+    if (NJ == 1 && pieces > 1) {
+      // two row fragments and more each: one for each of the two wavefronts of a column strip
+      const int frags = (rows + 31) / 32, most = (frags + 1) / 2, cut = pieces < most ? pieces : most;
+      const int part = (frags + cut - 1) / cut * 32, from = slot % pieces * part;
+      if (from >= rows) return false;
+      r0 += from;
+      rows = rows - from < part ? rows - from : part;
+    }
     // the chunk's nf row fragments are split between the two wavefronts of a column strip: the
     // first takes the first ceil(nf / 2), the second the rest (none when nf = 1: it then only copies)
     const int nf = (rows + 31) / 32;
@@ -565,8 +636,8 @@ __global__ __launch_bounds__(THREADS, 1) void gmm_fp8_skinny_kernel(GmmParams p)
       }
     }
     if (NT) {
-      // weights [M,K]: copy t of wavefront w fills block 2*w + t: columns 16*(2*w + t) .. + 15,
-      // lane L the 16-byte unit (L % 4) ^ ((col >> 2) & 3) of column 16*(2*w + t) + L / 4
+      // weights [M,K]: copy t of wavefront w fills block NJ*w + t: columns 16*(NJ*w + t) .. + 15,
+      // lane L the 16-byte unit (L % 4) ^ ((col >> 2) & 3) of column 16*(NJ*w + t) + L / 4
       const int64_t cols = M - col0 < BN ? M - col0 : BN;
       ln.rsrc_b = make_raw_rsrc(p.b + ((int64_t)e * M + col0) * K, cols * K);
 #pragma unroll
@@ -576,20 +647,21 @@ __global__ __launch_bounds__(THREADS, 1) void gmm_fp8_skinny_kernel(GmmParams p)
       }
       ln.b_kstep = BKS;
     } else {
-      // weights [K,M]: block 2*w + t holds k rows 4*(2*w + t) .. + 3, lane L the 16-byte unit U of
-      // its row with U = (((L%16) >> 1) ^ (krow & 7)) << 1 | (L & 1)
+      // weights [K,M]: block NJ*w + t holds 1 KiB of k rows, BN / 16 lanes each: unit L % (BN / 16) of a row the
+      // 16 bytes U of it with U = ((unit >> 1) ^ seg_swizzle(krow)) << 1 | (L & 1)
       ln.rsrc_b = make_raw_rsrc(p.b + (int64_t)e * K * M + col0, K * M - col0);
 #pragma unroll
       for (int t = 0; t < B_LOADS; ++t) {
-        const int krow = 4 * (wave * B_LOADS + t) + (lane >> 4);
-        const int U = ((((lane & 15) >> 1) ^ (krow & 7)) << 1) | (lane & 1);
+        constexpr int UNITS = BN / 16;
+        const int krow = 64 / UNITS * (wave * B_LOADS + t) + lane / UNITS;
+        const int U = ((((lane % UNITS) >> 1) ^ seg_swizzle<NJ>(krow)) << 1) | (lane & 1);
         ln.voff_b[t] = (uint32_t)((int64_t)krow * M + U * 16);
       }
       ln.b_kstep = (uint32_t)(BKS * M);
     }
-    // this wavefront's 64 columns lie inside one 128-column scale block; one load per register
+    // this wavefront's columns lie inside one 128-column scale block; one load per register
     const int kbs = (int)((K + 127) / 128), mbs = (int)((M + 127) / 128);
-    const int mb = (int)((col0 + 64 * cs) / 128);
+    const int mb = (int)((col0 + STRIP * cs) / 128);
     const int mbu = mb < mbs ? mb : mbs - 1;
     const uint16_t* sbase = reinterpret_cast<const uint16_t*>(p.b_scale) + (int64_t)e * kbs * mbs;
 #pragma unroll
@@ -608,33 +680,49 @@ __global__ __launch_bounds__(THREADS, 1) void gmm_fp8_skinny_kernel(GmmParams p)
   // at once), and after one barrier (every wavefront is done reading the last stage) the next
   // item's first two stages are requested.
   Item cur;
-  if (!setup(first, cur)) return;
-  static_for<0, C::AHEAD>([&](auto s_c) { issue_stage<NT, A8>(lds0, ln, wave, decltype(s_c)::value); });
-  for (long long base = first;;) {
+  int item_at = first + slot / pieces;
+  if (!setup(item_at, cur)) return;
+  // the first stages of an item, and its reduction
+  auto request = [&]() {
+    if constexpr (A8) {
+      static_for<0, C::AHEAD>([&](auto s_c) { issue_stage<NT, NJ>(lds0, ln, wave, decltype(s_c)::value); });
+      return 0;
+    } else {
+      Ahead<NJ> a(ln);
+      static_for<0, C::AHEAD>([&](auto) {
+        issue_stage<NT, NJ>(lds0, ln, wave, a);
+        a.advance();
+      });
+      return a;
+    }
+  };
+  auto at = request();
+  for (;;) {
     Item nxt;
     bool more = false;
     auto item = [&](auto nf_c) {
       constexpr int NF = decltype(nf_c)::value;
-      f32x16 acc[NF > 0 ? NF : 1][2];
+      f32x16 acc[NF > 0 ? NF : 1][NJ];
 #pragma unroll
       for (int i = 0; i < NF; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < NJ; ++j)
 #pragma unroll
           for (int vv = 0; vv < 16; ++vv) acc[i][j][vv] = 0.f;
-      run_item<NT, NF>(lds, lds0, ln, scale, kt_cnt, wave, cur.frag0, acc);  // overload on the lane type
-      base += per_xcd;
-      more = setup(base, nxt);
+      if constexpr (A8) run_item<NT, NF, NJ>(lds, lds0, ln, scale, kt_cnt, wave, cur.frag0, acc);
+      else run_item<NT, NF, NJ>(lds, lds0, ln, scale, kt_cnt, wave, cur.frag0, at, acc);
+      item_at += per_xcd;
+      more = setup(item_at, nxt);
       // lane holds row (lane % 32), columns 8*(v/4) + 4*(lane/32) + v%4 of each 32 x 32 block
 #pragma unroll
       for (int i = 0; i < NF; ++i) {
         const int row = (cur.frag0 + i) * 32 + (lane & 31);
         if (row >= cur.rows) continue;
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < NJ; ++j)
 #pragma unroll
           for (int vq = 0; vq < 4; ++vq) {
-            const int64_t n = cur.col0 + cs * 64 + j * 32 + 8 * vq + 4 * (lane >> 5);
+            const int64_t n = cur.col0 + cs * STRIP + j * 32 + 8 * vq + 4 * (lane >> 5);
             if (n < M)
               *reinterpret_cast<u32x2*>(cur.c_base + ((int64_t)row * M + n) * 2) =
                   pack4<GMOE_BF16>(acc[i][j][4 * vq], acc[i][j][4 * vq + 1], acc[i][j][4 * vq + 2],
@@ -652,16 +740,16 @@ __global__ __launch_bounds__(THREADS, 1) void gmm_fp8_skinny_kernel(GmmParams p)
     __syncthreads();
     if (!more) break;
     cur = nxt;
-    static_for<0, C::AHEAD>([&](auto s_c) { issue_stage<NT, A8>(lds0, ln, wave, decltype(s_c)::value); });
+    at = request();
   }
   // the copies requested past the last reduction (zeros) land before the workgroup ends
   wait_dma_outstanding<0>();
 }
 
-template <bool NT, bool A8>
-static int launch(const GmmParams& p, hipStream_t st) {
-  constexpr size_t smem = (size_t)Cfg<A8>::NST * Cfg<A8>::STAGE_BYTES;
-  auto kern = gmm_fp8_skinny_kernel<NT, A8>;
+template <bool NT, bool A8, int NJ>
+static int launch_strips(const GmmParams& p, hipStream_t st) {
+  constexpr size_t smem = (size_t)Cfg<A8, NJ>::NST * Cfg<A8, NJ>::STAGE_BYTES;
+  auto kern = gmm_fp8_skinny_kernel<NT, A8, NJ>;
   static std::atomic<uint64_t> done_mask{0};
   if (!gmoe_once_per_device(done_mask, [&] {
         return hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
@@ -672,6 +760,22 @@ static int launch(const GmmParams& p, hipStream_t st) {
   if (grid < 8) grid = 8;
   hipLaunchKernelGGL(kern, dim3(grid), dim3(THREADS), smem, st, p);
   return gmoe_launch_status();
+}
+
+// Strips of 128 columns where that makes at most one item per compute unit (a third more rows than the average are
+// reckoned with, so that few experts have a chunk more).  Half the weights per item, and half the items' time where
+// copies are waited for, but twice the activation traffic and fragment reads.  Mean time of strips of 256 over that
+// of 128 in launches of 8 to 32 experts, 1 to 1000 rows each, 512 to 7168 deep and wide, by items of 128 columns and
+// rows per expert (up to 32 / to 96 / more): 64 to 95 items 1.16 / 1.21 / 1.12, 128 to 159 1.14 / 1.13 / 0.95, 192
+// to 223 1.17 / 1.11 / 0.97, 256 to 287 1.13 / 1.14 / 1.01, 288 to 319 0.94 / 0.94 / 1.02, 352 to 383 0.83 / 0.79 /
+// 0.90 (there the fragments of wide items were shared out like those of narrow ones).  Over all such launches, those
+// of wide strips included, 1.13 times as fast as with strips of 256 alone; 512 rows, 8 experts of 1024 x 2048: 132 ->
+// 117 us for the four products of forward and backward.
+template <bool NT, bool A8>
+static int launch(const GmmParams& p, hipStream_t st) {
+  const int64_t experts = p.E > 0 ? p.E : 1, chunks = (p.N * 4 / 3 + experts * MAX_ROWS - 1) / (experts * MAX_ROWS);
+  const bool narrow = experts * chunks * ((p.M + 127) / 128) <= gmoe_cu_count();
+  return narrow ? launch_strips<NT, A8, 1>(p, st) : launch_strips<NT, A8, 2>(p, st);
 }
 
 }  // namespace fp8s
