@@ -1003,6 +1003,41 @@ static inline bool gmm_tn_short_pays(const GmmParams& p) {
   return n <= 768;
 }
 
+// dW outside those two rules (narrow results: K under 512, M under 256, or fewer than 129 tiles of 256x256; and what
+// the 256x256 kernel takes): the kernel with the least estimated time, us, of n rows per expert in `rounds` rounds of
+// its tiles.  Two workgroups of the smaller tiles share a CU, and a last round of at most half their slots takes
+// `half` of one.  Fitted to 1400 launches of 1 to 64 experts, 100 to 9000 rows each, K and M of 128 to 16000, one of
+// them at most 1024; an estimate has to be 8 % better to change the kernel.  Over those launches 1.06 times as fast
+// as the two rules alone (total time 1.09), the changed ones 1.33 (128x128 to 256x256), 1.23 (to 128x256) and 1.22
+// (256x256 to 128x256) times; 9 are more than 3 % slower, down to 0.78.  E.g. 4382 rows, 8 experts, 256 x 19968 512 ->
+// 345 us, and in whole steps, bf16: 8765 tokens of 256, 8 experts of 9984, top 4 2927 -> 2793 us; 4000 of 384, 8 of
+// 6144 1265 -> 1235; 3000 of 320, 32 of 2048 504 -> 507.  Results of 256 MB and more stay with the 256x256 kernel: writes bind them (64 experts, 108 rows, 15480 x
+// 352 255 / 346).
+struct TnCosts {
+  int rows, cols, per_cu;
+  double launch, round, per_row, half;
+};
+constexpr TnCosts kTnSmall = {128, 128, 2, 6.4, 4.83, 0.0203, 0.39}, kTnLarge = {256, 256, 1, 1.8, 7.75, 0.0217, 1.0},
+                  kTnShort = {128, 256, 2, 5.7, 4.35, 0.0319, 0.42};
+static inline double tn_estimate(const TnCosts& c, const GmmParams& p) {
+  const int64_t experts = p.E > 0 ? p.E : 1;
+  const int64_t tiles = experts * ((p.K + c.rows - 1) / c.rows) * ((p.M + c.cols - 1) / c.cols);
+  const int64_t slots = (int64_t)c.per_cu * gmm_grid(1), rest = tiles % slots;
+  const double rounds = (double)(tiles / slots) + (rest == 0 ? 0.0 : rest * 2 <= slots ? c.half : 1.0);
+  return c.launch + rounds * (c.round + c.per_row * (double)(p.N / experts));
+}
+enum TnKernel { TN_SMALL, TN_LARGE, TN_SHORT };
+static inline TnKernel gmm_tn_kernel(const GmmParams& p) {
+  if (gmm_tn_short_pays(p)) return TN_SHORT;
+  const bool large = gmm_large_tiles(p, MODE_TN);
+  if (p.K < 128 || p.M < 128) return large ? TN_LARGE : TN_SMALL;
+  constexpr double margin = 0.92;
+  const double t_large = tn_estimate(kTnLarge, p), t_short = tn_estimate(kTnShort, p);
+  if (large) return !gmm_tn_streams(p) && t_short < margin * t_large ? TN_SHORT : TN_LARGE;
+  if ((t_large < t_short ? t_large : t_short) >= margin * tn_estimate(kTnSmall, p)) return TN_SMALL;
+  return t_large < t_short ? TN_LARGE : TN_SHORT;
+}
+
 // Whether reading the operands beforehand (warm_operands) pays: they take bytes / 5 TB/s, and the launch has to be
 // one of several times more result bytes.  In a whole step the operands partly lie in the memory-side cache and the
 // stores of one launch meet the loads of the next, so the line is drawn there (us of a step without / with, result
@@ -1061,8 +1096,13 @@ static int launch_gmm_16bit(const GmmParams& p, int dtype, int out_dtype, hipStr
   if constexpr (MODE == MODE_TN) {
     GmmParams q = p;
     q.warm = gmm_tn_warm_pays(p);
-    if (gmm_tn_short_pays(p)) return launch_gmm_tn_short(q, dtype, out_dtype, st);
-    if (gmm_large_tiles(p, MODE)) return launch_gmm_dtl_tn(q, dtype, out_dtype, st);
+    // 32-bit results (the gate's) were not part of the fit
+    const TnKernel kernel = ODT != GMOE_F32          ? gmm_tn_kernel(p)
+                            : gmm_tn_short_pays(p)   ? TN_SHORT
+                            : gmm_large_tiles(p, MODE) ? TN_LARGE
+                                                       : TN_SMALL;
+    if (kernel == TN_SHORT) return launch_gmm_tn_short(q, dtype, out_dtype, st);
+    if (kernel == TN_LARGE) return launch_gmm_dtl_tn(q, dtype, out_dtype, st);
   } else {
     if (gmm_rows_pays(p, MODE, EPI)) return launch_gmm_rows(p, MODE, dtype, out_dtype, EPI, st);
   }

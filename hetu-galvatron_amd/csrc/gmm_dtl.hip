@@ -29,9 +29,10 @@
 //     transposing LDS load ds_read_b64_tr_b16: a group of 16 lanes reads a 4(k) x 16(outer) block
 //     and every lane receives the 4 k-values of its own column.
 //
-// For NN and NT the register-staged kernel of gmm.hip measured faster: copies of an operand whose
-// reduction index is contiguous arrive as 64-byte row pieces here, which the address path handles
-// at half the rate of the 128-byte pieces that kernel requests.
+// NN and NT have a kernel of their own (gmm_rows_kernel.h): 32-deep copies of an operand whose reduction
+// index is contiguous would be 64-byte row pieces, which the address path handles at half the rate of whole lines.
+// What did not help: stores issued by two wavefronts and copies by the other two, so that no copy waits behind a
+// store (5 to 7 % slower at 383 to 4096 rows per expert: 16 copies per K tile from one wavefront).
 #include "gmm_common.h"
 
 namespace gmoe {
