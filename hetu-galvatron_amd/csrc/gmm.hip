@@ -1003,16 +1003,14 @@ static inline bool gmm_tn_short_pays(const GmmParams& p) {
   return n <= 768;
 }
 
-// dW outside those two rules (narrow results: K under 512, M under 256, or fewer than 129 tiles of 256x256; and what
-// the 256x256 kernel takes): the kernel with the least estimated time, us, of n rows per expert in `rounds` rounds of
-// its tiles.  Two workgroups of the smaller tiles share a CU, and a last round of at most half their slots takes
-// `half` of one.  Fitted to 1400 launches of 1 to 64 experts, 100 to 9000 rows each, K and M of 128 to 16000, one of
-// them at most 1024; an estimate has to be 8 % better to change the kernel.  Over those launches 1.06 times as fast
-// as the two rules alone (total time 1.09), the changed ones 1.33 (128x128 to 256x256), 1.23 (to 128x256) and 1.22
-// (256x256 to 128x256) times; 9 are more than 3 % slower, down to 0.78.  E.g. 4382 rows, 8 experts, 256 x 19968 512 ->
-// 345 us, and in whole steps, bf16: 8765 tokens of 256, 8 experts of 9984, top 4 2927 -> 2793 us; 4000 of 384, 8 of
-// 6144 1265 -> 1235; 3000 of 320, 32 of 2048 504 -> 507.  Results of 256 MB and more stay with the 256x256 kernel: writes bind them (64 experts, 108 rows, 15480 x
-// 352 255 / 346).
+// dW outside those two rules (narrow results: K under 512, M under 256, or fewer than 129 tiles of 256x256): the
+// kernel with the least estimated time, us, of n rows per expert in `rounds` rounds of its tiles.  Two workgroups of
+// the smaller tiles share a CU, and a last round of at most half their slots takes `half` of one.  Fitted to 1400
+// launches of 1 to 64 experts, 100 to 9000 rows each, K and M of 128 to 16000, one of them at most 1024; an estimate
+// has to be 8 % better to leave the 128x128 tiles.  Over those launches 1.05 times as fast as the two rules alone
+// (total time 1.08), the changed ones 1.33 (to 256x256) and 1.23 times (to 128x256); 9 are more than 3 % slower, down
+// to 0.78.  E.g. 4382 rows, 8 experts, 256 x 19968 512 -> 345 us, and in whole steps, bf16: 8765 tokens of 256, 8
+// experts of 9984, top 4 2927 -> 2793 us; 4000 of 384, 8 of 6144 1265 -> 1235; 3000 of 320, 32 of 2048 504 -> 507.
 struct TnCosts {
   int rows, cols, per_cu;
   double launch, round, per_row, half;
@@ -1029,12 +1027,10 @@ static inline double tn_estimate(const TnCosts& c, const GmmParams& p) {
 enum TnKernel { TN_SMALL, TN_LARGE, TN_SHORT };
 static inline TnKernel gmm_tn_kernel(const GmmParams& p) {
   if (gmm_tn_short_pays(p)) return TN_SHORT;
-  const bool large = gmm_large_tiles(p, MODE_TN);
-  if (p.K < 128 || p.M < 128) return large ? TN_LARGE : TN_SMALL;
-  constexpr double margin = 0.92;
+  if (gmm_large_tiles(p, MODE_TN)) return TN_LARGE;
+  if (p.K < 128 || p.M < 128) return TN_SMALL;
   const double t_large = tn_estimate(kTnLarge, p), t_short = tn_estimate(kTnShort, p);
-  if (large) return !gmm_tn_streams(p) && t_short < margin * t_large ? TN_SHORT : TN_LARGE;
-  if ((t_large < t_short ? t_large : t_short) >= margin * tn_estimate(kTnSmall, p)) return TN_SMALL;
+  if ((t_large < t_short ? t_large : t_short) >= 0.92 * tn_estimate(kTnSmall, p)) return TN_SMALL;
   return t_large < t_short ? TN_LARGE : TN_SHORT;
 }
 

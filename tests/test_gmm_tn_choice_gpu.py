@@ -11,7 +11,7 @@ CASES = [  # rows per expert, K, M
     ([1024, 1], 8200, 128),             # ... the narrowest
     ([900] * 24, 184, 872),             # 128x256 tiles beyond 768 rows
     ([130] * 12, 2048, 136),            # ... with few rows and one column tile, mostly padding
-    ([160] * 6, 8192, 1016),            # 256x256 tiles of half a round more, now 128x256
+    ([160] * 6, 8192, 1016),            # 256x256 tiles, a little over half a round
     ([3000], 128, 136),                 # a few tiles
 ]
 
