@@ -5,9 +5,22 @@
 
 namespace gmoe {
 
+// What a tile costs besides 4 KiB of rows per unit (of 64) and stage (of 32 reduction elements), as KiB of operand
+// stream: per stage, around the tile, around each unit of it; and by which factor chunks of more than four units cost more.
+struct ChunkCosts {
+  float stage, tile, unit, tall;
+};
+constexpr ChunkCosts kChunkCosts{16.f, 250.f, 0.f, 1.f};
+// The activation backward reads fc1 and writes d(fc1) around a tile, four times the bytes of a plain result, with every
+// compute unit at it at once: taller chunks save little and leave a part empty last round longer.  us in chunks of up to
+// 128 / 192 / 256 / 320 / 384 rows (K x F): 16 experts of 640, 1024 x 2816 115 / 108 / 122 / 122 / 122; 8 of 366 to 402,
+// 4096 x 14336 477 / 489 / 454 / 447 / 474; 60 of 386, 6272 x 2688 1070 / 1009 / 953 / 957 / 943; 8 of 1000, 4096 x 14336
+// 1017 / 992 / 867 / 871 / 975.  Over 1059 launches (E 1-64, 40-6000 rows per expert, even and uneven loads, K and F
+// 128-16384) the costs above lose 0.9 % against the best size of each (p95 6 %), these 0.3 % (2 %).
+constexpr ChunkCosts kChunkCostsGluBwd{8.f, 120.f, 650.f, 1.04f};
+
 // Rows of a chunk, in units of 64: of the sizes SIZES - 1 to 2 the one that ends first.  v[0]: units of all experts,
-// v[u]: their chunks of up to u units.  A stage of a tile of u units takes as long as its operands stream, 16 + 4 u KiB;
-// prologue and epilogue take as long as 250 KiB.  Smaller chunks are taken where they cost less than `ahead` of the
+// v[u]: their chunks of up to u units.  Smaller chunks are taken where they cost less than `ahead` of the
 // best larger ones.  The kernel asks with ahead 1: over 8600 launches of 96 rows per expert and more that costs 1.1 %
 // against the best size of each, 0.95 costs 2.0 % (us in chunks of up to 128 / 192 / 256 / 320 / 384 rows, rows per
 // expert: with activation 383, 4096 x 28672, 8 experts 890 / 776 / 739 / 745 / 686; 640, 1024 x 5632, 16 172 / 152 /
@@ -16,14 +29,14 @@ constexpr int kRowsMaxUnits = 4;
 constexpr int kTallMaxUnits = 6;
 template <int SIZES>
 __host__ __device__ inline int rows_chunk_units(const int (&v)[SIZES], int col_tiles, int grid, int64_t K,
-                                                float ahead = 0.95f) {
-  const float fixed = 16.f + 250.f / (float)((K + 31) / 32);
+                                                float ahead = 0.95f, ChunkCosts c = kChunkCosts) {
+  const float stages = (float)((K + 31) / 32), fixed = c.stage + c.tile / stages, unit = 4.f + c.unit / stages;
   int best = SIZES - 1;
   float least = 0.f;
 #pragma unroll
   for (int u = SIZES - 1; u >= 2; --u) {
     const int rounds = (int)(((long long)v[u] * col_tiles + grid - 1) / grid);
-    const float cost = (float)rounds * (fixed + 4.f * (float)v[0] / (float)(v[u] > 0 ? v[u] : 1));
+    const float cost = (float)rounds * (fixed + unit * (float)v[0] / (float)(v[u] > 0 ? v[u] : 1)) * (u > 4 ? c.tall : 1.f);
     if (u == SIZES - 1 || cost < ahead * least) {
       best = u;
       least = cost;
