@@ -963,22 +963,12 @@ static inline bool gmm_large_tiles(const GmmParams& p, int mode) {
 }
 
 // Row-adaptive tiles (gmm_rows_kernel.h) for 16-bit NN / NT: tiles of 64 to 384 rows x 256 columns that share an expert's
-// rows evenly, one workgroup per CU; the rules with both sides' times are in rows_rule.h.  Launches that could fill
-// 256x256 tiles are 12 to 17 % faster here (us there / here, rows per expert, K x M, experts: with activation 4096, 4096
-// x 28672, 8 6211 / 5836; 1024, 7168 x 4096, 32 1661 / 1525; NN 4096, 14336 x 4096, 8 3023 / 2790; activation backward
-// 1024, 7168 x 2048, 32 915 / 838; NT 4096, 28672 x 4096, 8 6010 / 5659; of 3340 such launches 3 % are slower by
-// more than 2 %, where the loads decide whether a round more is needed), so of those only plain NT ones of
-// fewer than 768 rows per expert are left there, where the rules see no gain (600, 2056 x 4104, 8 120 / 123).
-// The kernel's resource of a tile spans 384 rows.
-constexpr int64_t kNtTallRows = 768;
+// rows evenly, one workgroup per CU; the rule with both sides' times is in rows_rule.h.  The kernel's resource of a tile
+// spans 384 rows.
 static inline bool gmm_rows_pays(const GmmParams& p, int mode, int epi) {
   const RowsKind kind = mode == MODE_NN ? (epi == EPI_NONE ? ROWS_NN : ROWS_NN_GLU)
                                         : (epi == EPI_NONE ? ROWS_NT : ROWS_NT_GLU_BWD);
-  if (kTallMaxUnits * 64 * p.K * 2 >= (1ll << 31)) return false;
-  const int64_t experts = p.E > 0 ? p.E : 1;
-  if (nn_large_tiles(experts, p.N, p.M))
-    return kind != ROWS_NT || p.N / experts >= kNtTallRows || rows_pays(kind, p.E, p.N, p.K, p.M, gmm_grid(1));
-  return rows_pays(kind, p.E, p.N, p.K, p.M, gmm_grid(1)) || tall_pays(kind, p.E, p.N, p.K, p.M, gmm_grid(1));
+  return kTallMaxUnits * 64 * p.K * 2 < (1ll << 31) && rows_pays(kind, p.E, p.N, p.K, p.M, gmm_grid(1));
 }
 
 // dW of 16-bit operands with a short reduction (gmm_tn.hip: 128x256 tiles, two workgroups per CU) against the

@@ -74,7 +74,7 @@ __device__ __forceinline__ int best_max_units(int (&v)[kMaxUnits + 1], int nt_cn
     for (int w = 0; w < kGemmThreads / 64; ++w) v[i] += sums[w * (kMaxUnits + 1) + i];
   }
   constexpr bool bwd = EPI == EPI_GLU_BWD_SILU || EPI == EPI_GLU_BWD_GELU;
-  return rows_chunk_units(v, nt_cnt, grid, K, 1.f, bwd ? kChunkCostsGluBwd : kChunkCosts);
+  return rows_chunk_units(v, nt_cnt, grid, K, bwd ? kChunkCostsGluBwd : kChunkCosts);
 }
 // first unit and unit count of chunk c of cnt
 __device__ __forceinline__ void chunk_units(long long n, int cnt, int c, int& first, int& units) {

@@ -1,6 +1,8 @@
 // Which 16-bit NN / NT launches go to the row-adaptive tiles (gmm_rows_kernel.h), and into which chunks the kernel cuts an
 // expert's rows.
 #pragma once
+#include <cmath>
+
 #include "split_rule.h"
 
 namespace gmoe {
@@ -19,25 +21,21 @@ constexpr ChunkCosts kChunkCosts{16.f, 250.f, 0.f, 1.f};
 // 128-16384) the costs above lose 0.9 % against the best size of each (p95 6 %), these 0.3 % (2 %).
 constexpr ChunkCosts kChunkCostsGluBwd{8.f, 120.f, 650.f, 1.04f};
 
-// Rows of a chunk, in units of 64: of the sizes SIZES - 1 to 2 the one that ends first.  v[0]: units of all experts,
-// v[u]: their chunks of up to u units.  Smaller chunks are taken where they cost less than `ahead` of the
-// best larger ones.  The kernel asks with ahead 1: over 8600 launches of 96 rows per expert and more that costs 1.1 %
-// against the best size of each, 0.95 costs 2.0 % (us in chunks of up to 128 / 192 / 256 / 320 / 384 rows, rows per
-// expert: with activation 383, 4096 x 28672, 8 experts 890 / 776 / 739 / 745 / 686; 640, 1024 x 5632, 16 172 / 152 /
+// Rows of a chunk, in units of 64: of the sizes kTallMaxUnits to 2 the one that ends first.  v[0]: units of all experts,
+// v[u]: their chunks of up to u units.  Over 8600 launches of 96 rows per expert and more it costs 1.1 % against the best size
+// of each (us in chunks of up to 128 / 192 / 256 / 320 / 384 rows, rows per expert: with activation 383, 4096 x 28672, 8 experts 890 / 776 / 739 / 745 / 686; 640, 1024 x 5632, 16 172 / 152 /
 // 150 / 147 / 135; NN 640, 2816 x 1024, 16 86 / 60 / 67 / 73 / 81; NT 383, 28672 x 4096, 8 817 / 935 / 691 / 700 / 926).
-constexpr int kRowsMaxUnits = 4;
 constexpr int kTallMaxUnits = 6;
-template <int SIZES>
-__host__ __device__ inline int rows_chunk_units(const int (&v)[SIZES], int col_tiles, int grid, int64_t K,
-                                                float ahead = 0.95f, ChunkCosts c = kChunkCosts) {
+__host__ __device__ inline int rows_chunk_units(const int (&v)[kTallMaxUnits + 1], int col_tiles, int grid, int64_t K,
+                                                ChunkCosts c) {
   const float stages = (float)((K + 31) / 32), fixed = c.stage + c.tile / stages, unit = 4.f + c.unit / stages;
-  int best = SIZES - 1;
+  int best = kTallMaxUnits;
   float least = 0.f;
 #pragma unroll
-  for (int u = SIZES - 1; u >= 2; --u) {
+  for (int u = kTallMaxUnits; u >= 2; --u) {
     const int rounds = (int)(((long long)v[u] * col_tiles + grid - 1) / grid);
     const float cost = (float)rounds * (fixed + unit * (float)v[0] / (float)(v[u] > 0 ? v[u] : 1)) * (u > 4 ? c.tall : 1.f);
-    if (u == SIZES - 1 || cost < ahead * least) {
+    if (u == kTallMaxUnits || cost < least) {
       best = u;
       least = cost;
     }
@@ -46,28 +44,6 @@ __host__ __device__ inline int rows_chunk_units(const int (&v)[SIZES], int col_t
 }
 
 enum RowsKind { ROWS_NN, ROWS_NN_GLU, ROWS_NT, ROWS_NT_GLU_BWD };
-
-// Times in ns, rates in bytes or operations per ns.
-struct RowsCosts {
-  // row-adaptive: around a tile, around each 64 rows of it, a stage of 32 reduction elements, share of a tile's
-  // time that a round saves as its tiles get fewer, around the launch, operations
-  double tile, unit, stage, lone_gain, launch, ops;
-  // 256x256 tiles: around one, 64 reduction elements, operations
-  double large_tile, large_step, large_ops;
-  // 128x128 tiles: around one, 64 reduction elements with two tiles on a CU and with one, around the split's sums
-  double small_tile, small_pair, small_lone, sums;
-  // around either launch; the weights' stream
-  double other_launch, weights;
-};
-constexpr RowsCosts kRowsCosts[] = {
-    {5320, 795, 721, 0.44, 6650, 1.14e6, 8000, 1410, 1.0e6, 3540, 1250, 563, 8890, 5550, 4470},
-    {2610, 1850, 814, 0.52, 7170, 1.6e6, 8610, 1500, 1.06e6, 4900, 1250, 753, 0, 1120, 4840},
-    {4310, 918, 778, 0.05, 6170, 1.6e6, 6170, 1360, 1.37e6, 831, 1420, 365, 0, 8230, 5380},
-    {0, 5240, 848, 0.11, 8970, 1.03e6, 22600, 1410, 1.57e6, 1360, 1580, 387, 4680, 15000, 4120}};
-constexpr double kRowsWeights = 6000;
-
-// Rows per expert from which rows_pays is not asked (gmm.hip).
-constexpr int64_t kRowsManyRows = 2048;
 
 // 256x256 tiles for NN / NT: an expert's share of rows can fill them and there are enough for every CU.
 inline bool nn_large_tiles(int64_t E, int64_t N, int64_t M) {
@@ -91,120 +67,108 @@ inline int64_t over_loads(int64_t E, int64_t n, F f) {
   return sum;
 }
 
-// The line for chunks of up to 256 rows, with constants fitted to 3400 shapes measured both ways (E 1-64, 72-2040 rows
-// per expert, K 256-28672, M 128-28672) when the kernel had no larger ones and streamed its rows in half cache lines: a
-// launch that paid then pays more now, and tall_pays adds those that pay only now.
-// K, M as in the product (with the activation M = 2F); cus: workgroups of a persistent grid, one per CU.
-inline bool rows_pays(RowsKind kind, int64_t E, int64_t N, int64_t K, int64_t M, int64_t cus) {
-  const int64_t n = N / (E > 0 ? E : 1);
-  // fewer rows: an expert is one tile either way, and its weights bound the launch; shorter reductions:
-  // prologue and epilogue weigh as much
-  if (n < 96 || n >= kRowsManyRows || K <= 512) return false;
-  const RowsCosts& c = kRowsCosts[kind];
-  const bool glu = kind == ROWS_NN_GLU, large = nn_large_tiles(E, N, M);
-  const double weights = (double)E * K * M * 2, ops = 2.0 * N * K * M;
-  auto cdiv = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
-  auto most = [](double a, double b) { return a > b ? a : b; };
-
-  // the chunk size that ends first, as the kernel chooses it
-  const int64_t cols = glu ? cdiv(M / 2, 128) : cdiv(M, 256);
-  const int64_t units = over_loads(E, n, [&](int64_t r) { return cdiv(r, 64); });
-  double rows = 0;
-  for (int u = 4; u >= 2; --u) {
-    const int64_t chunks = over_loads(E, n, [&](int64_t r) { return cdiv(cdiv(r, 64), u); });
-    const int64_t tiles = cdiv(E * chunks * cols, 5), rounds = cdiv(tiles, cus), last = tiles - (rounds - 1) * cus;
-    const double tile = c.tile + c.unit * units / chunks + c.stage * cdiv(K, 32);
-    const double t = tile * (rounds - c.lone_gain * (1 - (double)last / cus));
-    if (u == 4 || t < rows) rows = t;
-  }
-  rows = most(most(rows, weights / kRowsWeights), ops / c.ops) + c.launch;
-
-  const int64_t edge = large ? 256 : 128, steps = cdiv(K, 64);
-  const int64_t tiles = cdiv(E * over_loads(E, n, [&](int64_t r) { return cdiv(r, edge); }) * cdiv(M, edge), 5);
-  const int pieces = large || glu || kind == ROWS_NT_GLU_BWD ? 1 : nn_split_pieces(E, N, K, M);
-  double other;
-  if (large) {
-    other = most(cdiv(tiles, cus) * (c.large_tile + c.large_step * steps), ops / c.large_ops);
-  } else if (pieces > 1) {
-    other = (tiles * pieces > cus ? c.small_pair : c.small_lone) * steps / pieces + c.sums +
-            (double)kSplitNsPerPiece * tiles * pieces;
-  } else {
-    const int64_t rounds = tiles / (2 * cus), rest = tiles % (2 * cus);
-    const double pair = c.small_tile + c.small_pair * steps, lone = c.small_tile + c.small_lone * steps;
-    other = rounds * pair;
-    if (rest > 0) other += rest <= cus ? lone : lone + (pair - lone) * (rest - cus) / cus;
-  }
-  other = most(other, weights / c.weights) + c.other_launch;
-  // the activation as a launch of its own
-  if (glu && !large) other += 3000 + (double)N * M * 3 / 4000;
-  return rows < other;
-}
-
-// Times in ns as above: row-adaptive tiles with chunks of up to 384 rows (a stage is stage + unit_stage per 64 rows),
-// then 128x128 tiles.
-struct TallCosts {
-  double tile, unit, stage, unit_stage, lone_gain, launch, weights, ops;
-  double small_tile, small_pair, small_lone, sums, small_launch, small_weights, small_ops, act;
+// Times in ns, rates in bytes or operations per ns.
+struct RowsCosts {
+  // row-adaptive tiles: around a tile and each 64 rows of it, a stage of 32 reduction elements of it and of each 64
+  // rows, share of a tile's time that a round saves as its tiles get fewer, around the launch, traffic, operations
+  double tile, unit, stage, unit_stage, lone_gain, launch, bytes, ops;
+  // 128x128 tiles: around one, 64 reduction elements with two tiles on a CU and with one, around the launch, traffic,
+  // operations; around a split's sums; the activation's launch
+  double small_tile, small_pair, small_lone, small_launch, small_bytes, small_ops, sums, act;
+  // 256x256 tiles (plain NT): around one, 64 reduction elements, operations
+  double large_tile, large_step, large_ops;
 };
-constexpr TallCosts kTallCosts[] = {
-    {4620, 960, 217, 141, 0.31, 4200, 4830, 1.48e6, 3760, 1260, 520, 8700, 6300, 4320, 1e6, 0},
-    {3130, 1900, 386, 109, 0.38, 5100, 5700, 1.487e6, 2170, 1180, 500, 22300, 6200, 5540, 0.783e6, 3500},
-    {3840, 1140, 223, 144, 0.30, 4100, 4390, 1.41e6, 2860, 1240, 530, 7400, 6900, 4080, 1e6, 0},
-    {690, 5880, 294, 127, 0.36, 5200, 4080, 1.487e6, 9950, 1350, 560, 0, 3800, 3640, 1e6, 0}};
+constexpr RowsCosts kRowsCosts[] = {
+    {2840, 741, 275, 69.3, 0.0819, 9590, 7840, 0.991e6, 2730, 1250, 628, 2260, 4810, 0.563e6, 1990, 0, 0, 0, 0},
+    {3820, 2080, 343, 111, 0.0366, 1890, 6840, 1.49e6, 1110, 1310, 417, 3670, 5580, 0.484e6, 0, 2070, 0, 0, 0},
+    {2990, 1340, 176, 159, 0.14, 4650, 6800, 1.62e6, 2320, 1270, 614, 2730, 4720, 0.551e6, 4720, 0, 6670, 1630, 1.16e6},
+    {6890, 6480, 123, 102, 0.0491, 1020, 6580, 1.0e6, 10600, 1430, 422, 2500, 5630, 1.0e6, 0, 0, 0, 0, 0}};
 
-// Whether a launch that has too few rows or tiles for 256x256 ones is faster in row-adaptive tiles than in 128x128
-// ones.  Fitted to 15000 launches measured both ways (E 1-64, 2-8192 rows per expert, K 128-28672, M 128-28672, 2e8 to
-// 6e12 operations, operands from HBM, loads that differ by 6 or 30 %).  From 96 rows per expert on it costs 0.9 to 2.4
-// % against the better side of each, all of them in 128x128 tiles 6 to 27 %, rows_pays alone 2 to 22 %.  Below 96 rows
-// an expert's weights bound the launch on either side; there only the launch with the activation may come here, which
-// is two on the other tiles (1.9 % against the better side, the other tiles 5.4 %, without the host's time for the
-// second launch), and only where those are not split, which spreads the weights' stream evenly over the CUs.  us in
-// 128x128 tiles / in these (rows per expert, K x M, experts): NN 137, 2560 x 10240, 24 389 / 264; 656, 1280 x 1280, 2
-// 18.0 / 24.6; with activation 389, 512 x 14336, 64 924 / 562; 121, 7168 x 256, 8 72 / 101; 3, 4096 x 28672, 8 317 /
-// 346; 3, 4096 x 14336, 8 176 / 172; NT 938, 12544 x 2112, 4 280 / 217; 866, 19968 x 1536, 1 97 / 260; activation
-// backward 386, 6272 x 2688, 60 1210 / 956; 599, 304 x 544, 6 15.8 / 26.4.
-inline bool tall_pays(RowsKind kind, int64_t E, int64_t N, int64_t K, int64_t M, int64_t cus) {
-  const int64_t n = N / (E > 0 ? E : 1);
-  const bool glu = kind == ROWS_NN_GLU;
-  if (n < (glu ? 1 : 96)) return false;
-  const TallCosts& c = kTallCosts[kind];
-  const double weights = (double)E * K * M * 2, ops = 2.0 * N * K * M;
+// Whether a 16-bit NN / NT launch is faster in row-adaptive tiles than in the others: 128x128 ones, for plain NT that
+// could fill them 256x256 ones (only the host asks).  K, M as in the product (with the activation M = 2F); cus:
+// workgroups of a persistent grid, one per CU.
+//
+// Fitted to 6600 launches measured both ways, half of them of layers as they are trained, half spread over E 1-64, 1-9000
+// rows per expert, K and M 128-16384 (operands from HBM, loads that differ by 2 to 80 %), a third of them under 30 us.
+// Over them it costs 0.5 % (NN), 0.8 % (with activation), 0.8 % (NT) and 1.1 % (activation backward) against the better
+// side of each; the others throughout 11, 12, 6 and 7 %, these throughout 19, 8, 20 and 12 %.  The 3 % that these have to
+// be ahead by cost nothing and keep launches at the line where they were.
+//
+// Fewer than 96 rows per expert: an expert is one row tile and its weights bound the launch on either side.  Only the launch
+// with the activation, which is two on the other tiles, may come here, and only where its tiles fill their rounds: a
+// workgroup per CU streams the weights at the chip's rate only while all of them have a tile (rows per expert, K x M,
+// experts; 3, 4096 x 28672, 8, 3.5 rounds 319 / 350 others; 16, 2048 x 2816, 64, 2.75 rounds 142 / 131 these; 16, 1024 x
+// 5632, 16, 1.4 rounds 43 / 46 others).  Over 3500 such launches 1.8 % are lost against the better side, in the other tiles
+// throughout 2.3 %, here 9.8 %.
+//
+// us in the other tiles / in these (rows per expert, K x M, experts):
+//   * NN: 382, 14336 x 4096, 8 437 / 337 these; 363, 512 x 5120, 8 32 / 32; 267, 576 x 832, 64 45 / 36 these; 941, 768 x
+//     128, 32 18 / 24 others; 656, 1280 x 1280, 2 14 / 23 others; 1701, 10848 x 160, 4 79 / 133 others.
+//   * With activation: 382, 4096 x 28672, 8 976 / 650 these; 640, 1024 x 5632, 16 189 / 138 these; 208, 128 x 512, 32 12
+//     / 13 others; 103, 768 x 1024, 4 13 / 18 others; 121, 7168 x 256, 8 65 / 95 others.
+//   * NT: 382, 28672 x 4096, 8 860 / 628 these; 600, 2056 x 4104, 8 116 / 112 these; 1111, 5632 x 2048, 1 49 / 77 others;
+//     1769, 1408 x 512, 4 16 / 24 others; 1000, 28672 x 4096, 8 1439 / 1413 these.
+//     Short reductions of fewer than 768 rows per expert that fill 256x256 tiles stay there: of 36 such launches a third is
+//     slower here, by up to 7 %.
+//   * Activation backward: 382, 4096 x 14336, 8 470 / 382 these; 1024, 7168 x 2048, 32 1119 / 835 these; 640, 1024 x 2816,
+//     16 103 / 111 others; 599, 304 x 544, 6 15 / 29 others; 322, 4992 x 1024, 4 53 / 73 others.
+// It knows the average load only, and where that is close to whole rounds it can be wrong.
+inline bool rows_pays(RowsKind kind, int64_t E, int64_t N, int64_t K, int64_t M, int64_t cus) {
+  if (E < 1) E = 1;
+  const int64_t n = N / E;
+  const bool glu = kind == ROWS_NN_GLU, bwd = kind == ROWS_NT_GLU_BWD;
   auto cdiv = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
   auto most = [](double a, double b) { return a > b ? a : b; };
-
-  const int64_t cols = glu ? cdiv(M / 2, 128) : cdiv(M, 256), stages = 2 * cdiv(K, 64);
+  const int64_t cols = glu ? cdiv(M / 2, 128) : cdiv(M, 256);
+  if (n < 96) {
+    if (!glu || N < 1) return false;
+    const double tiles = E * (1 - std::pow(1 - 1.0 / E, (double)N)) * cols;  // of the experts that have rows
+    return tiles >= 0.9 * cus * std::ceil(tiles / cus);
+  }
+  const bool large = kind == ROWS_NT && nn_large_tiles(E, N, M);
+  if (large && n < 768 && K <= 2560) return false;
+  const RowsCosts& c = kRowsCosts[kind];
+  const double out = (double)N * M * (glu ? 3 : bwd ? 8 : 2), ops = 2.0 * N * K * M;
+  const double bytes = 2.0 * E * K * M + 2.0 * N * K + out;
+  const int64_t stages = 2 * cdiv(K, 64);
   const int64_t units = over_loads(E, n, [&](int64_t r) { return cdiv(r, 64); });
-  double tall = 0, idle = 0;
+  double rows = 0, idle = 0;
   for (int u = kTallMaxUnits; u >= 2; --u) {
     const int64_t chunks = over_loads(E, n, [&](int64_t r) { return cdiv(cdiv(r, 64), u); });
     const int64_t tiles = cdiv(E * chunks * cols, 5), rounds = cdiv(tiles, cus), last = tiles - (rounds - 1) * cus;
-    const double average = (double)units / chunks;
+    const double average = (double)units / chunks, part = 1 - (double)last / cus;
     const double tile = c.tile + c.unit * average + (c.stage + c.unit_stage * average) * stages;
-    const double t = tile * (rounds - c.lone_gain * (1 - (double)last / cus));
-    if (u == kTallMaxUnits || t < tall) {
-      tall = t;
-      idle = rounds > 0 ? (1 - (double)last / cus) / rounds : 0;
+    const double t = tile * (rounds - c.lone_gain * part);
+    if (u == kTallMaxUnits || t < rows) {
+      rows = t;
+      idle = part / rounds;
     }
   }
-  // a last round that is part empty does not stream the weights at the whole chip's rate
-  tall = most(most(tall, weights / c.weights * (1 + 0.6 * idle)), ops / c.ops) + c.launch;
+  // a last round that is part empty does not stream at the whole chip's rate
+  rows = most(most(rows, bytes / c.bytes * (1 + 0.6 * idle)), ops / c.ops) + c.launch;
 
-  const int64_t steps = cdiv(K, 64), tiles = cdiv(E * over_loads(E, n, [&](int64_t r) { return cdiv(r, 128); }) * cdiv(M, 128), 5);
-  const int pieces = kind == ROWS_NT_GLU_BWD ? 1 : nn_split_pieces(E, N, K, M);
-  if (n < 96 && pieces > 1) return false;
-  double small;
-  if (pieces > 1) {
-    small = (tiles * pieces > cus ? c.small_pair : c.small_lone) * steps / pieces + c.sums +
-            (double)kSplitNsPerPiece * tiles * pieces;
+  const int64_t edge = large ? 256 : 128, steps = cdiv(K, 64);
+  const int64_t tiles = cdiv(E * over_loads(E, n, [&](int64_t r) { return cdiv(r, edge); }) * cdiv(M, edge), 5);
+  // the launches with an activation have no workspace for a split
+  const int pieces = large || glu || bwd ? 1 : nn_split_pieces(E, N, K, M);
+  double other;
+  if (large) {
+    other = most(cdiv(tiles, cus) * (c.large_tile + c.large_step * steps), ops / c.large_ops);
   } else {
-    const int64_t rounds = tiles / (2 * cus), rest = tiles % (2 * cus);
-    const double pair = c.small_tile + c.small_pair * steps, lone = c.small_tile + c.small_lone * steps;
-    small = rounds * pair;
-    if (rest > 0) small += rest <= cus ? lone : lone + (pair - lone) * (rest - cus) / cus;
+    if (pieces > 1) {
+      other = (tiles * pieces > cus ? c.small_pair : c.small_lone) * steps / pieces + c.sums +
+              (double)kSplitNsPerPiece * tiles * pieces;
+    } else {
+      const int64_t rounds = tiles / (2 * cus), rest = tiles % (2 * cus);
+      const double pair = c.small_tile + c.small_pair * steps, lone = c.small_tile + c.small_lone * steps;
+      other = rounds * pair;
+      if (rest > 0) other += rest <= cus ? lone : lone + (pair - lone) * (rest - cus) / cus;
+    }
+    other = most(most(other, bytes / c.small_bytes), ops / c.small_ops);
   }
-  small = most(most(small, weights / c.small_weights), ops / c.small_ops) + c.small_launch;
-  if (glu) small += c.act + (double)N * M * 3 / 4000;  // the activation as a launch of its own
-  return tall < (glu ? 1.0 : 0.97) * small;
+  other += c.small_launch;
+  if (glu) other += c.act + (double)N * M * 3 / 4000;
+  return rows < 0.97 * other;
 }
 
 }  // namespace gmoe

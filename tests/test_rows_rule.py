@@ -1,12 +1,10 @@
-"""The choice between the row-adaptive tiles and the others (csrc/rows_rule.h) where both were measured and one is
-clearly ahead, and at the limits of what it looks at; and the chunks that the row-adaptive tiles cut rows into."""
+"""The choice between the row-adaptive tiles and the others (csrc/rows_rule.h) where both were measured, and at the limits of
+what it looks at."""
 import os
 import shutil
 import subprocess
 
 import pytest
-
-from test_gmm_rows_gpu import EDGES, ROWS
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "hetu-galvatron_amd", "csrc")
 PROGRAM = """
@@ -16,28 +14,37 @@ PROGRAM = """
 #include <cstdio>
 int main() {
   long long v, a, b, c, d, e;
-  while (std::scanf("%lld %lld %lld %lld %lld %lld", &v, &a, &b, &c, &d, &e) == 6) {
-    const int units[5] = {(int)a, 0, (int)b, (int)c, (int)d};
-    const int col_tiles = (int)(e >> 32);
-    std::printf("%d\\n", v < 0 ? gmoe::rows_chunk_units(units, col_tiles, 256, e & 0xffffffff)
-                               : gmoe::rows_pays((gmoe::RowsKind)v, a, b, c, d, e));
-  }
+  while (std::scanf("%lld %lld %lld %lld %lld %lld", &v, &a, &b, &c, &d, &e) == 6)
+    std::printf("%d\\n", gmoe::rows_pays((gmoe::RowsKind)v, a, b, c, d, e));
 }
 """
 NN, GLU, NT, GLU_BWD = range(4)
 # kind, experts, rows per expert, K, M, us on the other tiles and on the row-adaptive ones
 MEASURED = [
-    (GLU, 8, 382, 4096, 28672, 1004, 724), (GLU, 64, 139, 2048, 2816, 238, 188), (GLU, 16, 640, 1024, 5632, 162, 168),
-    (GLU, 2, 668, 3936, 6400, 95, 73), (GLU, 4, 608, 3232, 1024, 33, 46),
-    (NN, 8, 382, 14336, 4096, 537, 330), (NN, 64, 139, 1408, 2048, 122, 94), (NN, 16, 640, 2816, 1024, 84, 69),
-    (NN, 32, 1024, 2048, 7168, 893, 857), (NN, 64, 267, 576, 832, 34, 41), (NN, 64, 921, 1536, 128, 39, 55),
-    (NN, 24, 1832, 640, 4480, 291, 327), (NN, 4, 336, 4832, 2432, 44, 58),
-    (NT, 8, 382, 28672, 4096, 1074, 737), (NT, 16, 640, 5632, 1024, 158, 137), (NT, 1, 1111, 2048, 11264, 72, 59),
-    (NT, 1, 1111, 5632, 2048, 51, 78), (NT, 8, 740, 14336, 4096, 644, 729), (NT, 64, 1000, 640, 128, 29, 38),
-    (NT, 8, 1000, 28672, 4096, 1809, 1891), (NT, 8, 600, 2056, 4104, 120, 156),
-    (GLU_BWD, 8, 382, 4096, 14336, 525, 455), (GLU_BWD, 16, 640, 1024, 2816, 128, 119),
-    (GLU_BWD, 8, 1000, 4096, 14336, 886, 945), (GLU_BWD, 48, 192, 1024, 1024, 55, 60),
-    (GLU_BWD, 32, 1024, 7168, 2048, 911, 1004),
+    (GLU, 8, 382, 4096, 28672, 975.7, 649.6), (GLU, 64, 139, 2048, 2816, 258.8, 165.3),
+    (GLU, 16, 640, 1024, 5632, 188.6, 138.3), (GLU, 2, 668, 3936, 6400, 105.5, 79.09),
+    (GLU, 4, 608, 3232, 1024, 39.14, 55.32), (NN, 8, 382, 14336, 4096, 437.4, 336.5),
+    (NN, 64, 139, 1408, 2048, 120, 89.89), (NN, 16, 640, 2816, 1024, 81.26, 62.77),
+    (NN, 32, 1024, 2048, 7168, 1165, 808.8), (NN, 64, 267, 576, 832, 44.72, 36.03),
+    (NN, 64, 921, 1536, 128, 52.02, 58.89), (NN, 24, 1832, 640, 4480, 380.2, 284.4),
+    (NN, 4, 336, 4832, 2432, 53.2, 72.43), (NT, 8, 382, 28672, 4096, 860.3, 628.4),
+    (NT, 16, 640, 5632, 1024, 159.3, 116.2), (NT, 1, 1111, 2048, 11264, 68.47, 53.81),
+    (NT, 1, 1111, 5632, 2048, 49.44, 77.36), (NT, 8, 740, 14336, 4096, 636.2, 530),
+    (NT, 64, 1000, 640, 128, 27.89, 30.87), (NT, 8, 1000, 28672, 4096, 1439, 1413),
+    (NT, 8, 600, 2056, 4104, 115.9, 112), (GLU_BWD, 8, 382, 4096, 14336, 469.8, 381.9),
+    (GLU_BWD, 16, 640, 1024, 2816, 102.7, 110.8), (GLU_BWD, 8, 1000, 4096, 14336, 1138, 835.9),
+    (GLU_BWD, 48, 192, 1024, 1024, 48.16, 47.56), (GLU_BWD, 32, 1024, 7168, 2048, 1119, 834.7),
+    (NN, 8, 363, 512, 5120, 32.26, 31.75), (NN, 24, 137, 2560, 10240, 414.5, 268),
+    (NN, 24, 5374, 2688, 224, 246, 174.1), (NN, 32, 941, 768, 128, 17.59, 24.39),
+    (NN, 2, 656, 1280, 1280, 14.29, 23.23), (NN, 4, 1701, 10848, 160, 79.07, 132.5),
+    (GLU, 32, 208, 128, 512, 12.15, 13.35), (GLU, 64, 389, 512, 14336, 908.1, 621.9),
+    (GLU, 4, 1318, 1952, 1504, 60.4, 49.96), (GLU, 4, 103, 768, 1024, 12.61, 18.11),
+    (GLU, 8, 121, 7168, 256, 64.92, 94.84), (NT, 1, 1185, 1792, 7552, 45.63, 42.35),
+    (NT, 4, 938, 12544, 2112, 282.8, 216.3), (NT, 32, 203, 1392, 1968, 76.45, 59.1),
+    (NT, 24, 222, 12256, 192, 81.63, 193.8), (NT, 4, 1769, 1408, 512, 16.43, 23.71),
+    (NT, 1, 866, 19968, 1536, 95.51, 260.5), (GLU_BWD, 60, 386, 6272, 2688, 1231, 909.3),
+    (GLU_BWD, 24, 124, 128, 2560, 20.62, 22.03), (GLU_BWD, 2, 1917, 1888, 3936, 96.82, 75.48),
+    (GLU_BWD, 6, 599, 304, 544, 15.36, 29.33), (GLU_BWD, 4, 322, 4992, 1024, 52.84, 73.34),
 ]
 
 
@@ -60,36 +67,31 @@ def evaluate(tmp_path_factory):
 
 
 def test_choice(evaluate):
+    """Over the measured launches, short reductions and small launches among them, the choice takes less than 1 % longer than
+    the better side of each on average and 15 % at most."""
     got = evaluate([(kind, E, n * E, K, M, 256) for kind, E, n, K, M, _, _ in MEASURED])
-    wrong = [c for c, v in zip(MEASURED, got) if v != (c[6] < c[5])]
-    assert not wrong, wrong
-    # no rows, fewer than 96, reductions of up to 512, 2048 rows and more: never; one expert and a thousand: an answer
-    shapes = [(E, n, K, M) for E in (1, 8, 1024) for n in (0, 1, 95, 96, 2047, 2048) for K in (8, 512, 520, 4096)
-              for M in (8, 128, 4096)]
+    lost = [(c[5], c[6])[v] / min(c[5], c[6]) - 1 for c, v in zip(MEASURED, got)]
+    worst = max(zip(lost, MEASURED))
+    assert worst[0] < 0.15 and sum(lost) / len(lost) < 0.01, (sum(lost) / len(lost), worst)
+
+
+def test_few_rows(evaluate):
+    """The launch with the activation: where its tiles fill nine tenths of their rounds or more.  us in the other tiles and in
+    these, as above but with all rows."""
+    measured = [(8, 26, 4096, 28672, 319.1, 350.5), (8, 128, 4096, 28672, 331.5, 363.4), (64, 1024, 2048, 2816, 142.1, 131.4),
+                (64, 2664, 2048, 2816, 152.3, 139.8), (16, 256, 1024, 5632, 42.6, 46.5), (16, 1024, 1024, 5632, 47, 54.5),
+                (32, 8, 7168, 4096, 83.7, 104.9), (4, 128, 128, 512, 8.3, 9.6), (4, 104, 2368, 6400, 30.6, 38.4)]
+    got = evaluate([(GLU, *c[:4], 256) for c in measured])
+    assert got == [int(c[5] < c[4]) for c in measured]
+    assert not any(evaluate([(kind, *c[:4], 256) for c in measured for kind in (NN, NT, GLU_BWD)]))
+
+
+def test_limits(evaluate):
+    """Fewer than 96 rows per expert, with the activation none at all: never; one expert and a thousand, the smallest and
+    the longest reductions: an answer; the largest launches: always."""
+    shapes = [(E, n, K, M) for E in (1, 8, 1024) for n in (0, 1, 95, 96, 2048, 65536) for K in (8, 512, 65536) for M in (8, 4096)]
+    large = [(8, 4096, 4096, 28672), (8, 16384, 14336, 4096), (64, 4096, 2048, 2816), (1, 32768, 8192, 8192)]
     for kind in (NN, GLU, NT, GLU_BWD):
         for (E, n, K, M), v in zip(shapes, evaluate([(kind, E, n * E, K, M, 256) for E, n, K, M in shapes])):
-            assert v in (0, 1) and not (v and (n < 96 or n >= 2048 or K <= 512)), (kind, E, n, K, M)
-
-
-def test_chunks(evaluate):
-    """Chunks of up to 256, 192 and 128 rows against the rule in Python, for the edge test on the GPU, which reaches all
-    three; no rows at all; one tile."""
-    def units(rows):
-        u = [-(-r // 64) for r in rows]
-        return [sum(u)] + [sum(-(-x // size) for x in u) for size in (2, 3, 4)]
-
-    def model(counts, col_tiles, K):
-        best, least = 4, None
-        for size in (4, 3, 2):
-            chunks = counts[size - 1]
-            cost = -(-chunks * col_tiles // 256) * (16 + 250 / -(-K // 32) + 4 * counts[0] / max(chunks, 1))
-            if least is None or cost < 0.95 * least:
-                best, least = size, cost
-        return best
-
-    edges = [(units(ROWS * times), cols, K) for K, F, times in EDGES for cols in (-(-F // 128), -(-F // 256))]
-    other = [(units(rows), cols, K) for rows in ([0, 0], [1], [640] * 16, [256] * 64, [370] * 8) for cols in (1, 4, 6, 25)
-             for K in (520, 1024, 5632)]
-    got = evaluate([(-1, *counts, cols << 32 | K) for counts, cols, K in edges + other])
-    assert got == [model(*c) for c in edges + other]
-    assert set(got[:len(edges)]) == {2, 3, 4}
+            assert v in (0, 1) and not (v and n < (1 if kind == GLU else 96)), (kind, E, n, K, M)
+        assert all(evaluate([(kind, E, n * E, K, M, 256) for E, n, K, M in large])), kind

@@ -1,11 +1,11 @@
-"""Which 16-bit NN / NT launches go to the row-adaptive tiles beyond those of rows_pays, where both sides were measured,
-and the chunks of up to 384 rows (csrc/rows_rule.h)."""
+"""The chunks of up to 384 rows that the row-adaptive tiles cut an expert's rows into (csrc/rows_rule.h)."""
 import os
 import shutil
 import subprocess
 
 import pytest
 
+from test_gmm_rows_gpu import EDGES, ROWS
 from test_gmm_tall_gpu import TALL
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "hetu-galvatron_amd", "csrc")
@@ -15,31 +15,14 @@ PROGRAM = """
 #include "rows_rule.h"
 #include <cstdio>
 int main() {
-  long long v, a, b, c, d;
-  while (std::scanf("%lld %lld %lld %lld %lld", &v, &a, &b, &c, &d) == 5) {
-    if (v >= 0) {
-      std::printf("%d\\n", gmoe::tall_pays((gmoe::RowsKind)v, a, b, c, d, 256));
-      continue;
-    }
+  long long a, b, c, d;
+  while (std::scanf("%lld %lld %lld %lld", &a, &b, &c, &d) == 4) {
     int u[7] = {};
     for (int i = 0; i < 7; ++i) if (std::scanf("%d", u + i) != 1) return 1;
-    std::printf("%d\\n", gmoe::rows_chunk_units(u, (int)a, (int)b, c, 1.f, d ? gmoe::kChunkCostsGluBwd : gmoe::kChunkCosts));
+    std::printf("%d\\n", gmoe::rows_chunk_units(u, (int)a, (int)b, c, d ? gmoe::kChunkCostsGluBwd : gmoe::kChunkCosts));
   }
 }
 """
-NN, GLU, NT, GLU_BWD = range(4)
-# kind, experts, rows per expert, K, M, us on 128x128 tiles and on the row-adaptive ones
-MEASURED = [
-    (NN, 8, 363, 512, 5120, 35.1, 28.6), (NN, 24, 137, 2560, 10240, 389, 264), (NN, 24, 5374, 2688, 224, 241, 176),
-    (NN, 32, 941, 768, 128, 18.0, 20.4), (NN, 2, 656, 1280, 1280, 18.0, 24.6), (NN, 4, 1701, 10848, 160, 80.4, 130),
-    (GLU, 32, 208, 128, 512, 16.6, 13.8), (GLU, 64, 389, 512, 14336, 924, 562), (GLU, 4, 1318, 1952, 1504, 60.0, 48.4),
-    (GLU, 4, 103, 768, 1024, 15.8, 19.4), (GLU, 8, 121, 7168, 256, 71.9, 101),
-    (NT, 1, 1185, 1792, 7552, 50.9, 38.3), (NT, 4, 938, 12544, 2112, 280, 217), (NT, 32, 203, 1392, 1968, 80.5, 54.8),
-    (NT, 24, 222, 12256, 192, 83.5, 199), (NT, 4, 1769, 1408, 512, 19.7, 25.5), (NT, 1, 866, 19968, 1536, 97.1, 260),
-    (GLU_BWD, 60, 386, 6272, 2688, 1210, 956), (GLU_BWD, 24, 124, 128, 2560, 30.0, 23.3),
-    (GLU_BWD, 2, 1917, 1888, 3936, 95.1, 69.2), (GLU_BWD, 6, 599, 304, 544, 15.8, 26.4),
-    (GLU_BWD, 4, 322, 4992, 1024, 53.6, 72.7),
-]
 
 
 @pytest.fixture(scope="module")
@@ -60,40 +43,33 @@ def evaluate(tmp_path_factory):
     return run
 
 
-def test_choice(evaluate):
-    got = evaluate([(kind, E, n * E, K, M) for kind, E, n, K, M, _, _ in MEASURED])
-    wrong = [c for c, v in zip(MEASURED, got) if v != (c[6] < c[5])]
-    assert not wrong, wrong
-    # fewer than 96 rows, with the activation less than one: never; one expert and a thousand, the smallest and long
-    # reductions: an answer
-    shapes = [(E, n, K, M) for E in (1, 8, 1024) for n in (0, 1, 95, 96, 2048, 65536) for K in (8, 512, 65536) for M in (8, 4096)]
-    for kind in (NN, GLU, NT, GLU_BWD):
-        for (E, n, K, M), v in zip(shapes, evaluate([(kind, E, n * E, K, M) for E, n, K, M in shapes])):
-            assert v in (0, 1) and not (v and n < (1 if kind == GLU else 96)), (kind, E, n, K, M)
+def counts(rows):
+    u = [-(-r // 64) for r in rows]
+    return [sum(u), 0] + [sum(-(-x // size) for x in u) for size in range(2, 7)]
 
 
 def test_chunks(evaluate):
-    """Chunks of up to 384 rows against the rule in Python, for the edge test on the GPU, which reaches tiles of five and
-    six units (of 64 rows); no rows at all; one tile."""
-    def units(rows):
-        u = [-(-r // 64) for r in rows]
-        return [sum(u), 0] + [sum(-(-x // size) for x in u) for size in range(2, 7)]
-
-    def model(counts, col_tiles, K):
-        best, least = 6, None
+    """The rule against one in Python, for the edge tests on the GPU, which reach tiles of two, three, five and six units (of
+    64 rows), in the activation backward of six; no rows at all; one tile."""
+    def model(counts, col_tiles, K, bwd):
+        per_stage, around, unit, tall = (8, 120, 650, 1.04) if bwd else (16, 250, 0, 1)
+        best, least, stages = 6, None, -(-K // 32)
         for size in range(6, 1, -1):
             chunks = counts[size]
-            cost = -(-chunks * col_tiles // 256) * (16 + 250 / -(-K // 32) + 4 * counts[0] / max(chunks, 1))
+            cost = -(-chunks * col_tiles // 256) * (
+                per_stage + around / stages + (4 + unit / stages) * counts[0] / max(chunks, 1)) * (tall if size > 4 else 1)
             if least is None or cost < least:
                 best, least = size, cost
         return best
 
-    edges = [(units(rows), cols, K) for rows, K, F in TALL for cols in (-(-F // 128), -(-F // 256))]
-    other = [(units(rows), cols, K) for rows in ([0, 0], [1], [640] * 16, [256] * 64, [370] * 8, [1024] * 64)
-             for cols in (1, 4, 6, 25) for K in (520, 1024, 5632)]
-    got = evaluate([(-1, cols, 256, K, 0, *counts) for counts, cols, K in edges + other])
+    edges = [(counts(rows), cols, K, bwd) for rows, K, F in [(ROWS * times, K, F) for K, F, times in EDGES] + TALL
+             for cols, bwd in ((-(-F // 128), 0), (-(-F // 256), 0), (-(-F // 256), 1))]
+    other = [(counts(rows), cols, K, bwd) for rows in ([0, 0], [1], [640] * 16, [256] * 64, [370] * 8, [1024] * 64)
+             for cols in (1, 4, 6, 25) for K in (520, 1024, 5632) for bwd in (0, 1)]
+    got = evaluate([(cols, 256, K, bwd, *units) for units, cols, K, bwd in edges + other])
     assert got == [model(*c) for c in edges + other]
-    assert {5, 6} <= set(got[:len(edges)])
+    for bwd, sizes in ((0, {2, 3, 5, 6}), (1, {2, 3, 6})):
+        assert sizes <= {u for u, c in zip(got, edges) if c[3] == bwd}
 
 
 # rows of the experts, K, F, us of the activation backward in chunks of up to 128 / 192 / 256 / 320 / 384 rows
@@ -110,12 +86,8 @@ BACKWARD = [
 def test_chunks_of_the_activation_backward(evaluate):
     """Its chunks take 2.5 % longer than the best of those measured on average and 6 % at most; chosen by the other products'
     costs they take 6 % and 14 %.  No rows at all has an answer."""
-    def counts(rows):
-        u = [-(-r // 64) for r in rows]
-        return [sum(u), 0] + [sum(-(-x // size) for x in u) for size in range(2, 7)]
-
-    cases = [(-1, -(-F // 256), 256, K, 1, *counts(rows)) for rows, K, F, _ in BACKWARD]
-    got = evaluate(cases + [(-1, 4, 256, 8, 1, *counts([0, 0]))])
+    cases = [(-(-F // 256), 256, K, 1, *counts(rows)) for rows, K, F, _ in BACKWARD]
+    got = evaluate(cases + [(4, 256, 8, 1, *counts([0, 0]))])
     lost = [c[3][u - 2] / min(c[3]) - 1 for c, u in zip(BACKWARD, got)]
     assert max(lost) < 0.06 and sum(lost) / len(lost) < 0.025, list(zip(got, lost))
     assert 2 <= got[-1] <= 6
