@@ -951,15 +951,11 @@ static int launch_gmm_cfg(const GmmParams& p, hipStream_t st, int blocks_per_cu 
   return gmoe_launch_status();
 }
 
-// Large tiles once an expert's share of rows (NN/NT, nn_large_tiles) or the output itself (TN) can fill them and
-// there are enough of them for every CU; smaller problems spread over more, smaller tiles.
+// Large tiles once an expert's share of rows (NN/NT, nn_large_tiles) or the output itself (TN, tn_large_tiles) can fill
+// them and there are enough of them for every CU; smaller problems spread over more, smaller tiles.
 static inline bool gmm_large_tiles(const GmmParams& p, int mode) {
   const int64_t experts = p.E > 0 ? p.E : 1;
-  if (mode != MODE_TN) return nn_large_tiles(experts, p.N, p.M);
-  // TN: the 128x128 kernel runs at about 0.4 of the large one's rate per FLOP, so the large tiles win
-  // as soon as the small ones need a second round of their 512 slots (C3's shared experts, 176 large
-  // tiles: 0.29 -> 0.22 ms)
-  return p.K >= 512 && p.M >= 256 && experts * ((p.K + 255) / 256) * ((p.M + 255) / 256) >= 129;
+  return mode == MODE_TN ? tn_large_tiles(experts, p.K, p.M) : nn_large_tiles(experts, p.N, p.M);
 }
 
 // Row-adaptive tiles (gmm_rows_kernel.h) for 16-bit NN / NT: tiles of 64 to 384 rows x 256 columns that share an expert's
@@ -969,59 +965,6 @@ static inline bool gmm_rows_pays(const GmmParams& p, int mode, int epi) {
   const RowsKind kind = mode == MODE_NN ? (epi == EPI_NONE ? ROWS_NN : ROWS_NN_GLU)
                                         : (epi == EPI_NONE ? ROWS_NT : ROWS_NT_GLU_BWD);
   return kTallMaxUnits * 64 * p.K * 2 < (1ll << 31) && rows_pays(kind, p.E, p.N, p.K, p.M, gmm_grid(1));
-}
-
-// dW of 16-bit operands with a short reduction (gmm_tn.hip: 128x256 tiles, two workgroups per CU) against the
-// 256x256 LDS-DMA kernel, or 128x128 tiles where that one does not apply; n = rows per expert, us of that kernel /
-// of this one.  From one round of 256x256 tiles on that kernel, whose tiles run into each other, is the faster one
-// (n 128 402 / 484, n 383 784 / 879, n 1024 1671 / 1875, 8 experts of 4096 x 28672) except for few rows: n 24, 8
-// experts of 6144 x 16384 291 / 266, n 48 291 / 297, n 96 299 / 368; in whole steps n 8 717 / 707, n 32 1662 / 1649,
-// n 45 1693 / 1692, n 56 834 / 846, n 75 1752 / 1824, n 100 1128 / 1182 us. A result under 256 MB has the ordinary
-// stores there and nontemporal ones here, which moves the line: 1024 x 5632, 16 n 24 44 / 41, n 64 45 / 44, n 96 49
-// / 47; 1024 x 1024, 64 n 64 33 / 34, n 96 37 / 36; 2048 x 1184, 32 n 64 40 / 40, n 96 42 / 43.  With less than a
-// round of 256x256 tiles, and where its rows would be padding (K under 512), the smaller tiles spread better: 128
-// tiles of 256x256 14.0 / 11.1 (n 256, 1024 x 1024, 8), 240 17.8 / 15.4 (n 300, 640 x 1280, 16), n 384 of 384 x
-// 4096 over 64 159 / 117.  That holds beyond the 768 rows up to which it is used (n 1024 of 1024 x 1024 29.4 /
-// 22.5).  Fewer than three quarters of a tile per CU stay with 128x128 ones (128 tiles of 1024 x 512, 8: 10.1 /
-// 9.9).
-constexpr int64_t kTnFewRows = 112, kTnFewRowsStreamed = 48;
-static inline bool gmm_tn_short_pays(const GmmParams& p) {
-  const int64_t n = p.N / (p.E > 0 ? p.E : 1), col_tiles = (p.M + 255) / 256;
-  if (p.K < 128 || p.M < 256 || p.E * ((p.K + 127) / 128) * col_tiles * 4 < gmm_grid(1) * 3) return false;
-  const bool few = n < (gmm_tn_streams(p) ? kTnFewRowsStreamed : kTnFewRows);
-  if (!few && p.K >= 512 && p.E * ((p.K + 255) / 256) * col_tiles >= gmm_grid(1)) return false;
-  return n <= 768;
-}
-
-// dW outside those two rules (narrow results: K under 512, M under 256, or fewer than 129 tiles of 256x256): the
-// kernel with the least estimated time, us, of n rows per expert in `rounds` rounds of its tiles.  Two workgroups of
-// the smaller tiles share a CU, and a last round of at most half their slots takes `half` of one.  Fitted to 1400
-// launches of 1 to 64 experts, 100 to 9000 rows each, K and M of 128 to 16000, one of them at most 1024; an estimate
-// has to be 8 % better to leave the 128x128 tiles.  Over those launches 1.05 times as fast as the two rules alone
-// (total time 1.08), the changed ones 1.33 (to 256x256) and 1.23 times (to 128x256); 9 are more than 3 % slower, down
-// to 0.78.  E.g. 4382 rows, 8 experts, 256 x 19968 512 -> 345 us, and in whole steps, bf16: 8765 tokens of 256, 8
-// experts of 9984, top 4 2927 -> 2793 us; 4000 of 384, 8 of 6144 1265 -> 1235; 3000 of 320, 32 of 2048 504 -> 507.
-struct TnCosts {
-  int rows, cols, per_cu;
-  double launch, round, per_row, half;
-};
-constexpr TnCosts kTnSmall = {128, 128, 2, 6.4, 4.83, 0.0203, 0.39}, kTnLarge = {256, 256, 1, 1.8, 7.75, 0.0217, 1.0},
-                  kTnShort = {128, 256, 2, 5.7, 4.35, 0.0319, 0.42};
-static inline double tn_estimate(const TnCosts& c, const GmmParams& p) {
-  const int64_t experts = p.E > 0 ? p.E : 1;
-  const int64_t tiles = experts * ((p.K + c.rows - 1) / c.rows) * ((p.M + c.cols - 1) / c.cols);
-  const int64_t slots = (int64_t)c.per_cu * gmm_grid(1), rest = tiles % slots;
-  const double rounds = (double)(tiles / slots) + (rest == 0 ? 0.0 : rest * 2 <= slots ? c.half : 1.0);
-  return c.launch + rounds * (c.round + c.per_row * (double)(p.N / experts));
-}
-enum TnKernel { TN_SMALL, TN_LARGE, TN_SHORT };
-static inline TnKernel gmm_tn_kernel(const GmmParams& p) {
-  if (gmm_tn_short_pays(p)) return TN_SHORT;
-  if (gmm_large_tiles(p, MODE_TN)) return TN_LARGE;
-  if (p.K < 128 || p.M < 128) return TN_SMALL;
-  const double t_large = tn_estimate(kTnLarge, p), t_short = tn_estimate(kTnShort, p);
-  if ((t_large < t_short ? t_large : t_short) >= 0.92 * tn_estimate(kTnSmall, p)) return TN_SMALL;
-  return t_large < t_short ? TN_LARGE : TN_SHORT;
 }
 
 // Whether reading the operands beforehand (warm_operands) pays: they take bytes / 5 TB/s, and the launch has to be
@@ -1083,10 +1026,7 @@ static int launch_gmm_16bit(const GmmParams& p, int dtype, int out_dtype, hipStr
     GmmParams q = p;
     q.warm = gmm_tn_warm_pays(p);
     // 32-bit results (the gate's) were not part of the fit
-    const TnKernel kernel = ODT != GMOE_F32          ? gmm_tn_kernel(p)
-                            : gmm_tn_short_pays(p)   ? TN_SHORT
-                            : gmm_large_tiles(p, MODE) ? TN_LARGE
-                                                       : TN_SMALL;
+    const TnKernel kernel = tn_kernel(p.E, p.N, p.K, p.M, gmm_grid(1), ODT != GMOE_F32);
     if (kernel == TN_SHORT) return launch_gmm_tn_short(q, dtype, out_dtype, st);
     if (kernel == TN_LARGE) return launch_gmm_dtl_tn(q, dtype, out_dtype, st);
   } else {

@@ -6,6 +6,7 @@
 #include "gmoe_common.h"
 #include "copy_range.h"
 #include "rows_rule.h"
+#include "tn_rule.h"
 #include "split_rule.h"
 
 namespace gmoe {
@@ -97,7 +98,7 @@ __host__ __device__ __forceinline__ int64_t tn_segment_rows(int64_t K, int64_t M
 }
 
 // TN: a result that does not fit the memory-side cache (256 MB) beside the operands.
-static inline bool gmm_tn_streams(const GmmParams& p) { return p.E * p.K * p.M * 2 >= (256ll << 20); }
+static inline bool gmm_tn_streams(const GmmParams& p) { return tn_streams(p.E, p.K, p.M); }
 
 // TN of few rows per expert: the results are most of the traffic, and copies of operands that come from
 // HBM queue behind the stores, a latency that the few K tiles of an output tile cannot hide.  One pass over
