@@ -235,13 +235,23 @@ __attribute__((noinline)) __device__ void glu_bwd_rows(const unsigned char* lds,
 }
 
 // acc += b a with the accumulators in architectural registers: the compiler puts those of the builtin into the
-// accumulation registers, which hold 16 fragments.
+// accumulation registers, which hold 16 fragments.  It inserts no wait states around assembly: mma_ready and mma_settle bring
+// those before the first and after the last, and in between no vector instruction may write an operand in the two wait
+// states before, or touch the result in the 18 after, which the built kernels are tested for.  (The two wait states in
+// front of each one: 1 % slower, NN and NT of 4096 rows, 14336 x 4096 and 28672 x 4096, 8 experts.)
 template <int DT>
 __device__ __forceinline__ void mma_vgpr(const u32x4& a, const u32x4& b, f32x16& acc) {
   if constexpr (DT == GMOE_BF16)
     asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(b), "v"(a));
   else
     asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+v"(acc) : "v"(b), "v"(a));
+}
+
+// Between vector instructions that wrote operands of mma_vgpr and the first of them.
+__device__ __forceinline__ void mma_ready() {
+  GMOE_SCHED_FENCE();
+  asm volatile("s_nop 1");
+  GMOE_SCHED_FENCE();
 }
 
 // Before vector instructions read what mma_vgpr wrote: the compiler does not know how long that takes (up to 16 passes
@@ -297,7 +307,6 @@ __device__ __forceinline__ void run_tile(const GmmParams& p, const Item& it, uns
     for (int j = 0; j < 4; ++j)
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
-
   OpA oa;
   OpB ob;
   oa.init(p.a + it.row0 * K * 2, K, 0, it.n, RF * kUnit, K, wave, lane, wm * RF * 32);
@@ -369,6 +378,7 @@ __device__ __forceinline__ void run_tile(const GmmParams& p, const Item& it, uns
     wait_dma_outstanding<wait_y + N3>();
     __syncthreads();
     static_for<0, NREAD>(read_frags(c0, lds, ring_b));
+    if constexpr (RF > 4) mma_ready();
     int sa = 0, sb = 0;            // slots of tile kt
     int la = NA - 1, lb = NB - 1;  // slots of tiles kt - 1 + NA of A and kt - 1 + NB of B
     for (int kt = 0; kt < kt_cnt; ++kt) {
@@ -430,6 +440,7 @@ __device__ __forceinline__ void run_tile(const GmmParams& p, const Item& it, uns
     __syncthreads();
     static_for<0, NREAD>(read_frags(c0, lds, ring_b));
     static_for<0, A3>([&](auto q) { issue_a(q, NA - 1, oa.offset(NA - 1), NA - 1); });
+    if constexpr (RF > 4) mma_ready();
     int sa = 0, sb = 0;    // slots of tiles p of A and 2 p of B
     int la = NA - 1, lb = NB - 1;  // slots of tiles p - 1 + NA of A and 2 p - 1 + NB of B
     for (int p2 = 0; p2 < kt_cnt; ++p2) {
