@@ -298,7 +298,7 @@ class SharedExpertMLP(torch.nn.Module):
     enqueue on the current one."""
 
     stream = None  # shared by all instances, default priority
-    overlap_min_us = 150.0  # see _stage_stream
+    overlap_min_us, overlap_min_us_captured = 150.0, 1.0  # see _stage_stream
 
     def __init__(self, config: MoEConfig, gate: bool = False, device=None):
         super().__init__()
@@ -364,7 +364,10 @@ class SharedExpertMLP(torch.nn.Module):
         whichever is longer.  us per step with the side stream / without (estimate): 708 tokens of 192, 32 experts
         of 512, shared 4336 685 / 520 (5); 8345 of 1408, 8 of 384, top 4, shared 384 843 / 1005 (169); 512 of
         2048, 64 of 1408, top 6, shared 2816 977 / 999 (248); forward alone 512 of 1024, 16 of 2048, shared 4096 216
-        / 162 (50); 16 of 2048, 64 of 1408, top 6, shared 2816 245 / 269 (248)."""
+        / 162 (50); 16 of 2048, 64 of 1408, top 6, shared 2816 245 / 269 (248).
+        A graph that is being captured costs the host nothing when it is replayed, so all but the smallest layers take the
+        second stream there.  us of a replayed forward: 512 of 1024, 16 of 2048, shared 4096 125 / 136 (50); 4 of 512, 8 of
+        1024, shared 1024 68 / 71 (6); 128 of 128, 4 of 256, shared 512 70 / 63 (0.3)."""
         cfg, H = self.config, x.shape[-1]
         tokens = x.numel() // H if H else 0
         experts, rows = cfg.num_moe_experts or 0, tokens * (cfg.moe_router_topk or 0)
@@ -372,7 +375,8 @@ class SharedExpertMLP(torch.nn.Module):
         weights = 3.0 * x.element_size() * H * (min(experts, rows) * routed + shared)
         products = 6.0 * H * (rows * routed + tokens * shared)
         us = max(weights / 4.5e6, products / (1.2e8 if x.dtype == torch.float32 else 8e8))
-        return SharedExpertMLP.stream if us >= self.overlap_min_us else torch.cuda.current_stream()
+        least = self.overlap_min_us_captured if torch.cuda.is_current_stream_capturing() else self.overlap_min_us
+        return SharedExpertMLP.stream if us >= least else torch.cuda.current_stream()
 
     def _stage(self):
         stream = self._staged["stream"]

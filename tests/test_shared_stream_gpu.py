@@ -83,3 +83,34 @@ def test_captured_side_stream_replays_the_eager_bits(pkg, dev, monkeypatch):
             torch.cuda.synchronize()
             assert torch.equal(out, want)
             torch.cuda.synchronize()
+
+
+def test_small_layers_overlap_in_a_captured_graph(pkg, dev):
+    """A layer that stays on the current stream when it is called takes the second one when it is captured, and replays the
+    same bits; the smallest stay on one stream there too."""
+    _, router, mlp = build(pkg, dev, torch.bfloat16, overlap=True, E=16, H=1024, F=512, Fs=1024, k=2)
+    _, _, least = build(pkg, dev, torch.bfloat16, overlap=True)
+    shared, side = mlp.shared_experts, pkg.SharedExpertMLP.stream
+    g = torch.Generator().manual_seed(9)
+    x = torch.randn(32, 2, 1024, generator=g).bfloat16().to(dev)
+    little = torch.zeros(1, 1, 256, device=dev, dtype=torch.bfloat16)
+    assert shared._stage_stream(x) != side
+    with torch.no_grad():
+        want = mlp(x, x, *router(x))
+        warm = torch.cuda.Stream()
+        warm.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(warm):
+            for _ in range(2):
+                mlp(x, x, *router(x))
+        torch.cuda.current_stream().wait_stream(warm)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            chosen = shared._stage_stream(x), least.shared_experts._stage_stream(little)
+            out = mlp(x, x, *router(x))
+        assert chosen[0] == side and chosen[1] != side
+        for _ in range(3):
+            out.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want)
+            assert torch.equal(mlp(x, x, *router(x)), want)
