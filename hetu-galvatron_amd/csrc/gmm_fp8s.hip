@@ -123,10 +123,14 @@ __device__ __forceinline__ u32x4 uniform_rsrc(const u32x4& r) {
   return u32x4{(uint32_t)__builtin_amdgcn_readfirstlane(r[0]), (uint32_t)__builtin_amdgcn_readfirstlane(r[1]),
                (uint32_t)__builtin_amdgcn_readfirstlane(r[2]), (uint32_t)__builtin_amdgcn_readfirstlane(r[3])};
 }
-// bf16 activations: where the next stage's copies go and come from, carried from stage to stage.  Stages past the
-// reduction are requested too: at the resource's end.  (Everything in scalar registers, and computed under the
-// MFMAs: 4096 rows x 7168 x 4096 over 30 experts 335 -> 320 us.  Stages of fp8 activations are shorter and gain
-// nothing; there the copies are placed from the stage's number.)
+// bf16 activations: where the next stage's copies go and come from, carried from stage to stage.  (Everything in scalar
+// registers, and computed under the MFMAs: 4096 rows x 7168 x 4096 over 30 experts 335 -> 320 us.  Stages of fp8
+// activations are shorter and gain nothing; there the copies are placed from the stage's number.)
+//
+// Stages past the reduction are requested too.  Those of NN weights begin at the resource's end and read nothing; the
+// activations and NT weights, which are contiguous in the reduction, go on with the first elements of their next rows,
+// which nothing multiplies.  Begun at the resource's end they cost no traffic, but the choice costs more than that: bf16
+// rows, 7168 x 4096, 30 experts, NT of 13 rows 178 -> 177 us, NN of 136 rows 306 -> 311; fp8 rows 181 -> 177 and 211 -> 216.
 template <int NJ>
 struct Ahead {
   u32x4 rsrc_a, rsrc_b;
@@ -306,7 +310,7 @@ __device__ __forceinline__ void run_item(unsigned char* lds, uint32_t lds0, cons
   for (int kt = 0; kt < kt_cnt; ++kt) {
     // stage kt has landed (those after it may still be in flight); after the barrier every wavefront
     // sees it and has finished with stage kt-1, whose buffer the next copies overwrite.  Copies
-    // past the reduction read zeros: the count of outstanding copies stays the same to the end.
+    // are requested past the reduction too: the count of outstanding ones stays the same to the end.
     wait_dma_outstanding<(C::AHEAD - 1) * C::LOADS_PER_STAGE>();
     __syncthreads();
     issue_stage<NT, NJ>(lds0, ln, wave, at);
@@ -742,7 +746,7 @@ __global__ __launch_bounds__(THREADS, 1) void gmm_fp8_skinny_kernel(GmmParams p)
     cur = nxt;
     at = request();
   }
-  // the copies requested past the last reduction (zeros) land before the workgroup ends
+  // the copies requested past the last reduction land before the workgroup ends
   wait_dma_outstanding<0>();
 }
 
