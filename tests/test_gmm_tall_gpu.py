@@ -59,6 +59,41 @@ def test_tall_edges(pkg, dev, dtype, rows, K, F, act):
         s += n
 
 
+# rows of the experts, K, F: averages of 1 to 95 rows, where tiles of the experts that have rows fill a round
+FEW = [
+    ([0, 1] * 32 + [3, 0, 0, 95], 264, 1024),          # most experts empty, one row
+    ([1] * 64, 72, 768),
+    ([63, 64, 65, 0, 127, 128, 129, 1] * 4, 1160, 1016),  # around one and two units (of 64 rows), ragged K and F
+    ([95, 0, 200, 33, 7, 383, 1, 0], 520, 4088),
+    ([17], 2056, 32760),
+]
+
+
+@pytest.mark.parametrize("act", ["silu", "gelu"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,K,F", FEW)
+def test_few_rows_with_the_activation(pkg, dev, dtype, rows, K, F, act):
+    """fc1 against float64, and the activation to the bits of its own kernel."""
+    E, N = len(rows), sum(rows)
+    assert N // E < 96
+    g = torch.Generator(device=dev).manual_seed(K + F)
+    print("case", dtype, K, F, act, flush=True)
+    off = torch.tensor([0] + rows, device=dev).cumsum(0)
+    a = torch.empty(N, K, device=dev).normal_(generator=g).to(dtype)
+    w1 = torch.empty(E, K, 2 * F, device=dev).normal_(0.0, K ** -0.5, generator=g).to(dtype)
+    fc1, h = on_kernel("gmm_rows_kernel", lambda: pkg.ops.gmm_glu(a, w1, off, act))
+    assert torch.equal(h, pkg.ops.glu_fwd(fc1, act))
+    # as above, and half a unit of 8 or 11 bits for the 16-bit result
+    tol = 8 * 2.0 ** -24 * max(K, 64) ** 0.5 * 4
+    half = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    s = 0
+    for e, n in enumerate(rows):
+        if n:
+            want = a[s:s + n].double() @ w1[e].double()
+            assert ((fc1[s:s + n].double() - want).abs() - want.abs() * half).max().item() < tol + 2.0 ** -25, e
+        s += n
+
+
 @pytest.mark.parametrize("K,M", [(8, 2056), (72, 2312), (4104, 2056), (1000, 2304)])
 def test_tall_transposed(pkg, dev, K, M):
     """Plain NT of 768 rows per expert and more, with reductions of a few elements up to many rounds."""
