@@ -961,10 +961,21 @@ static inline bool gmm_large_tiles(const GmmParams& p, int mode) {
 // Row-adaptive tiles (gmm_rows_kernel.h) for 16-bit NN / NT: tiles of 64 to 384 rows x 256 columns that share an expert's
 // rows evenly, one workgroup per CU; the rule with both sides' times is in rows_rule.h.  The kernel's resource of a tile
 // spans 384 rows.
+static inline bool gmm_rows_fits(const GmmParams& p) { return kTallMaxUnits * 64 * p.K * 2 < (1ll << 31); }
 static inline bool gmm_rows_pays(const GmmParams& p, int mode, int epi) {
   const RowsKind kind = mode == MODE_NN ? (epi == EPI_NONE ? ROWS_NN : ROWS_NN_GLU)
                                         : (epi == EPI_NONE ? ROWS_NT : ROWS_NT_GLU_BWD);
-  return kTallMaxUnits * 64 * p.K * 2 < (1ll << 31) && rows_pays(kind, p.E, p.N, p.K, p.M, gmm_grid(1));
+  return gmm_rows_fits(p) && rows_pays(kind, p.E, p.N, p.K, p.M, gmm_grid(1));
+}
+// The same for fc1 with its activation where the host's time decides.
+static inline bool gmm_one_launch_pays(const GmmParams& p, hipStream_t st) {
+  if (!gmm_rows_fits(p) || !rows_one_launch_pays(p.E, p.N, p.K, p.M, gmm_grid(1))) return false;
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &capture) != hipSuccess) {
+    (void)hipGetLastError();  // the launch that follows says what is wrong with the stream
+    return false;
+  }
+  return capture == hipStreamCaptureStatusNone;
 }
 
 // Whether reading the operands beforehand (warm_operands) pays: they take bytes / 5 TB/s, and the launch has to be
@@ -1021,7 +1032,6 @@ static int launch_gmm_split(const GmmParams& p, hipStream_t st) {
 // MFMA with a smaller error; the fp32 MFMA kernels serve dW of operands beyond 2 GiB.
 template <int DT, int ODT, int MODE, int EPI>
 static int launch_gmm_16bit(const GmmParams& p, int dtype, int out_dtype, hipStream_t st) {
-  constexpr bool glu_fwd = EPI == EPI_GLU_FWD_SILU || EPI == EPI_GLU_FWD_GELU;
   if constexpr (MODE == MODE_TN) {
     GmmParams q = p;
     q.warm = gmm_tn_warm_pays(p);
@@ -1035,15 +1045,10 @@ static int launch_gmm_16bit(const GmmParams& p, int dtype, int out_dtype, hipStr
   if (MODE != MODE_TN && gmm_large_tiles(p, MODE)) {
     if constexpr (MODE == MODE_NT && EPI == EPI_NONE) return launch_gmm_cfg<DT, ODT, MODE_NT, 256, 256, EPI_NONE>(p, st);
   }
-  if constexpr (glu_fwd) {
-    return GMOE_ERR_UNSUPPORTED;  // the caller runs the GEMM and the activation kernel instead
-  } else {
-    if constexpr (MODE != MODE_TN && EPI == EPI_NONE) {
-      if (p.ws != nullptr && p.ws_floats >= 2 * 128 * 128 && gmm_split_pays(p))
-        return launch_gmm_split<DT, ODT, MODE>(p, st);
-    }
-    return launch_gmm_cfg<DT, ODT, MODE, 128, 128, EPI>(p, st, 2);
+  if constexpr (MODE != MODE_TN && EPI == EPI_NONE) {
+    if (p.ws != nullptr && p.ws_floats >= 2 * 128 * 128 && gmm_split_pays(p)) return launch_gmm_split<DT, ODT, MODE>(p, st);
   }
+  return launch_gmm_cfg<DT, ODT, MODE, 128, 128, EPI>(p, st, 2);
 }
 
 template <int MODE, int EPI>
@@ -1075,10 +1080,6 @@ static int launch_gmm(const GmmParams& p, int mode, int dtype, int out_dtype, in
   if (epi != EPI_NONE) {
     // fused activation epilogues keep the operand type
     if constexpr (DT == ODT) {
-      if (mode == MODE_NN && Elem<DT>::bytes == 2) {
-        if (epi == EPI_GLU_FWD_SILU) return launch_gmm_mode<DT, ODT, MODE_NN, EPI_GLU_FWD_SILU>(p, dtype, out_dtype, st);
-        if (epi == EPI_GLU_FWD_GELU) return launch_gmm_mode<DT, ODT, MODE_NN, EPI_GLU_FWD_GELU>(p, dtype, out_dtype, st);
-      }
       if (mode == MODE_NT) {
         if (epi == EPI_GLU_BWD_SILU) return launch_gmm_mode<DT, ODT, MODE_NT, EPI_GLU_BWD_SILU>(p, dtype, out_dtype, st);
         if (epi == EPI_GLU_BWD_GELU) return launch_gmm_mode<DT, ODT, MODE_NT, EPI_GLU_BWD_GELU>(p, dtype, out_dtype, st);
@@ -1216,8 +1217,8 @@ extern "C" int gmoe_gmm_glu(const void* a, const void* w1, void* fc1, void* act_
   hipStream_t st = static_cast<hipStream_t>(stream);
   p.c2 = static_cast<unsigned char*>(act_out);
   p.F = F;
-  if (dtype != GMOE_F32 && F % 8 == 0 && gmm_rows_pays(p, MODE_NN, EPI_GLU_FWD_SILU))
-    return gmm_dispatch(p, MODE_NN, dtype, dtype, act == GMOE_ACT_SILU ? EPI_GLU_FWD_SILU : EPI_GLU_FWD_GELU, st);
+  if (dtype != GMOE_F32 && F % 8 == 0 && (gmm_rows_pays(p, MODE_NN, EPI_GLU_FWD_SILU) || gmm_one_launch_pays(p, st)))
+    return launch_gmm_rows(p, MODE_NN, dtype, dtype, act == GMOE_ACT_SILU ? EPI_GLU_FWD_SILU : EPI_GLU_FWD_GELU, st);
   // small groups / fp32: the GEMM followed by the activation kernel
   const int rc2 = gmm_dispatch(p, MODE_NN, dtype, dtype, EPI_NONE, st);
   if (rc2 != GMOE_OK) return rc2;

@@ -1,8 +1,6 @@
 // Which 16-bit NN / NT launches go to the row-adaptive tiles (gmm_rows_kernel.h), and into which chunks the kernel cuts an
 // expert's rows.
 #pragma once
-#include <cmath>
-
 #include "split_rule.h"
 
 namespace gmoe {
@@ -84,69 +82,19 @@ constexpr RowsCosts kRowsCosts[] = {
     {2990, 1340, 176, 159, 0.14, 4650, 6800, 1.62e6, 2320, 1270, 614, 2730, 4720, 0.551e6, 4720, 0, 6670, 1630, 1.16e6},
     {6890, 6480, 123, 102, 0.0491, 1020, 6580, 1.0e6, 10600, 1430, 422, 2500, 5630, 1.0e6, 0, 0, 0, 0, 0}};
 
-// Whether a 16-bit NN / NT launch is faster in row-adaptive tiles than in the others: 128x128 ones, for plain NT that
-// could fill them 256x256 ones (only the host asks).  K, M as in the product (with the activation M = 2F); cus:
-// workgroups of a persistent grid, one per CU.
-//
-// Fitted to 6600 launches measured both ways, half of them of layers as they are trained, half spread over E 1-64, 1-9000
-// rows per expert, K and M 128-16384 (operands from HBM, loads that differ by 2 to 80 %), a third of them under 30 us.
-// Over them it costs 0.5 % (NN), 0.8 % (with activation), 0.8 % (NT) and 1.1 % (activation backward) against the better
-// side of each; the others throughout 11, 12, 6 and 7 %, these throughout 19, 8, 20 and 12 %.  The 3 % that these have to
-// be ahead by cost nothing and keep launches at the line where they were.
-//
-// Fewer than 96 rows per expert: an expert is one row tile and its weights bound the launch on either side.  Only the launch
-// with the activation, which is two on the other tiles, may come here, and only where its tiles fill their rounds: a
-// workgroup per CU streams the weights at the chip's rate only while all of them have a tile (rows per expert, K x M,
-// experts; 3, 4096 x 28672, 8, 3.5 rounds 319 / 350 others; 16, 2048 x 2816, 64, 2.75 rounds 142 / 131 these; 16, 1024 x
-// 5632, 16, 1.4 rounds 43 / 46 others).  Over 3500 such launches 1.8 % are lost against the better side, in the other tiles
-// throughout 2.3 %, here 9.8 %.
-//
-// us in the other tiles / in these (rows per expert, K x M, experts):
-//   * NN: 382, 14336 x 4096, 8 437 / 337 these; 363, 512 x 5120, 8 32 / 32; 267, 576 x 832, 64 45 / 36 these; 941, 768 x
-//     128, 32 18 / 24 others; 656, 1280 x 1280, 2 14 / 23 others; 1701, 10848 x 160, 4 79 / 133 others.
-//   * With activation: 382, 4096 x 28672, 8 976 / 650 these; 640, 1024 x 5632, 16 189 / 138 these; 208, 128 x 512, 32 12
-//     / 13 others; 103, 768 x 1024, 4 13 / 18 others; 121, 7168 x 256, 8 65 / 95 others.
-//   * NT: 382, 28672 x 4096, 8 860 / 628 these; 600, 2056 x 4104, 8 116 / 112 these; 1111, 5632 x 2048, 1 49 / 77 others;
-//     1769, 1408 x 512, 4 16 / 24 others; 1000, 28672 x 4096, 8 1439 / 1413 these.
-//     Short reductions of fewer than 768 rows per expert that fill 256x256 tiles stay there: of 36 such launches a third is
-//     slower here, by up to 7 %.
-//   * Activation backward: 382, 4096 x 14336, 8 470 / 382 these; 1024, 7168 x 2048, 32 1119 / 835 these; 640, 1024 x 2816,
-//     16 103 / 111 others; 599, 304 x 544, 6 15 / 29 others; 322, 4992 x 1024, 4 53 / 73 others.
-// It knows the average load only, and where that is close to whole rounds it can be wrong.
-inline bool rows_pays(RowsKind kind, int64_t E, int64_t N, int64_t K, int64_t M, int64_t cus) {
-  if (E < 1) E = 1;
+// What a launch reads and writes once.
+inline double rows_bytes(RowsKind kind, int64_t E, int64_t N, int64_t K, int64_t M) {
+  return 2.0 * E * K * M + 2.0 * N * K + (double)N * M * (kind == ROWS_NN_GLU ? 3 : kind == ROWS_NT_GLU_BWD ? 8 : 2);
+}
+
+// Time of a launch in the other tiles (with the activation of two), ns, from one row per expert on.
+inline double others_ns(RowsKind kind, int64_t E, int64_t N, int64_t K, int64_t M, int64_t cus) {
+  const RowsCosts& c = kRowsCosts[kind];
   const int64_t n = N / E;
-  const bool glu = kind == ROWS_NN_GLU, bwd = kind == ROWS_NT_GLU_BWD;
+  const bool glu = kind == ROWS_NN_GLU, bwd = kind == ROWS_NT_GLU_BWD, large = kind == ROWS_NT && nn_large_tiles(E, N, M);
+  const double ops = 2.0 * N * K * M, bytes = rows_bytes(kind, E, N, K, M);
   auto cdiv = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
   auto most = [](double a, double b) { return a > b ? a : b; };
-  const int64_t cols = glu ? cdiv(M / 2, 128) : cdiv(M, 256);
-  if (n < 96) {
-    if (!glu || N < 1) return false;
-    const double tiles = E * (1 - std::pow(1 - 1.0 / E, (double)N)) * cols;  // of the experts that have rows
-    return tiles >= 0.9 * cus * std::ceil(tiles / cus);
-  }
-  const bool large = kind == ROWS_NT && nn_large_tiles(E, N, M);
-  if (large && n < 768 && K <= 2560) return false;
-  const RowsCosts& c = kRowsCosts[kind];
-  const double out = (double)N * M * (glu ? 3 : bwd ? 8 : 2), ops = 2.0 * N * K * M;
-  const double bytes = 2.0 * E * K * M + 2.0 * N * K + out;
-  const int64_t stages = 2 * cdiv(K, 64);
-  const int64_t units = over_loads(E, n, [&](int64_t r) { return cdiv(r, 64); });
-  double rows = 0, idle = 0;
-  for (int u = kTallMaxUnits; u >= 2; --u) {
-    const int64_t chunks = over_loads(E, n, [&](int64_t r) { return cdiv(cdiv(r, 64), u); });
-    const int64_t tiles = cdiv(E * chunks * cols, 5), rounds = cdiv(tiles, cus), last = tiles - (rounds - 1) * cus;
-    const double average = (double)units / chunks, part = 1 - (double)last / cus;
-    const double tile = c.tile + c.unit * average + (c.stage + c.unit_stage * average) * stages;
-    const double t = tile * (rounds - c.lone_gain * part);
-    if (u == kTallMaxUnits || t < rows) {
-      rows = t;
-      idle = part / rounds;
-    }
-  }
-  // a last round that is part empty does not stream at the whole chip's rate
-  rows = most(most(rows, bytes / c.bytes * (1 + 0.6 * idle)), ops / c.ops) + c.launch;
-
   const int64_t edge = large ? 256 : 128, steps = cdiv(K, 64);
   const int64_t tiles = cdiv(E * over_loads(E, n, [&](int64_t r) { return cdiv(r, edge); }) * cdiv(M, edge), 5);
   // the launches with an activation have no workspace for a split
@@ -168,7 +116,80 @@ inline bool rows_pays(RowsKind kind, int64_t E, int64_t N, int64_t K, int64_t M,
   }
   other += c.small_launch;
   if (glu) other += c.act + (double)N * M * 3 / 4000;
-  return rows < 0.97 * other;
+  return other;
+}
+
+// Whether a 16-bit NN / NT launch is faster in row-adaptive tiles than in the others: 128x128 ones, for plain NT that
+// could fill them 256x256 ones (only the host asks).  K, M as in the product (with the activation M = 2F); cus:
+// workgroups of a persistent grid, one per CU.
+//
+// Fitted to 6600 launches measured both ways, half of them of layers as they are trained, half spread over E 1-64, 1-9000
+// rows per expert, K and M 128-16384 (operands from HBM, loads that differ by 2 to 80 %), a third of them under 30 us.
+// Over them it costs 0.5 % (NN), 0.8 % (with activation), 0.8 % (NT) and 1.1 % (activation backward) against the better
+// side of each; the others throughout 11, 12, 6 and 7 %, these throughout 19, 8, 20 and 12 %.  The 3 % that these have to
+// be ahead by cost nothing and keep launches at the line where they were.
+//
+// Fewer than 96 rows per expert: an expert is one row tile and its weights bound the launch on either side.  Only the launch
+// with the activation, which is two on the other tiles, may come here, and only where its tiles fill their rounds: a
+// workgroup per CU streams the weights at the chip's rate only while all of them have a tile (rows per expert, K x M,
+// experts; 3, 4096 x 28672, 8, 3.5 rounds 319 / 350 others; 16, 2048 x 2816, 64, 2.75 rounds 142 / 131 these; 16, 1024 x
+// 5632, 16, 1.4 rounds 43 / 46 others).  Under 4 rows per expert the host cannot tell how many experts have any.  Over 3500
+// such launches 1.9 % are lost against the better side, in the other tiles throughout 2.3 %, here 9.8 %.
+//
+// us in the other tiles / in these (rows per expert, K x M, experts):
+//   * NN: 382, 14336 x 4096, 8 437 / 337 these; 363, 512 x 5120, 8 32 / 32; 267, 576 x 832, 64 45 / 36 these; 941, 768 x
+//     128, 32 18 / 24 others; 656, 1280 x 1280, 2 14 / 23 others; 1701, 10848 x 160, 4 79 / 133 others.
+//   * With activation: 382, 4096 x 28672, 8 976 / 650 these; 640, 1024 x 5632, 16 189 / 138 these; 208, 128 x 512, 32 12
+//     / 13 others; 103, 768 x 1024, 4 13 / 18 others; 121, 7168 x 256, 8 65 / 95 others.
+//   * NT: 382, 28672 x 4096, 8 860 / 628 these; 600, 2056 x 4104, 8 116 / 112 these; 1111, 5632 x 2048, 1 49 / 77 others;
+//     1769, 1408 x 512, 4 16 / 24 others; 1000, 28672 x 4096, 8 1439 / 1413 these.
+//     Short reductions of fewer than 768 rows per expert that fill 256x256 tiles stay there: of 36 such launches a third is
+//     slower here, by up to 7 %.
+//   * Activation backward: 382, 4096 x 14336, 8 470 / 382 these; 1024, 7168 x 2048, 32 1119 / 835 these; 640, 1024 x 2816,
+//     16 103 / 111 others; 599, 304 x 544, 6 15 / 29 others; 322, 4992 x 1024, 4 53 / 73 others.
+// It knows the average load only, and where that is close to whole rounds it can be wrong.
+inline bool rows_pays(RowsKind kind, int64_t E, int64_t N, int64_t K, int64_t M, int64_t cus) {
+  if (E < 1) E = 1;
+  const int64_t n = N / E;
+  const bool glu = kind == ROWS_NN_GLU;
+  auto cdiv = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
+  auto most = [](double a, double b) { return a > b ? a : b; };
+  const int64_t cols = glu ? cdiv(M / 2, 128) : cdiv(M, 256);
+  if (n < 96) {
+    const int64_t tiles = E * cols;
+    return glu && n >= 4 && 10 * tiles >= 9 * cus * cdiv(tiles, cus);
+  }
+  if (kind == ROWS_NT && n < 768 && K <= 2560 && nn_large_tiles(E, N, M)) return false;
+  const RowsCosts& c = kRowsCosts[kind];
+  const double ops = 2.0 * N * K * M, bytes = rows_bytes(kind, E, N, K, M);
+  const int64_t stages = 2 * cdiv(K, 64);
+  const int64_t units = over_loads(E, n, [&](int64_t r) { return cdiv(r, 64); });
+  double rows = 0, idle = 0;
+  for (int u = kTallMaxUnits; u >= 2; --u) {
+    const int64_t chunks = over_loads(E, n, [&](int64_t r) { return cdiv(cdiv(r, 64), u); });
+    const int64_t tiles = cdiv(E * chunks * cols, 5), rounds = cdiv(tiles, cus), last = tiles - (rounds - 1) * cus;
+    const double average = (double)units / chunks, part = 1 - (double)last / cus;
+    const double tile = c.tile + c.unit * average + (c.stage + c.unit_stage * average) * stages;
+    const double t = tile * (rounds - c.lone_gain * part);
+    if (u == kTallMaxUnits || t < rows) {
+      rows = t;
+      idle = part / rounds;
+    }
+  }
+  // a last round that is part empty does not stream at the whole chip's rate
+  rows = most(most(rows, bytes / c.bytes * (1 + 0.6 * idle)), ops / c.ops) + c.launch;
+
+  return rows < 0.97 * others_ns(kind, E, N, K, M, cus);
+}
+
+// Whether fc1 and its activation are so short that one launch is better than two for the host's sake, although these tiles
+// take longer for it: programs of such launches wait for the host, which a launch costs 3 to 4 us.  us in one launch / in
+// two, and of the whole step called eagerly: 128 rows, 4 experts, 128 x 512 9.4 / 8.2 and 272 / 277; 128 rows, 8 experts,
+// forward, 512 x 1024 68.4 / 71.1.  Of 1600 launches these are 850; they take 1.3 us longer than two would.  Not asked while a
+// graph is captured, whose replay takes the host no time.
+inline bool rows_one_launch_pays(int64_t E, int64_t N, int64_t K, int64_t M, int64_t cus) {
+  if (E < 1) E = 1;
+  return N >= 1 && others_ns(ROWS_NN_GLU, E, N, K, M, cus) < 12000;
 }
 
 }  // namespace gmoe

@@ -59,10 +59,10 @@ def test_tall_edges(pkg, dev, dtype, rows, K, F, act):
         s += n
 
 
-# rows of the experts, K, F: averages of 1 to 95 rows, where tiles of the experts that have rows fill a round
+# rows of the experts, K, F: averages of 4 to 90 rows, where a tile of each expert fills a round
 FEW = [
-    ([0, 1] * 32 + [3, 0, 0, 95], 264, 1024),          # most experts empty, one row
-    ([1] * 64, 72, 768),
+    ([0, 1] * 15 + [0] * 30 + [95, 70, 60, 55], 264, 1024),  # most experts empty, some with one row
+    ([4] * 64, 72, 512),
     ([63, 64, 65, 0, 127, 128, 129, 1] * 4, 1160, 1016),  # around one and two units (of 64 rows), ragged K and F
     ([95, 0, 200, 33, 7, 383, 1, 0], 520, 4088),
     ([17], 2056, 32760),
@@ -92,6 +92,34 @@ def test_few_rows_with_the_activation(pkg, dev, dtype, rows, K, F, act):
             want = a[s:s + n].double() @ w1[e].double()
             assert ((fc1[s:s + n].double() - want).abs() - want.abs() * half).max().item() < tol + 2.0 ** -25, e
         s += n
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,K,F", [([32, 0, 95, 1], 128, 256), ([1], 136, 72), ([0, 0, 5, 0, 0, 0, 0, 0], 264, 520), ([70] * 8, 72, 136)])
+def test_short_launches_with_the_activation(pkg, dev, dtype, rows, K, F):
+    """One launch when they are called, two where a graph is captured: the same bits from both, in every replay."""
+    g = torch.Generator(device=dev).manual_seed(K + F)
+    off = torch.tensor([0] + rows, device=dev).cumsum(0)
+    a = torch.empty(sum(rows), K, device=dev).normal_(generator=g).to(dtype)
+    w1 = torch.empty(len(rows), K, 2 * F, device=dev).normal_(0.0, K ** -0.5, generator=g).to(dtype)
+    print("case", dtype, rows, K, F, flush=True)
+    fc1, h = on_kernel("gmm_rows_kernel", lambda: pkg.ops.gmm_glu(a, w1, off, "silu"))
+    assert torch.equal(h, pkg.ops.glu_fwd(fc1, "silu"))
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        pkg.ops.gmm(a, w1, off)
+        pkg.ops.glu_fwd(fc1, "silu")
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        fc1_graph, h_graph = pkg.ops.gmm_glu(a, w1, off, "silu")
+    for _ in range(3):
+        fc1_graph.zero_()
+        h_graph.zero_()
+        on_kernel("gmm_kernel", graph.replay)
+        assert torch.equal(fc1_graph, fc1) and torch.equal(h_graph, h)
+        assert torch.equal(pkg.ops.gmm_glu(a, w1, off, "silu")[1], h)
 
 
 @pytest.mark.parametrize("K,M", [(8, 2056), (72, 2312), (4104, 2056), (1000, 2304)])

@@ -15,7 +15,7 @@ PROGRAM = """
 int main() {
   long long v, a, b, c, d, e;
   while (std::scanf("%lld %lld %lld %lld %lld %lld", &v, &a, &b, &c, &d, &e) == 6)
-    std::printf("%d\\n", gmoe::rows_pays((gmoe::RowsKind)v, a, b, c, d, e));
+    std::printf("%d\\n", v < 0 ? gmoe::rows_one_launch_pays(a, b, c, d, e) : gmoe::rows_pays((gmoe::RowsKind)v, a, b, c, d, e));
 }
 """
 NN, GLU, NT, GLU_BWD = range(4)
@@ -76,22 +76,35 @@ def test_choice(evaluate):
 
 
 def test_few_rows(evaluate):
-    """The launch with the activation: where its tiles fill nine tenths of their rounds or more.  us in the other tiles and in
-    these, as above but with all rows."""
+    """The launch with the activation, from 4 rows per expert on: where its tiles fill nine tenths of their rounds or more.  us in
+    the other tiles and in these, as above but with all rows."""
     measured = [(8, 26, 4096, 28672, 319.1, 350.5), (8, 128, 4096, 28672, 331.5, 363.4), (64, 1024, 2048, 2816, 142.1, 131.4),
                 (64, 2664, 2048, 2816, 152.3, 139.8), (16, 256, 1024, 5632, 42.6, 46.5), (16, 1024, 1024, 5632, 47, 54.5),
                 (32, 8, 7168, 4096, 83.7, 104.9), (4, 128, 128, 512, 8.3, 9.6), (4, 104, 2368, 6400, 30.6, 38.4)]
     got = evaluate([(GLU, *c[:4], 256) for c in measured])
     assert got == [int(c[5] < c[4]) for c in measured]
     assert not any(evaluate([(kind, *c[:4], 256) for c in measured for kind in (NN, NT, GLU_BWD)]))
+    # fewer: how many experts have rows is not known
+    assert not any(evaluate([(GLU, E, N, 2048, 2816, 256) for E in (1, 8, 64) for N in (1, 2, 3 * E, 4 * E - 1) if N < 4 * E]))
+
+
+def test_one_launch(evaluate):
+    """Short launches of fc1 with its activation are one launch where the host's time decides; longer ones, and none at all, are
+    not.  us in one launch and in two."""
+    measured = [(4, 128, 128, 512, 9.4, 8.2), (4, 26, 128, 512, 9.2, 8.1), (64, 64, 128, 256, 9.1, 10.9), (8, 128, 512, 1024, 12.5, 10.9),
+                (8, 26, 4096, 28672, 350.5, 319.1), (16, 64, 1024, 5632, 45.2, 42.2), (4, 104, 2368, 6400, 38.4, 30.6),
+                (6, 132, 1664, 6400, 36, 31)]
+    got = evaluate([(-1, *c[:4], 256) for c in measured])
+    assert got == [int(c[4] < 15) for c in measured]
+    assert not any(evaluate([(-1, E, 0, 128, 512, 256) for E in (1, 64)]))
 
 
 def test_limits(evaluate):
-    """Fewer than 96 rows per expert, with the activation none at all: never; one expert and a thousand, the smallest and
+    """Fewer than 96 rows per expert, with the activation fewer than four: never; one expert and a thousand, the smallest and
     the longest reductions: an answer; the largest launches: always."""
     shapes = [(E, n, K, M) for E in (1, 8, 1024) for n in (0, 1, 95, 96, 2048, 65536) for K in (8, 512, 65536) for M in (8, 4096)]
     large = [(8, 4096, 4096, 28672), (8, 16384, 14336, 4096), (64, 4096, 2048, 2816), (1, 32768, 8192, 8192)]
     for kind in (NN, GLU, NT, GLU_BWD):
         for (E, n, K, M), v in zip(shapes, evaluate([(kind, E, n * E, K, M, 256) for E, n, K, M in shapes])):
-            assert v in (0, 1) and not (v and n < (1 if kind == GLU else 96)), (kind, E, n, K, M)
+            assert v in (0, 1) and not (v and n < (4 if kind == GLU else 96)), (kind, E, n, K, M)
         assert all(evaluate([(kind, E, n * E, K, M, 256) for E, n, K, M in large])), kind
