@@ -15,9 +15,10 @@ constexpr ChunkCosts kChunkCosts{16.f, 250.f, 0.f, 1.f};
 // compute unit at it at once: taller chunks save little and leave a part empty last round longer.  us in chunks of up to
 // 128 / 192 / 256 / 320 / 384 rows (K x F): 16 experts of 640, 1024 x 2816 115 / 108 / 122 / 122 / 122; 8 of 366 to 402,
 // 4096 x 14336 477 / 489 / 454 / 447 / 474; 60 of 386, 6272 x 2688 1070 / 1009 / 953 / 957 / 943; 8 of 1000, 4096 x 14336
-// 1017 / 992 / 867 / 871 / 975.  Over 1059 launches (E 1-64, 40-6000 rows per expert, even and uneven loads, K and F
-// 128-16384) the costs above lose 0.9 % against the best size of each (p95 6 %), these 0.3 % (2 %).
-constexpr ChunkCosts kChunkCostsGluBwd{8.f, 120.f, 650.f, 1.04f};
+// 1017 / 992 / 867 / 871 / 975; 8 of 358, 61, 931, 83, 155, 6, 730 and 738, 4096 x 14336 471 / 454 / 426 / 470 / 488.
+// Over 1059 launches (E 1-64, 40-6000 rows per expert, even and uneven loads, K and F 128-16384) the costs above lose
+// 0.9 % against the best size of each (p95 6 %), these 0.3 % (2 %).
+constexpr ChunkCosts kChunkCostsGluBwd{7.3f, 390.f, 866.f, 1.07f};
 
 // Rows of a chunk, in units of 64: of the sizes kTallMaxUnits to 2 the one that ends first.  v[0]: units of all experts,
 // v[u]: their chunks of up to u units.  Over 8600 launches of 96 rows per expert and more it costs 1.1 % against the best size

@@ -52,7 +52,7 @@ def test_chunks(evaluate):
     """The rule against one in Python, for the edge tests on the GPU, which reach tiles of two, three, five and six units (of
     64 rows), in the activation backward of six; no rows at all; one tile."""
     def model(counts, col_tiles, K, bwd):
-        per_stage, around, unit, tall = (8, 120, 650, 1.04) if bwd else (16, 250, 0, 1)
+        per_stage, around, unit, tall = (7.3, 390, 866, 1.07) if bwd else (16, 250, 0, 1)
         best, least, stages = 6, None, -(-K // 32)
         for size in range(6, 1, -1):
             chunks = counts[size]
@@ -80,6 +80,7 @@ BACKWARD = [
     ([700] * 8, 4096, 14336, (794.2, 718.0, 696.6, 684.7, 682.9)),
     ([300] * 24, 1024, 4096, (131.2, 124.3, 123.7, 130.1, 128.0)),
     ([1024] * 32, 7168, 2048, (1010.1, 932.5, 821.8, 821.1, 861.6)),
+    ([358, 61, 931, 83, 155, 6, 730, 738], 4096, 14336, (471.1, 453.7, 425.9, 469.9, 487.9)),
 ]
 
 
