@@ -58,7 +58,7 @@ __device__ __forceinline__ int chunk_count(long long n, int max_units) {
 }
 // rows_chunk_units for the launch; v: units and chunks of this thread's experts, summed over the workgroup here.
 template <int EPI>
-__device__ __forceinline__ int best_max_units(int (&v)[kMaxUnits + 1], int nt_cnt, int grid, int64_t K, int* sums,
+__device__ __forceinline__ int best_max_units(int (&v)[kMaxUnits + 1], int nt_cnt, int grid, int E, int64_t K, int* sums,
                                               int lane, int wave) {
 #pragma unroll
   for (int i = 0; i <= kMaxUnits; ++i) {
@@ -74,7 +74,7 @@ __device__ __forceinline__ int best_max_units(int (&v)[kMaxUnits + 1], int nt_cn
     for (int w = 0; w < kGemmThreads / 64; ++w) v[i] += sums[w * (kMaxUnits + 1) + i];
   }
   constexpr bool bwd = EPI == EPI_GLU_BWD_SILU || EPI == EPI_GLU_BWD_GELU;
-  return rows_chunk_units(v, nt_cnt, grid, K, bwd ? kChunkCostsGluBwd : kChunkCosts);
+  return rows_chunk_units(v, nt_cnt, grid, K, chunk_costs(bwd, v[0], E));
 }
 // first unit and unit count of chunk c of cnt
 __device__ __forceinline__ void chunk_units(long long n, int cnt, int c, int& first, int& units) {
@@ -596,7 +596,7 @@ __global__ __launch_bounds__(kGemmThreads, 1) void gmm_rows_kernel(GmmParams p) 
 #pragma unroll
       for (int u = 2; u <= kMaxUnits; ++u) v[u] += chunk_count(rows_of[j], u);
     }
-    max_units = best_max_units<EPI>(v, nt_cnt, (int)gridDim.x, p.K, scratch + kWaves, lane, wave);
+    max_units = best_max_units<EPI>(v, nt_cnt, (int)gridDim.x, E, p.K, scratch + kWaves, lane, wave);
     int cnt[kPer], local = 0;
 #pragma unroll
     for (int j = 0; j < kPer; ++j) {

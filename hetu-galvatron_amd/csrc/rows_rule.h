@@ -17,8 +17,14 @@ constexpr ChunkCosts kChunkCosts{16.f, 250.f, 0.f, 1.f};
 // 4096 x 14336 477 / 489 / 454 / 447 / 474; 60 of 386, 6272 x 2688 1070 / 1009 / 953 / 957 / 943; 8 of 1000, 4096 x 14336
 // 1017 / 992 / 867 / 871 / 975; 8 of 358, 61, 931, 83, 155, 6, 730 and 738, 4096 x 14336 471 / 454 / 426 / 470 / 488.
 // Over 1059 launches (E 1-64, 40-6000 rows per expert, even and uneven loads, K and F 128-16384) the costs above lose
-// 0.9 % against the best size of each (p95 6 %), these 0.3 % (2 %).
+// 0.9 % against the best size of each (p95 6 %), these 0.3 % (2 %).  With more than 1024 rows per expert the costs above
+// stay: there are many rounds, little is lost (1 %), and what a part empty one leaves idle is used by what runs beside (8192
+// tokens of 2048, 64 experts of 1408, top 8, the shared experts on their own stream: the step 5085 us, with these 5115).
 constexpr ChunkCosts kChunkCostsGluBwd{7.3f, 390.f, 866.f, 1.07f};
+// units: of all E experts
+__host__ __device__ inline ChunkCosts chunk_costs(bool glu_bwd, int units, int E) {
+  return glu_bwd && units <= 16 * E ? kChunkCostsGluBwd : kChunkCosts;
+}
 
 // Rows of a chunk, in units of 64: of the sizes kTallMaxUnits to 2 the one that ends first.  v[0]: units of all experts,
 // v[u]: their chunks of up to u units.  Over 8600 launches of 96 rows per expert and more it costs 1.1 % against the best size

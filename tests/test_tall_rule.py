@@ -19,7 +19,7 @@ int main() {
   while (std::scanf("%lld %lld %lld %lld", &a, &b, &c, &d) == 4) {
     int u[7] = {};
     for (int i = 0; i < 7; ++i) if (std::scanf("%d", u + i) != 1) return 1;
-    std::printf("%d\\n", gmoe::rows_chunk_units(u, (int)a, (int)b, c, d ? gmoe::kChunkCostsGluBwd : gmoe::kChunkCosts));
+    std::printf("%d\\n", gmoe::rows_chunk_units(u, (int)a, (int)b, c, gmoe::chunk_costs(d > 0, u[0], (int)d)));
   }
 }
 """
@@ -51,8 +51,8 @@ def counts(rows):
 def test_chunks(evaluate):
     """The rule against one in Python, for the edge tests on the GPU, which reach tiles of two, three, five and six units (of
     64 rows), in the activation backward of six; no rows at all; one tile."""
-    def model(counts, col_tiles, K, bwd):
-        per_stage, around, unit, tall = (7.3, 390, 866, 1.07) if bwd else (16, 250, 0, 1)
+    def model(counts, col_tiles, K, bwd):  # bwd: experts of the activation backward, 0 for the others
+        per_stage, around, unit, tall = (7.3, 390, 866, 1.07) if counts[0] <= 16 * bwd else (16, 250, 0, 1)
         best, least, stages = 6, None, -(-K // 32)
         for size in range(6, 1, -1):
             chunks = counts[size]
@@ -63,13 +63,13 @@ def test_chunks(evaluate):
         return best
 
     edges = [(counts(rows), cols, K, bwd) for rows, K, F in [(ROWS * times, K, F) for K, F, times in EDGES] + TALL
-             for cols, bwd in ((-(-F // 128), 0), (-(-F // 256), 0), (-(-F // 256), 1))]
-    other = [(counts(rows), cols, K, bwd) for rows in ([0, 0], [1], [640] * 16, [256] * 64, [370] * 8, [1024] * 64)
-             for cols in (1, 4, 6, 25) for K in (520, 1024, 5632) for bwd in (0, 1)]
+             for cols, bwd in ((-(-F // 128), 0), (-(-F // 256), 0), (-(-F // 256), len(rows)))]
+    other = [(counts(rows), cols, K, bwd) for rows in ([0, 0], [1], [640] * 16, [256] * 64, [370] * 8, [1024] * 64, [1025] * 64)
+             for cols in (1, 4, 6, 25) for K in (520, 1024, 5632) for bwd in (0, len(rows))]
     got = evaluate([(cols, 256, K, bwd, *units) for units, cols, K, bwd in edges + other])
     assert got == [model(*c) for c in edges + other]
-    for bwd, sizes in ((0, {2, 3, 5, 6}), (1, {2, 3, 6})):
-        assert sizes <= {u for u, c in zip(got, edges) if c[3] == bwd}
+    for bwd, sizes in ((False, {2, 3, 5, 6}), (True, {2, 3, 6})):
+        assert sizes <= {u for u, c in zip(got, edges) if (c[3] > 0) == bwd}
 
 
 # rows of the experts, K, F, us of the activation backward in chunks of up to 128 / 192 / 256 / 320 / 384 rows
@@ -87,7 +87,7 @@ BACKWARD = [
 def test_chunks_of_the_activation_backward(evaluate):
     """Its chunks take 2.5 % longer than the best of those measured on average and 6 % at most; chosen by the other products'
     costs they take 6 % and 14 %.  No rows at all has an answer."""
-    cases = [(-(-F // 256), 256, K, 1, *counts(rows)) for rows, K, F, _ in BACKWARD]
+    cases = [(-(-F // 256), 256, K, len(rows), *counts(rows)) for rows, K, F, _ in BACKWARD]
     got = evaluate(cases + [(4, 256, 8, 1, *counts([0, 0]))])
     lost = [c[3][u - 2] / min(c[3]) - 1 for c, u in zip(BACKWARD, got)]
     assert max(lost) < 0.06 and sum(lost) / len(lost) < 0.025, list(zip(got, lost))
