@@ -431,7 +431,7 @@ def run_fp8_shard(args, torch, pkg, dev):
                    "launch": "HIP graph replay" if args.graph else "eager"},
         "pct_mfma_peak": round(100 * value / (5000.0 if args.fp8_activations else MFMA_PEAK["bf16"]), 2),
         # weight-streaming regime (128 rows per expert): both rooflines of the largest launch
-        "roofline": {"bound": "hbm", "kernel": "gmm_kernel (fp8 weights) " + dom_key,
+        "roofline": {"bound": "hbm", "kernel": "gmm_fp8_skinny_kernel " + dom_key,
                      "achieved": round(d["bytes"] / (d_ms * 1e-3) / 1e9, 1), "peak": HBM_PEAK_GBPS,
                      "unit": "GB/s", "frac": round(d["bytes"] / (d_ms * 1e-3) / 1e9 / HBM_PEAK_GBPS, 4),
                      "traffic": None,
@@ -678,13 +678,14 @@ def main():
     # command, FETCH_SIZE and WRITE_SIZE scaled by what the 1 GiB copy above reads back), so
     # `traffic` stays null here and the profiled figure is quoted with its source.
     profiled_traffic = {("mixtral", "gmm_NN+glu 32768x4096x28672"):
-                        {"bytes_per_launch": 17.1e9, "source": "profiles/bench_mixtral_hbm_traffic.md"}}
+                        {"bytes_per_launch": 17.4e9, "source": "profiles/bench_mixtral_hbm_traffic.md"}}
     dom_key = max(gemm, key=lambda k: gemm[k]["work"] * (1 if k.startswith("gmm_NN") else 0.5)) if gemm else None
     roofline = None
     if dom_key:
         d = gemm[dom_key]
         ach = d["work"] / (d["ms"] / d["calls"] * 1e-3) / 1e12
-        roofline = {"bound": "mfma", "kernel": "gmm_kernel " + dom_key, "achieved": round(ach, 1),
+        kernel = "gmm_f32_kernel " if w.dtype == torch.float32 else "gmm_rows_kernel "
+        roofline = {"bound": "mfma", "kernel": kernel + dom_key, "achieved": round(ach, 1),
                     "peak": peak, "unit": "TFLOP/s", "frac": round(ach / peak, 4),
                     "traffic": None,
                     "traffic_profiled": profiled_traffic.get((w.name, dom_key)),

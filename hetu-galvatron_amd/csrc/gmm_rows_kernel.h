@@ -1,6 +1,6 @@
 // Grouped GEMM with row-adaptive tiles for 16-bit operands (bf16 / fp16) on gfx950: NN and NT of
-// gmm.hip's contract, with the fused gated-activation epilogues, from 96 rows per expert on (the rules with
-// both sides' times are in rows_rule.h and gmm.hip).
+// gmm.hip's contract, with the fused gated-activation epilogues: from 96 rows per expert on what rows_rule.h prices cheaper
+// here, with the activation from 4 rows on where the tiles fill their rounds, and its short launches from one row on.
 //
 //   * A tile is RF*64 rows (RF = 1..6, chosen per tile) x 256 columns of C.  An expert's rows are cut
 //     into chunks of up to 384 (320 .. 128 where those fill the rounds better: best_max_units) that are as

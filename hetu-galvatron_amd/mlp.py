@@ -79,10 +79,9 @@ class _FusedGatedExperts:
     # The fused d(act) GEMM + activation backward gives the same bits as the two launches.  Its
     # epilogue reads fc1 and writes d(fc1) (4 bytes of HBM traffic per accumulator) while the matrix
     # cores of that workgroup's CU idle, which the separate activation-backward kernel at HBM speed
-    # nearly makes up for: measured in the same run the fused form is 0.06 ms per step faster on the
-    # Mixtral shape (3.55 ms against 2.85 + 0.86 ms in isolation), 0.03 ms slower on the fine-grained
-    # one and equal on the DeepSeek-V3-shape shard; it never materialises d(act) (0.94 GB at the
-    # Mixtral shape), which decides it.
+    # does not make up for (us fused / apart: 8 experts of 4096 rows, 4096 x 14336 3202 / 3642, of 383 369 / 385; 64 of
+    # 1024, 2048 x 1408 421 / 508; 32 of 1024, 7168 x 2048 776 / 846), and it never materialises d(act) (0.94 GB at the
+    # first of these).
     fuse_backward = True
 
     @staticmethod

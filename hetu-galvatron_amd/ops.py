@@ -659,7 +659,7 @@ def gmm(a: torch.Tensor, b: torch.Tensor, expert_offsets: torch.Tensor, trans_a:
 
 def gmm_glu(a: torch.Tensor, w1: torch.Tensor, expert_offsets: torch.Tensor, act: str = "silu"):
     """fc1 = gmm(a, w1 [E,K,2F]); act_out = act(fc1[:, :F]) * fc1[:, F:], one launch for large
-    16-bit groups.  Returns (fc1 [N,2F], act_out [N,F])."""
+    16-bit groups and, outside of graph capture, for short launches.  Returns (fc1 [N,2F], act_out [N,F])."""
     dev = _check_dev(a, w1, expert_offsets)
     assert a.dim() == 2 and w1.dim() == 3 and a.dtype == w1.dtype and w1.shape[1] == a.shape[1]
     assert expert_offsets.dtype == torch.int64 and w1.shape[2] % 2 == 0

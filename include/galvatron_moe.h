@@ -315,10 +315,10 @@ int gmoe_bias_rows_bwd(const void* grad, int dtype, int64_t N, int64_t M,
  * K and M must be multiples of 8 (16-byte rows).  One persistent kernel walks a device-side tile
  * list built from expert_offsets; no host synchronisation.
  * workspace (optional, 16-byte aligned, workspace_bytes long): scratch for fp32 partial results.  With
- * gmoe_gmm_workspace_bytes(...) bytes, launches of few tiles, and the one for the experts' short last
- * row tiles with large groups, split their reduction over otherwise idle CUs; a smaller one is used as
- * far as it goes, without one they run unsplit.  The result does not depend on the contents of the
- * workspace, only (in the last bits: another order of the same fp32 additions) on its size.
+ * gmoe_gmm_workspace_bytes(...) bytes, launches of few tiles split their reduction over otherwise idle
+ * CUs; a smaller one is used as far as it goes, without one they run unsplit.  The result does not
+ * depend on the contents of the workspace, only (in the last bits: another order of the same fp32
+ * additions) on its size.
  */
 int64_t gmoe_gmm_workspace_bytes(int E, int64_t N, int64_t K, int64_t M, int trans_a, int trans_b,
                                  int dtype);
@@ -326,11 +326,12 @@ int gmoe_gmm(const void* a, const void* b, void* c, const int64_t* expert_offset
              int64_t N, int64_t K, int64_t M, int trans_a, int trans_b, int dtype, int out_dtype,
              void* workspace, int64_t workspace_bytes, void* stream);
 
-/* Forward of the gated expert MLP's first half in one launch: fc1 = gmm(a, w1) with w1 [E,K,2F]
+/* Forward of the gated expert MLP's first half: fc1 = gmm(a, w1) with w1 [E,K,2F]
  * ([gate | up] columns, moe/mlp.py:80-95) and act_out [N,F] = act(fc1[:, :F]) * fc1[:, F:]
- * (moe/mlp.py:106-110: gmm followed by the activation closure).  fc1 [N,2F] is written too (the
- * backward needs it).  act_out is computed from fc1 as rounded to `dtype`, so it is bit-identical
- * to gmoe_gmm followed by gmoe_glu_fwd. */
+ * (moe/mlp.py:106-110: gmm followed by the activation closure), in one launch or, where those are
+ * faster, two (short launches: two only while the stream is capturing).  fc1 [N,2F] is written too (the
+ * backward needs it).  act_out is computed from fc1 as rounded to `dtype`, so it is bit-identical to
+ * gmoe_gmm followed by gmoe_glu_fwd. */
 int gmoe_gmm_glu(const void* a, const void* w1, void* fc1, void* act_out,
                  const int64_t* expert_offsets, int E, int64_t N, int64_t K, int64_t F, int act,
                  int dtype, void* stream);
