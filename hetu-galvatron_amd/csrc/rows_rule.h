@@ -27,9 +27,10 @@ __host__ __device__ inline ChunkCosts chunk_costs(bool glu_bwd, int units, int E
 }
 
 // Rows of a chunk, in units of 64: of the sizes kTallMaxUnits to 2 the one that ends first.  v[0]: units of all experts,
-// v[u]: their chunks of up to u units.  Over 8600 launches of 96 rows per expert and more it costs 1.1 % against the best size
-// of each (us in chunks of up to 128 / 192 / 256 / 320 / 384 rows, rows per expert: with activation 383, 4096 x 28672, 8 experts 890 / 776 / 739 / 745 / 686; 640, 1024 x 5632, 16 172 / 152 /
-// 150 / 147 / 135; NN 640, 2816 x 1024, 16 86 / 60 / 67 / 73 / 81; NT 383, 28672 x 4096, 8 817 / 935 / 691 / 700 / 926).
+// v[u]: their chunks of up to u units.  Over 8600 launches of 96 rows per expert and more it costs 1.1 % against the best
+// size of each (us in chunks of up to 128 / 192 / 256 / 320 / 384 rows, rows per expert: with activation 383, 4096 x
+// 28672, 8 experts 890 / 776 / 739 / 745 / 686; 640, 1024 x 5632, 16 172 / 152 / 150 / 147 / 135; NN 640, 2816 x 1024, 16
+// 86 / 60 / 67 / 73 / 81; NT 383, 28672 x 4096, 8 817 / 935 / 691 / 700 / 926).
 constexpr int kTallMaxUnits = 6;
 __host__ __device__ inline int rows_chunk_units(const int (&v)[kTallMaxUnits + 1], int col_tiles, int grid, int64_t K,
                                                 ChunkCosts c) {
@@ -192,8 +193,8 @@ inline bool rows_pays(RowsKind kind, int64_t E, int64_t N, int64_t K, int64_t M,
 // Whether fc1 and its activation are so short that one launch is better than two for the host's sake, although these tiles
 // take longer for it: programs of such launches wait for the host, which a launch costs 3 to 4 us.  us in one launch / in
 // two, and of the whole step called eagerly: 128 rows, 4 experts, 128 x 512 9.4 / 8.2 and 272 / 277; 128 rows, 8 experts,
-// forward, 512 x 1024 68.4 / 71.1.  Of 1600 launches these are 850; they take 1.3 us longer than two would.  Not asked while a
-// graph is captured, whose replay takes the host no time.
+// forward, 512 x 1024 68.4 / 71.1.  Of 3500 launches of few rows these are 850; they take 1.3 us longer than two would.
+// Not asked while a graph is captured, whose replay takes the host no time.
 inline bool rows_one_launch_pays(int64_t E, int64_t N, int64_t K, int64_t M, int64_t cus) {
   if (E < 1) E = 1;
   return N >= 1 && others_ns(ROWS_NN_GLU, E, N, K, M, cus) < 12000;
